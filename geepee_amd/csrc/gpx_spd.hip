@@ -8,137 +8,304 @@
 // 16 x 16 pivot blocks, on the FP64 matrix cores (spd_gj_kernel below).
 #include "gpx_common.h"
 
+#include <utility>
+
 namespace {
 
-template <int MT>
-struct SpdLds {
-  static constexpr int MP = 16 * MT, RS = MP + 1;  // RS: LDS row stride (doubles)
-  // rowK: block row K (read by the panel only, so one buffer); colT: block column K,
-  // transposed (read by the tile updates while the next block's column is published,
-  // so two); rvK, Pi: the panel's results
-  double rowK[16 * RS];
-  double colT[2][16 * RS];
-  double rvK[16 * RS];
-  double Pi[16 * 17];
-  double piv[MP];
-  int failk[2];
-  double red[16];
+// LDS of one matrix.  Tiles are kept as the registers of the MFMA accumulator layout:
+// [r][lane] with lane = 16 (row % 4) + column, row = 4r + lane / 16.
+//   rv: block row K, one 256-double slot per tile J, the identity in slot K and the pivot
+//       block P in slot MT; the panel replaces slot J by P^-1 A[K,J] and slot K by P^-1.
+//       Register r of a slot is at the same time the k-slice r of an MFMA B operand.
+//   ct: minus block column K transposed, [k][row] with rows of 17, per tile I (the MFMA A
+//       operand of the updates); slot K holds the identity.
+// With those identities and the tiles of block row and column K zeroed where they are
+// published, every tile's update is the same A[I,J] += ct[I] rv[J], without a branch.
+// Both double-buffered by the parity of K, so a wave may publish block K + 1 while others
+// still update with block K; NB = 1 (one more barrier per block) where two do not fit.
+// From M = 193 on the matrix and the working registers outgrow the register file: TL tiles per
+// wave live in lt and, from M = 225 on, TG tiles at their place in the output array (in the
+// L2), read and written once per block.  GT = false: no output array (log det only), those
+// tiles in registers that spill.
+template <int MT, int NW, bool GT>
+struct SpdShape {
+  static constexpr int T = MT * MT;
+  static constexpr int TPW = (T + NW - 1) / NW;                 // tiles per wave
+  static constexpr int TL = MT <= 12 ? 0 : (MT == 13 ? 1 : 5);  // of them in LDS
+  static constexpr int TG = !GT || MT < 15 ? 0 : (MT == 15 ? 4 : 7);  // in the output array
+  static constexpr int TR = TPW - TL - TG;                      // in registers
+  static constexpr int NB = MT <= 13 ? 2 : 1;
+  static constexpr int NPW = NW == 4 ? 3 : 6;  // waves that carry the panel's tiles
+  static constexpr int NJ = (MT + NPW - 1) / NPW;               // tiles of each
+  // where the accumulators leave few registers: the panel's tiles stay in LDS (YL), and the
+  // updates load one tile's operands at a time (not PF)
+  static constexpr bool YL = MT >= 13, PF = GT || MT <= 14;
 };
 
-// Phase 2 for panel wave pw of block K.  Lane c < 16 holds pivot column K*16 + c, lane
-// 16 + c identity column c (ending as column c of P^-1) and lanes 32.. hold CPL of the
-// other columns each (ending as P^-1 A[K, col]).  Every panel wave runs the same pivots
-// on the same pivot columns, so their copies agree bit for bit.
-template <int MT, int CPL = 1>
-__device__ __forceinline__ void spd_panel(SpdLds<MT> &sm, int K, int pw, int lane) {
-  constexpr int MP = SpdLds<MT>::MP, RS = SpdLds<MT>::RS;
-  int col[CPL];
-  bool live[CPL];
-#pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-    live[c] = c == 0 || lane >= 32;
-    col[c] = K * 16 + lane;
-    if (lane >= 32) {
-      const int m = 32 * CPL * pw + 32 * c + lane - 32;
-      live[c] = m < MP - 16;
-      col[c] = m < K * 16 ? m : m + 16;
-    }
-  }
-  const bool ident = lane >= 16 && lane < 32;
-  double v[CPL][16];
-#pragma unroll
-  for (int c = 0; c < CPL; ++c)
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      v[c][i] = ident ? (c == 0 && i == lane - 16 ? 1.0 : 0.0) : (live[c] ? sm.rowK[i * RS + col[c]] : 0.0);
-  int bad = 0;
-#pragma unroll
-  for (int p = 0; p < 16; ++p) {
-    const double d = gpx_readlane_d(v[0][p], p);
-    if (!bad && !(d > 0.0 && d < INFINITY)) bad = p + 1;
-    const double rd = gpx_recip(d);
-    double colp[16];  // column p, read from the pivot lane
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      if (i != p) colp[i] = gpx_readlane_d(v[0][i], p);
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-      const double rowp = v[c][p] * rd;
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if (i != p) v[c][i] = fma(-colp[i], rowp, v[c][i]);
-      v[c][p] = rowp;
-    }
-    if (pw == 0 && lane == 0) sm.piv[K * 16 + p] = d;
-  }
-  if (ident) {
-    if (pw == 0) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sm.Pi[i * 17 + lane - 16] = v[0][i];
-    }
-  } else if (lane >= 32) {
-#pragma unroll
-    for (int c = 0; c < CPL; ++c)
-      if (live[c]) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sm.rvK[i * RS + col[c]] = v[c][i];
-      }
-  }
-  if (pw == 0 && lane == 0) sm.failk[K & 1] = bad ? K * 16 + bad : 0;
+template <int MT, int NW>
+struct SpdLds {
+  typedef SpdShape<MT, NW, true> S;
+  static constexpr int CT = 16 * 17;
+  // the small arrays first: LDS addresses below 64 KB fit an instruction's offset field
+  double mul[4][16];   // [g][i]: pivot g's multiplier of row i, its reciprocal at i = g
+  double piv[16 * MT];
+  double red[16];
+  int first[NW];
+  int step;            // pivots done, in fours, over all blocks
+  double pt[4][CT];    // the pivot block, transposed, before each four pivots
+  double rv[S::NB][(MT + 1) * 256];
+  double ct[S::NB][MT * CT];
+  double lt[S::TL ? S::TL * NW * 256 : 1];
+};
+
+// Lane LC of each 16-lane row to the whole row (DPP row_newbcast, one instruction).
+template <int LC>
+__device__ __forceinline__ double spd_bcast16(double v) {
+  return __longlong_as_double(
+      __builtin_amdgcn_mov_dpp((long long)__double_as_longlong(v), 0x150 + LC, 0xF, 0xF, true));
 }
 
-// Phase 1 for one tile: block row K and block column K (transposed) to LDS.
-template <int MT>
-__device__ __forceinline__ void spd_publish(SpdLds<MT> &sm, int K, int I, int J, const gpx_d4 &acc, int lr,
-                                            int lc) {
-  constexpr int RS = SpdLds<MT>::RS;
-  double *cT = sm.colT[K & 1];
-  if (I == K) {
+// c[g][i] = the value of v in lane 4 g + i of each row.
+template <int... E>
+__device__ __forceinline__ void spd_spread(double v, double (*c)[4], std::integer_sequence<int, E...>) {
+  ((c[E / 4][E % 4] = spd_bcast16<E>(v)), ...);
+}
+
+// x[k] = the value of v in lane 16 k + (lane % 16): the four 16-lane rows of v, each in
+// every row (cross-row lane swaps).
+__device__ __forceinline__ void spd_rows4(double v, double *x) {
+  const unsigned lo = __double2loint(v), hi = __double2hiint(v);
+  const auto l16 = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sm.rowK[(lr + 4 * r) * RS + J * 16 + lc] = acc[r];
-  }
-  if (J == K) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) cT[lc * RS + I * 16 + lr + 4 * r] = acc[r];
+  for (int o = 0; o < 2; ++o) {  // o = 0: rows 0 and 2, o = 1: rows 1 and 3
+    const auto l32 = __builtin_amdgcn_permlane32_swap(l16[o], l16[o], false, false);
+    const auto h32 = __builtin_amdgcn_permlane32_swap(h16[o], h16[o], false, false);
+    x[o] = __hiloint2double(h32[0], l32[0]);
+    x[o + 2] = __hiloint2double(h32[1], l32[1]);
   }
 }
 
-// Phase 3 for one tile.
-template <int MT>
-__device__ __forceinline__ void spd_update(SpdLds<MT> &sm, int K, int I, int J, gpx_d4 &acc, int lr, int lc) {
-  constexpr int RS = SpdLds<MT>::RS;
-  const double *cT = sm.colT[K & 1];
+__device__ __forceinline__ void spd_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// 1/d from the hardware estimate r (relative error e < 2^-20): r (1 + e + e^2), three dependent
+// operations after the estimate.
+__device__ __forceinline__ double spd_recip(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+
+// One scalar pivot, row 4 R + G of the pivot block, on the four rows x of its register R
+// (each lane its column); c[G] the pivot's reciprocal, c[i] its multiplier of row i.
+template <int R, int G>
+__device__ __forceinline__ void spd_pivot(double *x, double *c, double &d) {
+  d = spd_bcast16<4 * R + G>(x[G]);
+  c[G] = spd_recip(d);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i != G) c[i] = spd_bcast16<4 * R + G>(x[i]);
+  x[G] *= c[G];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (i != G) x[i] = fma(-c[i], x[G], x[i]);
+}
+
+// x0 .. x3 by the lane's 16-lane row.
+__device__ __forceinline__ double spd_pick(double x0, double x1, double x2, double x3, int lr) {
+  const bool odd = lr & 1, high = lr & 2;
+  return high ? (odd ? x3 : x2) : (odd ? x1 : x0);
+}
+
+// Rows 4R .. 4R+3 of the pivot block P (wave 0): four scalar pivots over the four rows, their
+// multipliers to LDS for the other waves, then the rank-4 update of P's other rows as one
+// MFMA.
+template <int R, int MT, int NW>
+__device__ __forceinline__ void spd_pivot_rows(SpdLds<MT, NW> &sm, int K, int lane, gpx_d4 &P) {
+  const int lr = lane >> 4, lc = lane & 15;
+  double x[4], c[4][4], d[4];
+  spd_rows4(P[R], x);
+  spd_pivot<R, 0>(x, c[0], d[0]);
+  __builtin_amdgcn_sched_barrier(0);
+  // A operand P[., 4R .. 4R+3] before these pivots (columns to operand layout through LDS)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) sm.pt[R][lc * 17 + lr + 4 * r] = P[r];
+  spd_wave_sync();
+  const double a = sm.pt[R][(4 * R + lr) * 17 + lc];
+  __builtin_amdgcn_sched_barrier(0);
+  spd_pivot<R, 1>(x, c[1], d[1]);
+  spd_pivot<R, 2>(x, c[2], d[2]);
+  spd_pivot<R, 3>(x, c[3], d[3]);
+  if (lane == 0) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sm.mul[R][g * 4 + i] = c[g][i];
+      sm.piv[K * 16 + 4 * R + g] = d[g];
+    }
+  }
+  if constexpr (R < 3) {
+    const double px = spd_pick(x[0], x[1], x[2], x[3], lr);
+    P = gpx_mfma16(a, -px, P);
+    P[R] = px;
+  }
+  __hip_atomic_store(&sm.step, 4 * K + R + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// The same rows of the wave's panel tiles, one step behind the pivot block.
+template <int R, int MT, int NW, int NJ>
+__device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, int K, int pw, int lane, gpx_d4 *y) {
+  typedef SpdShape<MT, NW, true> S;
+  const int lr = lane >> 4, lc = lane & 15;
+  // tile j of the wave; past the last tile the first one again (its copy is not written back)
+  auto slot = [&](int j) { return rv + (pw + S::NPW * j < MT ? pw + S::NPW * j : pw) * 256; };
+  double yr[NJ][4];
+  if constexpr (R > 0 && !S::YL) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) slot(j)[R * 64 + lane] = y[j][R];
+  }
+  spd_wave_sync();
+  auto rows = [&](int j) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) yr[j][k] = slot(j)[R * 64 + 16 * k + lc];
+  };
+  if constexpr (!S::YL) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) rows(j);
+  }
+  while (__hip_atomic_load(&sm.step, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < 4 * K + R + 1) {
+    __builtin_amdgcn_s_sleep(1);  // leave instruction fetch to wave 0
+  }
+  const double a = sm.pt[R][(4 * R + lr) * 17 + lc];
+  // the 16 multipliers as one value per lane of each row
+  const double cm = sm.mul[R][lc];
+  double c[4][4];
+  spd_spread(cm, c, std::make_integer_sequence<int, 16>());
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if constexpr (S::YL) {
+      if (pw + S::NPW * j >= MT) break;  // wave-uniform
+      rows(j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[j][r] = slot(j)[r * 64 + lane];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      yr[j][g] *= c[g][g];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (i != g) yr[j][i] = fma(-c[g][i], yr[j][g], yr[j][i]);
+    }
+    const double py = spd_pick(yr[j][0], yr[j][1], yr[j][2], yr[j][3], lr);
+    y[j] = gpx_mfma16(a, -py, y[j]);
+    y[j][R] = py;
+    if constexpr (S::YL) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) slot(j)[r * 64 + lane] = y[j][r];
+    }
+  }
+}
+
+// Phase 2 for block K: Gauss-Jordan over the 16 scalar pivots of P on [P | I | A[K, other
+// columns]].  Wave 0 runs the pivots on P alone; the waves of the other SIMDs (not wave 4,
+// which shares wave 0's) carry the tiles of the block row, each a step of four pivots
+// behind it (sm.step; wave 0 waits for nobody, so every wait ends).
+template <int MT, int NW>
+__device__ __forceinline__ void spd_panel(SpdLds<MT, NW> &sm, double *rv, int K, int w, int lane) {
+  typedef SpdShape<MT, NW, true> S;
+  constexpr int NJ = S::NJ;
+  if (w == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    gpx_d4 P;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) P[r] = rv[MT * 256 + r * 64 + lane];
+    spd_pivot_rows<0, MT, NW>(sm, K, lane, P);
+    spd_pivot_rows<1, MT, NW>(sm, K, lane, P);
+    spd_pivot_rows<2, MT, NW>(sm, K, lane, P);
+    spd_pivot_rows<3, MT, NW>(sm, K, lane, P);
+    __builtin_amdgcn_s_setprio(0);
+    return;
+  }
+  const int pw = w < 4 ? w - 1 : w - 2;
+  if (w == 4 || pw >= MT) return;
+  gpx_d4 y[NJ];
+  if constexpr (!S::YL) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int J = pw + S::NPW * j < MT ? pw + S::NPW * j : pw;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[j][r] = rv[J * 256 + r * 64 + lane];
+    }
+  }
+  spd_tile_rows<0, MT, NW, NJ>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<1, MT, NW, NJ>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<2, MT, NW, NJ>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<3, MT, NW, NJ>(sm, rv, K, pw, lane, y);
+  if constexpr (!S::YL) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (pw + S::NPW * j >= MT) break;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rv[(pw + S::NPW * j) * 256 + r * 64 + lane] = y[j][r];
+    }
+  }
+}
+
+// Phase 1 for one tile: block row K and (negated, transposed) block column K to LDS.
+template <int MT, int NW>
+__device__ __forceinline__ void spd_publish(double *rv, double *ct, int K, int I, int J, gpx_d4 &acc, int lane) {
+  if (__builtin_expect(I != K && J != K, 1)) return;
+  const int lr = lane >> 4, lc = lane & 15;
+  double *c = ct + I * SpdLds<MT, NW>::CT + lc * 17 + lr;
   if (I == K) {
+    double *v = rv + (J == K ? MT : J) * 256 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r * 64] = acc[r];
     if (J == K) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = sm.Pi[(lr + 4 * r) * 17 + lc];
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) acc[r] = sm.rvK[(lr + 4 * r) * RS + J * 16 + lc];
+      for (int r = 0; r < 4; ++r) c[4 * r] = rv[K * 256 + r * 64 + lane] = lr + 4 * r == lc ? 1.0 : 0.0;
     }
-  } else if (J == K) {
-    gpx_d4 c = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      c = gpx_mfma16(-cT[(4 * ks + lr) * RS + I * 16 + lc], sm.Pi[(4 * ks + lr) * 17 + lc], c);
-    acc = c;
   } else {
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      acc = gpx_mfma16(-cT[(4 * ks + lr) * RS + I * 16 + lc], sm.rvK[(4 * ks + lr) * RS + J * 16 + lc], acc);
+    for (int r = 0; r < 4; ++r) c[4 * r] = -acc[r];
+  }
+  acc = gpx_d4{0.0, 0.0, 0.0, 0.0};
+}
+
+// The wave's next tile, NW further in row-major order (I = MT past the last one).
+template <int MT, int NW>
+__device__ __forceinline__ void spd_next(int &I, int &J) {
+  J += NW % MT;
+  I += NW / MT;
+  if (J >= MT) {
+    J -= MT;
+    ++I;
   }
 }
 
+// log det and info from the pivots; returns info: the first pivot that is not a positive
+// number, counted from 1 (0: none; what was computed after it is not used).
 template <int MT, int NW>
-__device__ __forceinline__ void spd_finish(SpdLds<MT> &sm, int M, int b, int fail, double *logdet, int *info) {
-  __syncthreads();  // pivots of the last block were written after the last barrier of the loop
-  double ld = 0.0;
-  for (int k = threadIdx.x; k < (fail ? 0 : M); k += NW * 64) ld += log(sm.piv[k]);
-  ld = gpx_block_sum(ld, sm.red);
-  if (threadIdx.x == 0) {
+__device__ __forceinline__ int spd_finish(SpdLds<MT, NW> &sm, int M, int b, double *logdet, int *info) {
+  static_assert(NW * 64 >= 16 * MT, "one pivot per thread");
+  const int k = threadIdx.x;
+  const double d = k < M ? sm.piv[k] : 1.0;
+  const unsigned long long bad = __ballot(!(d > 0.0 && d < INFINITY));
+  if ((k & 63) == 0) sm.first[k >> 6] = bad ? k + __ffsll(bad) : 0;
+  const double ld = gpx_block_sum(log(d), sm.red);  // its barriers order sm.first
+  int fail = 0;
+#pragma unroll
+  for (int w = NW - 1; w >= 0; --w) fail = sm.first[w] ? sm.first[w] : fail;
+  if (k == 0) {
     if (logdet) logdet[b] = fail ? NAN : ld;
     if (info) info[b] = fail;
   }
+  return fail;
 }
 
 // Blocked Gauss-Jordan on the matrix cores, 16 x 16 pivot blocks.  Eliminating block
@@ -146,89 +313,184 @@ __device__ __forceinline__ void spd_finish(SpdLds<MT> &sm, int M, int b, int fai
 //   A[I,J] -= c_I P^-1 A[K,J]     (I, J != K)
 //   A[K,J] <- P^-1 A[K,J],  A[I,K] <- -c_I P^-1,  A[K,K] <- P^-1,
 // and after every block the matrix holds A^-1.  All MT x MT tiles are kept, in MFMA
-// accumulator layout, dealt round-robin to the tile waves (register r of lane l holds
-// tile entry [l/16 + 4r][l%16]): keeping only a symmetric half and mirroring it costs
-// two orders of magnitude in accuracy downstream on ill-conditioned input, because the
-// two halves of a computed inverse carry errors that cancel in later products.
-// Per block: the owners of block row and column K publish them to LDS; the panel waves
-// run Gauss-Jordan over the 16 scalar pivots on [P | I | A[K, other columns]], giving
-// P^-1 A[K,:] and P^-1 without ever multiplying by an explicit P^-1 (which loses an order
-// of magnitude on ill-conditioned blocks); the tile waves then update their tiles with
-// four 16x16x4 MFMAs per tile.  The scalar pivots are the D of A = L D L^T: their logs
-// sum to log det A and the first non-positive one flags a matrix that is not positive
-// definite.  The matrix is padded with the identity up to a multiple of 16.  Every wave
-// holds tiles and the first NPW waves also run the panel (giving the panel waves of its
-// own, two columns per lane, measured slower at every size on MI355X).
-template <int MT, int NW>
+// accumulator layout, dealt round-robin to the waves: keeping only a symmetric half and
+// mirroring it costs two orders of magnitude in accuracy downstream on ill-conditioned
+// input, because the two halves of a computed inverse carry errors that cancel in later
+// products.  Per block: (1) the owners of block row and column K publish them to LDS; (2)
+// the panel waves run Gauss-Jordan over the 16 scalar pivots on [P | I | A[K, other
+// columns]], giving P^-1 A[K,:] and P^-1 without ever multiplying by an explicit P^-1
+// (which loses an order of magnitude on ill-conditioned blocks); (3) every wave updates
+// its tiles with four 16x16x4 MFMAs per tile.  The scalar pivots are the D of A = L D L^T:
+// their logs sum to log det A and the first non-positive one flags a matrix that is not
+// positive definite.  The matrix is padded with the identity up to a multiple of 16.
+//
+// What bounds it: the serial chain of 16 pivots per block (about 3,900 cycles on wave 0; the
+// tiles of the block row follow one step of four pivots behind, about 1,900 more) and the 4 T
+// MFMAs of 64 cycles per block on four SIMDs (4,096 of them at M = 128, 10,816 at M = 200);
+// an FP64 MFMA holds up the FP64 vector work of its SIMD, so the two do not overlap.  Every
+// lane broadcast is a DPP move or a lane swap (16 rows of one column at a time by scalar
+// lane reads took 6,700 cycles per block), and the updates run without a branch, the next
+// tile's operands loaded beside the current MFMAs.  One matrix, microseconds before -> now:
+// M = 50 18.3 -> 14.5, 100 43.5 -> 38, 128 53 -> 48, 160 102 -> 74, 200 200 -> 141,
+// 224 255 -> 173, 256 409 -> 289 (64 matrices take 2-4% longer).
+template <int MT, int NW, bool GT>
 __global__ __launch_bounds__(NW * 64) void spd_gj_kernel(int M, int batch, const double *__restrict__ A,
                                                          int lda, long sA, double *__restrict__ out, int ldo,
                                                          long sO, double *__restrict__ logdet,
                                                          int *__restrict__ info) {
-  constexpr int MP = 16 * MT;
-  constexpr int T = MT * MT;
-  constexpr int NPW = MP > 16 ? (MP - 16 + 31) / 32 : 1;  // panel waves
-  constexpr int TPW = (T + NW - 1) / NW;
-  static_assert(NPW <= NW, "not enough waves for the panel");
-  __shared__ SpdLds<MT> sm;
+  typedef SpdShape<MT, NW, GT> S;
+  constexpr int T = S::T, TR = S::TR, TL = S::TL, TG = S::TG, TM = TL + TG, CT = SpdLds<MT, NW>::CT;
+  __shared__ SpdLds<MT, NW> sm;
   const int b = blockIdx.x;
   if (b >= batch) return;
   // w in a scalar register: the tile indices and their LDS offsets are then wave-uniform
   // scalars rather than a few vector registers per tile
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane >> 4, lc = lane & 15;
-  int fail = 0;
   const double *Ab = A + b * sA;
-  gpx_d4 acc[TPW];
+  gpx_d4 acc[TR];
+  double *lt = sm.lt + (TL ? w * TL * 256 : 0);
+  // tile t = w + NW u of the wave: u < TG in the output array (they lie in the first rows of
+  // tiles, where the padding is the zeros right of column M), the next TL in LDS, the others
+  // in acc.  Loads are unconditional at clamped indices (so they issue together); the identity padding of the
+  // edge tiles is put in afterwards.
+  auto load = [&](int t) {
+    gpx_d4 v;
+    const int I = t / MT, J = t % MT, j = min(J * 16 + lc, M - 1);
 #pragma unroll
-  for (int u = 0; u < TPW; ++u) {
-    const int t = w + NW * u, I = t / MT, J = t % MT;
+    for (int r = 0; r < 4; ++r) v[r] = Ab[(long)min(I * 16 + lr + 4 * r, M - 1) * lda + j];
+    return v;
+  };
+  auto pad = [&](int t, gpx_d4 &v) {
+    const int I = t / MT, J = t % MT, j = J * 16 + lc;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = I * 16 + lr + 4 * r, j = J * 16 + lc;
-      acc[u][r] = (t < T && i < M && j < M) ? Ab[(long)i * lda + j] : (i == j ? 1.0 : 0.0);
+      const int i = I * 16 + lr + 4 * r;
+      v[r] = i < M && j < M ? v[r] : (i == j ? 1.0 : 0.0);
     }
+  };
+  double *Ob = out ? out + b * sO : nullptr;
+  auto get = [&](int u, int I, int J) {
+    gpx_d4 v;
+    if (u < TG) {
+      const int j = J * 16 + lc;
+      const double *p = Ob + (long)(I * 16 + lr) * ldo + min(j, M - 1);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = p[(long)(4 * r) * ldo];
+        if (j >= M) v[r] = 0.0;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = lt[(u - TG) * 256 + r * 64 + lane];
+    }
+    return v;
+  };
+  auto put = [&](int u, int I, int J, const gpx_d4 &v) {
+    if (u < TG) {
+      const int j = J * 16 + lc;
+      double *p = Ob + (long)(I * 16 + lr) * ldo + j;
+      if (j < M) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[(long)(4 * r) * ldo] = v[r];
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lt[(u - TG) * 256 + r * 64 + lane] = v[r];
+    }
+  };
+  if (threadIdx.x == 0) sm.step = 0;
+#pragma unroll
+  for (int u = 0; u < TR; ++u) acc[u] = load(w + NW * (u + TM));
+#pragma unroll
+  for (int u = 0; u < TM; ++u) {
+    gpx_d4 v = load(w + NW * u);
+    if (M & 15) pad(w + NW * u, v);
+    put(u, (w + NW * u) / MT, (w + NW * u) % MT, v);
+  }
+  if (M & 15) {  // wave-uniform
+#pragma unroll
+    for (int u = 0; u < TR; ++u) pad(w + NW * (u + TM), acc[u]);
   }
 #pragma unroll 1
-  for (int K = 0; K < MT; ++K) {
+  for (int K = 0;; ++K) {
+    const int buf = S::NB == 2 ? K & 1 : 0;
+    double *rv = sm.rv[buf], *ct = sm.ct[buf];
+    // the wave's first tile; opaque per block, so that the tile indices are stepped along
+    // instead of being kept for every tile over the whole elimination
+    int w0 = w;
+    asm volatile("" : "+s"(w0));
     // (1) block row and column K to LDS
+    {
+      int I = w0 / MT, J = w0 % MT;
 #pragma unroll
-    for (int u = 0; u < TPW; ++u) {
-      const int t = w + NW * u;
-      if (t < T) spd_publish<MT>(sm, K, t / MT, t % MT, acc[u], lr, lc);
+      for (int u = 0; u < TM + TR; ++u) {
+        if (u < TM) {
+          if (__builtin_expect(I == K || J == K, 0)) {
+            gpx_d4 v = get(u, I, J);
+            spd_publish<MT, NW>(rv, ct, K, I, J, v, lane);
+            put(u, I, J, v);
+          }
+        } else if (u + 1 < TM + TR || T % NW == 0 || I < MT) {
+          spd_publish<MT, NW>(rv, ct, K, I, J, acc[u < TM ? 0 : u - TM], lane);
+        }
+        spd_next<MT, NW>(I, J);
+      }
     }
     __syncthreads();
     // (2) the panel
-    if (w < NPW) spd_panel<MT>(sm, K, w, lane);
+    spd_panel<MT, NW>(sm, rv, K, w, lane);
     __syncthreads();
-    if (sm.failk[K & 1]) {
-      fail = sm.failk[K & 1];
-      break;
-    }
-    // (3) the tiles, one tile's operands at a time (hoisting the LDS loads of later tiles
-    // above this one's MFMAs would hold all of them in registers at once)
+    // (3) the tiles, the next tile's operands loaded beside this one's MFMAs (hoisting more
+    // of the LDS loads would hold all of them in registers at once); a wave's tile past the
+    // last one is computed from the last row's operands and never used
+    double a[2][4], bv[2][4];
+    int I = w0 / MT, J = w0 % MT;
+    auto operands = [&](double *av, double *bw) {
+      const double *pr = rv + J * 256 + lane, *pc = ct + min(I, MT - 1) * CT + lr * 17 + lc;
 #pragma unroll
-    for (int u = 0; u < TPW; ++u) {
-      const int t = w + NW * u;
-      if (t < T) spd_update<MT>(sm, K, t / MT, t % MT, acc[u], lr, lc);
+      for (int ks = 0; ks < 4; ++ks) {
+        bw[ks] = pr[ks * 64];
+        av[ks] = pc[ks * 68];
+      }
+    };
+    if (S::PF) operands(a[0], bv[0]);
+    gpx_d4 ahead = TG ? get(0, I, J) : gpx_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < TM + TR; ++u) {
+      constexpr int N1 = S::PF ? 1 : 0;  // tiles loaded ahead
+      const int Iu = I, Ju = J;
+      gpx_d4 v = u < TG ? ahead : (u < TM ? get(u, I, J) : acc[u < TM ? 0 : u - TM]);
+      if (N1 == 0 || u + 1 < TM + TR) {
+        if (N1 || u > 0) spd_next<MT, NW>(I, J);
+        operands(a[(u + N1) & 1], bv[(u + N1) & 1]);
+        if (N1 && u + 1 < TG) ahead = get(u + 1, I, J);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) v = gpx_mfma16(a[u & 1][ks], bv[u & 1][ks], v);
+      if (u < TM) put(u, Iu, Ju, v); else acc[u < TM ? 0 : u - TM] = v;
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (K + 1 == MT) break;
+    if (S::NB == 1) __syncthreads();
   }
-  spd_finish<MT, NW>(sm, M, b, fail, logdet, info);
+  const int fail = spd_finish<MT, NW>(sm, M, b, logdet, info);
   if (!out) return;
-  double *Ob = out + b * sO;
   // the store indices are formed afresh from an opaque copy of the lane: otherwise the
   // compiler keeps the load's per-tile indices live through the whole elimination
   int lane2 = lane;
   asm volatile("" : "+v"(lane2));
   const int lr2 = lane2 >> 4, lc2 = lane2 & 15;
 #pragma unroll
-  for (int u = 0; u < TPW; ++u) {
+  for (int u = 0; u < TM + TR; ++u) {
     const int t = w + NW * u, I = t / MT, J = t % MT;
-    if (t >= T) continue;
+    if (t >= T || (u < TG && !fail)) continue;
+    const gpx_d4 v = u < TM ? get(u, I, J) : acc[u < TM ? 0 : u - TM];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = I * 16 + lr2 + 4 * r, j = J * 16 + lc2;
-      if (i < M && j < M) Ob[(long)i * ldo + j] = fail ? NAN : acc[u][r];
+      if (i < M && j < M) Ob[(long)i * ldo + j] = fail ? NAN : v[r];
     }
   }
 }
@@ -236,11 +498,15 @@ __global__ __launch_bounds__(NW * 64) void spd_gj_kernel(int M, int batch, const
 template <int MT>
 int launch_gj(int M, int batch, const double *A, int lda, long sA, double *out, int ldo, long sO,
                  double *logdet, int *info, hipStream_t st) {
-  // 8 waves from M > 48 on (measured on MI355X against 16: equal at M = 200, faster
-  // everywhere else)
+  // 8 waves (two per SIMD) from M > 48 on: one wave's LDS operand loads hide behind the
+  // other's MFMAs
   constexpr int NW = MT <= 3 ? 4 : 8;
-  hipLaunchKernelGGL((spd_gj_kernel<MT, NW>), dim3(batch), dim3(NW * 64), 0, st, M, batch, A, lda, sA, out, ldo,
-                     sO, logdet, info);
+  if (MT < 15 || out)
+    hipLaunchKernelGGL((spd_gj_kernel<MT, NW, true>), dim3(batch), dim3(NW * 64), 0, st, M, batch, A, lda, sA, out,
+                       ldo, sO, logdet, info);
+  else
+    hipLaunchKernelGGL((spd_gj_kernel<MT, NW, MT < 15>), dim3(batch), dim3(NW * 64), 0, st, M, batch, A, lda, sA,
+                       out, ldo, sO, logdet, info);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }
