@@ -8,15 +8,12 @@ sums), so any of them meets the same tolerance.
 
 Knobs
   fused forward   nsub (16*nsub points per workgroup), splits_f (pair-tile splits)
-  fused backward  splits_b (column-tile splits of the per-point pass),
-                  nsplit (point ranges of the per-pair pass)
+  fused backward  nsplit (point ranges)
   gemm            tile (32 or 64 rows/cols per workgroup), split-K factor
 
-Cache: ``$GEEPEE_AMD_TUNE_CACHE`` if set, else ``~/.cache/geepee_amd/tune.json``, over
-the plans shipped in ``tuned_plans.json`` (the benchmark shapes, tuned on MI355X).
+Cache: ``$GEEPEE_AMD_TUNE_CACHE`` if set, else ``~/.cache/geepee_amd/tune.json``.
 ``lookup`` is consulted by dops.fused_plan and dops.mm before their heuristics.
 """
-import itertools
 import json
 import os
 
@@ -46,9 +43,6 @@ def _device_tag():
     return _tag
 
 
-SHIPPED = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'tuned_plans.json')
-
-
 def _read(path):
     try:
         with open(path) as f:
@@ -58,14 +52,11 @@ def _read(path):
 
 
 def _load():
-    """Plans shipped with the package (tuned on MI355X for the benchmark shapes),
-    overridden by the user's cache."""
+    """The plans of the user's cache file."""
     global _cache
     if _cache is None:
-        _cache = dict(_read(SHIPPED)) if os.path.exists(SHIPPED) else {}
         p = cache_path()
-        if os.path.exists(p):
-            _cache.update(_read(p))
+        _cache = _read(p) if os.path.exists(p) else {}
     return _cache
 
 
@@ -129,14 +120,13 @@ def fused_candidates(N, M):
     ntiles = T * (T + 1) // 2
     fwd = [{'nsub': ns, 'splits_f': s} for ns in (1, 2, 4) for s in _pow2_upto(1, min(ntiles, 64))
            if -(-N // (16 * ns)) * s >= 64]
-    bwd_points = [s for s in _pow2_upto(1, min(T, 64)) if -(-N // 16) * s >= 64]
-    bwd_pairs = [s for s in _pow2_upto(1, min(-(-N // 16), 64)) if ntiles * 4 * s >= 64]
+    bwd = [s for s in _pow2_upto(1, min(-(-N // 16), 64)) if ntiles * 4 * s >= 64]
     # point-range counts that fill whole rounds of 256 workgroups over the tiles (the
-    # merged adjoint kernel of D > 16 runs one workgroup per CU)
-    bwd_pairs = sorted(set(bwd_pairs) | {k * 256 // ntiles for k in (1, 2, 3, 4)
-                                         if 1 <= k * 256 // ntiles <= min(-(-N // 16), 64)})
-    return fwd or [{'nsub': 1, 'splits_f': min(ntiles, 64)}], bwd_points or [min(T, 64)], \
-        bwd_pairs or [min(-(-N // 16), 64)]
+    # adjoint kernel runs one workgroup per CU)
+    bwd = sorted(set(bwd) | {k * 256 // ntiles for k in (1, 2, 3, 4)
+                             if 1 <= k * 256 // ntiles <= min(-(-N // 16), 64)})
+    # (the middle list: the adjoint's splits_b, which no longer splits anything)
+    return fwd or [{'nsub': 1, 'splits_f': min(ntiles, 64)}], [1], bwd or [min(-(-N // 16), 64)]
 
 
 def tune_fused(N, M, Q, D, reps=5, seed=0, save=True, verbose=False):
@@ -152,7 +142,7 @@ def tune_fused(N, M, Q, D, reps=5, seed=0, save=True, verbose=False):
     Ahat = dev(rs.randn(D, M) * 0.1)
     Bp = dops.sym_pairmajor(dev(rs.randn(D, M, M) * 0.01))
     dm_all, dv = dev(rs.randn(N, D)), dev(rs.randn(N, D))
-    fwd, bpt, bpr = fused_candidates(N, M)
+    fwd, _, bwd = fused_candidates(N, M)
     base = dops.fused_plan(N, M, Q, D, tuned=False)
     table = {'fwd': {}, 'bwd': {}}
     best_f, tf = None, float('inf')
@@ -163,12 +153,12 @@ def tune_fused(N, M, Q, D, reps=5, seed=0, save=True, verbose=False):
             best_f, tf = c, t
     psi1, _, _ = dops.fused_mm_fwd(mx, vx, z, ls, sf, Ahat, Bp, plan=dict(base, **best_f))
     best_b, tb = None, float('inf')
-    for sb, ns in itertools.product(bpt, bpr):
-        p = dict(base, splits_b=sb, nsplit=ns)
+    for ns in bwd:
+        p = dict(base, nsplit=ns)
         t = _time(lambda: dops.fused_mm_bwd(mx, vx, z, ls, sf, Ahat, Bp, psi1, dm_all, dv, plan=p), reps)
-        table['bwd']['%d/%d' % (sb, ns)] = t
+        table['bwd']['%d' % ns] = t
         if t < tb:
-            best_b, tb = {'splits_b': sb, 'nsplit': ns}, t
+            best_b, tb = {'splits_b': base['splits_b'], 'nsplit': ns}, t
     plan = dict(best_f, **best_b)
     plan['ms_fwd'], plan['ms_bwd'] = tf, tb
     store('fused', (N, M, Q, D), plan, save=save)

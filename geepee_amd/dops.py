@@ -366,9 +366,19 @@ def fused_fits(M, Q, D):
 
 
 def fused_plan(N, M, Q=None, D=None, tuned=True):
-    """Launch shape of the fused moment-matched kernels: points per block (16*nsub), pair-tile
-    splits of the forward / per-point pass, point ranges of the per-pair pass.  A plan
-    stored by the autotuner for (N, M, Q, D) wins over the heuristic."""
+    """Launch shape of the fused moment-matched kernels: points per block (16*nsub) and pair-tile
+    splits of the forward, point ranges of the adjoint (splits_b is accepted by the adjoint's
+    entry points and no longer splits anything).  A plan stored by the autotuner for
+    (N, M, Q, D) wins over the heuristic.
+
+    Forward: two point tiles per workgroup (one B-hat load for both) once they leave two
+    workgroups per CU, and 4 splits, whose share of B-hat one XCD's L2 keeps; 8 where fewer
+    than 400 workgroups would hold many tiles each.  (Microseconds at (N, M, Q, D), plan
+    nsub/splits: (3001, 190, 10, 12) 1/4 133, 1/8 137, 2/8 146, 2/11 180; (500, 200, 8, 16) 1/8
+    49, 1/16 50, 1/32 60; (9999, 200, 4, 4) 2/4 285, 2/3 295, 4/8 328.)
+    Adjoint: one workgroup per CU takes ceil(blocks / k) 16-point blocks plus about two
+    blocks' worth of set-up and stores, in ceil(tiles k / 256) rounds; the k with the least
+    product.  ((900, 256, 10, 12): k = 2 316, 3 246, 4 256, 8 244.)"""
     if tuned and Q is not None:
         from . import autotune
         hit = autotune.lookup('fused', (N, M, Q, D))
@@ -376,16 +386,13 @@ def fused_plan(N, M, Q=None, D=None, tuned=True):
             return hit
     T = (M + 15) // 16
     ntiles = T * (T + 1) // 2
-    nsub = 4 if N >= 4096 else (2 if N >= 512 else 1)
-    fwd_blocks = -(-N // (16 * nsub))
-    splits_f = max(1, min(ntiles, -(-1024 // fwd_blocks)))
-    pt_blocks = -(-N // 16)
-    splits_b = max(1, min(T, -(-1024 // pt_blocks)))
-    nsplit = max(1, min(-(-N // 16), -(-1024 // (ntiles * 4))))
-    if D is not None and (D > 16 or N >= 1000):
-        # the merged adjoint kernel: one workgroup per CU, one round of 256 over the tiles
-        nsplit = max(1, min(-(-N // 16), 256 // ntiles))
-    return {'nsub': nsub, 'splits_f': splits_f, 'splits_b': splits_b, 'nsplit': nsplit}
+    nsub = 2 if N >= 4096 else 1
+    blocks = -(-N // (16 * nsub))
+    splits_f = 8 if 4 * blocks < 400 and (ntiles >= 56 or blocks < 32) else 4
+    splits_f = min(ntiles, splits_f)
+    nb = -(-N // 16)
+    nsplit = min(range(1, min(nb, 32) + 1), key=lambda k: (-(-ntiles * k // 256) * (-(-nb // k) + 2), k))
+    return {'nsub': nsub, 'splits_f': splits_f, 'splits_b': 1, 'nsplit': nsplit}
 
 
 def sym_pairmajor(B):
@@ -436,7 +443,7 @@ def fused_mm_bwd(mx, vx, z, ls, sf, Ahat, Bp, psi1, dm_all, dv, plan=None):
 
 
 class FusedBwdRest(object):
-    """The rest of a split fused adjoint (the per-pair pass and the tail): call() on the
+    """The rest of a split fused adjoint (the per-pair sums and the tail): call() on the
     stream it should run on, after that stream has waited for the first part, to get
     (dBhat, dsf2, dell, dZ).  The tensors in `keep` must stay alive until then."""
 

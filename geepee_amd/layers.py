@@ -539,7 +539,7 @@ class SGP_Layer(object):
         dAhat = mm(dm_all, psi1, tA=True)
         rest = None
         if psi2 is None and side is not None:
-            # the psi adjoint's per-pair pass and hyper-parameter tail join the forked chain
+            # the psi adjoint's per-pair sums and hyper-parameter tail join the forked chain
             # below: the layer below needs only dmx, dvx
             dmx, dvx, rest = dops.fused_mm_bwd_split(
                 mx, vx, self.zu, self.ls, self.sf, self.Ahat, self._Bp, psi1, dm_all, dv)

@@ -345,7 +345,7 @@ int gpx_sym_pairmajor(int D, int M, const double *B, double *out, void *stream);
 
 /* Forward of a Gaussian-input layer: psi1 (N x M), mout = psi1 Ahat^T and
  * vout = sf2 + <Bhat[d], psi2_n> - mout^2 with psi2 recomputed per 16x16 tile (FP64 MFMA for
- * the exponent GEMM and the Bhat contraction).  splits (grid.y over pair tiles) and nsub
+ * the exponent's cross terms and the Bhat contraction).  splits (grid.y over pair tiles) and nsub
  * (1, 2, 4: 16*nsub points per block) are tuning knobs; `work` holds
  * gpx_fused_fwd_workspace(N, M, D, splits) doubles.  Replaces compute_psi_weave followed by
  * the einsums of geepee/aep_models.py:193-198 (and base_models.py:298-304). */
@@ -371,7 +371,8 @@ int gpx_fused_mm_fwd_noalloc(int N, int M, int Q, int D, const double *mx, const
 
 /* Adjoint of the same layer without psi2 or dL/dpsi2 in HBM: from dm_all = dm - 2 dv m and dv
  * (N x D) produces dBhat = sum_n dv_nd psi2_n (D x M x M), and the psi adjoints dsf2, dell, dZ,
- * dmx, dvx.  Replaces geepee/aep_models.py:235-243 with compute_psi_derivatives
+ * dmx, dvx.  nsplit: point ranges (a tuning knob); splits (1 .. ceil(M/16)) is range-checked
+ * and otherwise unused.  Replaces geepee/aep_models.py:235-243 with compute_psi_derivatives
  * (geepee/kernels.py:302-309, 355-444). */
 long gpx_fused_bwd_workspace(int N, int M, int Q, int D, int splits, int nsplit);
 int gpx_fused_mm_bwd(int N, int M, int Q, int D, const double *mx, const double *vx, const double *z,

@@ -1,0 +1,89 @@
+"""The fused moment-matched kernels at the edges of their dispatch (GPU only): every count of
+exponent slices (Q = 1 .. 16) and of output slices (D = 1 .. 32), partial 16-row tiles and
+point blocks, the point counts per workgroup that fall back for lack of LDS, and far-away
+points whose psi2 underflows.
+
+Oracle: the moment-matching formulas in float64 on the CPU with torch's autograd.
+Tolerance: an exponent of magnitude E carries an absolute error of a few E eps, E < 300 here, so
+every psi2 entry is within 4 * 300 * 2.2e-16 = 2.7e-13 relative; sums of products of mixed
+sign lose at most one to two digits more at these sizes: 1e-11 normwise.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-11
+
+
+def _problem(N, M, Q, D, far=False):
+    rs = np.random.RandomState(N + 7 * M + 11 * Q + 13 * D)
+    t = lambda a: torch.as_tensor(a, dtype=torch.float64)
+    mx, vx = t(rs.randn(N, Q)), t(rs.uniform(0.0, 0.5, (N, Q)))
+    if far:
+        mx[: (N + 1) // 2] += 60.0
+    z, ls, sf = t(rs.randn(M, Q)), t(0.2 * rs.randn(Q) + 0.4), t(np.array([0.3]))
+    B = rs.randn(D, M, M) / M
+    return mx, vx, z, ls, sf, t(rs.randn(D, M)), t(0.5 * (B + B.transpose(0, 2, 1)))
+
+
+def _reference(mx, vx, z, ls, sf, A, B):
+    l = torch.exp(2 * ls)
+    e1, e2 = 0.0, 0.0
+    for q in range(mx.shape[1]):
+        s1, s2 = l[q] + vx[:, q:q + 1], l[q] + 2 * vx[:, q, None, None]
+        h = 0.5 * (z[:, None, q] + z[None, :, q])
+        e1 = e1 + 0.5 * torch.log(l[q] / s1) - 0.5 * (mx[:, q:q + 1] - z[None, :, q]) ** 2 / s1
+        e2 = e2 + 0.5 * torch.log(l[q] / s2) - (mx[:, q, None, None] - h) ** 2 / s2 \
+            - (z[:, None, q] - z[None, :, q]) ** 2 / (4 * l[q])
+    psi1, psi2 = torch.exp(2 * sf + e1), torch.exp(4 * sf + e2)
+    m = psi1 @ A.T
+    v = torch.exp(2 * sf) + torch.einsum('nab,dab->nd', psi2, B) - m ** 2
+    return m, v
+
+
+def _close(x, y):
+    x, y = x.cpu(), y.detach()
+    assert torch.isfinite(x).all()
+    assert torch.linalg.norm(x - y) <= TOL * max(float(torch.linalg.norm(y)), 1e-300), \
+        float(torch.linalg.norm(x - y) / torch.linalg.norm(y))
+
+
+SHAPES = [(1, 1, 1, 1), (16, 16, 4, 4), (17, 15, 5, 5), (33, 17, 8, 8), (65, 40, 9, 9), (31, 33, 12, 16),
+          (50, 31, 13, 17), (20, 48, 15, 32), (70, 130, 3, 2), (40, 250, 2, 3), (23, 256, 15, 4), (300, 20, 6, 31)]
+
+
+@pytest.mark.parametrize('far', [False, True])
+@pytest.mark.parametrize('N,M,Q,D', SHAPES)
+def test_fused_edges(N, M, Q, D, far):
+    from geepee_amd import dops
+    print('fused edges', N, M, Q, D, far, flush=True)
+    P = _problem(N, M, Q, D, far)
+    rs = np.random.RandomState(5)
+    gm, gv = (torch.as_tensor(rs.randn(N, D)) for _ in range(2))
+    ins = [p.clone().requires_grad_(True) for p in P]
+    m, v = _reference(*ins)
+    dmx, dvx, dz, _, _, _, dB = torch.autograd.grad([m, v], ins, [gm, gv])
+    mx, vx, z, ls, sf, A, B = [p.cuda() for p in P]
+    Bp = dops.sym_pairmajor(B)
+    nt = (M + 15) // 16 * ((M + 15) // 16 + 1) // 2
+    for nsub, splits in ((1, 1), (2, min(nt, 3)), (4, min(nt, 8))):
+        plan = {'nsub': nsub, 'splits_f': splits, 'splits_b': 1, 'nsplit': nsub}
+        psi1, mo, vo = dops.fused_mm_fwd(mx, vx, z, ls, sf, A, Bp, plan=plan)
+        _close(mo, m)
+        _close(vo, v)
+        dm = gm.cuda() - 2 * gv.cuda() * mo
+        out = dops.fused_mm_bwd(mx, vx, z, ls, sf, A, Bp, psi1, dm, gv.cuda(), plan=plan)
+        for got, want in zip((out[0], out[3], out[4], out[5]), (dB, dz, dmx, dvx)):
+            _close(got, want)
+
+
+def test_fused_forward_sixteen_inputs():
+    from geepee_amd import dops
+    P = _problem(19, 37, 16, 3)
+    m, v = _reference(*P)
+    mx, vx, z, ls, sf, A, B = [p.cuda() for p in P]
+    _, mo, vo = dops.fused_mm_fwd(mx, vx, z, ls, sf, A, dops.sym_pairmajor(B))
+    _close(mo, m)
+    _close(vo, v)
