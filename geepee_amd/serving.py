@@ -186,7 +186,7 @@ class ModelStore(object):
     def predict_many(self, reqs, noisy=False):
         return self.collect(self.launch(reqs, noisy))
 
-    # -- per-request plain path (one op per reference call, psi2 materialised) --
+    # -- per-request plain path (one layer call after the other) --
     def predict_plain(self, mid, X, noisy=False):
         x = torch.as_tensor(np.asarray(X, dtype=np.float64), device='cuda')
         mf = vf = None

@@ -87,3 +87,22 @@ def test_fused_forward_sixteen_inputs():
     _, mo, vo = dops.fused_mm_fwd(mx, vx, z, ls, sf, A, dops.sym_pairmajor(B))
     _close(mo, m)
     _close(vo, v)
+
+
+@pytest.mark.parametrize('N,M,Q,D', [(1, 5, 1, 1), (17, 16, 3, 2), (40, 50, 15, 32), (33, 256, 4, 1), (20, 20, 16, 2),
+                                     (9, 12, 2, 33)])
+def test_posterior_propagation_without_psi2(N, M, Q, D):
+    """forward_prop_thru_post at Gaussian inputs folds psi2 into the contraction where the fused
+    kernels take the shape (Q <= 15, D <= 32); with return_info it stores psi2, and at the last
+    two shapes it always does."""
+    from geepee_amd.layers import SGP_Layer
+    P = _problem(N, M, Q, D)
+    L = SGP_Layer(100, Q, D, M)
+    mx, vx, L.zu, L.ls, L.sf, L.A, L.B_sto = [p.cuda().contiguous() for p in P]
+    L._pred_ready, L._Bp_post = True, None
+    m, v = L.forward_prop_thru_post(mx, vx)
+    m2, v2, psi1, psi2 = L.forward_prop_thru_post(mx, vx, return_info=True)
+    assert psi1.shape == (N, M) and psi2.shape == (N, M, M)
+    for got in ((m, v), (m2, v2)):
+        for x, y in zip(got, _reference(*P)):
+            _close(x, y)
