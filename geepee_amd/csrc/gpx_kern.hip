@@ -3,14 +3,17 @@
 // hyper-parameters (ls, sf, sn, R) are read from the device so no host sync is needed.
 #include "gpx_common.h"
 
+#include <algorithm>
+
 namespace {
 
 // ---------------------------------------------------------------------------
 // SE kernel: compute_kernel (kernels.py:10-22), K = sf2 exp(-sum_q (x-z)^2 / (2 l_q))
 // ---------------------------------------------------------------------------
-__global__ void se_kernel(int N, int M, int Q, const double *__restrict__ x, int ldx,
-                          const double *__restrict__ z, const double *__restrict__ ls,
-                          const double *__restrict__ sf, double jitter, double *__restrict__ K) {
+// Q > 16 (any Q): one thread per entry.
+__global__ void se_any_kernel(int N, int M, int Q, const double *__restrict__ x, int ldx,
+                              const double *__restrict__ z, const double *__restrict__ ls,
+                              const double *__restrict__ sf, double jitter, double *__restrict__ K) {
   const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (e >= (long)N * M) return;
   const int n = (int)(e / M), m = (int)(e % M);
@@ -24,108 +27,166 @@ __global__ void se_kernel(int N, int M, int Q, const double *__restrict__ x, int
   K[e] = k;
 }
 
-// kfucompDer (kernels.py:381-399) with L = dK * K, pass 1 over slabs of KFU_NB rows, one
-// slab per workgroup staged in LDS (rows past N as zeros): part[blk][m] = [colsum_m,
-// sum_n L x_nq (Q), sum_n L (z_mq - x_nq)^2 (Q)], one thread per (m, q') entry with the
-// slab's rows unrolled so their LDS reads issue together;
-// dx_nq = sum_m L_nm (z_mq - x_nq) / l_q.
-constexpr int KFU_NB = 16;
-__global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, const double *__restrict__ dK,
+// Q <= QC: a block takes SE_ROWS rows by 64 columns, each wave every fourth row.  x, 1/l and
+// sf2 are formed once per block, a thread's z row stays in registers.  Bound by its exps and
+// its writes (N = 20000, M = 200, Q = 8: 58 -> 22 us; with the lengthscales' exps and divisions
+// per entry it was bound by those).
+constexpr int SE_ROWS = 16;
+template <int QC>
+__global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const double *__restrict__ x, int ldx,
+                                                 const double *__restrict__ z, const double *__restrict__ ls,
+                                                 const double *__restrict__ sf, double jitter,
+                                                 double *__restrict__ K) {
+  __shared__ double xs[SE_ROWS][QC], il[QC], s2;
+  const int tid = threadIdx.x, n0 = blockIdx.x * SE_ROWS, m = blockIdx.y * 64 + (tid & 63);
+  if (tid < QC) il[tid] = tid < Q ? exp(-2.0 * ls[tid]) : 0.0;
+  if (tid == 255) s2 = exp(2.0 * sf[0]);
+  for (int e = tid; e < SE_ROWS * QC; e += 256) {
+    const int i = e / QC, q = e % QC;
+    xs[i][q] = q < Q ? x[(long)min(n0 + i, N - 1) * ldx + q] : 0.0;
+  }
+  double zr[QC];
+#pragma unroll
+  for (int q = 0; q < QC; ++q) zr[q] = q < Q ? z[min(m, M - 1) * Q + q] : 0.0;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < SE_ROWS / 4; ++u) {
+    const int i = (tid >> 6) + 4 * u, n = n0 + i;
+    double r2 = 0.0;
+#pragma unroll
+    for (int q = 0; q < QC; ++q) {
+      const double d = xs[i][q] - zr[q];
+      r2 = fma(d * il[q], d, r2);
+    }
+    double k = s2 * exp(-0.5 * r2);
+    if (n == m) k += jitter;
+    if (n < N && m < M) K[(long)n * M + m] = k;
+  }
+}
+
+// kfucompDer (kernels.py:381-399) with L = dK * K.  Pass 1: block b takes the rows b G + g,
+// b G + g + nblk G, ...; thread (g, m) (m < MP, the columns rounded up to 64, 128 or 256;
+// G = 256 / MP row groups) keeps colsum_m, sum_n L x_nq and sum_n L (z_mq - x_nq)^2 in
+// registers (QC >= Q), the groups are added in order through LDS, and the W = 2Q + 1
+// sums go to part[b][w][m].  Bound by reading dK and K once; partials of 16-row slabs summed
+// by 14 workgroups were most of the adjoint before (three passes at N = 20000, M = 200, Q = 8
+// 104 -> 38 us; N = 1000, M = 100, Q = 10 17 -> 18 us).
+template <int QC>
+__global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, int MP, const double *__restrict__ dK,
                                                        const double *__restrict__ K,
                                                        const double *__restrict__ x,
                                                        const double *__restrict__ z,
-                                                       const double *__restrict__ ls,
-                                                       double *__restrict__ part,
-                                                       double *__restrict__ dx) {
-  __shared__ double xs[KFU_NB][17];
-  __shared__ double Ls[KFU_NB][257];
-  const int n0 = blockIdx.x * KFU_NB, nb = min(KFU_NB, N - n0), tid = threadIdx.x;
-  for (int e = tid; e < KFU_NB * Q; e += 256) {
-    const int i = e / Q, q = e % Q;
-    xs[i][q] = i < nb ? x[(long)(n0 + i) * Q + q] : 0.0;
+                                                       double *__restrict__ part) {
+  __shared__ double red[2 * QC + 1][256];
+  // g is uniform over a wave (MP a multiple of 64): its x rows are scalar loads
+  const int tid = threadIdx.x, m = tid % MP, g = __builtin_amdgcn_readfirstlane(tid / MP), G = 256 / MP,
+            mc = min(m, M - 1);
+  double zr[QC], lx[QC], ld2[QC], cs = 0.0;
+#pragma unroll
+  for (int q = 0; q < QC; ++q) {
+    zr[q] = q < Q ? z[mc * Q + q] : 0.0;
+    lx[q] = ld2[q] = 0.0;
   }
-  for (int e = tid; e < KFU_NB * M; e += 256) {
-    const int i = e / M, m = e % M;
-    const long o = (long)(n0 + i) * M + m;
-    Ls[i][m] = i < nb ? dK[o] * K[o] : 0.0;
+  const int step = gridDim.x * G;
+  // four rows' loads in flight together (rows past the end clamped, their L zeroed)
+  for (int n = blockIdx.x * G + g; n < N; n += 4 * step) {
+    double L[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long o = (long)min((long)n + (long)u * step, N - 1L) * M + mc;
+      L[u] = dK[o] * K[o];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const long r = (long)n + (long)u * step;
+      const double Lu = r < N ? L[u] : 0.0;
+      const double *xr = x + min(r, N - 1L) * Q;
+      cs += Lu;
+#pragma unroll
+      for (int q = 0; q < QC; ++q) {
+        const double xv = xr[min(q, Q - 1)], d = zr[q] - xv;  // q >= Q: never stored
+        lx[q] = fma(Lu, xv, lx[q]);
+        ld2[q] = fma(Lu * d, d, ld2[q]);
+      }
+    }
+  }
+  red[0][tid] = cs;
+#pragma unroll
+  for (int q = 0; q < QC; ++q) {
+    red[1 + q][tid] = lx[q];
+    red[1 + QC + q][tid] = ld2[q];
   }
   __syncthreads();
   const int W = 2 * Q + 1;
-  for (int e = tid; e < M * (Q + 1); e += 256) {
-    const int m = e / (Q + 1), q1 = e % (Q + 1);
-    double *P = part + ((long)blockIdx.x * M + m) * W;
-    if (q1 == 0) {
-      double cs = 0.0;
-#pragma unroll
-      for (int i = 0; i < KFU_NB; ++i) cs += Ls[i][m];
-      P[0] = cs;
-    } else {
-      const int q = q1 - 1;
-      const double zq = z[m * Q + q];
-      double lx = 0.0, ld2 = 0.0;
-#pragma unroll
-      for (int i = 0; i < KFU_NB; ++i) {
-        const double L = Ls[i][m], xv = xs[i][q], d = zq - xv;
-        lx += L * xv;
-        ld2 += L * d * d;
-      }
-      P[1 + q] = lx;
-      P[1 + Q + q] = ld2;
-    }
-  }
-  if (!dx) return;
-  for (int e = tid; e < nb * Q; e += 256) {
-    const int i = e / Q, q = e % Q;
-    double s = 0.0;
-    for (int m = 0; m < M; ++m) s += Ls[i][m] * (z[m * Q + q] - xs[i][q]);
-    dx[(long)(n0 + i) * Q + q] = s / exp(2.0 * ls[q]);
+  for (int e = tid; e < W * M; e += 256) {
+    const int w = e / M, c = e % M, r = w <= Q ? w : w - Q + QC;
+    double s = red[r][c];
+    for (int h = 1; h < G; ++h) s += red[r][h * MP + c];
+    part[((long)blockIdx.x * W + w) * M + c] = s;
   }
 }
 
-// Pass 2: workgroup g sums the slabs' partials (in slab order) for the rows
-// m in [g mb, (g + 1) mb), mb = 256 / (2Q + 1), one thread per partial column with its
-// loads issued KFU_LB at a time; then dZ_mq = -(z_mq colsum_m - Lx_mq) / l_q, and
-// colsum_m, Ld2_mq go to `red` (M x (Q + 1)) for pass 3.
-constexpr int KFU_LB = 16;
-__global__ __launch_bounds__(256) void kfu_bwd_final(int nblk, int M, int Q, const double *__restrict__ part,
-                                                     const double *__restrict__ z,
-                                                     const double *__restrict__ ls, double *__restrict__ dZ,
-                                                     double *__restrict__ red) {
-  __shared__ double sm[256];
-  const int W = 2 * Q + 1, mb = 256 / W, m0 = blockIdx.x * mb, tid = threadIdx.x;
-  const int ncol = min(mb, M - m0) * W;
-  const long bs = (long)M * W;
-  if (tid < ncol) {
-    const double *P = part + (long)m0 * W + tid;
-    double s = 0.0;
-    for (int b0 = 0; b0 < nblk; b0 += KFU_LB) {
-      double v[KFU_LB];
+// dx_nq = sum_m L_nm (z_mq - x_nq) / l_q, one wave per row, its lanes over m.
+__global__ __launch_bounds__(256) void kfu_dx_kernel(int N, int M, int Q, const double *__restrict__ dK,
+                                                     const double *__restrict__ K, const double *__restrict__ x,
+                                                     const double *__restrict__ z, const double *__restrict__ ls,
+                                                     double *__restrict__ dx) {
+  const int lane = threadIdx.x & 63;
+  const long n = blockIdx.x * 4L + (threadIdx.x >> 6);
+  if (n >= N) return;  // whole wave, no barriers
+  double L[4];
 #pragma unroll
-      for (int u = 0; u < KFU_LB; ++u) v[u] = b0 + u < nblk ? P[(b0 + u) * bs] : 0.0;
-#pragma unroll
-      for (int u = 0; u < KFU_LB; ++u)
-        if (b0 + u < nblk) s += v[u];
-    }
-    sm[tid] = s;
+  for (int j = 0; j < 4; ++j) {
+    const int m = min(lane + 64 * j, M - 1);
+    L[j] = dK[n * M + m] * K[n * M + m] * (lane + 64 * j < M ? 1.0 : 0.0);
   }
+  for (int q = 0; q < Q; ++q) {
+    const double xv = x[n * Q + q];
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s = fma(L[j], z[min(lane + 64 * j, M - 1) * Q + q] - xv, s);
+    s = gpx_wave_sum(s);
+    if (lane == 0) dx[n * Q + q] = s / exp(2.0 * ls[q]);
+  }
+}
+
+// Pass 2: red[w][m] = sum over the blocks of part[b][w][m]: 64 columns by 16 groups of blocks
+// (loads eight at a time), the groups added in order.
+__global__ __launch_bounds__(1024) void kfu_bwd_final(int nblk, int M, int W, const double *__restrict__ part,
+                                                      double *__restrict__ red) {
+  __shared__ double sm[16][64];
+  const int c = threadIdx.x & 63, g = threadIdx.x >> 6, m = blockIdx.x * 64 + c, w = blockIdx.y;
+  const double *P = part + (long)w * M + min(m, M - 1);
+  const long bs = (long)W * M;
+  double s = 0.0;
+#pragma unroll 8
+  for (int b = g; b < nblk; b += 16) s += P[b * bs];
+  sm[g][c] = s;
   __syncthreads();
-  for (int e = tid; e < min(mb, M - m0) * Q; e += 256) {
-    const int ml = e / Q, q = e % Q, m = m0 + ml;
-    dZ[m * Q + q] = -(z[m * Q + q] * sm[ml * W] - sm[ml * W + 1 + q]) / exp(2.0 * ls[q]);
-    red[m * (Q + 1) + 1 + q] = sm[ml * W + 1 + Q + q];
+  if (g == 0 && m < M) {
+    double t = sm[0][c];
+#pragma unroll
+    for (int h = 1; h < 16; ++h) t += sm[h][c];
+    red[(long)w * M + m] = t;
   }
-  if (tid < min(mb, M - m0)) red[(m0 + tid) * (Q + 1)] = sm[tid * W];
 }
 
-// pass 3, one wave per output j <= Q, lanes over m and a fixed-order wave reduction:
-// dsf2 = sum_m colsum_m / sf2, dell_q = sum_m Ld2_mq / ell^3.
+// Pass 3, one wave per output j <= Q, lanes over m and a fixed-order wave reduction:
+// dsf2 = sum_m colsum_m / sf2, dell_q = sum_m Ld2_mq / ell^3, and
+// dZ_mq = -(z_mq colsum_m - Lx_mq) / l_q.
 __global__ __launch_bounds__(64) void kfu_bwd_scalars(int M, int Q, const double *__restrict__ red,
+                                                      const double *__restrict__ z,
                                                       const double *__restrict__ ls,
                                                       const double *__restrict__ sf, double *__restrict__ dsf2,
-                                                      double *__restrict__ dell) {
+                                                      double *__restrict__ dell, double *__restrict__ dZ) {
   const int j = blockIdx.x, lane = threadIdx.x;
+  const double l = j ? exp(2.0 * ls[j - 1]) : 1.0;
   double s = 0.0;
-  for (int m = lane; m < M; m += 64) s += red[m * (Q + 1) + j];
+  for (int m = lane; m < M; m += 64) {
+    const double cs = red[m];
+    s += j == 0 ? cs : red[(long)(Q + j) * M + m];
+    if (j) dZ[m * Q + j - 1] = -(z[m * Q + j - 1] * cs - red[(long)j * M + m]) / l;
+  }
   s = gpx_wave_sum(s);
   if (lane == 0) {
     if (j == 0)
@@ -761,20 +822,27 @@ struct KuuLayers {
 };
 __global__ __launch_bounds__(256) void kuu_batched_kernel(int nl, KuuLayers L, int M, double jitter,
                                                           double *__restrict__ K) {
+  __shared__ double il[16], s2;
   const long MM = (long)M * M;
-  const long e = blockIdx.x * 256L + threadIdx.x;
-  if (e >= nl * MM) return;
-  const int l = (int)(e / MM), n = (int)((e % MM) / M), m = (int)(e % M);
+  const int l = blockIdx.y, Q = L.Q[l];
   const double *z = L.z[l], *ls = L.ls[l];
-  const int Q = L.Q[l];
+  if (threadIdx.x < 16) il[threadIdx.x] = (int)threadIdx.x < Q ? exp(-2.0 * ls[threadIdx.x]) : 0.0;
+  if (threadIdx.x == 255) s2 = exp(2.0 * L.sf[l][0]);
+  __syncthreads();
+  const long e = blockIdx.x * 256L + threadIdx.x;
+  if (e >= MM) return;
+  const int n = (int)(e / M), m = (int)(e % M);
   double r2 = 0.0;
   for (int q = 0; q < Q; ++q) {
     const double d = z[n * Q + q] - z[m * Q + q];
-    r2 += d * d / exp(2.0 * ls[q]);
+    if (Q <= 16)
+      r2 = fma(d * il[q], d, r2);  // the operations of se_kernel
+    else
+      r2 += d * d / exp(2.0 * ls[q]);  // those of se_any_kernel
   }
-  double k = exp(2.0 * L.sf[l][0]) * exp(-0.5 * r2);
+  double k = s2 * exp(-0.5 * r2);
   if (n == m) k += jitter;
-  K[e] = k;
+  K[l * MM + e] = k;
 }
 
 // Posterior and cavity precisions of several layers of one M from X = R^T R (the
@@ -810,15 +878,29 @@ int gpx_se_kernel(int N, int M, int Q, const double *x, int ldx, const double *z
   if (N < 0 || M < 0 || Q < 1 || ldx < Q) return GPX_EINVAL;
   if (N == 0 || M == 0) return GPX_OK;
   if (!x || !z || !ls || !sf || !K) return GPX_EINVAL;
-  hipLaunchKernelGGL(se_kernel, dim3(gpx_cdiv((long)N * M, 256)), dim3(256), 0, (hipStream_t)stream, N,
-                     M, Q, x, ldx, z, ls, sf, jitter, K);
+  hipStream_t st = (hipStream_t)stream;
+  if (Q > 16 || M > 64 * 65535) {
+    hipLaunchKernelGGL(se_any_kernel, dim3(gpx_cdiv((long)N * M, 256)), dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf,
+                       jitter, K);
+  } else {
+    const dim3 grid(gpx_cdiv(N, SE_ROWS), gpx_cdiv(M, 64));
+    if (Q <= 4)
+      hipLaunchKernelGGL(se_kernel<4>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+    else if (Q <= 8)
+      hipLaunchKernelGGL(se_kernel<8>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+    else
+      hipLaunchKernelGGL(se_kernel<16>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+  }
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }
 
-long gpx_kfu_bwd_workspace(int N, int M, int Q) {
-  return (long)gpx_cdiv(N, KFU_NB) * M * (2 * Q + 1) + (long)M * (Q + 1);
-}
+// Columns of the adjoint's thread layout, and its number of blocks: at least eight rows a
+// thread, at most two blocks per CU (their partials are read again by pass 2).
+static int kfu_cols(int M) { return M <= 64 ? 64 : (M <= 128 ? 128 : 256); }
+static int kfu_blocks(int N, int M) { return (int)std::min<long>(512, gpx_cdiv(N, 8L * (256 / kfu_cols(M)))); }
+
+long gpx_kfu_bwd_workspace(int N, int M, int Q) { return ((long)kfu_blocks(N, M) + 1) * M * (2 * Q + 1); }
 
 // Adjoint of K(x, Z): dsf2 (w.r.t. sf2), dell (w.r.t. ell), dZ (M x Q), dx (N x Q, optional).
 int gpx_kfu_bwd(int N, int M, int Q, const double *dK, const double *K, const double *x,
@@ -827,14 +909,25 @@ int gpx_kfu_bwd(int N, int M, int Q, const double *dK, const double *K, const do
   if (N < 1 || M < 1 || M > 256 || Q < 1 || Q > 16) return GPX_EINVAL;
   if (!dK || !K || !x || !z || !ls || !sf || !dsf2 || !dell || !dZ || !work) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  const unsigned nblk = gpx_cdiv(N, KFU_NB);
-  double *red = work + (long)nblk * M * (2 * Q + 1);
-  hipLaunchKernelGGL(kfu_bwd_partial, dim3(nblk), dim3(256), 0, st, N, M, Q, dK, K, x, z, ls, work, dx);
+  const int nblk = kfu_blocks(N, M), MP = kfu_cols(M), W = 2 * Q + 1;
+  double *red = work + (long)nblk * M * W;
+  if (Q <= 4)
+    hipLaunchKernelGGL(kfu_bwd_partial<4>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
+  else if (Q <= 8)
+    hipLaunchKernelGGL(kfu_bwd_partial<8>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
+  else if (Q <= 12)
+    hipLaunchKernelGGL(kfu_bwd_partial<12>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
+  else
+    hipLaunchKernelGGL(kfu_bwd_partial<16>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
   GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(kfu_bwd_final, dim3(gpx_cdiv(M, 256 / (2 * Q + 1))), dim3(256), 0, st, (int)nblk, M, Q,
-                     (const double *)work, z, ls, dZ, red);
+  if (dx) {
+    hipLaunchKernelGGL(kfu_dx_kernel, dim3(gpx_cdiv(N, 4)), dim3(256), 0, st, N, M, Q, dK, K, x, z, ls, dx);
+    GPX_CHECK_LAUNCH();
+  }
+  hipLaunchKernelGGL(kfu_bwd_final, dim3(gpx_cdiv(M, 64), W), dim3(1024), 0, st, nblk, M, W, (const double *)work, red);
   GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(kfu_bwd_scalars, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)red, ls, sf, dsf2, dell);
+  hipLaunchKernelGGL(kfu_bwd_scalars, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)red, z, ls, sf, dsf2, dell,
+                     dZ);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }
@@ -927,7 +1020,7 @@ int gpx_kuu_batched(int nl, int M, const double *const *z, const int *Q, const d
     L.sf[l] = sf[l];
     L.Q[l] = Q[l];
   }
-  hipLaunchKernelGGL(kuu_batched_kernel, dim3(gpx_cdiv((long)nl * M * M, 256)), dim3(256), 0, (hipStream_t)stream, nl,
+  hipLaunchKernelGGL(kuu_batched_kernel, dim3(gpx_cdiv((long)M * M, 256), nl), dim3(256), 0, (hipStream_t)stream, nl,
                      L, M, jitter, K);
   GPX_CHECK_LAUNCH();
   return GPX_OK;

@@ -1,0 +1,47 @@
+"""The SE kernel matrix and its adjoint at the edges of their thread layouts (GPU only): columns
+per block (64, 128, 256), row batches of four, register widths (Q = 4, 8, 12, 16) and the
+general path beyond 16 inputs.
+
+Tolerance: r^2/2 of magnitude E < 200 carries an absolute error of a few E eps into the
+exponential (< 2e-13 relative); the adjoint's sums of up to 20000 terms of mixed sign lose at
+most two digits more: 1e-11 normwise.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _nrel(a, b):
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+@pytest.mark.parametrize('N,M,Q', [(1, 1, 1), (15, 63, 4), (16, 64, 5), (17, 65, 8), (100, 128, 9), (33, 129, 12),
+                                   (64, 256, 13), (2049, 200, 16), (20001, 40, 3), (5, 70, 17), (40, 9, 30)])
+def test_se_and_adjoint(N, M, Q):
+    from geepee_amd import dops
+    print('se', N, M, Q, flush=True)
+    rs = np.random.RandomState(N + M + Q)
+    x, z, ls, sf = rs.randn(N, Q), rs.randn(M, Q), 0.2 * rs.randn(Q) + 0.5, np.array([0.3])
+    G = rs.randn(N, M)
+    t = [torch.as_tensor(a, device='cuda') for a in (x, z, ls, sf, G)]
+    il = np.exp(-2 * ls)
+    K = np.exp(2 * sf[0] - 0.5 * (((x * np.sqrt(il)) ** 2).sum(1)[:, None] + ((z * np.sqrt(il)) ** 2).sum(1)[None]
+                                  - 2 * (x * il).dot(z.T)))
+    got = dops.se(t[0], t[1], t[2], t[3])
+    assert _nrel(got.cpu().numpy(), K) < 1e-11
+    if N == 1 or M < 2:
+        return
+    Kzz = dops.se(t[1], t[1], t[2], t[3], jitter=0.25).cpu().numpy()
+    assert np.array_equal(Kzz, Kzz.T) and np.allclose(np.diag(Kzz), np.exp(2 * sf[0]) + 0.25, rtol=1e-14)
+    if Q > 16:
+        return
+    L = G * K
+    dsf2, dell, dz, dx = dops.kfu_bwd(t[4], got, t[0], t[1], t[2], t[3], want_dx=True)
+    cs = L.sum(0)
+    assert abs(float(dsf2) - L.sum() / np.exp(2 * sf[0])) < 1e-11 * np.abs(L).sum() / np.exp(2 * sf[0])
+    wl = np.array([(L * (z[None, :, q] - x[:, q:q + 1]) ** 2).sum() for q in range(Q)]) * np.exp(-3 * ls)
+    assert _nrel(dell.cpu().numpy(), wl) < 1e-10
+    assert _nrel(dz.cpu().numpy(), -(z * cs[:, None] - L.T.dot(x)) * il) < 1e-11
+    assert _nrel(dx.cpu().numpy(), (L.dot(z) - x * L.sum(1)[:, None]) * il) < 1e-11
