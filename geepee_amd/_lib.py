@@ -63,6 +63,8 @@ SIGNATURES = {
     'gpx_lvm_vfe_x_grads': (_i, [_i, _i, _p, _p, _p, _p, _p, _d, _d, _i, _d, _p, _p, _p, _p]),
     'gpx_ssm_vfe_x_grads': (_i, [_i, _i, _i, _i, _p, _p, _d, _d, _p, _p, _i, _p, _p, _p, _p, _i, _d,
                                  _p, _p, _p, _p]),
+    'gpx_gram_workspace': (_l, [_i, _i, _i]),
+    'gpx_gram': (_i, [_i, _i, _i, _p, _p, _i, _d, _p, _l, _p, _i, _p, _p]),
     'gpx_rowscale': (_i, [_i, _i, _i, _p, _p, _p, _p]),
     'gpx_wsum': (_i, [_i, _i, _i, _d, _p, _p, _d, _p, _p]),
     'gpx_dmall': (_i, [_l, _p, _p, _p, _p, _p]),

@@ -9,7 +9,7 @@ sums), so any of them meets the same tolerance.
 Knobs
   fused forward   nsub (16*nsub points per workgroup), splits_f (pair-tile splits)
   fused backward  nsplit (point ranges)
-  gemm            tile (32 or 64 rows/cols per workgroup), split-K factor
+  gemm            tile (32 or 64 rows/cols per wave, 0 = by size), split-K factor
 
 Cache: ``$GEEPEE_AMD_TUNE_CACHE`` if set, else ``~/.cache/geepee_amd/tune.json``.
 ``lookup`` is consulted by dops.fused_plan and dops.mm before their heuristics.
@@ -168,10 +168,9 @@ def tune_fused(N, M, Q, D, reps=5, seed=0, save=True, verbose=False):
 
 
 def gemm_candidates(m, n, k, batch):
-    tiles = [32, 64]
     out = []
-    for tile in tiles:
-        nt = -(-m // tile) * -(-n // tile) * batch
+    for tile in (0, 32, 64):
+        nt = -(-m // (tile or 32)) * -(-n // (tile or 32)) * batch
         for s in _pow2_upto(1, 64):
             if s > 1 and (k // s < 64 or nt * s > 4096):
                 continue

@@ -10,8 +10,6 @@
 
 namespace {
 
-constexpr int BK = 32;
-
 // Output epilogue: C = v + beta C + gamma E (beta == 0 never reads C; E may be NULL; an
 // E stride of 0 broadcasts one matrix over the batch).
 struct GemmEpi {
@@ -26,150 +24,6 @@ __device__ __forceinline__ void epi_store(double *c, double v, const GemmEpi &ep
   if (ep.beta != 0.0) r += ep.beta * *c;
   if (ep.E) r += ep.gamma * ep.E[b * ep.sE + (long)i * ep.ldE + j];
   *c = r;
-}
-
-// Stage one BK-slice of op(A) (BM x BK) and op(B) (BK x BN) into registers.
-template <int BM, int BN>
-__device__ __forceinline__ void gemm_load(double *ra, double *rb, const double *__restrict__ A,
-                                          const double *__restrict__ B, int tA, int tB, int lda, int ldb,
-                                          int m, int n, int m0, int n0, int k0, int kend) {
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int u = 0; u < LA; ++u) {
-    const int e = tid + 256 * u;
-    int mm, kk;
-    if (tA) { kk = e / BM; mm = e % BM; } else { mm = e / BK; kk = e % BK; }
-    const int gm = m0 + mm, gk = k0 + kk;
-    ra[u] = (gm < m && gk < kend) ? (tA ? A[(long)gk * lda + gm] : A[(long)gm * lda + gk]) : 0.0;
-  }
-#pragma unroll
-  for (int u = 0; u < LB; ++u) {
-    const int e = tid + 256 * u;
-    int nn, kk;
-    if (tB) { nn = e / BK; kk = e % BK; } else { kk = e / BN; nn = e % BN; }
-    const int gn = n0 + nn, gk = k0 + kk;
-    rb[u] = (gn < n && gk < kend) ? (tB ? B[(long)gn * ldb + gk] : B[(long)gk * ldb + gn]) : 0.0;
-  }
-}
-
-template <int BM, int BN>
-__device__ __forceinline__ void gemm_store(const double *ra, const double *rb, double (*As)[BM + 1],
-                                           double (*Bs)[BN + 1], int tA, int tB) {
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int u = 0; u < LA; ++u) {
-    const int e = tid + 256 * u;
-    int mm, kk;
-    if (tA) { kk = e / BM; mm = e % BM; } else { mm = e / BK; kk = e % BK; }
-    As[kk][mm] = ra[u];
-  }
-#pragma unroll
-  for (int u = 0; u < LB; ++u) {
-    const int e = tid + 256 * u;
-    int nn, kk;
-    if (tB) { nn = e / BK; kk = e % BK; } else { kk = e / BN; nn = e % BN; }
-    Bs[kk][nn] = rb[u];
-  }
-}
-
-// Block -> (column tile, row tile, z) of a batched product (z = batch element, or batch
-// element and split).  With xcd the launch is 1-D and all the tiles of one z run on one
-// XCD: blocks are dealt to the eight XCDs round-robin by id, so block p runs on XCD p % 8;
-// z takes XCD z % 8 and its tiles are the blocks p = 8 (tpz (z / 8) + t) + z % 8.  The
-// operand panels that a z's tiles re-read then stay in that XCD's L2.
-struct TileIdx {
-  int x, y, z;
-};
-__device__ __forceinline__ TileIdx gemm_tile(int xcd, int tx, int ty) {
-  if (!xcd) return {(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
-  const int tpz = tx * ty, p = blockIdx.x, j = p >> 3;
-  const int t = j % tpz;
-  return {t % tx, t / tx, (p & 7) + 8 * (j / tpz)};
-}
-
-// 4 waves as 2x2; each wave owns (BM/2) x (BN/2) of 16x16 MFMA tiles.  K advances in
-// slices of BK through two LDS buffers; the next slice is fetched from global memory into
-// registers while the current one feeds the matrix cores (one barrier per slice).
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void gemm_kernel(
-    int m, int n, int k, int tA, int tB, double alpha,
-    const double *__restrict__ A, int lda, long sA,
-    const double *__restrict__ B, int ldb, long sB,
-    GemmEpi ep, double *__restrict__ C, int ldc, long sC,
-    int batch, int splits, int kchunk, double *__restrict__ part, int xcd) {
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  constexpr int LA = BM * BK / 256, LB = BN * BK / 256;
-  __shared__ double As[2][BK][BM + 1];
-  __shared__ double Bs[2][BK][BN + 1];
-  const TileIdx ti = gemm_tile(xcd, (n + BN - 1) / BN, (m + BM - 1) / BM);
-  const int z = ti.z;
-  const int bidx = z / splits, sidx = z % splits;
-  if (bidx >= batch) return;
-  A += bidx * sA;
-  B += bidx * sB;
-  const int m0 = ti.y * BM, n0 = ti.x * BN;
-  const int kbeg = sidx * kchunk, kend = min(k, kbeg + kchunk);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  gpx_d4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
-  double ra[LA], rb[LB];
-  int cur = 0;
-  if (kbeg < kend) {
-    gemm_load<BM, BN>(ra, rb, A, B, tA, tB, lda, ldb, m, n, m0, n0, kbeg, kend);
-    gemm_store<BM, BN>(ra, rb, As[0], Bs[0], tA, tB);
-  }
-  __syncthreads();
-  for (int k0 = kbeg; k0 < kend; k0 += BK) {
-    const bool more = k0 + BK < kend;
-    if (more) gemm_load<BM, BN>(ra, rb, A, B, tA, tB, lda, ldb, m, n, m0, n0, k0 + BK, kend);
-#pragma unroll
-    for (int kq = 0; kq < BK; kq += 4) {
-      double a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = As[cur][kq + (lane >> 4)][wm * WM + i * 16 + (lane & 15)];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) b[j] = Bs[cur][kq + (lane >> 4)][wn * WN + j * 16 + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = gpx_mfma16(a[i], b[j], acc[i][j]);
-    }
-    if (more) gemm_store<BM, BN>(ra, rb, As[cur ^ 1], Bs[cur ^ 1], tA, tB);
-    __syncthreads();
-    cur ^= 1;
-  }
-
-  if (part) {
-    double *P = part + ((long)sidx * batch + bidx) * (long)m * n;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gm = m0 + wm * WM + i * 16 + (lane >> 4) + 4 * r;
-          const int gn = n0 + wn * WN + j * 16 + (lane & 15);
-          if (gm < m && gn < n) P[(long)gm * n + gn] = acc[i][j][r];
-        }
-    return;
-  }
-  C += bidx * sC;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gm = m0 + wm * WM + i * 16 + (lane >> 4) + 4 * r;
-        const int gn = n0 + wn * WN + j * 16 + (lane & 15);
-        if (gm < m && gn < n) epi_store(C + (long)gm * ldc + gn, alpha * acc[i][j][r], ep, bidx, gm, gn);
-      }
 }
 
 // Sum of the split-K partials part[q][b][i][j] (q < splits) and the epilogue.  A workgroup
@@ -200,76 +54,6 @@ __global__ __launch_bounds__(256) void splitk_reduce(int m, int n, int batch, in
     const long r = e % mn;
     const int i = (int)(r / n), j = (int)(r % n);
     epi_store(C + b * sC + (long)i * ldc + j, alpha * t, ep, b, i, j);
-  }
-}
-
-// Short contractions (k <= FULLK_MAX): every operand element of the block's 32-row
-// panel of op(A) and 32-column panel of op(B) is fetched in one round into LDS (one
-// memory latency instead of one per K slice), then the 2x2 waves run their MFMAs over
-// the whole K.  Same output layout and epilogue as gemm_kernel; no split-K.
-constexpr int FULLK_MAX = 128;
-
-__global__ __launch_bounds__(256) void gemm_fullk_kernel(
-    int m, int n, int k, int tA, int tB, double alpha,
-    const double *__restrict__ A, int lda, long sA,
-    const double *__restrict__ B, int ldb, long sB,
-    GemmEpi ep, double *__restrict__ C, int ldc, long sC, int batch, int xcd) {
-  __shared__ double As[FULLK_MAX][33];
-  __shared__ double Bs[FULLK_MAX][33];
-  const TileIdx ti = gemm_tile(xcd, (n + 31) / 32, (m + 31) / 32);
-  const int bidx = ti.z;
-  if (bidx >= batch) return;
-  A += bidx * sA;
-  B += bidx * sB;
-  const int m0 = ti.y * 32, n0 = ti.x * 32;
-  const int kp = (k + 3) & ~3;
-  const int tid = threadIdx.x;
-  // all loads first (16 + 16 per thread in flight), then the LDS stores.  Thread t covers
-  // k = k0 + 8j of one row / column (shifts only, no division), reading along the
-  // operand's contiguous dimension.
-  constexpr int U = FULLK_MAX / 8;
-  double ra[U], rb[U];
-  // op(A)[mm][kk]: A stored (m x k) reads 8 consecutive k of a row; A^T stored (k x m)
-  // reads 32 consecutive m of a k-row
-  const int am = tA ? (tid & 31) : (tid >> 3), ak = tA ? (tid >> 5) : (tid & 7);
-  const int bn = tB ? (tid >> 3) : (tid & 31), bk = tB ? (tid & 7) : (tid >> 5);
-  const int gam = m0 + am, gbn = n0 + bn;
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int kka = ak + 8 * u, kkb = bk + 8 * u;
-    ra[u] = (gam < m && kka < k) ? (tA ? A[(long)kka * lda + gam] : A[(long)gam * lda + kka]) : 0.0;
-    rb[u] = (gbn < n && kkb < k) ? (tB ? B[(long)gbn * ldb + kkb] : B[(long)kkb * ldb + gbn]) : 0.0;
-  }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int kka = ak + 8 * u, kkb = bk + 8 * u;
-    if (kka < kp) As[kka][am] = ra[u];
-    if (kkb < kp) Bs[kkb][bn] = rb[u];
-  }
-  __syncthreads();
-  const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-  gpx_d4 acc = gpx_d4{0.0, 0.0, 0.0, 0.0};
-  // eight 4-wide slices at a time: their LDS reads issue ahead of the MFMAs, which then
-  // run back to back on one accumulator (same order as one slice at a time)
-  const int ar = wm * 16 + (lane & 15), bc = wn * 16 + (lane & 15), g = lane >> 4;
-  int kq = 0;
-  for (; kq + 32 <= kp; kq += 32) {
-    double a[8], b[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      a[u] = As[kq + 4 * u + g][ar];
-      b[u] = Bs[kq + 4 * u + g][bc];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc = gpx_mfma16(a[u], b[u], acc);
-  }
-  for (; kq < kp; kq += 4) acc = gpx_mfma16(As[kq + g][ar], Bs[kq + g][bc], acc);
-  C += bidx * sC;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int gm = m0 + wm * 16 + (lane >> 4) + 4 * r;
-    const int gn = n0 + wn * 16 + (lane & 15);
-    if (gm < m && gn < n) epi_store(C + (long)gm * ldc + gn, alpha * acc[r], ep, bidx, gm, gn);
   }
 }
 
@@ -306,9 +90,417 @@ __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB,
   if (lane == 0) epi_store(C + b * sC + (long)i * ldc, alpha * s, ep, b, i, 0);
 }
 
+// ---------------------------------------------------------------------------
+// Register-direct products.  One wave owns a (16 TM) x (16 TN) tile of C and feeds the matrix
+// cores straight from global memory: no LDS staging, no barriers, every wave at its own pace.
+// K advances in groups of 8; of a group, lane group g = lane / 16 supplies k = 2 g + s to MFMA
+// step s = 0, 1 (the same permutation of k in both operands), so an operand whose rows run
+// along k is read as one 16-byte load per lane and one whose rows run across k as 128-byte row
+// segments.  The next group is in flight while the current one is multiplied.  Rows and columns
+// past the edge re-read the last valid one (their results are not stored); a last partial group
+// is masked to zero in both operands.  Large products are bound by the matrix cores, small ones
+// by one launch and one round of loads.  Against tiles staged through LDS (64 x 64 or 32 x 32
+// per workgroup), us: 20000 x 200 x 200, 4 products 245 -> 125 (26 -> 51 TF); 4001 x 256 x 256, 2
+// 34 -> 29; 10000 x 6 x 1000 55 -> 17; 256^3, 2 9.6 -> 6.0; 100^3, 5 6.3 -> 4.3; 50^3 5.3 -> 4.1.
+// ---------------------------------------------------------------------------
+typedef double gemm_d2 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int T>
+struct GemmFrag {
+  double v[2][T];
+};
+
+// Operand view of one wave: `p` is uniform (tile origin), `off[i]` the lane's offset in tile i.
+// KC: k is the contiguous dimension (row stride ld); otherwise k-rows of stride ld.
+template <int T, bool KC>
+struct GemmOp {
+  const double *p;
+  long off[T];
+  int ld;
+  __device__ __forceinline__ GemmOp(const double *base, int ld_, int r0, int rows, int lane) : ld(ld_) {
+    const int g = lane >> 4, last = rows - r0 - 1;
+    p = KC ? base + (long)r0 * ld : base + r0;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      const int r = min(16 * i + (lane & 15), last);
+      off[i] = KC ? (long)r * ld + 2 * g : 2L * g * ld + r;
+    }
+  }
+  __device__ __forceinline__ void load(GemmFrag<T> &f, int k0) const {
+    const double *q = p + (KC ? (long)k0 : (long)k0 * ld);
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+      if constexpr (KC) {
+        const gemm_d2 t = *(const gemm_d2 *)(q + off[i]);
+        f.v[0][i] = t.x;
+        f.v[1][i] = t.y;
+      } else {
+        f.v[0][i] = q[off[i]];
+        f.v[1][i] = (q + ld)[off[i]];
+      }
+    }
+  }
+  // the `kr` (1..7) valid k of a last group; lanes past them re-read the group's first
+  __device__ __forceinline__ void load_tail(GemmFrag<T> &f, int k0, int kr, int lane) const {
+    const double *q = p + (KC ? (long)k0 : (long)k0 * ld);
+    const int g = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bool on = 2 * g + s < kr;
+      const long back = on ? s : -2 * g;
+#pragma unroll
+      for (int i = 0; i < T; ++i) {
+        f.v[s][i] = 0.0;
+        if constexpr (T > 2) {  // no registers for the clamped addresses
+          if (on) f.v[s][i] = q[off[i] + (KC ? s : (long)s * ld)];
+        } else {
+          const double t = q[off[i] + (KC ? back : back * ld)];
+          if (on) f.v[s][i] = t;
+        }
+      }
+    }
+  }
+};
+
+template <int TM, int TN, bool TA, bool TB, int KW>
+__device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int kend, double alpha, const double *A,
+                                                 int lda, const double *B, int ldb, const GemmEpi &ep, double *C,
+                                                 int ldc, int m0, int n0, int bidx, bool raw, double *red) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const GemmOp<TM, !TA> oa(A, lda, m0, m, lane);
+  const GemmOp<TN, TB> ob(B, ldb, n0, n, lane);
+  gpx_d4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+  auto mul = [&](const GemmFrag<TM> &fa, const GemmFrag<TN> &fb) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = gpx_mfma16(fa.v[s][i], fb.v[s][j], acc[i][j]);
+  };
+  const int kw = KW > 1 ? wave : 0;
+  const int groups = (kend - kbeg) >> 3, mine = (groups - kw + KW - 1) / KW;  // group kw + KW t of this wave
+  const int kr = (kend - kbeg) & 7;
+  const bool tail = kr && kw == groups % KW;
+  constexpr bool EARLY = TM <= 2;  // registers to hold the tail from the start
+  GemmFrag<EARLY ? TM : 1> ta;
+  GemmFrag<EARLY ? TN : 1> tb;
+  if constexpr (EARLY)
+    if (tail) {
+      oa.load_tail(ta, kbeg + 8 * groups, kr, lane);
+      ob.load_tail(tb, kbeg + 8 * groups, kr, lane);
+    }
+  if (mine > 0) {
+    constexpr int P = TM == 1 ? 4 : 2;  // groups in flight
+    GemmFrag<TM> fa[P];
+    GemmFrag<TN> fb[P];
+    auto load = [&](int u, int t) {
+      const int k0 = kbeg + 8 * (kw + KW * min(t, mine - 1));
+      oa.load(fa[u], k0);
+      ob.load(fb[u], k0);
+    };
+#pragma unroll
+    for (int u = 0; u < P - 1; ++u) load(u, u);
+    int t = 0;
+    for (; t + P <= mine; t += P)
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        load((u + P - 1) % P, t + u + P - 1);
+        mul(fa[u], fb[u]);
+      }
+#pragma unroll
+    for (int u = 0; u < P - 1; ++u)
+      if (t + u < mine) mul(fa[u], fb[u]);
+  }
+  if (tail) {
+    if constexpr (EARLY) {
+      mul(ta, tb);
+    } else {
+      GemmFrag<TM> fa;
+      GemmFrag<TN> fb;
+      oa.load_tail(fa, kbeg + 8 * groups, kr, lane);
+      ob.load_tail(fb, kbeg + 8 * groups, kr, lane);
+      mul(fa, fb);
+    }
+  }
+  if constexpr (KW > 1) {
+    // the waves' partial tiles, one row of 16 x 16 tiles at a time: wave r adds accumulator
+    // register r (rows g + 4 r of each tile) of all four in wave order, and stores it
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (i) __syncthreads();
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[((wave * TN + j) * 4 + r) * 64 + lane] = acc[i][j][r];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int gm = m0 + i * 16 + (lane >> 4) + 4 * wave, gn = n0 + j * 16 + (lane & 15);
+        double v = red[(j * 4 + wave) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < KW; ++w) v += red[((w * TN + j) * 4 + wave) * 64 + lane];
+        if (gm < m && gn < n) {
+          double *c = C + (long)gm * ldc + gn;
+          if (raw) *c = v;
+          else epi_store(c, alpha * v, ep, bidx, gm, gn);
+        }
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gm = m0 + i * 16 + (lane >> 4) + 4 * r, gn = n0 + j * 16 + (lane & 15);
+        if (gm < m && gn < n) {
+          double *c = C + (long)gm * ldc + gn;
+          if (raw) *c = acc[i][j][r];
+          else epi_store(c, alpha * acc[i][j][r], ep, bidx, gm, gn);
+        }
+      }
+}
+
+// Tiles are numbered column band fastest, then row band, then z = (batch, split).  KW = 1: the
+// four waves of a workgroup take four consecutive tiles; KW = 4: they share one tile, each with
+// every fourth group of K.  The n columns are cut into bands of ceil- or floor-balanced counts
+// of 16-column tiles (n = 200: 4 + 3 + 3 + 3), so padding is below 16 columns in all.
+// Workgroups are dealt to the XCDs in contiguous runs of tiles, which share operand panels.
+template <int TM, int TX, bool TA, bool TB, int KW>
+__global__ __launch_bounds__(256, 2) void gemm_direct_kernel(int m, int n, int k, double alpha, const double *__restrict__ A,
+                                                          int lda, long sA, const double *__restrict__ B, int ldb,
+                                                          long sB, GemmEpi ep, double *__restrict__ C, int ldc,
+                                                          long sC, int batch, int splits, int kchunk,
+                                                          double *__restrict__ part) {
+  __shared__ double red[KW > 1 ? KW * TX * 256 : 1];
+  const int nt = (n + 15) >> 4, cb = (nt + TX - 1) / TX, rb = (m + 16 * TM - 1) / (16 * TM);
+  const long tiles = (long)rb * cb * batch * splits;
+  const long chunk = gridDim.x >> 3, blk = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
+  long t = KW > 1 ? blk : blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t >= tiles) return;
+  const int c = (int)(t % cb);
+  t /= cb;
+  const int r = (int)(t % rb), z = (int)(t / rb);
+  const int b = z / splits, q = z % splits;
+  const int lo = nt / cb, hi = nt % cb;  // the first `hi` bands have lo + 1 tiles
+  const int tn = lo + (c < hi), n0 = 16 * (c * lo + min(c, hi)), m0 = 16 * TM * r;
+  const int kbeg = q * kchunk, kend = min(k, kbeg + kchunk);
+  A += b * sA;
+  B += b * sB;
+  const bool raw = part != nullptr;
+  double *Cb = raw ? part + ((long)q * batch + b) * (long)m * n : C + b * sC;
+  if (raw) ldc = n;
+#define GEMM_TILE(TN)                                                                                               \
+  gemm_direct_tile<TM, TN, TA, TB, KW>(m, n, kbeg, kend, alpha, A, lda, B, ldb, ep, Cb, ldc, m0, n0, b, raw, red)
+  if constexpr (TX >= 4) {
+    if (tn == 4) return GEMM_TILE(4);
+    if (tn == 3) return GEMM_TILE(3);
+  }
+  if constexpr (TX >= 2)
+    if (tn == 2) return GEMM_TILE(2);
+  GEMM_TILE(1);
+#undef GEMM_TILE
+}
+
+template <int TM, int KW>
+int gemm_direct(int tA, int tB, int m, int n, int k, double alpha, const double *A, int lda, long sA, const double *B,
+                int ldb, long sB, const GemmEpi &ep, double *C, int ldc, long sC, int batch, int splits, int kchunk,
+                double *part, hipStream_t st) {
+  const long cb = gpx_cdiv(gpx_cdiv(n, 16), TM), rb = gpx_cdiv(m, 16 * TM), tiles = rb * cb * batch * splits;
+  const long blocks = KW > 1 ? tiles : (tiles + 3) / 4;
+  const dim3 grid(8 * gpx_cdiv(blocks, 8));
+#define GEMM_GO(TA, TB)                                                                                          \
+  hipLaunchKernelGGL((gemm_direct_kernel<TM, TM, TA, TB, KW>), grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sA, B, \
+                     ldb, sB, ep, C, ldc, sC, batch, splits, kchunk, part)
+  if (tA) {
+    if (tB) GEMM_GO(true, true); else GEMM_GO(true, false);
+  } else {
+    if (tB) GEMM_GO(false, true); else GEMM_GO(false, false);
+  }
+#undef GEMM_GO
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Weighted Gram matrices: out[d] = sum_n w_nd x_n x_n^T (+ gamma E[d]), symmetric, so only the
+// 16 x 16 tiles on and above the diagonal are formed: pairs (r <= c) of column bands of at most
+// four tiles (balanced, n = 200: 4 + 3 + 3 + 3), the weight applied to one operand's fragments
+// as they arrive.  A workgroup owns one (pair, d, share of the points); its four waves take every
+// fourth group of 8 points and are added in wave order.  Bound by the matrix cores (N = 20000,
+// M = 200, 4 outputs: 84 us of which 47 are its products; a scaled copy of x and a full product
+// took 45 + 317 us; N = 200, M = 50, 1 output 11 -> 9 us).
+// ---------------------------------------------------------------------------
+template <int TM, int TN, bool DIAG>
+__device__ __forceinline__ void gram_tile(int N, int D, int M, int kbeg, int kend, const double *w, const double *X,
+                                          int ldx, int m0, int n0, double *out, double *red) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
+  const GemmOp<TM, false> oa(X, ldx, m0, M, lane);
+  const GemmOp<TN, false> ob(X, ldx, n0, M, lane);
+  gpx_d4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+  auto mul = [&](const GemmFrag<TM> &fa, const GemmFrag<TN> &fb, const double *wv) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      double b[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = wv[s] * (DIAG ? fa.v[s][j] : fb.v[s][j]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = DIAG ? i : 0; j < TN; ++j) acc[i][j] = gpx_mfma16(fa.v[s][i], b[j], acc[i][j]);
+    }
+  };
+  const int groups = (kend - kbeg) >> 3, mine = (groups - wave + 3) / 4;
+  if (mine > 0) {
+    GemmFrag<TM> fa[2];
+    GemmFrag<TN> fb[2];
+    double wv[2][2];
+    auto load = [&](int u, int t) {
+      const int k0 = kbeg + 8 * (wave + 4 * min(t, mine - 1));
+      oa.load(fa[u], k0);
+      if constexpr (!DIAG) ob.load(fb[u], k0);
+      const double *wk = w + (long)k0 * D;
+      wv[u][0] = wk[2L * g * D];
+      wv[u][1] = wk[2L * g * D + D];
+    };
+    load(0, 0);
+    int t = 0;
+    for (; t + 2 <= mine; t += 2) {
+      load(1, t + 1);
+      mul(fa[0], fb[0], wv[0]);
+      load(0, t + 2);
+      mul(fa[1], fb[1], wv[1]);
+    }
+    if (t < mine) mul(fa[0], fb[0], wv[0]);
+  }
+  const int kr = (kend - kbeg) & 7;
+  if (kr && wave == groups % 4) {
+    const int k0 = kbeg + 8 * groups;
+    GemmFrag<TM> fa;
+    GemmFrag<TN> fb;
+    oa.load_tail(fa, k0, kr, lane);
+    ob.load_tail(fb, k0, kr, lane);
+    double wv[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) wv[s] = 2 * g + s < kr ? w[(long)(k0 + 2 * g + s) * D] : 0.0;
+    mul(fa, fb, wv);
+  }
+  // the waves' partial tiles, one row of 16 x 16 tiles at a time: wave r adds accumulator
+  // register r of all four in wave order, and stores it
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    if (i) __syncthreads();
+#pragma unroll
+    for (int j = DIAG ? i : 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[((wave * TN + j) * 4 + r) * 64 + lane] = acc[i][j][r];
+    __syncthreads();
+#pragma unroll
+    for (int j = DIAG ? i : 0; j < TN; ++j) {
+      const int gm = m0 + i * 16 + g + 4 * wave, gn = n0 + j * 16 + (lane & 15);
+      double v = red[(j * 4 + wave) * 64 + lane];
+#pragma unroll
+      for (int u = 1; u < 4; ++u) v += red[((u * TN + j) * 4 + wave) * 64 + lane];
+      if (gm < M && gn < M) out[(long)gm * M + gn] = v;
+    }
+  }
+}
+
+// Grid: (splits, pairs, D), largest pairs (lowest bands) first.
+__global__ __launch_bounds__(256, 2) void gram_kernel(int N, int D, int M, int kchunk, const double *__restrict__ w,
+                                                      const double *__restrict__ X, int ldx, double *__restrict__ part) {
+  __shared__ double red[16 * 256];
+  const int nt = (M + 15) >> 4, cb = (nt + 3) / 4, lo = nt / cb, hi = nt % cb, d = blockIdx.z;
+  int r = 0, c = blockIdx.y;
+  while (c >= cb - r) {  // pair index -> (r, r + c)
+    c -= cb - r;
+    ++r;
+  }
+  c += r;
+  const int tm = lo + (r < hi), tn = lo + (c < hi), m0 = 16 * (r * lo + min(r, hi)), n0 = 16 * (c * lo + min(c, hi));
+  const int kbeg = blockIdx.x * kchunk, kend = min(N, kbeg + kchunk);
+  double *out = part + ((long)blockIdx.x * D + d) * M * M;
+#define GRAM_TILE(TM, TN, DIAG) gram_tile<TM, TN, DIAG>(N, D, M, kbeg, kend, w + d, X, ldx, m0, n0, out, red)
+  if (r == c) {
+    if (tm == 4) GRAM_TILE(4, 4, true);
+    else if (tm == 3) GRAM_TILE(3, 3, true);
+    else if (tm == 2) GRAM_TILE(2, 2, true);
+    else GRAM_TILE(1, 1, true);
+  } else if (tm == 4) {
+    if (tn == 4) GRAM_TILE(4, 4, false); else GRAM_TILE(4, 3, false);
+  } else {  // two bands or more: at least 3 + 2 tiles
+    if (tn == 3) GRAM_TILE(3, 3, false); else GRAM_TILE(3, 2, false);
+  }
+#undef GRAM_TILE
+}
+
+// Sum of the partial Gram matrices over the splits (fixed order) for i <= j, stored at (i, j)
+// and (j, i); same thread layout as splitk_reduce.
+__global__ __launch_bounds__(256) void gram_reduce(int D, int M, int splits, const double *__restrict__ part,
+                                                   GemmEpi ep, double *__restrict__ out) {
+  __shared__ double red[8][SPLITK_OUT + 1];
+  const long mm = (long)M * M, total = mm * D;
+  const int o = threadIdx.x & (SPLITK_OUT - 1), g = threadIdx.x / SPLITK_OUT;
+  const long e = (long)blockIdx.x * SPLITK_OUT + o;
+  const int b = (int)(e / mm), r = (int)(e - b * mm), i = r / M, j = r - i * M;
+  const bool on = e < total && i <= j;
+  double s = 0.0;
+  if (on) {
+#pragma unroll 4
+    for (int q = g; q < splits; q += 8) s += part[(long)q * total + e];
+  }
+  red[g][o] = s;
+  __syncthreads();
+  if (g == 0 && on) {
+    double t = red[0][o];
+#pragma unroll
+    for (int h = 1; h < 8; ++h) t += red[h][o];
+    out += b * mm;
+    epi_store(out + (long)i * M + j, t, ep, b, i, j);
+    if (i != j) epi_store(out + (long)j * M + i, t, ep, b, j, i);
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+long gpx_gram_workspace(int D, int M, int splits) { return (long)splits * D * M * M; }
+
+int gpx_gram(int N, int D, int M, const double *w, const double *X, int ldx, double gamma, const double *E,
+             long strideE, double *out, int splits, double *work, void *stream) {
+  if (N < 0 || D < 0 || M < 0 || splits < 1 || D > 65535) return GPX_EINVAL;
+  if (E && strideE < 0) return GPX_EINVAL;
+  if (D == 0 || M == 0) return GPX_OK;
+  if (!out || (N > 0 && (!w || !X || !work || ldx < M))) return GPX_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  int kchunk = (N + splits - 1) / splits;
+  kchunk = (kchunk + 7) / 8 * 8;
+  splits = kchunk ? (N + kchunk - 1) / kchunk : 0;
+  const GemmEpi ep{0.0, gamma, E, M, strideE};
+  if (splits) {
+    const int cb = (int)gpx_cdiv(gpx_cdiv(M, 16), 4);
+    if ((long)cb * (cb + 1) / 2 > 65535) return GPX_ETOOBIG;
+    hipLaunchKernelGGL(gram_kernel, dim3(splits, cb * (cb + 1) / 2, D), dim3(256), 0, st, N, D, M, kchunk, w, X, ldx,
+                       work);
+    GPX_CHECK_LAUNCH();
+  }
+  hipLaunchKernelGGL(gram_reduce, dim3(gpx_cdiv((long)D * M * M, SPLITK_OUT)), dim3(256), 0, st, D, M, splits,
+                     (const double *)work, ep, out);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
 
 // Workspace (doubles) that gpx_gemm_batched needs for a given split count.
 long gpx_gemm_workspace(int m, int n, int batch, int splits) {
@@ -347,35 +539,29 @@ int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alph
     GPX_CHECK_LAUNCH();
     return GPX_OK;
   }
-  if (splits == 1 && k <= FULLK_MAX && tile != 64 &&
-      (tile == 32 || (long)gpx_cdiv(m, 64) * gpx_cdiv(n, 64) * batch < 256)) {
-    if (batch > 65535) return GPX_EINVAL;
-    const int xcd = batch >= 8;
-    const unsigned tpz = gpx_cdiv(n, 32) * gpx_cdiv(m, 32);
-    dim3 grid = xcd ? dim3(8 * gpx_cdiv(batch, 8) * tpz) : dim3(gpx_cdiv(n, 32), gpx_cdiv(m, 32), batch);
-    hipLaunchKernelGGL(gemm_fullk_kernel, grid, dim3(256), 0, st, m, n, k, transA, transB, alpha, A, lda, strideA,
-                       B, ldb, strideB, ep, C, ldc, strideC, batch, xcd);
-    GPX_CHECK_LAUNCH();
-    return GPX_OK;
-  }
   int kchunk = (k + splits - 1) / splits;
-  kchunk = ((kchunk + BK - 1) / BK) * BK;
+  kchunk = (kchunk + 7) / 8 * 8;
   splits = (k + kchunk - 1) / kchunk;
   double *part = splits > 1 ? work : nullptr;
   if ((long)batch * splits > 65535L) return GPX_EINVAL;
-  const int nz = batch * splits, xcd = nz >= 8;
-  if (tile == 32 || (tile == 0 && (long)gpx_cdiv(m, 64) * gpx_cdiv(n, 64) * batch * splits < 256)) {
-    const unsigned tpz = gpx_cdiv(n, 32) * gpx_cdiv(m, 32);
-    dim3 grid = xcd ? dim3(8 * gpx_cdiv(nz, 8) * tpz) : dim3(gpx_cdiv(n, 32), gpx_cdiv(m, 32), nz);
-    hipLaunchKernelGGL((gemm_kernel<32, 32>), grid, dim3(256), 0, st, m, n, k, transA, transB, alpha,
-                       A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch, splits, kchunk, part, xcd);
-  } else {
-    const unsigned tpz = gpx_cdiv(n, 64) * gpx_cdiv(m, 64);
-    dim3 grid = xcd ? dim3(8 * gpx_cdiv(nz, 8) * tpz) : dim3(gpx_cdiv(n, 64), gpx_cdiv(m, 64), nz);
-    hipLaunchKernelGGL((gemm_kernel<64, 64>), grid, dim3(256), 0, st, m, n, k, transA, transB, alpha,
-                       A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch, splits, kchunk, part, xcd);
-  }
-  GPX_CHECK_LAUNCH();
+  const long z = (long)batch * splits, t4 = z * gpx_cdiv(m, 64) * gpx_cdiv(n, 64),
+             t2 = z * gpx_cdiv(m, 32) * gpx_cdiv(n, 32), t1 = z * gpx_cdiv(m, 16) * gpx_cdiv(n, 16);
+  int rc;
+#define GEMM_DIRECT(TM, KW)                                                                                       \
+  gemm_direct<TM, KW>(transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch, \
+                      splits, kchunk, part, st)
+  // 64 x 64 per wave once there are two such tiles per SIMD (20000 x n x n, 4 products, us
+  // against 32 x 32: n = 256 172 : 228, 200 125 : 133, 128 (2504 tiles) 63 : 65; 5000 x 100 x 100, 4
+  // (632 tiles) 24 : 18).  16 x 16 per workgroup, its waves sharing k, where those are at most three
+  // per CU (against 32 x 32: 128^3 4.4 : 5.5, 200^3, 4 (676 tiles) 5.8 : 6.0, 128^3, 32 (2048) 13 : 7.8).
+  // Else 32 x 32, a tile per wave if that makes a wave per SIMD (4001 x 256 x 256 (1008) 17.4 : 18.3;
+  // 128^3, 32 (512) 10.5 : 8.8) or if k leaves four waves nothing to share.
+  if (tile == 64 || (tile != 32 && t4 >= 2048 && k >= 64)) rc = GEMM_DIRECT(4, 1);
+  else if (tile != 32 && t1 <= 768) rc = GEMM_DIRECT(1, 4);
+  else if (t2 >= 1024 || k <= 32) rc = GEMM_DIRECT(2, 1);
+  else rc = GEMM_DIRECT(2, 4);
+#undef GEMM_DIRECT
+  if (rc != GPX_OK) return rc;
   if (part) {
     const long total = (long)batch * m * n;
     hipLaunchKernelGGL(splitk_reduce, dim3(gpx_cdiv(total, SPLITK_OUT)), dim3(256), 0, st, m, n, batch, splits, alpha,

@@ -36,11 +36,11 @@ def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=Non
         if hit:
             splits, tile = hit['splits'], hit['tile']
         else:
-            tiles = -(-m // 64) * -(-n // 64) * batch
+            tiles = -(-m // 32) * -(-n // 32) * batch
             splits = 1
-            if tiles < 256 and k >= 256:
+            if tiles < 512 and k >= 1024:
                 # long, skinny contractions: split K so that enough workgroups run
-                splits = max(1, min(-(-256 // tiles), k // 128, 64))
+                splits = max(1, min(-(-512 // tiles), k // 512, 64))
     return _lib.mm(A, B, C, tA=tA, tB=tB, alpha=alpha, beta=beta, splits=splits, tile=tile,
                    E=E, gamma=gamma)
 
@@ -151,6 +151,24 @@ def rowscale(w, X):
     M = X.shape[1]
     out = empty(D, N, M, like=X)
     call('gpx_rowscale', N, D, M, P(w), P(X), P(out), S())
+    return out
+
+
+def gram(w, X, E=None, gamma=0.0, splits=None):
+    """(D, M, M): sum_n w_nd x_n x_n^T + gamma E, for w (N, D), X (N, M)."""
+    N, D = w.shape
+    M = X.shape[1]
+    if splits is None:
+        cb = -(-M // 64)
+        pairs = D * cb * (cb + 1) // 2
+        # four workgroups per CU of 256 points or more, at least one of 64; a multiple of 8 keeps
+        # a share's rows on one XCD (N = 20000, M = 200, D = 4: 24 shares 84 us, 25 94, 8 132)
+        splits = max(1, min(256 // pairs, N // 64, 128), min(1024 // pairs, N // 256))
+        splits -= splits % 8 if splits > 8 else 0
+    out = empty(D, M, M, like=X)
+    work = empty(query('gpx_gram_workspace', D, M, splits), like=X)
+    call('gpx_gram', N, D, M, P(w), P(X), M, float(gamma), P(E) if E is not None else None,
+         M * M if E is not None and E.dim() == 3 else 0, P(out), splits, P(work), S())
     return out
 
 

@@ -402,7 +402,7 @@ class SGP_Layer(object):
         sumdv = colsum(dv, B * D, 1)
         # cavity mean / covariance
         dmucav = mm(dm, kfuKi, tA=True)
-        dSucav = mm(dops.rowscale(dv, kfuKi), kfuKi, tA=True)
+        dSucav = dops.gram(dv, kfuKi)
         Suinvmuhat = mm(self.Suhatinv, _col(self.muhat)).reshape(D, M)
         lincomb(dmucav, 1.0, dmucav, scale_cav, Suinvmuhat)
         lincomb(dSucav, 1.0, dSucav, 0.5 * scale_cav, self.Suhatinv)
@@ -418,7 +418,7 @@ class SGP_Layer(object):
         dAhat = mm(dm, kfu, tA=True)
         dKi = mm(dAhat, self.muhat, tA=True)
         lincomb(dKi, 1.0, dKi, -0.5 * D, self.Kuu)
-        dBhat = mm(dops.rowscale(dv, kfu), kfu, tA=True)
+        dBhat = dops.gram(dv, kfu)
         KiS = mm(Ki, self.Suhat)
         mm(KiS.reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, alpha=2.0, beta=1.0)
         colsum(dBhat, D, M * M, out=dKi.reshape(-1), alpha=-1.0, beta=1.0)
@@ -460,7 +460,7 @@ class SGP_Layer(object):
         dsf2, dell, dzu, _ = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf)
         sumdv = colsum(dv, B * D, 1)
         dAhat = mm(dm, kfu, tA=True)
-        dBhat = mm(dops.rowscale(dv, kfu), kfu, tA=True)
+        dBhat = dops.gram(dv, kfu)
         # cavity: dmu_cav, dSu_cav (+ the normalising factor), then dSuinv_cav
         c = self._adjoint('reg', alpha)
         dmucav = mm(dAhat, Ki, E=th, gamma=scale_cav * beta)
@@ -499,7 +499,7 @@ class SGP_Layer(object):
         dsf2, dell, dzu, dx = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf, want_dx=True)
         sumdv = colsum(dv, B * D, 1)
         dmucav = mm(dm, kfuKi, tA=True)
-        dSucav = mm(dops.rowscale(dv, kfuKi), kfuKi, tA=True)
+        dSucav = dops.gram(dv, kfuKi)
         dSinv = _sandwich(self.Suhat, dSucav, self.Suhat, alpha=-1.0)
         dSinvM = mm(self.Suhat, _col(dmucav)).reshape(D, M)
         _add_outer(dSinv, dSinvM, self.muhat, -1.0)
@@ -510,7 +510,7 @@ class SGP_Layer(object):
         dAhat = mm(dm, kfu, tA=True)
         dKi = colsum(dSinv, D, M * M).reshape(M, M)
         mm(dAhat, self.muhat, dKi, tA=True, beta=1.0)
-        dBhat = mm(dops.rowscale(dv, kfu), kfu, tA=True)
+        dBhat = dops.gram(dv, kfu)
         KiS2 = mm(Ki, self.Suhat, alpha=2.0, E=_eye(M, Ki), gamma=-1.0)
         mm(KiS2.reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0)
         Minner = lincomb(torch.empty_like(dKi), 1.0, c['Mc'], -2.0, dKi)

@@ -167,11 +167,11 @@ class SGP_Layer(_Layer):
         kfuKi = mm(kfu, Ki)
         # dmu = dm^T kfu Kuu^-1 + Kuu^-1 mu (A = mu Kuu^-1), dSu = sum_n dv kfuKi kfuKi^T + C0
         dmu = mm(dm, kfuKi, tA=True, E=self.A, gamma=1.0)
-        dSu = mm(dops.rowscale(dv, kfuKi), kfuKi, tA=True, E=self._C0, gamma=1.0)
+        dSu = dops.gram(dv, kfuKi, E=self._C0, gamma=1.0)
         deta1, deta2, dKi_u = self._post_grad_u(dmu, dSu)
         dA = mm(dm, kfu, tA=True)
         dKi = mm(dA, self.mu, tA=True, E=self._Kc, gamma=1.0)
-        dB = mm(dops.rowscale(dv, kfu), kfu, tA=True)
+        dB = dops.gram(dv, kfu)
         mm(self._kis2('det').reshape(D * M, M), dB.reshape(D * M, M), dKi, tA=True, beta=1.0)
         if dKi_u is not None:
             lincomb(dKi, 1.0, dKi, 1.0, dKi_u)

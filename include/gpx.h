@@ -32,7 +32,8 @@ extern "C" {
 
 /* C[b] = alpha op(A[b]) op(B[b]) + beta C[b] on the FP64 matrix cores; strides of 0
  * broadcast an operand over the batch; splits > 1 splits K into partial slabs summed in a
- * fixed order (needs gpx_gemm_workspace doubles); tile = 0 (auto), 32 or 64.
+ * fixed order (needs gpx_gemm_workspace doubles); tile = 0 (auto), 32 or 64
+ * (rows and columns of C per tile).
  * Replaces the np.dot / np.einsum contractions of geepee/aep_models.py:156, 197, 239-258,
  * 453-493, 525-546 and geepee/base_models.py:470-488, 497. */
 long gpx_gemm_workspace(int m, int n, int batch, int splits);
@@ -170,6 +171,15 @@ int gpx_mm_var(long n, const double *m, const double *Bp, const double *sf, doub
 /* out[b] = sum_i x[b,i] y[b,i] (the mu^T Sigma^-1 mu terms of aep_models.py:80, 93). */
 int gpx_batched_dot(int batch, int n, const double *x, const double *y, double *out,
                     void *stream);
+
+/* out[d] = sum_n w[n,d] x_n x_n^T + gamma E[d] (out D x M x M, symmetric, fully stored; w N x D,
+ * X N x M with row stride ldx; E NULL or M x M matrices strideE apart, 0 = one for all; must
+ * not alias out): the einsums 'nd,na,nb->dab' (geepee/aep_models.py:464, 490) without the
+ * weighted copy of X.  `splits` shares of the points are summed in a fixed order (work:
+ * gpx_gram_workspace doubles). */
+long gpx_gram_workspace(int D, int M, int splits);
+int gpx_gram(int N, int D, int M, const double *w, const double *X, int ldx, double gamma, const double *E,
+             long strideE, double *out, int splits, double *work, void *stream);
 
 /* out[d][n][m] = w[n,d] X[n][m]: the dv-weighted rows behind the syrk-like einsums
  * 'nd,na,nb->dab' (geepee/aep_models.py:464, 490). */
