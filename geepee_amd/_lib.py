@@ -103,6 +103,8 @@ SIGNATURES = {
                               _p, _p]),
     'gpx_psi_qmax': (_i, []),
     'gpx_psi_fwd': (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p]),
+    'gpx_psi_bwd_gen_workspace': (_l, [_i, _i, _i]),
+    'gpx_psi_bwd_gen': (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     'gpx_psi_bwd_workspace': (_l, [_i, _i, _i]),
     'gpx_psi_bwd': (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p,
                          _p, _p]),

@@ -6,7 +6,7 @@
 // base_models.py:470-488, 497), including the N x M^2 projections of psi2.
 // Split-K partial slabs (one per z-slice of the grid) are summed by a deterministic
 // second pass, so results do not depend on scheduling.
-#include "gpx_common.h"
+#include "gpx_frag.h"
 
 namespace {
 
@@ -103,78 +103,19 @@ __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB,
 // per workgroup), us: 20000 x 200 x 200, 4 products 245 -> 125 (26 -> 51 TF); 4001 x 256 x 256, 2
 // 34 -> 29; 10000 x 6 x 1000 55 -> 17; 256^3, 2 9.6 -> 6.0; 100^3, 5 6.3 -> 4.3; 50^3 5.3 -> 4.1.
 // ---------------------------------------------------------------------------
-typedef double gemm_d2 __attribute__((ext_vector_type(2), aligned(8)));
-
-template <int T>
-struct GemmFrag {
-  double v[2][T];
-};
-
-// Operand view of one wave: `p` is uniform (tile origin), `off[i]` the lane's offset in tile i.
-// KC: k is the contiguous dimension (row stride ld); otherwise k-rows of stride ld.
-template <int T, bool KC>
-struct GemmOp {
-  const double *p;
-  long off[T];
-  int ld;
-  __device__ __forceinline__ GemmOp(const double *base, int ld_, int r0, int rows, int lane) : ld(ld_) {
-    const int g = lane >> 4, last = rows - r0 - 1;
-    p = KC ? base + (long)r0 * ld : base + r0;
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-      const int r = min(16 * i + (lane & 15), last);
-      off[i] = KC ? (long)r * ld + 2 * g : 2L * g * ld + r;
-    }
-  }
-  __device__ __forceinline__ void load(GemmFrag<T> &f, int k0) const {
-    const double *q = p + (KC ? (long)k0 : (long)k0 * ld);
-#pragma unroll
-    for (int i = 0; i < T; ++i) {
-      if constexpr (KC) {
-        const gemm_d2 t = *(const gemm_d2 *)(q + off[i]);
-        f.v[0][i] = t.x;
-        f.v[1][i] = t.y;
-      } else {
-        f.v[0][i] = q[off[i]];
-        f.v[1][i] = (q + ld)[off[i]];
-      }
-    }
-  }
-  // the `kr` (1..7) valid k of a last group; lanes past them re-read the group's first
-  __device__ __forceinline__ void load_tail(GemmFrag<T> &f, int k0, int kr, int lane) const {
-    const double *q = p + (KC ? (long)k0 : (long)k0 * ld);
-    const int g = lane >> 4;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const bool on = 2 * g + s < kr;
-      const long back = on ? s : -2 * g;
-#pragma unroll
-      for (int i = 0; i < T; ++i) {
-        f.v[s][i] = 0.0;
-        if constexpr (T > 2) {  // no registers for the clamped addresses
-          if (on) f.v[s][i] = q[off[i] + (KC ? s : (long)s * ld)];
-        } else {
-          const double t = q[off[i] + (KC ? back : back * ld)];
-          if (on) f.v[s][i] = t;
-        }
-      }
-    }
-  }
-};
-
 template <int TM, int TN, bool TA, bool TB, int KW>
 __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int kend, double alpha, const double *A,
                                                  int lda, const double *B, int ldb, const GemmEpi &ep, double *C,
                                                  int ldc, int m0, int n0, int bidx, bool raw, double *red) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const GemmOp<TM, !TA> oa(A, lda, m0, m, lane);
-  const GemmOp<TN, TB> ob(B, ldb, n0, n, lane);
+  const GpxOperand<TM, !TA> oa(A, lda, m0, m, lane);
+  const GpxOperand<TN, TB> ob(B, ldb, n0, n, lane);
   gpx_d4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
-  auto mul = [&](const GemmFrag<TM> &fa, const GemmFrag<TN> &fb) {
+  auto mul = [&](const GpxFrag<TM> &fa, const GpxFrag<TN> &fb) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -187,8 +128,8 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
   const int kr = (kend - kbeg) & 7;
   const bool tail = kr && kw == groups % KW;
   constexpr bool EARLY = TM <= 2;  // registers to hold the tail from the start
-  GemmFrag<EARLY ? TM : 1> ta;
-  GemmFrag<EARLY ? TN : 1> tb;
+  GpxFrag<EARLY ? TM : 1> ta;
+  GpxFrag<EARLY ? TN : 1> tb;
   if constexpr (EARLY)
     if (tail) {
       oa.load_tail(ta, kbeg + 8 * groups, kr, lane);
@@ -196,8 +137,8 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
     }
   if (mine > 0) {
     constexpr int P = TM == 1 ? 4 : 2;  // groups in flight
-    GemmFrag<TM> fa[P];
-    GemmFrag<TN> fb[P];
+    GpxFrag<TM> fa[P];
+    GpxFrag<TN> fb[P];
     auto load = [&](int u, int t) {
       const int k0 = kbeg + 8 * (kw + KW * min(t, mine - 1));
       oa.load(fa[u], k0);
@@ -220,8 +161,8 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
     if constexpr (EARLY) {
       mul(ta, tb);
     } else {
-      GemmFrag<TM> fa;
-      GemmFrag<TN> fb;
+      GpxFrag<TM> fa;
+      GpxFrag<TN> fb;
       oa.load_tail(fa, kbeg + 8 * groups, kr, lane);
       ob.load_tail(fb, kbeg + 8 * groups, kr, lane);
       mul(fa, fb);
@@ -342,14 +283,14 @@ template <int TM, int TN, bool DIAG>
 __device__ __forceinline__ void gram_tile(int N, int D, int M, int kbeg, int kend, const double *w, const double *X,
                                           int ldx, int m0, int n0, double *out, double *red) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
-  const GemmOp<TM, false> oa(X, ldx, m0, M, lane);
-  const GemmOp<TN, false> ob(X, ldx, n0, M, lane);
+  const GpxOperand<TM, false> oa(X, ldx, m0, M, lane);
+  const GpxOperand<TN, false> ob(X, ldx, n0, M, lane);
   gpx_d4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
-  auto mul = [&](const GemmFrag<TM> &fa, const GemmFrag<TN> &fb, const double *wv) {
+  auto mul = [&](const GpxFrag<TM> &fa, const GpxFrag<TN> &fb, const double *wv) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       double b[TN];
@@ -363,8 +304,8 @@ __device__ __forceinline__ void gram_tile(int N, int D, int M, int kbeg, int ken
   };
   const int groups = (kend - kbeg) >> 3, mine = (groups - wave + 3) / 4;
   if (mine > 0) {
-    GemmFrag<TM> fa[2];
-    GemmFrag<TN> fb[2];
+    GpxFrag<TM> fa[2];
+    GpxFrag<TN> fb[2];
     double wv[2][2];
     auto load = [&](int u, int t) {
       const int k0 = kbeg + 8 * (wave + 4 * min(t, mine - 1));
@@ -387,8 +328,8 @@ __device__ __forceinline__ void gram_tile(int N, int D, int M, int kbeg, int ken
   const int kr = (kend - kbeg) & 7;
   if (kr && wave == groups % 4) {
     const int k0 = kbeg + 8 * groups;
-    GemmFrag<TM> fa;
-    GemmFrag<TN> fb;
+    GpxFrag<TM> fa;
+    GpxFrag<TN> fb;
     oa.load_tail(fa, k0, kr, lane);
     ob.load_tail(fb, k0, kr, lane);
     double wv[2];

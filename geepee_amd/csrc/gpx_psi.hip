@@ -9,17 +9,15 @@
 //
 // Adjoint: compute_psi_derivatives -> psi1compDer / psi2compDer (kernels.py:302-309,
 // 355-444), restated with per-point sufficient statistics.  With
-// L[n,a,b] = dpsi2[n,a,b] psi2[n,a,b] (dpsi2 symmetric), T_na = sum_b L_nab,
+// L[n,a,b] = dpsi2[n,a,b] psi2[n,a,b], T_na = sum_b L_nab,
 // V_nq = sum_ab L_nab z_aq z_bq, S0 = sum_a T_a, S1_q = sum_a T_a z_aq,
 // S2_q = (sum_a T_a z_aq^2 + V_q)/2 and d = 1/(2v+l):
 //   dmu = -2 d (mu S0 - S1),  dv = 2 d^2 (mu^2 S0 - 2 mu S1 + S2) - d S0,
 //   dell (per n) = 2 ell [(v/l) d S0 + d^2 (mu^2 S0 - 2 mu S1 + S2)
 //                         + (sum_a T_a z_aq^2 - V_q) / (2 l^2)],
-//   dZ_aq = -(z_aq R_a - (Lsum z)_aq)/l + 2 P_aq - z_aq R'_aq - sum_b W_abq z_bq,
-// where Lsum = sum_n L_n, R = rowsum(Lsum), W_abq = sum_n L_nab d_nq,
-// P_aq = sum_n T_na d_nq mu_nq, R'_aq = sum_n T_na d_nq (the n-reductions run as
-// MFMA GEMMs on the host side of this file's entry points).
-#include "gpx_common.h"
+//   dZ_aq = sum_n [(U_naq - z_aq T_na)/l + d (2 mu T_na - z_aq T_na - U_naq)],  U_n = L_n z.
+// A dpsi2 that is not symmetric enters as its symmetric part.
+#include "gpx_frag.h"
 
 #include <cstdint>
 
@@ -216,115 +214,256 @@ __global__ __launch_bounds__(256) void psi2_kernel(int N, int M, int Q, const do
 }
 
 // ---------------------------------------------------------------------------
-// adjoint, per-point pass (one block per n, thread b owns column b of L_n)
+// adjoint, materialised psi2
 // ---------------------------------------------------------------------------
 
-constexpr int NRED = 5 * GPX_QMAX + 2;
+// One workgroup per point, point after point.  With L = dpsi2_n * psi2_n the matrix cores form
+// U = L z (as U^T = z^T L: L's elements are the B operand exactly as they are read, 128-byte row
+// segments), T = the row sums of L ride along on the vector ALU, and everything the adjoint needs
+// is linear in U, T and Lp = dpsi1 * psi1:
+//   dZ_aq += (U - z T)/l + d (2 mu T - z T - U) + Lp e (mu - z),  d = 1/(2v+l), e = 1/(v+l),
+// summed over the workgroup's points in registers (lane (g, c): q = g + 4 r, a = n0 + 16 j + c),
+// and the per-point sums S0, S1, TZ2, V and the psi1 terms, reduced over a across the 16 lanes of
+// a row and then over the waves.  The L array, its product with [1 | d] and the T, Lp products
+// are not formed.  SYM: dpsi2 is symmetric; otherwise L uses (dpsi2 + dpsi2^T)/2, whose transposed
+// reads come from the caches.  Bound by reading psi2 and dpsi2 once: N = 1501, M = 100, Q = 5 65 us
+// (78 with the symmetric part taken here), 50 at the rate of a large copy; one thread per column,
+// with L stored and its product, 260 + 66 (and 122 for a symmetrising pass).  N = 1000 134 -> 48.
+// part[block]: [dZ (M x Q) | sum of H (Q) | S0, A1].
+constexpr int PSI_NRED = 5 * GPX_QMAX + 2;
+constexpr int PSI_ZLD = GPX_QMAX + 1;
 
-__global__ __launch_bounds__(256) void psi_bwd_rows_kernel(
+__device__ __forceinline__ double psi_row_sum(double v) {  // over the 16 lanes of a row
+  v = gpx_dpp_add<0x140>(v);
+  v = gpx_dpp_add<0x141>(v);
+  v = gpx_dpp_add<0x4E>(v);
+  return gpx_dpp_add<0xB1>(v);
+}
+
+template <int TN, int W, bool SYM>
+__global__ __launch_bounds__(64 * W, 3) void psi_bwd_points_kernel(
     int N, int M, int Q, const double *__restrict__ mx, const double *__restrict__ vx,
-    const double *__restrict__ z, const double *__restrict__ ls,
-    const double *__restrict__ dpsi1, const double *__restrict__ psi1,
-    const double *__restrict__ dpsi2, const double *__restrict__ psi2,
-    double *__restrict__ dmx, double *__restrict__ dvx,
-    double *__restrict__ Lout,    // N x M x M
-    double *__restrict__ Tout,    // N x M
-    double *__restrict__ Lpout,   // N x M
-    double *__restrict__ Hout,    // N x Q   per-point d/d ell contribution
-    double *__restrict__ s0out,   // N x 2   (S0, sum Lp)
-    double *__restrict__ Dn,      // N x (Q+1): [1 | d]
-    double *__restrict__ Pn,      // N x 2Q : [d*mu | d]
-    double *__restrict__ En) {    // N x 2Q : [e | e*mu]
-  __shared__ double zs[256][GPX_QMAX];
-  __shared__ double red[4][NRED];
-  __shared__ double tot[NRED];
-  const int n = blockIdx.x, b = threadIdx.x, lane = b & 63, w = b >> 6;
-  for (int e = b; e < M * Q; e += 256) zs[e / Q][e % Q] = z[e];
+    const double *__restrict__ z, const double *__restrict__ ls, const double *__restrict__ dpsi1,
+    const double *__restrict__ psi1, const double *__restrict__ dpsi2, const double *__restrict__ psi2,
+    double *__restrict__ dmx, double *__restrict__ dvx, double *__restrict__ part) {
+  extern __shared__ double psi_lds[];
+  const int Mp = (M + 7) & ~7, tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  double *zs = psi_lds;                                             // Mp x PSI_ZLD, zero padded
+  double(*red)[W][PSI_NRED] = (double(*)[W][PSI_NRED])(zs + Mp * PSI_ZLD);  // [2][W][PSI_NRED]
+  for (int e = tid; e < Mp * PSI_ZLD; e += 64 * W) {
+    const int a = e / PSI_ZLD, q = e % PSI_ZLD;
+    zs[e] = (a < M && q < Q) ? z[a * Q + q] : 0.0;
+  }
   __syncthreads();
-  double mu[GPX_QMAX];
+  const int nt = (M + 15) >> 4, lo = nt / W, hi = nt % W, tn = lo + (w < hi);
+  const int first = 16 * (w * lo + min(w, hi)), n0 = min(first, M - 1);
+  bool on[TN];
+  double dz[TN][4];
 #pragma unroll
-  for (int q = 0; q < GPX_QMAX; ++q) mu[q] = (q < Q) ? mx[(long)n * Q + q] : 0.0;
-  double T = 0.0, U[GPX_QMAX];
+  for (int j = 0; j < TN; ++j) {
+    on[j] = j < tn && first + 16 * j + c < M;
 #pragma unroll
-  for (int q = 0; q < GPX_QMAX; ++q) U[q] = 0.0;
-  double Lp = 0.0;
-  if (b < M) {
-    const double *P2 = psi2 + (long)n * M * M + b;
-    const double *G2 = dpsi2 + (long)n * M * M + b;
-    double *Lo = Lout ? Lout + (long)n * M * M + b : nullptr;
-    for (int a = 0; a < M; ++a) {
-      const double l = G2[(long)a * M] * P2[(long)a * M];
-      if (Lo) Lo[(long)a * M] = l;
-      T += l;
+    for (int r = 0; r < 4; ++r) dz[j][r] = 0.0;
+  }
+  double l[4], il[4];
 #pragma unroll
-      for (int q = 0; q < GPX_QMAX; ++q)
-        if (q < Q) U[q] = fma(l, zs[a][q], U[q]);
+  for (int r = 0; r < 4; ++r) {
+    l[r] = g + 4 * r < Q ? exp(2.0 * ls[g + 4 * r]) : 1.0;
+    il[r] = 1.0 / l[r];
+  }
+  const GpxOperand<TN, false> off(psi2, M, n0, M, lane);  // lane offsets of a point's matrix
+  const GpxOperand<TN, true> offT(dpsi2, M, n0, M, lane);
+  const int groups = M >> 3, kr = M & 7;
+  const double *zl = zs + 2 * g * PSI_ZLD + c;  // A operand: z^T[q = c][k = 2 g + s]
+  double hsum = 0.0, s0sum = 0.0, a1sum = 0.0;
+  int par = 0;
+  for (int n = blockIdx.x; n < N; n += gridDim.x, par ^= 1) {
+    GpxOperand<TN, false> op = off, og = off;
+    GpxOperand<TN, true> ot = offT;
+    op.p = psi2 + (long)n * M * M + n0;
+    og.p = dpsi2 + (long)n * M * M + n0;
+    ot.p = dpsi2 + (long)n * M * M + (long)n0 * M;
+    gpx_d4 U[TN];
+    double T[TN], Lp[TN], p1[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      U[j] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+      T[j] = 0.0;
+      const long e = (long)n * M + min(first + 16 * j + c, M - 1);
+      Lp[j] = dpsi1[e];
+      p1[j] = psi1[e];
     }
-    Lp = dpsi1[(long)n * M + b] * psi1[(long)n * M + b];
-    Tout[(long)n * M + b] = T;
-    Lpout[(long)n * M + b] = Lp;
-  }
-  // per-thread contributions, reduced over b:
-  // [0] S0, [1] sum Lp, [2+q] S1, [2+Q+q] sum T z^2, [2+2Q+q] V,
-  // [2+3Q+q] B1 = sum Lp (z-mu), [2+4Q+q] C1 = sum Lp (z-mu)^2
-  double c[NRED];
+    GpxFrag<TN> fp[2], fg[2], ft[2];
+    auto load = [&](int u, int t) {
+      const int k0 = 8 * min(t, groups - 1);
+      op.load(fp[u], k0);
+      og.load(fg[u], k0);
+      if constexpr (!SYM) ot.load(ft[u], k0);
+    };
+    auto mul = [&](int u, int t) {
 #pragma unroll
-  for (int i = 0; i < NRED; ++i) c[i] = 0.0;
-  c[0] = T;
-  c[1] = Lp;
-  if (b < M) {
+      for (int s = 0; s < 2; ++s) {
+        const double za = zl[(8 * t + s) * PSI_ZLD];
 #pragma unroll
-    for (int q = 0; q < GPX_QMAX; ++q)
-      if (q < Q) {
-        const double zq = zs[b][q], zm = zq - mu[q];
-        c[2 + q] = T * zq;
-        c[2 + GPX_QMAX + q] = T * zq * zq;
-        c[2 + 2 * GPX_QMAX + q] = U[q] * zq;
-        c[2 + 3 * GPX_QMAX + q] = Lp * zm;
-        c[2 + 4 * GPX_QMAX + q] = Lp * zm * zm;
+        for (int j = 0; j < TN; ++j) {
+          const double gg = SYM ? fg[u].v[s][j] : 0.5 * (fg[u].v[s][j] + ft[u].v[s][j]);
+          const double le = gg * fp[u].v[s][j];
+          T[j] += le;
+          U[j] = gpx_mfma16(za, le, U[j]);
+        }
       }
-  }
+    };
+    if (groups) {
+      load(0, 0);
+      int t = 0;
+      for (; t + 2 <= groups; t += 2) {
+        load(1, t + 1);
+        mul(0, t);
+        load(0, t + 2);
+        mul(1, t + 1);
+      }
+      if (t < groups) mul(0, t);
+    }
+    if (kr) {
+      op.load_tail(fp[0], 8 * groups, kr, lane);
+      og.load_tail(fg[0], 8 * groups, kr, lane);
+      if constexpr (!SYM) ot.load_tail(ft[0], 8 * groups, kr, lane);
+      mul(0, groups);
+    }
+    double S0 = 0.0, A1 = 0.0;
 #pragma unroll
-  for (int i = 0; i < NRED; ++i) {
-    if (i >= 2 && (i - 2) % GPX_QMAX >= Q) continue;  // unused q slots
-    const double s = gpx_wave_sum(c[i]);
-    if (lane == 0) red[w][i] = s;
+    for (int j = 0; j < TN; ++j) {
+      T[j] = on[j] ? gpx_swap_add<16>(gpx_swap_add<32>(T[j])) : 0.0;
+      Lp[j] = on[j] ? Lp[j] * p1[j] : 0.0;
+      S0 += T[j];
+      A1 += Lp[j];
+    }
+    double *rw = red[par][w];
+    int zo = first + c;  // opaque: z is re-read from LDS for each point, not kept in registers
+    asm volatile("" : "+v"(zo));
+    S0 = psi_row_sum(S0);
+    A1 = psi_row_sum(A1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (4 * r >= Q) break;
+      const int q = g + 4 * r, qc = min(q, Q - 1);
+      const double mu = mx[(long)n * Q + qc], vv = vx[(long)n * Q + qc];
+      const double d = 1.0 / (2.0 * vv + l[r]), e = 1.0 / (vv + l[r]);
+      double V = 0.0, S1 = 0.0, Z2 = 0.0, B1 = 0.0, C1 = 0.0;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const double u = on[j] ? U[j][r] : 0.0, zz = zs[min(zo + 16 * j, M - 1) * PSI_ZLD + q];
+        const double zm = zz - mu, tz = T[j] * zz, lz = Lp[j] * zm;
+        V = fma(u, zz, V);
+        S1 += tz;
+        Z2 = fma(tz, zz, Z2);
+        B1 += lz;
+        C1 = fma(lz, zm, C1);
+        dz[j][r] += fma(u - tz, il[r], d * (2.0 * mu * T[j] - tz - u)) - e * lz;
+      }
+      V = psi_row_sum(V);
+      S1 = psi_row_sum(S1);
+      Z2 = psi_row_sum(Z2);
+      B1 = psi_row_sum(B1);
+      C1 = psi_row_sum(C1);
+      if (c == 0) {
+        rw[2 + q] = S1;
+        rw[2 + GPX_QMAX + q] = Z2;
+        rw[2 + 2 * GPX_QMAX + q] = V;
+        rw[2 + 3 * GPX_QMAX + q] = B1;
+        rw[2 + 4 * GPX_QMAX + q] = C1;
+      }
+    }
+    if (lane == 0) {
+      rw[0] = S0;
+      rw[1] = A1;
+    }
+    __syncthreads();  // red[par] is next written two points on, behind the next point's barrier
+    if (tid < Q) {
+      const int q = tid;
+      auto sum = [&](int i) {
+        double t = red[par][0][i];
+        for (int u = 1; u < W; ++u) t += red[par][u][i];
+        return t;
+      };
+      const double s0 = sum(0), a1 = sum(1), s1 = sum(2 + q), tz2 = sum(2 + GPX_QMAX + q),
+                   vs = sum(2 + 2 * GPX_QMAX + q), b1 = sum(2 + 3 * GPX_QMAX + q), c1 = sum(2 + 4 * GPX_QMAX + q);
+      const double m = mx[(long)n * Q + q], v = vx[(long)n * Q + q];
+      const double ell = exp(ls[q]), lq = exp(2.0 * ls[q]);
+      const double d = 1.0 / (2.0 * v + lq), e = 1.0 / (v + lq);
+      const double quad = m * m * s0 - 2.0 * m * s1 + 0.5 * (tz2 + vs);
+      dmx[(long)n * Q + q] = -2.0 * d * (m * s0 - s1) + e * b1;
+      dvx[(long)n * Q + q] = 2.0 * d * d * quad - d * s0 + 0.5 * e * (e * c1 - a1);
+      hsum += 2.0 * ell * ((v / lq) * d * s0 + d * d * quad + (tz2 - vs) / (2.0 * lq * lq));
+      hsum += e * ell * (e * c1 + (v / lq) * a1);
+      s0sum += s0;
+      a1sum += a1;
+    }
   }
-  __syncthreads();
-  for (int i = b; i < NRED; i += 256) tot[i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
-  __syncthreads();
-  if (b < Q) {
-    const int q = b;
-    const double S0 = tot[0], A1 = tot[1];
-    const double S1 = tot[2 + q], TZ2 = tot[2 + GPX_QMAX + q], V = tot[2 + 2 * GPX_QMAX + q];
-    const double B1 = tot[2 + 3 * GPX_QMAX + q], C1 = tot[2 + 4 * GPX_QMAX + q];
-    const double l = exp(2.0 * ls[q]);
-    const double m = mx[(long)n * Q + q], vv = vx[(long)n * Q + q];
-    const double ell = exp(ls[q]);
-    const double d = 1.0 / (2.0 * vv + l), e = 1.0 / (vv + l);
-    const double S2 = 0.5 * (TZ2 + V);
-    const double quad = m * m * S0 - 2.0 * m * S1 + S2;
-    const double dmu = -2.0 * d * (m * S0 - S1) + e * B1;
-    const double dvv = 2.0 * d * d * quad - d * S0 + 0.5 * e * (e * C1 - A1);
-    const double h2 = 2.0 * ell * ((vv / l) * d * S0 + d * d * quad + (TZ2 - V) / (2.0 * l * l));
-    const double h1 = e * ell * (e * C1 + (vv / l) * A1);
-    dmx[(long)n * Q + q] = dmu;
-    dvx[(long)n * Q + q] = dvv;
-    Hout[(long)n * Q + q] = h1 + h2;
-    Dn[(long)n * (Q + 1) + 1 + q] = d;
-    Pn[(long)n * 2 * Q + q] = d * m;
-    Pn[(long)n * 2 * Q + Q + q] = d;
-    En[(long)n * 2 * Q + q] = e;
-    En[(long)n * 2 * Q + Q + q] = e * m;
-  }
-  if (b == 0) {
-    Dn[(long)n * (Q + 1)] = 1.0;
-    s0out[2 * n] = tot[0];
-    s0out[2 * n + 1] = tot[1];
+  double *po = part + (long)blockIdx.x * (M * Q + Q + 2);
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (on[j] && g + 4 * r < Q) po[(first + 16 * j + c) * Q + g + 4 * r] = dz[j][r];
+  if (tid < Q) po[M * Q + tid] = hsum;
+  if (tid == 0) {
+    po[M * Q + Q] = s0sum;
+    po[M * Q + Q + 1] = a1sum;
   }
 }
 
-// Final assembly for the hyper-parameter adjoints.  One block per inducing point a
+// Sums the workgroups' partials (fixed order: 8 interleaved groups, then the groups).  A workgroup
+// takes 32 of the M Q + Q + 1 outputs; the last output is dsf2 = (A1 + 2 S0) / sf2.
+__global__ __launch_bounds__(256) void psi_bwd_sum_kernel(int M, int Q, int blocks, const double *__restrict__ part,
+                                                          const double *__restrict__ sf, double *__restrict__ dsf2,
+                                                          double *__restrict__ dell, double *__restrict__ dZ) {
+  __shared__ double red[8][33];
+  const int o = threadIdx.x & 31, g = threadIdx.x >> 5, mq = M * Q, width = mq + Q + 2;
+  const int e = blockIdx.x * 32 + o;
+  double s = 0.0;
+  if (e < mq + Q) {
+#pragma unroll 4
+    for (int b = g; b < blocks; b += 8) s += part[(long)b * width + e];
+  } else if (e == mq + Q) {
+#pragma unroll 4
+    for (int b = g; b < blocks; b += 8) s += part[(long)b * width + e + 1] + 2.0 * part[(long)b * width + e];
+  }
+  red[g][o] = s;
+  __syncthreads();
+  if (g != 0 || e > mq + Q) return;
+  double t = red[0][o];
+#pragma unroll
+  for (int h = 1; h < 8; ++h) t += red[h][o];
+  if (e < mq) dZ[e] = t;
+  else if (e < mq + Q) dell[e - mq] = t;
+  else dsf2[0] = t / exp(2.0 * sf[0]);
+}
+
+// Workgroups of the point pass: what fills three waves per SIMD, each with as many points as the
+// others.
+int psi_bwd_blocks(int N, int M) {
+  const int most = M > 128 ? 256 : 768, rounds = (int)gpx_cdiv(N, most);
+  return (int)gpx_cdiv(N, rounds);
+}
+
+template <int TN, int W>
+int psi_bwd_launch(int blocks, int N, int M, int Q, int sym, const double *mx, const double *vx, const double *z,
+                   const double *ls, const double *dpsi1, const double *psi1, const double *dpsi2,
+                   const double *psi2, double *dmx, double *dvx, double *part, hipStream_t st) {
+  const int lds = (int)sizeof(double) * (((M + 7) & ~7) * PSI_ZLD + 2 * W * PSI_NRED);
+  if (sym)
+    hipLaunchKernelGGL((psi_bwd_points_kernel<TN, W, true>), dim3(blocks), dim3(64 * W), lds, st, N, M, Q, mx, vx, z,
+                       ls, dpsi1, psi1, dpsi2, psi2, dmx, dvx, part);
+  else
+    hipLaunchKernelGGL((psi_bwd_points_kernel<TN, W, false>), dim3(blocks), dim3(64 * W), lds, st, N, M, Q, mx, vx, z,
+                       ls, dpsi1, psi1, dpsi2, psi2, dmx, dvx, part);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
+// Final assembly for the hyper-parameter adjoints of the fused path.  One block per inducing point a
 // (threads over b), plus block M which finishes the scalar / per-q sums.
 //   LW:  M^2 x (Q+1)  [Lsum | W]          (sum_n L_nab [1 | d_nq])
 //   TP:  M x 2Q       [P | R']            (sum_n T_na [d mu | d])
@@ -404,7 +543,7 @@ extern "C" int gpx_gemm_batched(int transA, int transB, int m, int n, int k, dou
 
 extern "C" {
 
-// Shared tail of the psi adjoint (materialising and fused paths): from the per-point
+// Tail of the fused psi adjoint: from the per-point
 // outputs T, Lp (N x M), H (N x Q), s0 (N x 2), Dn, Pn, En and the pair sums LW
 // ((M*M) x (Q+1)) finish dsf2, dell (w.r.t. ell) and dZ.  TP, LE (M x 2Q) and cols0 (2)
 // are workspace.
@@ -473,49 +612,44 @@ int gpx_psi_fwd(int N, int M, int Q, const double *mx, const double *vx, const d
   return GPX_OK;
 }
 
-// Workspace (doubles) for gpx_psi_bwd.
-long gpx_psi_bwd_workspace(int N, int M, int Q) {
-  long s = (long)N * M * M;                 // L
-  s += 2L * N * M;                          // T, Lp
-  s += (long)N * Q + 2L * N;                // H, s0
-  s += (long)N * (Q + 1) + 4L * N * Q;      // Dn, Pn, En
-  s += (long)M * M * (Q + 1) + 4L * M * Q;  // LW, TP, LE
-  s += Q + 2;                               // colH, cols0
-  s += gpx_psi_tail_workspace(N, M, Q);     // split-K partials of the tail
-  return s;
+// Adjoint of gpx_psi_fwd given dL/dpsi1 (N x M) and dL/dpsi2 (N x M x M), symmetric or (sym = 0)
+// any: dsf2 (1, w.r.t. sf2), dell (Q, w.r.t. ell = exp(ls)), dZ (M x Q), dmx, dvx (N x Q).
+long gpx_psi_bwd_gen_workspace(int N, int M, int Q) {
+  return N < 1 ? 0 : (long)psi_bwd_blocks(N, M) * (M * Q + Q + 2);
 }
 
-// Adjoint of gpx_psi_fwd given dL/dpsi1 (N x M) and a symmetric dL/dpsi2 (N x M x M):
-// dsf2 (1, w.r.t. sf2), dell (Q, w.r.t. ell = exp(ls)), dZ (M x Q), dmx, dvx (N x Q).
+int gpx_psi_bwd_gen(int N, int M, int Q, int sym, const double *mx, const double *vx, const double *z,
+                    const double *ls, const double *sf, const double *dpsi1, const double *psi1,
+                    const double *dpsi2, const double *psi2, double *dsf2, double *dell, double *dZ,
+                    double *dmx, double *dvx, double *work, void *stream) {
+  if (N < 1 || M < 1 || M > 256 || Q < 1 || Q > GPX_QMAX) return GPX_EINVAL;
+  if (!mx || !vx || !z || !ls || !sf || !dpsi1 || !psi1 || !dpsi2 || !psi2 || !work) return GPX_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  const int blocks = psi_bwd_blocks(N, M);
+  int rc;
+#define PSI_GO(TN, W) \
+  psi_bwd_launch<TN, W>(blocks, N, M, Q, sym, mx, vx, z, ls, dpsi1, psi1, dpsi2, psi2, dmx, dvx, work, st)
+  if (M <= 64) rc = PSI_GO(1, 4);
+  else if (M <= 128) rc = PSI_GO(2, 4);
+  else rc = PSI_GO(2, 8);
+#undef PSI_GO
+  if (rc != GPX_OK) return rc;
+  hipLaunchKernelGGL(psi_bwd_sum_kernel, dim3(gpx_cdiv(M * Q + Q + 1, 32)), dim3(256), 0, st, M, Q, blocks,
+                     (const double *)work, sf, dsf2, dell, dZ);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
+// The same for a symmetric dpsi2; its workspace query covers N M^2 doubles as well, which callers
+// of this entry point may count on having reserved.
+long gpx_psi_bwd_workspace(int N, int M, int Q) { return (long)N * M * M + gpx_psi_bwd_gen_workspace(N, M, Q); }
+
 int gpx_psi_bwd(int N, int M, int Q, const double *mx, const double *vx, const double *z,
                 const double *ls, const double *sf, const double *dpsi1, const double *psi1,
                 const double *dpsi2, const double *psi2, double *dsf2, double *dell, double *dZ,
                 double *dmx, double *dvx, double *work, void *stream) {
-  if (N < 1 || M < 1 || M > 256 || Q < 1 || Q > GPX_QMAX) return GPX_EINVAL;
-  if (!mx || !vx || !z || !ls || !sf || !dpsi1 || !psi1 || !dpsi2 || !psi2 || !work) return GPX_EINVAL;
-  hipStream_t st = (hipStream_t)stream;
-  double *L = work;
-  double *T = L + (long)N * M * M;
-  double *Lp = T + (long)N * M;
-  double *H = Lp + (long)N * M;
-  double *s0 = H + (long)N * Q;
-  double *Dn = s0 + 2L * N;
-  double *Pn = Dn + (long)N * (Q + 1);
-  double *En = Pn + 2L * N * Q;
-  double *LW = En + 2L * N * Q;
-  double *TP = LW + (long)M * M * (Q + 1);
-  double *LE = TP + 2L * M * Q;
-  double *colH = LE + 2L * M * Q;
-  double *cols0 = colH + Q;
-  hipLaunchKernelGGL(psi_bwd_rows_kernel, dim3(N), dim3(256), 0, st, N, M, Q, mx, vx, z, ls, dpsi1,
-                     psi1, dpsi2, psi2, dmx, dvx, L, T, Lp, H, s0, Dn, Pn, En);
-  GPX_CHECK_LAUNCH();
-  // LW = L^T [1 | d]  (M^2 x (Q+1)), reduction over n
-  int rc = gpx_gemm_batched(1, 0, M * M, Q + 1, N, 1.0, L, M * M, 0, Dn, Q + 1, 0, 0.0, LW, Q + 1, 0, 1,
-                            1, nullptr, 0, stream);
-  if (rc) return rc;
-  return gpx_psi_bwd_tail(N, M, Q, z, ls, sf, T, Lp, H, s0, Dn, Pn, En, LW, TP, LE, cols0, dsf2, dell, dZ, cols0 + 2,
-                          stream);
+  return gpx_psi_bwd_gen(N, M, Q, 1, mx, vx, z, ls, sf, dpsi1, psi1, dpsi2, psi2, dsf2, dell, dZ, dmx, dvx, work,
+                         stream);
 }
 
 }  // extern "C"

@@ -236,13 +236,14 @@ def psi_fwd(mx, vx, z, ls, sf, with_psi2=True):
     return psi1, psi2
 
 
-def psi_bwd(mx, vx, z, ls, sf, dpsi1, psi1, dpsi2, psi2):
+def psi_bwd(mx, vx, z, ls, sf, dpsi1, psi1, dpsi2, psi2, symmetric=True):
+    """Adjoint of psi_fwd: dsf2, dell, dz, dmx, dvx; symmetric=False for a dpsi2 that is not."""
     N, Q = mx.shape
     M = z.shape[0]
     outs = [empty(1, like=mx), empty(Q, like=mx), empty(M, Q, like=mx), empty(N, Q, like=mx),
             empty(N, Q, like=mx)]
-    work = empty(query('gpx_psi_bwd_workspace', N, M, Q), like=mx)
-    call('gpx_psi_bwd', N, M, Q, P(mx), P(vx), P(z), P(ls), P(sf), P(dpsi1), P(psi1), P(dpsi2),
+    work = empty(query('gpx_psi_bwd_gen_workspace', N, M, Q), like=mx)
+    call('gpx_psi_bwd_gen', N, M, Q, int(symmetric), P(mx), P(vx), P(z), P(ls), P(sf), P(dpsi1), P(psi1), P(dpsi2),
          P(psi2), *[P(o) for o in outs], P(work), S())
     return outs
 

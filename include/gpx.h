@@ -98,6 +98,14 @@ int gpx_psi_bwd(int N, int M, int Q, const double *mx, const double *vx, const d
                 const double *dpsi2, const double *psi2, double *dsf2, double *dell, double *dZ,
                 double *dmx, double *dvx, double *work, void *stream);
 
+/* The same for any dL/dpsi2 (sym = 0: its symmetric part counts; sym = 1: it is symmetric), with
+ * gpx_psi_bwd_gen_workspace doubles of scratch (geepee/kernels.py:415-418). */
+long gpx_psi_bwd_gen_workspace(int N, int M, int Q);
+int gpx_psi_bwd_gen(int N, int M, int Q, int sym, const double *mx, const double *vx, const double *z,
+                    const double *ls, const double *sf, const double *dpsi1, const double *psi1,
+                    const double *dpsi2, const double *psi2, double *dsf2, double *dell, double *dZ,
+                    double *dmx, double *dvx, double *work, void *stream);
+
 /* Adjoint of K(x, Z): dsf2, dell, dZ and optionally dx (N x Q); M <= 256, Q <= 16.
  * Replaces compute_kfu_derivatives -> kfucompDer (geepee/kernels.py:312-313, 381-399). */
 long gpx_kfu_bwd_workspace(int N, int M, int Q);
@@ -411,7 +419,7 @@ int gpx_fused_mm_bwd_tail(int N, int M, int Q, int D, const double *z, const dou
                           int splits, int nsplit, double *dsf2, double *dell, double *dZ, double *work,
                           void *stream);
 
-/* Shared final stage of both psi adjoints (pair sums LW and per-point statistics in, dsf2,
+/* Final stage of the fused psi adjoint (pair sums LW and per-point statistics in, dsf2,
  * dell, dZ out); the tail of compute_psi_derivatives (geepee/kernels.py:430-442, 371-376). */
 int gpx_psi_bwd_tail(int N, int M, int Q, const double *z, const double *ls, const double *sf,
                      const double *T, const double *Lp, const double *H, const double *s0,
