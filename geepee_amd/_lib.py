@@ -24,6 +24,8 @@ SIGNATURES = {
                                  _d, _p, _i, _l, _i, _i, _p, _i, _p]),
     'gpx_spd_max_m': (_i, []),
     'gpx_spd_inv_batched': (_i, [_i, _i, _p, _i, _l, _p, _i, _l, _p, _p, _p]),
+    'gpx_spd_workspace': (_l, [_i, _i]),
+    'gpx_spd_inv_batched_ws': (_i, [_i, _i, _p, _i, _l, _p, _i, _l, _p, _p, _p, _p]),
     'gpx_status_fold': (_i, [_i, _p, _p, _p, _p]),
     'gpx_se_kernel': (_i, [_i, _i, _i, _p, _i, _p, _p, _p, _d, _p, _p]),
     'gpx_kfu_bwd_workspace': (_l, [_i, _i, _i]),
@@ -248,5 +250,7 @@ def spd_inv(A, out=None, logdet=None, info=None):
     """Batched SPD inverse / log-determinant of A (b, M, M) or (M, M)."""
     M = A.shape[-1]
     batch = A.shape[0] if A.dim() == 3 else 1
-    call('gpx_spd_inv_batched', M, batch, P(A), M, M * M, P(out), M, M * M, P(logdet), P(info), S())
+    need = query('gpx_spd_workspace', M, batch) if out is not None else 0
+    work = torch.empty(need, dtype=torch.float64, device=A.device) if need else None
+    call('gpx_spd_inv_batched_ws', M, batch, P(A), M, M * M, P(out), M, M * M, P(logdet), P(info), P(work), S())
     return out

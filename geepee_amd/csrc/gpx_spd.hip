@@ -1,4 +1,5 @@
-// Batched SPD inverse + log-determinant, one workgroup per M x M matrix.
+// Batched SPD inverse + log-determinant: one workgroup per M x M matrix, or many for a few large
+// ones.
 //
 // Replaces the per-output-dim np.linalg.inv / slogdet / solve calls of the layer
 // algebra (base_models.py:462-476; aep_models.py:62-95, 523-533).  The matrix stays in
@@ -45,7 +46,8 @@ struct SpdShape {
 template <int MT, int NW>
 struct SpdLds {
   typedef SpdShape<MT, NW, true> S;
-  static constexpr int CT = 16 * 17;
+  static constexpr int CT = 16 * 17, COLS = MT, WAVES = NW, NPW = S::NPW, NJ = S::NJ;
+  static constexpr bool YL = S::YL;
   // the small arrays first: LDS addresses below 64 KB fit an instruction's offset field
   double mul[4][16];   // [g][i]: pivot g's multiplier of row i, its reciprocal at i = g
   double piv[16 * MT];
@@ -124,8 +126,8 @@ __device__ __forceinline__ double spd_pick(double x0, double x1, double x2, doub
 // Rows 4R .. 4R+3 of the pivot block P (wave 0): four scalar pivots over the four rows, their
 // multipliers to LDS for the other waves, then the rank-4 update of P's other rows as one
 // MFMA.
-template <int R, int MT, int NW>
-__device__ __forceinline__ void spd_pivot_rows(SpdLds<MT, NW> &sm, int K, int lane, gpx_d4 &P) {
+template <int R, class L>
+__device__ __forceinline__ void spd_pivot_rows(L &sm, int K, int lane, gpx_d4 &P) {
   const int lr = lane >> 4, lc = lane & 15;
   double x[4], c[4][4], d[4];
   spd_rows4(P[R], x);
@@ -157,14 +159,14 @@ __device__ __forceinline__ void spd_pivot_rows(SpdLds<MT, NW> &sm, int K, int la
 }
 
 // The same rows of the wave's panel tiles, one step behind the pivot block.
-template <int R, int MT, int NW, int NJ>
-__device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, int K, int pw, int lane, gpx_d4 *y) {
-  typedef SpdShape<MT, NW, true> S;
+template <int R, class L>
+__device__ __forceinline__ void spd_tile_rows(L &sm, double *rv, int K, int pw, int lane, gpx_d4 *y) {
+  constexpr int MT = L::COLS, NJ = L::NJ;
   const int lr = lane >> 4, lc = lane & 15;
   // tile j of the wave; past the last tile the first one again (its copy is not written back)
-  auto slot = [&](int j) { return rv + (pw + S::NPW * j < MT ? pw + S::NPW * j : pw) * 256; };
+  auto slot = [&](int j) { return rv + (pw + L::NPW * j < MT ? pw + L::NPW * j : pw) * 256; };
   double yr[NJ][4];
-  if constexpr (R > 0 && !S::YL) {
+  if constexpr (R > 0 && !L::YL) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) slot(j)[R * 64 + lane] = y[j][R];
   }
@@ -173,7 +175,7 @@ __device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, in
 #pragma unroll
     for (int k = 0; k < 4; ++k) yr[j][k] = slot(j)[R * 64 + 16 * k + lc];
   };
-  if constexpr (!S::YL) {
+  if constexpr (!L::YL) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) rows(j);
   }
@@ -187,8 +189,8 @@ __device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, in
   spd_spread(cm, c, std::make_integer_sequence<int, 16>());
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    if constexpr (S::YL) {
-      if (pw + S::NPW * j >= MT) break;  // wave-uniform
+    if constexpr (L::YL) {
+      if (pw + L::NPW * j >= MT) break;  // wave-uniform
       rows(j);
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[j][r] = slot(j)[r * 64 + lane];
@@ -204,7 +206,7 @@ __device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, in
     const double py = spd_pick(yr[j][0], yr[j][1], yr[j][2], yr[j][3], lr);
     y[j] = gpx_mfma16(a, -py, y[j]);
     y[j][R] = py;
-    if constexpr (S::YL) {
+    if constexpr (L::YL) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) slot(j)[r * 64 + lane] = y[j][r];
     }
@@ -215,60 +217,60 @@ __device__ __forceinline__ void spd_tile_rows(SpdLds<MT, NW> &sm, double *rv, in
 // columns]].  Wave 0 runs the pivots on P alone; the waves of the other SIMDs (not wave 4,
 // which shares wave 0's) carry the tiles of the block row, each a step of four pivots
 // behind it (sm.step; wave 0 waits for nobody, so every wait ends).
-template <int MT, int NW>
-__device__ __forceinline__ void spd_panel(SpdLds<MT, NW> &sm, double *rv, int K, int w, int lane) {
-  typedef SpdShape<MT, NW, true> S;
-  constexpr int NJ = S::NJ;
+template <class L>
+__device__ __forceinline__ void spd_panel(L &sm, double *rv, int K, int w, int lane) {
+  constexpr int MT = L::COLS, NJ = L::NJ;
   if (w == 0) {
     __builtin_amdgcn_s_setprio(3);
     gpx_d4 P;
 #pragma unroll
     for (int r = 0; r < 4; ++r) P[r] = rv[MT * 256 + r * 64 + lane];
-    spd_pivot_rows<0, MT, NW>(sm, K, lane, P);
-    spd_pivot_rows<1, MT, NW>(sm, K, lane, P);
-    spd_pivot_rows<2, MT, NW>(sm, K, lane, P);
-    spd_pivot_rows<3, MT, NW>(sm, K, lane, P);
+    spd_pivot_rows<0>(sm, K, lane, P);
+    spd_pivot_rows<1>(sm, K, lane, P);
+    spd_pivot_rows<2>(sm, K, lane, P);
+    spd_pivot_rows<3>(sm, K, lane, P);
     __builtin_amdgcn_s_setprio(0);
     return;
   }
   const int pw = w < 4 ? w - 1 : w - 2;
   if (w == 4 || pw >= MT) return;
   gpx_d4 y[NJ];
-  if constexpr (!S::YL) {
+  if constexpr (!L::YL) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      const int J = pw + S::NPW * j < MT ? pw + S::NPW * j : pw;
+      const int J = pw + L::NPW * j < MT ? pw + L::NPW * j : pw;
 #pragma unroll
       for (int r = 0; r < 4; ++r) y[j][r] = rv[J * 256 + r * 64 + lane];
     }
   }
-  spd_tile_rows<0, MT, NW, NJ>(sm, rv, K, pw, lane, y);
-  spd_tile_rows<1, MT, NW, NJ>(sm, rv, K, pw, lane, y);
-  spd_tile_rows<2, MT, NW, NJ>(sm, rv, K, pw, lane, y);
-  spd_tile_rows<3, MT, NW, NJ>(sm, rv, K, pw, lane, y);
-  if constexpr (!S::YL) {
+  spd_tile_rows<0>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<1>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<2>(sm, rv, K, pw, lane, y);
+  spd_tile_rows<3>(sm, rv, K, pw, lane, y);
+  if constexpr (!L::YL) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-      if (pw + S::NPW * j >= MT) break;
+      if (pw + L::NPW * j >= MT) break;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) rv[(pw + S::NPW * j) * 256 + r * 64 + lane] = y[j][r];
+      for (int r = 0; r < 4; ++r) rv[(pw + L::NPW * j) * 256 + r * 64 + lane] = y[j][r];
     }
   }
 }
 
-// Phase 1 for one tile: block row K and (negated, transposed) block column K to LDS.
-template <int MT, int NW>
-__device__ __forceinline__ void spd_publish(double *rv, double *ct, int K, int I, int J, gpx_d4 &acc, int lane) {
-  if (__builtin_expect(I != K && J != K, 1)) return;
+// Phase 1 for one tile: block row K and (negated, transposed) block column KJ to LDS.
+template <class L>
+__device__ __forceinline__ void spd_publish(double *rv, double *ct, int K, int KJ, int I, int J, gpx_d4 &acc,
+                                            int lane) {
+  if (__builtin_expect(I != K && J != KJ, 1)) return;
   const int lr = lane >> 4, lc = lane & 15;
-  double *c = ct + I * SpdLds<MT, NW>::CT + lc * 17 + lr;
+  double *c = ct + I * L::CT + lc * 17 + lr;
   if (I == K) {
-    double *v = rv + (J == K ? MT : J) * 256 + lane;
+    double *v = rv + (J == KJ ? L::COLS : J) * 256 + lane;
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r * 64] = acc[r];
-    if (J == K) {
+    if (J == KJ) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) c[4 * r] = rv[K * 256 + r * 64 + lane] = lr + 4 * r == lc ? 1.0 : 0.0;
+      for (int r = 0; r < 4; ++r) c[4 * r] = rv[KJ * 256 + r * 64 + lane] = lr + 4 * r == lc ? 1.0 : 0.0;
     }
   } else {
 #pragma unroll
@@ -288,13 +290,13 @@ __device__ __forceinline__ void spd_next(int &I, int &J) {
   }
 }
 
-// log det and info from the pivots; returns info: the first pivot that is not a positive
+// log det and info from the pivots, thread k holding pivot k (1 past the last); returns info: the first pivot that is not a positive
 // number, counted from 1 (0: none; what was computed after it is not used).
-template <int MT, int NW>
-__device__ __forceinline__ int spd_finish(SpdLds<MT, NW> &sm, int M, int b, double *logdet, int *info) {
-  static_assert(NW * 64 >= 16 * MT, "one pivot per thread");
+template <class L>
+__device__ __forceinline__ int spd_finish(L &sm, double d, int b, double *logdet, int *info) {
+  constexpr int NW = L::WAVES;
+  static_assert(NW * 64 >= 16 * L::COLS, "one pivot per thread");
   const int k = threadIdx.x;
-  const double d = k < M ? sm.piv[k] : 1.0;
   const unsigned long long bad = __ballot(!(d > 0.0 && d < INFINITY));
   if ((k & 63) == 0) sm.first[k >> 6] = bad ? k + __ffsll(bad) : 0;
   const double ld = gpx_block_sum(log(d), sm.red);  // its barriers order sm.first
@@ -428,18 +430,18 @@ __global__ __launch_bounds__(NW * 64) void spd_gj_kernel(int M, int batch, const
         if (u < TM) {
           if (__builtin_expect(I == K || J == K, 0)) {
             gpx_d4 v = get(u, I, J);
-            spd_publish<MT, NW>(rv, ct, K, I, J, v, lane);
+            spd_publish<SpdLds<MT, NW>>(rv, ct, K, K, I, J, v, lane);
             put(u, I, J, v);
           }
         } else if (u + 1 < TM + TR || T % NW == 0 || I < MT) {
-          spd_publish<MT, NW>(rv, ct, K, I, J, acc[u < TM ? 0 : u - TM], lane);
+          spd_publish<SpdLds<MT, NW>>(rv, ct, K, K, I, J, acc[u < TM ? 0 : u - TM], lane);
         }
         spd_next<MT, NW>(I, J);
       }
     }
     __syncthreads();
     // (2) the panel
-    spd_panel<MT, NW>(sm, rv, K, w, lane);
+    spd_panel(sm, rv, K, w, lane);
     __syncthreads();
     // (3) the tiles, the next tile's operands loaded beside this one's MFMAs (hoisting more
     // of the LDS loads would hold all of them in registers at once); a wave's tile past the
@@ -475,7 +477,7 @@ __global__ __launch_bounds__(NW * 64) void spd_gj_kernel(int M, int batch, const
     if (K + 1 == MT) break;
     if (S::NB == 1) __syncthreads();
   }
-  const int fail = spd_finish<MT, NW>(sm, M, b, logdet, info);
+  const int fail = spd_finish(sm, (int)threadIdx.x < M ? sm.piv[threadIdx.x] : 1.0, b, logdet, info);
   if (!out) return;
   // the store indices are formed afresh from an opaque copy of the lane: otherwise the
   // compiler keeps the load's per-tile indices live through the whole elimination
@@ -516,6 +518,319 @@ const gj_fn kGJ[16] = {launch_gj<1>,  launch_gj<2>,  launch_gj<3>,  launch_gj<4>
                              launch_gj<5>,  launch_gj<6>,  launch_gj<7>,  launch_gj<8>,
                              launch_gj<9>,  launch_gj<10>, launch_gj<11>, launch_gj<12>,
                              launch_gj<13>, launch_gj<14>, launch_gj<15>, launch_gj<16>};
+
+// ---------------------------------------------------------------------------
+// The same elimination over many workgroups, four 16-blocks (one panel) at a time, two launches
+// per panel:
+//   spd_diag_kernel, one workgroup per matrix, runs the four blocks on the 64 x 64 diagonal block
+//     alone and records the steps: per block the pivot rows' multipliers (mul), the columns before
+//     each four pivots (aop), the columns c_I of the other three rows (cop) and the block row Wd;
+//   spd_sweep_kernel, per column tile J and three row tiles, replays the recorded steps on the
+//     panel's four tiles of column J (its last wave), which gives the block rows W_k[J] = P^-1 A[K,J] at
+//     their own stage, forms c_k = A[I,K0+k] - sum_{l<k} c_l Wd_l[k] for its row tiles (a wave each)
+//     and applies the four rank-16 updates.
+// These are the operations of the one-workgroup kernel, tile for tile and in its order; no product
+// with an explicit inverse of the 64 x 64 block, which would cost accuracy on ill-conditioned
+// panels.  Bound by the diagonal blocks' pivot chains (14 us per panel) and the replay (9 us).
+// Between panels the matrix lives in two scratch copies in tile order (a sweep reads one
+// and writes the other), padded with the identity.
+// ---------------------------------------------------------------------------
+constexpr int SPD_NB = 4;     // 16-blocks per panel
+constexpr int SPD_SWEEP = 3;  // row tiles of a sweep's workgroup, a wave each; its last wave replays
+
+// Scratch of one matrix, in doubles.
+struct SpdWork {
+  static constexpr int MUL = 0, AOP = MUL + 4 * 64, COP = AOP + 4 * 256, REC = COP + 16 * 256;
+  static constexpr int WD = REC, PIV = WD + 16 * 256, TMP = PIV + 256;
+  static constexpr long size(int MT) { return TMP + 2L * MT * MT * 256; }
+};
+
+// A panel step's matrix before (src, first panel: the caller's) and after it.
+struct SpdStep {
+  const double *A;  // caller's matrix, first panel only
+  int lda;
+  long sA;
+  double *out;  // caller's result, last panel only
+  int ldo;
+  long sO;
+  double *work;
+  int M, MT, K0, from, to;  // scratch copies read (-1: A) and written (-1: out)
+};
+
+__device__ __forceinline__ gpx_d4 spd_step_load(const SpdStep &p, int b, int I, int J, int lane) {
+  const int lr = lane >> 4, j = J * 16 + (lane & 15);
+  gpx_d4 v;
+  if (p.from >= 0) {
+    const double *t = p.work + b * SpdWork::size(p.MT) + SpdWork::TMP +
+                      ((long)(p.from * p.MT + I) * p.MT + J) * 256 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = t[r * 64];
+  } else {
+    const double *A = p.A + b * p.sA;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = I * 16 + lr + 4 * r;
+      const double x = A[(long)min(i, p.M - 1) * p.lda + min(j, p.M - 1)];
+      v[r] = i < p.M && j < p.M ? x : (i == j ? 1.0 : 0.0);
+    }
+  }
+  return v;
+}
+
+__device__ __forceinline__ void spd_step_store(const SpdStep &p, int b, int I, int J, int lane, const gpx_d4 &v,
+                                               bool fail) {
+  const int lr = lane >> 4, j = J * 16 + (lane & 15);
+  if (p.to >= 0) {
+    double *t = p.work + b * SpdWork::size(p.MT) + SpdWork::TMP + ((long)(p.to * p.MT + I) * p.MT + J) * 256 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t[r * 64] = v[r];
+  } else {
+    double *o = p.out + b * p.sO;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = I * 16 + lr + 4 * r;
+      if (i < p.M && j < p.M) o[(long)i * p.ldo + j] = fail ? NAN : v[r];
+    }
+  }
+}
+
+struct SpdDiagLds {
+  static constexpr int CT = 16 * 17, COLS = SPD_NB, WAVES = 8, NPW = 6, NJ = 1;
+  static constexpr bool YL = false;
+  double mul[4][16];
+  double piv[16 * SPD_NB];
+  double red[16];
+  int first[WAVES];
+  int step;
+  double pt[4][CT];
+  double rv[2][(SPD_NB + 1) * 256];
+  double ct[2][SPD_NB * CT];
+};
+
+__global__ __launch_bounds__(512) void spd_diag_kernel(SpdStep p, double *__restrict__ logdet, int *__restrict__ info) {
+  typedef SpdDiagLds L;
+  constexpr int CT = L::CT, NB = SPD_NB;
+  __shared__ L sm;
+  const int b = blockIdx.x, nb = min(NB, p.MT - p.K0), tid = threadIdx.x;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane >> 4, lc = lane & 15;
+  double *work = p.work + b * SpdWork::size(p.MT);
+  // tiles (w / 4, w % 4) and two rows below; those past a last panel's nb blocks are the identity
+  gpx_d4 acc[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int I = w / NB + 2 * u, J = w % NB;
+    acc[u] = spd_step_load(p, b, p.K0 + min(I, nb - 1), p.K0 + min(J, nb - 1), lane);
+    if (I >= nb || J >= nb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[u][r] = I == J && lr + 4 * r == lc ? 1.0 : 0.0;
+  }
+  if (tid == 0) sm.step = 0;
+#pragma unroll 1
+  for (int K = 0; K < nb; ++K) {
+    double *rv = sm.rv[K & 1], *ct = sm.ct[K & 1];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) spd_publish<L>(rv, ct, K, K, w / NB + 2 * u, w % NB, acc[u], lane);
+    __syncthreads();
+    spd_panel(sm, rv, K, w, lane);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const double *pr = rv + (w % NB) * 256 + lane, *pc = ct + (w / NB + 2 * u) * CT + lr * 17 + lc;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) acc[u] = gpx_mfma16(pc[ks * 68], pr[ks * 64], acc[u]);
+    }
+    // the record of this block
+    for (int e = tid; e < 1024; e += 512) {
+      work[SpdWork::WD + K * 1024 + e] = rv[e];
+      const int I = e >> 8, ks = (e >> 6) & 3, l = e & 63;
+      work[SpdWork::COP + K * 1024 + e] = ct[I * CT + (l >> 4) * 17 + (l & 15) + ks * 68];
+    }
+    if (tid < 256) {
+      const int R = tid >> 6;
+      work[SpdWork::AOP + K * 256 + tid] = sm.pt[R][(4 * R + lr) * 17 + lc];
+    }
+    if (tid < 64) work[SpdWork::MUL + K * 64 + tid] = sm.mul[tid >> 4][tid & 15];
+  }
+  double *pivots = work + SpdWork::PIV;
+  if (tid < 16 * nb) pivots[16 * p.K0 + tid] = sm.piv[tid];
+  int fail = 0;
+  if (p.to < 0) {  // the last panel: every pivot is known
+    const double d = tid >= p.M ? 1.0 : (tid < 16 * p.K0 ? pivots[tid] : sm.piv[tid - 16 * p.K0]);
+    fail = spd_finish(sm, d, b, logdet, info);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int I = w / NB + 2 * u, J = w % NB;
+    if (I < nb && J < nb) spd_step_store(p, b, p.K0 + I, p.K0 + J, lane, acc[u], fail);
+  }
+}
+
+struct SpdSweepLds {
+  double rec[SpdWork::REC];
+  double wl[SPD_NB][256];
+  double ct[SPD_SWEEP][16 * 17];
+};
+
+__global__ __launch_bounds__(256) void spd_sweep_kernel(SpdStep p) {
+  __shared__ SpdSweepLds sm;
+  constexpr int NB = SPD_NB;
+  const int J = blockIdx.x, b = blockIdx.z, nb = min(NB, p.MT - p.K0), tid = threadIdx.x;
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane >> 4, lc = lane & 15;
+  const int own = J >= p.K0 && J < p.K0 + nb ? J - p.K0 : -1;  // the panel's own columns
+  const int row = blockIdx.y * SPD_SWEEP + w, I = row < p.K0 ? row : row + nb;
+  const bool on = w < SPD_SWEEP && I < p.MT;
+  const double *work = p.work + b * SpdWork::size(p.MT);
+  // waves 0-2: their row's panel columns and its tile of column J; wave 3: the panel's tiles of
+  // column J
+  gpx_d4 c[NB], v = gpx_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int kk = p.K0 + min(k, nb - 1);
+    c[k] = w < SPD_SWEEP ? spd_step_load(p, b, min(I, p.MT - 1), kk, lane) : spd_step_load(p, b, kk, J, lane);
+  }
+  if (own < 0 && w < SPD_SWEEP) v = spd_step_load(p, b, min(I, p.MT - 1), J, lane);
+  double wd[NB][NB][4];  // waves 0-2: Wd_l[k], l < k; wave 3: wd[k][0] = Wd_k[own]
+  if (w < SPD_SWEEP) {
+#pragma unroll
+    for (int k = 1; k < NB; ++k)
+#pragma unroll
+      for (int l = 0; l < k; ++l)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          wd[l][k][r] = work[SpdWork::WD + (min(l, nb - 1) * NB + min(k, nb - 1)) * 256 + r * 64 + lane];
+  } else if (own >= 0) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) wd[k][0][r] = work[SpdWork::WD + (min(k, nb - 1) * NB + own) * 256 + r * 64 + lane];
+  }
+  if (own < 0) {  // 16 bytes a lane: REC is even, the scratch 16-byte aligned from its base
+#pragma unroll
+    for (int u = 0; u < (SpdWork::REC / 2 + 255) / 256; ++u) {
+      const int e = min(tid + 256 * u, SpdWork::REC / 2 - 1);
+      ((double2 *)sm.rec)[e] = ((const double2 *)work)[e];
+    }
+  }
+  __syncthreads();
+  double a[NB][4];
+  if (w < SPD_SWEEP) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      if (k >= nb) break;
+#pragma unroll
+      for (int l = 0; l < k; ++l)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+          c[k] = gpx_mfma16(a[l][ks], wd[l][k][ks], c[k]);
+      double *t = sm.ct[w];
+      spd_wave_sync();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t[lc * 17 + lr + 4 * r] = -c[k][r];
+      spd_wave_sync();
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) a[k][ks] = t[lr * 17 + lc + ks * 68];
+    }
+  } else if (own >= 0) {
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sm.wl[k][r * 64 + lane] = wd[k][0][r];
+  } else {
+    double mul[NB][4], aop[NB][4];
+#pragma unroll
+    for (int K = 0; K < NB; ++K)
+#pragma unroll
+      for (int R = 0; R < 4; ++R) {
+        mul[K][R] = sm.rec[SpdWork::MUL + K * 64 + R * 16 + lc];
+        aop[K][R] = sm.rec[SpdWork::AOP + K * 256 + R * 64 + lane];
+      }
+#pragma unroll
+    for (int K = 0; K < NB; ++K) {
+      if (K >= nb) break;
+      gpx_d4 y = c[K];
+#pragma unroll
+      for (int R = 0; R < 4; ++R) {
+        double yr[4], m[4][4];
+        spd_rows4(y[R], yr);
+        spd_spread(mul[K][R], m, std::make_integer_sequence<int, 16>());
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          yr[g] *= m[g][g];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (i != g) yr[i] = fma(-m[g][i], yr[g], yr[i]);
+        }
+        const double py = spd_pick(yr[0], yr[1], yr[2], yr[3], lr);
+        y = gpx_mfma16(aop[K][R], -py, y);
+        y[R] = py;
+      }
+      c[K] = y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sm.wl[K][r * 64 + lane] = y[r];
+#pragma unroll
+      for (int d = 1; d < NB; ++d) {  // the next block's row first
+        const int i = (K + d) % NB;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+          c[i] = gpx_mfma16(sm.rec[SpdWork::COP + (K * NB + i) * 256 + ks * 64 + lane], y[ks], c[i]);
+      }
+    }
+  }
+  bool fail = false;
+  if (p.to < 0) {  // the last panel's launch knows every pivot
+    for (int k = lane; k < p.M; k += 64) {
+      const double d = work[SpdWork::PIV + k];
+      fail |= !(d > 0.0 && d < INFINITY);
+    }
+    fail = __any(fail);
+  }
+  __syncthreads();
+  if (w == SPD_SWEEP) {
+    if (own < 0 && blockIdx.y == 0)
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+        if (k < nb) spd_step_store(p, b, p.K0 + k, J, lane, c[k], fail);
+    return;
+  }
+  if (!on) return;
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    if (k >= nb || k < own) continue;  // a column of the panel starts from zero at its stage
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) v = gpx_mfma16(a[k][ks], sm.wl[k][ks * 64 + lane], v);
+  }
+  spd_step_store(p, b, I, J, lane, v, fail);
+}
+
+int launch_split(int M, int batch, const double *A, int lda, long sA, double *out, int ldo, long sO, double *logdet,
+                 int *info, double *work, hipStream_t st) {
+  const int MT = (M + 15) / 16;
+  SpdStep p = {A, lda, sA, out, ldo, sO, work, M, MT, 0, -1, -1};
+  for (int t = 0; p.K0 < MT; ++t, p.K0 += SPD_NB) {
+    const int nb = MT - p.K0 < SPD_NB ? MT - p.K0 : SPD_NB;
+    p.from = t ? (t - 1) & 1 : -1;
+    p.to = p.K0 + nb < MT ? t & 1 : -1;
+    hipLaunchKernelGGL(spd_diag_kernel, dim3(batch), dim3(512), 0, st, p, logdet, info);
+    GPX_CHECK_LAUNCH();
+    hipLaunchKernelGGL(spd_sweep_kernel, dim3(MT, gpx_cdiv(MT - nb, SPD_SWEEP), batch), dim3(256), 0, st, p);
+    GPX_CHECK_LAUNCH();
+  }
+  return GPX_OK;
+}
+
+// Whether the many-workgroup form is the faster one: it costs about 23 us per panel while its
+// sweeps' workgroups fit the chip, the other 6 to 18 us per block on one CU per matrix.  us, 1 / 4 /
+// 16 / 64 matrices, against one workgroup each: M = 144 60 / 60 / 70 / 116 : 59 / 59 / 60 / 62, 160
+// 64 / 65 / 76 / 130 : 73 / 74 / 74 / 77, 176 69 / 70 / 91 / 167 : 89 / 90 / 91 / 93, 200 84 / 86 / 120 / 237 :
+// 139 / 141 / 142 / 145, 256 96 / 99 / 155 / 382 : 288 / 289 / 291 / 298.
+bool split_wins(int MT, int batch) {
+  const long blocks = (long)batch * MT * gpx_cdiv(MT - SPD_NB, SPD_SWEEP);
+  return MT >= 12 ? blocks <= 1024 : MT >= 10 && blocks <= 256;
+}
+
 
 // Pivot-failure flags of several SPD launches folded into one status word pair:
 // status[0] = the largest info entry (0 = every matrix was positive definite),
@@ -574,6 +889,22 @@ int gpx_spd_inv_batched(int M, int batch, const double *A, int lda, long strideA
   if (!A || lda < M || (out && ldo < M)) return GPX_EINVAL;
   return kGJ[(M + 15) / 16 - 1](M, batch, A, lda, strideA, out, ldo, strideOut, logdet, info,
                                    (hipStream_t)stream);
+}
+
+// Scratch (doubles) of gpx_spd_inv_batched_ws; 0 where one workgroup per matrix is used anyway.
+long gpx_spd_workspace(int M, int batch) {
+  const int MT = (M + 15) / 16;
+  return M < 1 || M > 256 || batch < 1 || !split_wins(MT, batch) ? 0 : batch * SpdWork::size(MT);
+}
+
+// gpx_spd_inv_batched with scratch (16-byte aligned; NULL, or out NULL: as without).
+int gpx_spd_inv_batched_ws(int M, int batch, const double *A, int lda, long strideA, double *out, int ldo,
+                           long strideOut, double *logdet, int *info, double *work, void *stream) {
+  if (M < 0 || batch < 0 || M > 256) return GPX_EINVAL;
+  if (!work || !out || gpx_spd_workspace(M, batch) == 0)
+    return gpx_spd_inv_batched(M, batch, A, lda, strideA, out, ldo, strideOut, logdet, info, stream);
+  if (!A || lda < M || ldo < M) return GPX_EINVAL;
+  return launch_split(M, batch, A, lda, strideA, out, ldo, strideOut, logdet, info, work, (hipStream_t)stream);
 }
 
 }  // extern "C"

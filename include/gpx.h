@@ -63,6 +63,12 @@ int gpx_spd_max_m(void);
 int gpx_spd_inv_batched(int M, int batch, const double *A, int lda, long strideA, double *out,
                         int ldo, long strideOut, double *logdet, int *info, void *stream);
 
+/* The same with gpx_spd_workspace doubles of scratch (16-byte aligned), which lets several
+ * workgroups share a large matrix; work NULL, out NULL or a workspace of 0: as above. */
+long gpx_spd_workspace(int M, int batch);
+int gpx_spd_inv_batched_ws(int M, int batch, const double *A, int lda, long strideA, double *out, int ldo,
+                           long strideOut, double *logdet, int *info, double *work, void *stream);
+
 /* Folds the `info` arrays of up to 16 gpx_spd_inv_batched calls (host arrays of nlists
  * device pointers and their lengths) into a device status pair: status[0] = the largest
  * entry (0 when every matrix was positive definite), status[1] = max(status[1],
