@@ -22,6 +22,10 @@ SIGNATURES = {
                               _i, _i, _p, _i, _p]),
     'gpx_gemm_batched_ex': (_i, [_i, _i, _i, _i, _i, _d, _p, _i, _l, _p, _i, _l, _d, _p, _i, _l,
                                  _d, _p, _i, _l, _i, _i, _p, _i, _p]),
+    'gpx_gemm_batched_tail': (_i, [_i, _i, _i, _i, _i, _d, _p, _i, _l, _p, _i, _l, _d, _p, _i, _l, _d, _p, _i, _l, _p,
+                                   _i, _i, _p, _i, _p]),
+    'gpx_moments': (_i, [_i, _i, _i, _p, _p, _d, _d, _p, _p, _p]),
+    'gpx_kuu_tail': (_i, [_i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     'gpx_spd_max_m': (_i, []),
     'gpx_spd_inv_batched': (_i, [_i, _i, _p, _i, _l, _p, _i, _l, _p, _p, _p]),
     'gpx_spd_workspace': (_l, [_i, _i]),
@@ -54,6 +58,8 @@ SIGNATURES = {
     'gpx_emission_workspace': (_l, [_i, _i, _i]),
     'gpx_emission_tilted': (_i, [_i, _i, _i, _p, _p, _p, _i, _p, _i, _p, _i, _d, _d, _p, _p, _p,
                                  _p, _p, _p, _p]),
+    'gpx_vfe_kl_workspace': (_l, [_i, _i]),
+    'gpx_vfe_kl_ws': (_i, [_i, _i, _p, _p, _d, _p, _p, _p, _p, _p]),
     'gpx_vfe_kl': (_i, [_i, _i, _p, _p, _d, _p, _p, _p, _p]),
     'gpx_gauss_lik_exp': (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _d, _p, _p, _p, _p]),
     'gpx_probit_lik_exp': (_i, [_i, _i, _i, _i, _p, _p, _p, _d, _p, _p, _p, _p]),
@@ -218,10 +224,19 @@ def gemm(tA, tB, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch
          float(beta), P(C), ldc, sC, batch, splits, P(work), tile, S())
 
 
+class GemmTail(ctypes.Structure):
+    """GpxGemmTail of include/gpx.h."""
+    _fields_ = [('delta', _d), ('U', _p), ('V', _p), ('terms', _i), ('sU', _l), ('sV', _l), ('C2', _p), ('sC2', _l),
+                ('a2', _d), ('E2', _p), ('sE2', _l)]
+
+
 def mm(A, B, C, tA=False, tB=False, alpha=1.0, beta=0.0, splits=1, work=None, tile=0,
-       E=None, gamma=0.0):
+       E=None, gamma=0.0, outer=None, second=None):
     """C = alpha op(A) op(B) + beta C + gamma E for 2-D or batched 3-D contiguous
-    tensors; a 2-D operand (E included) is broadcast over the batch of a 3-D one."""
+    tensors; a 2-D operand (E included) is broadcast over the batch of a 3-D one.
+    outer = (U, V, delta): + delta sum_t U_t V_t^T (2-D C), or + delta U_b V_b^T in member b (3-D
+    C), U (., m) and V (., n).  second = (C2, a2, E2): C without the outer term, C2 = a2 (C +
+    outer) + E2 (E2 may be None)."""
     batch = max(t.shape[0] if t.dim() == 3 else 1 for t in (A, B, C))
     ar, ac = A.shape[-2:]
     br, bc = B.shape[-2:]
@@ -236,11 +251,31 @@ def mm(A, B, C, tA=False, tB=False, alpha=1.0, beta=0.0, splits=1, work=None, ti
     sC = m * n if C.dim() == 3 else 0
     if splits > 1 and work is None:
         work = torch.empty(splits * batch * m * n, dtype=torch.float64, device=C.device)
-    if E is None:
+    if E is None and outer is None and second is None:
         gemm(tA, tB, m, n, k, alpha, A, ac, sA, B, bc, sB, beta, C, n, sC, batch, splits, work, tile)
         return C
-    assert E.is_contiguous() and E.dtype == torch.float64 and E.shape[-2:] == (m, n), E.shape
-    sE = m * n if E.dim() == 3 else 0
+    sE = 0
+    if E is not None:
+        assert E.is_contiguous() and E.dtype == torch.float64 and E.shape[-2:] == (m, n), E.shape
+        sE = m * n if E.dim() == 3 else 0
+    if outer is not None or second is not None:
+        t = GemmTail()
+        if outer is not None:
+            U, V, t.delta = outer
+            assert U.is_contiguous() and V.is_contiguous() and U.shape[0] == V.shape[0]
+            assert U.shape[1] == m and V.shape[1] == n and U.dtype == V.dtype == torch.float64
+            assert C.dim() == 2 or U.shape[0] == batch
+            t.U, t.V, t.terms = P(U), P(V), U.shape[0] if C.dim() == 2 else 1
+            t.sU, t.sV = (0, 0) if C.dim() == 2 else (m, n)
+        if second is not None:
+            C2, t.a2, E2 = second
+            for x in (C2, E2):
+                assert x is None or (x.is_contiguous() and x.shape == C.shape and x.dtype == torch.float64)
+            t.C2, t.sC2, t.E2, t.sE2 = P(C2), m * n, P(E2), m * n
+        call('gpx_gemm_batched_tail', int(tA), int(tB), m, n, k, float(alpha), P(A), ac, sA, P(B), bc, sB,
+             float(beta), P(C), n, sC, float(gamma), P(E), n, sE, ctypes.addressof(t), batch, splits, P(work), tile,
+             S())
+        return C
     call('gpx_gemm_batched_ex', int(tA), int(tB), m, n, k, float(alpha), P(A), ac, sA, P(B), bc, sB,
          float(beta), P(C), n, sC, float(gamma), P(E), n, sE, batch, splits, P(work), tile, S())
     return C

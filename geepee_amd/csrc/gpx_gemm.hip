@@ -7,22 +7,50 @@
 // Split-K partial slabs (one per z-slice of the grid) are summed by a deterministic
 // second pass, so results do not depend on scheduling.
 #include "gpx_frag.h"
+#include "../../include/gpx.h"
 
 namespace {
 
 // Output epilogue: C = v + beta C + gamma E (beta == 0 never reads C; E may be NULL; an
-// E stride of 0 broadcasts one matrix over the batch).
+// E stride of 0 broadcasts one matrix over the batch).  With a tail (EXT kernels): the outer
+// products delta sum_t U_t V_t^T are added, to C or, if there is a C2, to C2 = a2 (C + outer) + E2.
 struct GemmEpi {
   double beta, gamma;
   const double *E;
   int ldE;
   long sE;
+  int ext;      // whether `t` counts
+  int um, vn;   // its rows: m, n
+  GpxGemmTail t;
 };
 
-__device__ __forceinline__ void epi_store(double *c, double v, const GemmEpi &ep, int b, int i, int j) {
+// Terms t0, t0 + step, ... of the tail's sum_t U_t[i] V_t[j].
+__device__ __forceinline__ double epi_outer(const GemmEpi &ep, int b, int i, int j, int t0, int step) {
+  const double *u = ep.t.U + b * ep.t.sU + i, *w = ep.t.V + b * ep.t.sV + j;
+  double s = 0.0;
+#pragma unroll 4
+  for (int t = t0; t < ep.t.terms; t += step) s = fma(u[(long)t * ep.um], w[(long)t * ep.vn], s);
+  return s;
+}
+
+// `outer`: epi_outer over all terms (formed here unless the caller has it).
+template <bool EXT, bool HAVE = false>
+__device__ __forceinline__ void epi_store(double *c, double v, const GemmEpi &ep, int b, int i, int j,
+                                          double outer = 0.0) {
   double r = v;
   if (ep.beta != 0.0) r += ep.beta * *c;
   if (ep.E) r += ep.gamma * ep.E[b * ep.sE + (long)i * ep.ldE + j];
+  if constexpr (EXT) {
+    if (ep.ext) {
+      const double s = r + ep.t.delta * (HAVE ? outer : epi_outer(ep, b, i, j, 0, 1));
+      if (ep.t.C2) {
+        const long e = (long)i * ep.vn + j;
+        ep.t.C2[b * ep.t.sC2 + e] = ep.t.E2 ? ep.t.a2 * s + ep.t.E2[b * ep.t.sE2 + e] : ep.t.a2 * s;
+      } else {
+        r = s;
+      }
+    }
+  }
   *c = r;
 }
 
@@ -35,25 +63,30 @@ constexpr int SPLITK_OUT = 32;
 __global__ __launch_bounds__(256) void splitk_reduce(int m, int n, int batch, int splits, double alpha,
                                                      const double *__restrict__ part, GemmEpi ep,
                                                      double *__restrict__ C, int ldc, long sC) {
-  __shared__ double red[8][SPLITK_OUT + 1];
+  __shared__ double red[8][SPLITK_OUT + 1], redo[8][SPLITK_OUT + 1];
   const long mn = (long)m * n, total = (long)batch * mn;
   const int o = threadIdx.x & (SPLITK_OUT - 1), g = threadIdx.x / SPLITK_OUT;
   const long e = (long)blockIdx.x * SPLITK_OUT + o;
+  const int b = (int)(e / mn);
+  const long r = e - b * mn;
+  const int i = (int)(r / n), j = (int)(r - (long)i * n);
   double s = 0.0;
   if (e < total) {
 #pragma unroll 4
     for (int q = g; q < splits; q += 8) s += part[(long)q * total + e];
   }
   red[g][o] = s;
+  // the tail's outer products, shared by the groups like the splits
+  redo[g][o] = ep.ext && e < total ? epi_outer(ep, b, i, j, g, 8) : 0.0;
   __syncthreads();
   if (g == 0 && e < total) {
-    double t = red[0][o];
+    double t = red[0][o], u = redo[0][o];
 #pragma unroll
-    for (int h = 1; h < 8; ++h) t += red[h][o];
-    const int b = (int)(e / mn);
-    const long r = e % mn;
-    const int i = (int)(r / n), j = (int)(r % n);
-    epi_store(C + b * sC + (long)i * ldc + j, alpha * t, ep, b, i, j);
+    for (int h = 1; h < 8; ++h) {
+      t += red[h][o];
+      u += redo[h][o];
+    }
+    epi_store<true, true>(C + b * sC + (long)i * ldc + j, alpha * t, ep, b, i, j, u);
   }
 }
 
@@ -69,7 +102,7 @@ __global__ __launch_bounds__(256) void rank1_kernel(int m, int n, int tA, int tB
   const int b = (int)(e / mn), r = (int)(e - b * mn), i = r / n, j = r - i * n;
   const double a = tA ? A[b * sA + i] : A[b * sA + (long)i * lda];
   const double bb = tB ? B[b * sB + (long)j * ldb] : B[b * sB + j];
-  epi_store(C + b * sC + (long)i * ldc + j, alpha * (a * bb), ep, b, i, j);
+  epi_store<true>(C + b * sC + (long)i * ldc + j, alpha * (a * bb), ep, b, i, j);
 }
 
 // n == 1: matrix-vector products.  One wave per output row: lanes stride over k, then a
@@ -87,7 +120,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB,
   for (int kk = lane; kk < k; kk += 64)
     s = fma(tA ? Ab[(long)kk * lda + i] : Ab[(long)i * lda + kk], tB ? Bb[kk] : Bb[(long)kk * ldb], s);
   s = gpx_wave_sum(s);
-  if (lane == 0) epi_store(C + b * sC + (long)i * ldc, alpha * s, ep, b, i, 0);
+  if (lane == 0) epi_store<true>(C + b * sC + (long)i * ldc, alpha * s, ep, b, i, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -188,7 +221,7 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
         if (gm < m && gn < n) {
           double *c = C + (long)gm * ldc + gn;
           if (raw) *c = v;
-          else epi_store(c, alpha * v, ep, bidx, gm, gn);
+          else epi_store<(TM < 4)>(c, alpha * v, ep, bidx, gm, gn);
         }
       }
     }
@@ -204,7 +237,7 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
         if (gm < m && gn < n) {
           double *c = C + (long)gm * ldc + gn;
           if (raw) *c = acc[i][j][r];
-          else epi_store(c, alpha * acc[i][j][r], ep, bidx, gm, gn);
+          else epi_store<(TM < 4)>(c, alpha * acc[i][j][r], ep, bidx, gm, gn);
         }
       }
 }
@@ -408,8 +441,8 @@ __global__ __launch_bounds__(256) void gram_reduce(int D, int M, int splits, con
 #pragma unroll
     for (int h = 1; h < 8; ++h) t += red[h][o];
     out += b * mm;
-    epi_store(out + (long)i * M + j, t, ep, b, i, j);
-    if (i != j) epi_store(out + (long)j * M + i, t, ep, b, j, i);
+    epi_store<true>(out + (long)i * M + j, t, ep, b, i, j);
+    if (i != j) epi_store<true>(out + (long)j * M + i, t, ep, b, j, i);
   }
 }
 
@@ -429,7 +462,7 @@ int gpx_gram(int N, int D, int M, const double *w, const double *X, int ldx, dou
   int kchunk = (N + splits - 1) / splits;
   kchunk = (kchunk + 7) / 8 * 8;
   splits = kchunk ? (N + kchunk - 1) / kchunk : 0;
-  const GemmEpi ep{0.0, gamma, E, M, strideE};
+  const GemmEpi ep{0.0, gamma, E, M, strideE, 0, M, M, GpxGemmTail{}};
   if (splits) {
     const int cb = (int)gpx_cdiv(gpx_cdiv(M, 16), 4);
     if ((long)cb * (cb + 1) / 2 > 65535) return GPX_ETOOBIG;
@@ -448,17 +481,18 @@ long gpx_gemm_workspace(int m, int n, int batch, int splits) {
   return splits > 1 ? (long)splits * batch * m * n : 0;
 }
 
-int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alpha,
+int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double alpha,
                         const double *A, int lda, long strideA,
                         const double *B, int ldb, long strideB,
                         double beta, double *C, int ldc, long strideC,
-                        double gamma, const double *E, int ldE, long strideE,
+                        double gamma, const double *E, int ldE, long strideE, const GpxGemmTail *tail,
                         int batch, int splits, double *work, int tile, void *stream) {
   if (m < 0 || n < 0 || k < 0 || batch < 0 || splits < 1) return GPX_EINVAL;
   if (E && (ldE < n || strideE < 0)) return GPX_EINVAL;
-  GemmEpi ep{beta, gamma, E, ldE, strideE};
+  GemmEpi ep{beta, gamma, E, ldE, strideE, tail != nullptr, m, n, tail ? *tail : GpxGemmTail{}};
   if (m == 0 || n == 0 || batch == 0) return GPX_OK;
   if (!A || !B || !C) return GPX_EINVAL;
+  if (tail && (tail->terms < 0 || (tail->terms && (!tail->U || !tail->V)))) return GPX_EINVAL;
   if (splits > 1 && !work) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   if (k == 0) {  // C = beta * C
@@ -491,13 +525,14 @@ int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alph
 #define GEMM_DIRECT(TM, KW)                                                                                       \
   gemm_direct<TM, KW>(transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch, \
                       splits, kchunk, part, st)
+  // (with a tail never 64 x 64 per wave: its 64 stores per lane each carry the epilogue)
   // 64 x 64 per wave once there are two such tiles per SIMD (20000 x n x n, 4 products, us
   // against 32 x 32: n = 256 172 : 228, 200 125 : 133, 128 (2504 tiles) 63 : 65; 5000 x 100 x 100, 4
   // (632 tiles) 24 : 18).  16 x 16 per workgroup, its waves sharing k, where those are at most three
   // per CU (against 32 x 32: 128^3 4.4 : 5.5, 200^3, 4 (676 tiles) 5.8 : 6.0, 128^3, 32 (2048) 13 : 7.8).
   // Else 32 x 32, a tile per wave if that makes a wave per SIMD (4001 x 256 x 256 (1008) 17.4 : 18.3;
   // 128^3, 32 (512) 10.5 : 8.8) or if k leaves four waves nothing to share.
-  if (tile == 64 || (tile != 32 && t4 >= 2048 && k >= 64)) rc = GEMM_DIRECT(4, 1);
+  if (!tail && (tile == 64 || (tile != 32 && t4 >= 2048 && k >= 64))) rc = GEMM_DIRECT(4, 1);
   else if (tile != 32 && t1 <= 768) rc = GEMM_DIRECT(1, 4);
   else if (t2 >= 1024 || k <= 32) rc = GEMM_DIRECT(2, 1);
   else rc = GEMM_DIRECT(2, 4);
@@ -510,6 +545,16 @@ int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alph
     GPX_CHECK_LAUNCH();
   }
   return GPX_OK;
+}
+
+int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alpha,
+                        const double *A, int lda, long strideA,
+                        const double *B, int ldb, long strideB,
+                        double beta, double *C, int ldc, long strideC,
+                        double gamma, const double *E, int ldE, long strideE,
+                        int batch, int splits, double *work, int tile, void *stream) {
+  return gpx_gemm_batched_tail(transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
+                               strideC, gamma, E, ldE, strideE, nullptr, batch, splits, work, tile, stream);
 }
 
 int gpx_gemm_batched(int transA, int transB, int m, int n, int k, double alpha,

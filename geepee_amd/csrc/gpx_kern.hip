@@ -206,8 +206,8 @@ template <int QT>
 __global__ __launch_bounds__(256) void dtrace_kernel(int M, const double *__restrict__ Mm,
                                                      const double *__restrict__ z,
                                                      const double *__restrict__ ls,
-                                                     const double *__restrict__ sf,
-                                                     double *__restrict__ gz, double *__restrict__ part) {
+                                                     const double *__restrict__ sf, const double *dz0,
+                                                     double *gz, double *__restrict__ part) {
   __shared__ double zs[QT][256];
   __shared__ double ils[QT];
   const int tid = threadIdx.x, lane = tid & 63, a = blockIdx.x * 4 + (tid >> 6);
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(256) void dtrace_kernel(int M, const double *__rest
   for (int q = 0; q < QT; ++q)
     if (lane == q) {
       part[(long)a * (QT + 1) + 1 + q] = gl[q];
-      gz[a * QT + q] = -gzq[q] * il[q];
+      gz[a * QT + q] = dz0 ? dz0[a * QT + q] - gzq[q] * il[q] : -gzq[q] * il[q];
     }
 }
 
@@ -266,6 +266,75 @@ __global__ __launch_bounds__(64) void dtrace_final(int M, int Q, const double *_
   if (lane == 0) {
     if (j == 0) gsf[0] = s;
     else gls[j - 1] = s;
+  }
+}
+
+// dtrace_final with the chain rule of the log hyper-parameters (hyper_kernel) applied.
+__global__ __launch_bounds__(64) void kuu_tail_kernel(int M, int Q, const double *__restrict__ part,
+                                                      const double *__restrict__ ls, const double *__restrict__ sf,
+                                                      const double *__restrict__ dell,
+                                                      const double *__restrict__ dsf2,
+                                                      const double *__restrict__ sumdv, double *__restrict__ dls,
+                                                      double *__restrict__ dsf) {
+  const int j = blockIdx.x, lane = threadIdx.x;
+  double s = 0.0;
+  for (int a = lane; a < M; a += 64) s += part[(long)a * (Q + 1) + j];
+  s = gpx_wave_sum(s);
+  if (lane != 0) return;
+  if (j == 0) dsf[0] = 2.0 * exp(2.0 * sf[0]) * (dsf2[0] + sumdv[0]) + 2.0 * s;
+  else dls[j - 1] = dell[j - 1] * exp(ls[j - 1]) + 2.0 * s;
+}
+
+// mu_b = s_b S_b t_b and P_b = S_b + mu_b mu_b^T.  Workgroup (b, y) forms all of mu_b (a wave per
+// row, four rows in flight; the matrix comes from the caches the second time) and the rows of
+// P_b of its share y.  In place of a product and an outer product per set: M = 50, 2 sets 11 -> 3 us.
+__global__ __launch_bounds__(1024) void moments_kernel(int D, int M, const double *__restrict__ S,
+                                                       const double *__restrict__ theta, double s0, double s1,
+                                                       double *__restrict__ mu, double *__restrict__ P) {
+  __shared__ double m[256];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nj = (M + 63) >> 6;
+  const double *Sb = S + (long)b * M * M, *t = theta + (long)(b % D) * M;
+  const double scale = b < D ? s0 : s1;
+  double tv[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) tv[j] = lane + 64 * j < M ? t[lane + 64 * j] : 0.0;
+  for (int i0 = w; i0 < M; i0 += 64) {  // rows i0 + 16 u
+    double sv[4][4], acc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sv[u][j] = j < nj ? Sb[(long)min(i0 + 16 * u, M - 1) * M + min(lane + 64 * j, M - 1)] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      acc[u] = 0.0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (lane + 64 * j < M) acc[u] = fma(sv[u][j], tv[j], acc[u]);
+      acc[u] = gpx_wave_sum(acc[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (lane == 0 && i0 + 16 * u < M) m[i0 + 16 * u] = scale * acc[u];
+  }
+  __syncthreads();
+  if (blockIdx.y == 0 && tid < M) mu[(long)b * M + tid] = m[tid];
+  const int rows = (M + gridDim.y - 1) / gridDim.y, r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
+  double *Pb = P + (long)b * M * M;
+  for (int i0 = r0 + w; i0 < r1; i0 += 64) {
+    double sv[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sv[u][j] = j < nj ? Sb[(long)min(i0 + 16 * u, M - 1) * M + min(lane + 64 * j, M - 1)] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + 16 * u, c = lane + 64 * j;
+        if (i < r1 && c < M) Pb[(long)i * M + c] = m[i] * m[c] + sv[u][j];
+      }
   }
 }
 
@@ -934,6 +1003,21 @@ int gpx_kfu_bwd(int N, int M, int Q, const double *dK, const double *K, const do
 
 long gpx_dtrace_workspace(int M, int Q) { return (long)M * (Q + 1); }
 
+static int launch_dtrace(int M, int Q, const double *Mm, const double *z, const double *ls, const double *sf,
+                         const double *dz0, double *gz, double *work, hipStream_t st) {
+  switch (Q) {
+#define GPX_DT(QV)                                                                                               \
+  case QV:                                                                                                       \
+    hipLaunchKernelGGL((dtrace_kernel<QV>), dim3(gpx_cdiv(M, 4)), dim3(256), 0, st, M, Mm, z, ls, sf, dz0, gz, work); \
+    break;
+    GPX_DT(1) GPX_DT(2) GPX_DT(3) GPX_DT(4) GPX_DT(5) GPX_DT(6) GPX_DT(7) GPX_DT(8)
+    GPX_DT(9) GPX_DT(10) GPX_DT(11) GPX_DT(12) GPX_DT(13) GPX_DT(14) GPX_DT(15) GPX_DT(16)
+#undef GPX_DT
+  }
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
 // d tr(Mm Kzz) / d(lsf, lls, z) for Kzz = SE(z, z): gsf (1), gls (Q), gz (M x Q).
 int gpx_dtrace_kzz(int M, int Q, const double *Mm, const double *z, const double *ls,
                    const double *sf, double *gsf, double *gls, double *gz, double *work,
@@ -941,17 +1025,35 @@ int gpx_dtrace_kzz(int M, int Q, const double *Mm, const double *z, const double
   if (M < 1 || M > 256 || Q < 1 || Q > 16 || !Mm || !z || !ls || !sf || !gsf || !gls || !gz || !work)
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  switch (Q) {
-#define GPX_DT(QV)                                                                                        \
-  case QV:                                                                                                \
-    hipLaunchKernelGGL((dtrace_kernel<QV>), dim3(gpx_cdiv(M, 4)), dim3(256), 0, st, M, Mm, z, ls, sf, gz, work); \
-    break;
-    GPX_DT(1) GPX_DT(2) GPX_DT(3) GPX_DT(4) GPX_DT(5) GPX_DT(6) GPX_DT(7) GPX_DT(8)
-    GPX_DT(9) GPX_DT(10) GPX_DT(11) GPX_DT(12) GPX_DT(13) GPX_DT(14) GPX_DT(15) GPX_DT(16)
-#undef GPX_DT
-  }
-  GPX_CHECK_LAUNCH();
+  const int rc = launch_dtrace(M, Q, Mm, z, ls, sf, nullptr, gz, work, st);
+  if (rc != GPX_OK) return rc;
   hipLaunchKernelGGL(dtrace_final, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)work, gsf, gls);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
+int gpx_kuu_tail(int M, int Q, const double *Mm, const double *z, const double *ls, const double *sf,
+                 const double *dell, const double *dsf2, const double *sumdv, const double *dz0, double *dls,
+                 double *dsf, double *dZ, double *work, void *stream) {
+  if (M < 1 || M > 256 || Q < 1 || Q > 16 || !Mm || !z || !ls || !sf || !dell || !dsf2 || !sumdv || !dz0 || !dls ||
+      !dsf || !dZ || !work)
+    return GPX_EINVAL;
+  hipStream_t st = (hipStream_t)stream;
+  const int rc = launch_dtrace(M, Q, Mm, z, ls, sf, dz0, dZ, work, st);
+  if (rc != GPX_OK) return rc;
+  hipLaunchKernelGGL(kuu_tail_kernel, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)work, ls, sf, dell, dsf2,
+                     sumdv, dls, dsf);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
+int gpx_moments(int batch, int D, int M, const double *S, const double *theta, double s0, double s1, double *mu,
+                double *P, void *stream) {
+  if (batch < 0 || D < 1 || M < 1 || M > 256) return GPX_EINVAL;
+  if (batch == 0) return GPX_OK;
+  if (!S || !theta || !mu || !P) return GPX_EINVAL;
+  hipLaunchKernelGGL(moments_kernel, dim3(batch, gpx_cdiv(M, 64)), dim3(1024), 0, (hipStream_t)stream, D, M, S, theta,
+                     s0, s1, mu, P);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }

@@ -15,9 +15,10 @@ def empty(*shape, like=None, device='cuda'):
     return torch.empty(*shape, dtype=F64, device=like.device if like is not None else device)
 
 
-def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=None, gamma=0.0):
+def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=None, gamma=0.0, outer=None,
+       second=None):
     """C = alpha op(A) op(B) + beta C + gamma E (2-D or batched 3-D; 2-D operands
-    broadcast; E is added in the product's own epilogue).
+    broadcast; E, and outer and second as in _lib.mm, ride in the product's own epilogue).
     Picks a split-K factor when the output has few tiles and K is long (a tuned plan
     for the shape, if the autotuner stored one, wins)."""
     if C is None:
@@ -42,7 +43,7 @@ def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=Non
                 # long, skinny contractions: split K so that enough workgroups run
                 splits = max(1, min(-(-512 // tiles), k // 512, 64))
     return _lib.mm(A, B, C, tA=tA, tB=tB, alpha=alpha, beta=beta, splits=splits, tile=tile,
-                   E=E, gamma=gamma)
+                   E=E, gamma=gamma, outer=outer, second=second)
 
 
 def spd_inv(A, out=None):
@@ -265,6 +266,24 @@ def dtrace(Mm, z, ls, sf):
     work = empty(query('gpx_dtrace_workspace', M, Q), like=z)
     call('gpx_dtrace_kzz', M, Q, P(Mm), P(z), P(ls), P(sf), *[P(o) for o in outs], P(work), S())
     return outs
+
+
+def kuu_tail(Mm, z, ls, sf, dell, dsf2, sumdv, dz):
+    """(dls, dsf, dzu): the hyper-parameter gradients with the trace terms of Kuu's adjoint Mm."""
+    M, Q = z.shape
+    dls, dsf, dzu = torch.empty_like(ls), torch.empty_like(sf), torch.empty_like(dz)
+    work = empty(query('gpx_dtrace_workspace', M, Q), like=z)
+    call('gpx_kuu_tail', M, Q, P(Mm), P(z), P(ls), P(sf), P(dell), P(dsf2), P(sumdv), P(dz), P(dls), P(dsf), P(dzu),
+         P(work), S())
+    return dls, dsf, dzu
+
+
+def moments(cov, theta, s0, s1=0.0):
+    """mu (b, M) = s cov_b theta_(b mod D) and cov + mu mu^T, s = s0 for the first D, then s1."""
+    b, M = cov.shape[:2]
+    mu, second = empty(b, M, like=cov), torch.empty_like(cov)
+    call('gpx_moments', b, theta.shape[0], M, P(cov), P(theta), float(s0), float(s1), P(mu), P(second), S())
+    return mu, second
 
 
 def gauss_tilted(m, v, y, sn, alpha, scale, want_dmall=False):

@@ -130,11 +130,12 @@ class SGP_Layer(object):
         self.Su, self.Suhat = cov[:D], cov[D:]
         self.ld_Suinv, self.ld_Suhatinv = ld[:D], ld[D:]
         self.info_Su, self.info_Suhat = info[:D], info[D:]
-        self.mu = mm(self.Su, _col(self.theta_2)).reshape(D, M)
+        # posterior and cavity means and second moments in one launch
+        mu, second = dops.moments(cov, self.theta_2, 1.0, beta)
+        self.mu, self.muhat = mu[:D], mu[D:]
+        self.Splusmm, self.Splusmmhat = second[:D], second[D:]
         self._ld_post, self._sgn_post = self.ld_Suinv, -1.0
-        self.Splusmm = _plus_outer(self.Su, self.mu, self.mu)
         self._pred_ready = False
-        self.muhat = mm(self.Suhat, _col(self.theta_2), alpha=beta).reshape(D, M)
         self._beta, self._alpha = beta, alpha
         self._cavity_tail()
 
@@ -148,14 +149,14 @@ class SGP_Layer(object):
             R = self.theta_1_R
             self.Suinv = mm(R, R, dops.empty(D, M, M, like=self.Kuu), tA=True, E=self.Kuuinv, gamma=1.0)
             self.Su, self.ld_Suinv, self.info_Su = dops.spd_inv(self.Suinv)
-            self.mu = mm(self.Su, _col(self.theta_2)).reshape(D, M)
+            self.mu, self.Splusmm = dops.moments(self.Su, self.theta_2, 1.0)
             self._ld_post, self._sgn_post = self.ld_Suinv, -1.0
         else:
             self.Su = self.theta_1
             self.Suinv, self.ld_Su, self.info_Su = dops.spd_inv(self.Su)
             self.mu = self.theta_2
             self._ld_post, self._sgn_post = self.ld_Su, 1.0
-        self.Splusmm = _plus_outer(self.Su, self.mu, self.mu)
+            self.Splusmm = _plus_outer(self.Su, self.mu, self.mu)
         self._pred_ready = False
 
     def _posterior_predictive(self):
@@ -181,13 +182,14 @@ class SGP_Layer(object):
             R = self.theta_1_R
             self.Suhatinv = mm(R, R, dops.empty(D, M, M, like=Ki), tA=True, alpha=beta, E=Ki, gamma=1.0)
             self.Suhat, self.ld_Suhatinv, self.info_Suhat = dops.spd_inv(self.Suhatinv)
-            self.muhat = mm(self.Suhat, _col(self.theta_2), alpha=beta).reshape(D, M)
+            self.muhat, self.Splusmmhat = dops.moments(self.Suhat, self.theta_2, beta)
         else:
             # Kuuinv + beta (Suinv - Kuuinv);  muhat = Suhat beta Suinv mu
             self.Suhatinv = lincomb(dops.empty(D, M, M, like=Ki), 1.0 - beta, Ki, beta, self.Suinv)
             self.Suhat, self.ld_Suhatinv, self.info_Suhat = dops.spd_inv(self.Suhatinv)
             f2 = mm(self.Suinv, _col(self.mu))
             self.muhat = mm(self.Suhat, f2, alpha=beta).reshape(D, M)
+            self.Splusmmhat = _plus_outer(self.Suhat, self.muhat, self.muhat)
         self._cavity_tail()
 
     def adjoint_constants(self, kind, alpha=None):
@@ -235,15 +237,16 @@ class SGP_Layer(object):
         return c
 
     def _cavity_tail(self):
-        """Ahat, Bhat_sto, Bhat_det from muhat, Suhat (aep_models.py:535-546):
+        """Ahat, Bhat_sto, Bhat_det from muhat, Suhat (aep_models.py:535-546; muhat, Suhat and
+        Splusmmhat are there):
         Bhat_det = Ki Suhat Ki - Ki (the -Ki in the second product's epilogue) and
         Bhat_sto = Ki (Suhat + muhat muhat^T) Ki - Ki = Bhat_det + Ahat Ahat^T, since
         Ahat = Ki muhat."""
         Ki = self.Kuuinv
         self.Ahat = mm(self.muhat, Ki, tB=True)
-        self.Splusmmhat = _plus_outer(self.Suhat, self.muhat, self.muhat)
-        self.Bhat_det = _sandwich(Ki, self.Suhat, Ki, E=Ki, gamma=-1.0)
-        self.Bhat_sto = _plus_outer(self.Bhat_det, self.Ahat, self.Ahat)
+        self.Bhat_sto = torch.empty_like(self.Suhat)
+        self.Bhat_det = mm(Ki, mm(self.Suhat, Ki), E=Ki, gamma=-1.0, outer=(self.Ahat, self.Ahat, 1.0),
+                           second=(self.Bhat_sto, 1.0, None))
         # the fused kernels' operand layout, formed with the rest of the q(u) set-up (off the
         # forward pass's critical path in a deep GP)
         self._Bp = None
@@ -426,9 +429,7 @@ class SGP_Layer(object):
         if dKi_post is not None:
             lincomb(dKi, 1.0, dKi, 1.0, dKi_post)
         M_inner = _sandwich(Ki, dKi, Ki, alpha=-1.0)
-        gsf, gls, gz = dops.dtrace(M_inner, self.zu, self.ls, self.sf)
-        dls, dsf = dops.hyper(self.ls, self.sf, dell, gls, dsf2, sumdv, gsf)
-        lincomb(dzu, 1.0, dzu, 1.0, gz)
+        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
         deta1 = lincomb(deta1_cav, 1.0, deta1_cav, 1.0, deta1_post)
         deta2 = lincomb(deta2_cav, 1.0, deta2_cav, 1.0, deta2_post)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': deta2}
@@ -464,20 +465,18 @@ class SGP_Layer(object):
         # cavity: dmu_cav, dSu_cav (+ the normalising factor), then dSuinv_cav
         c = self._adjoint('reg', alpha)
         dmucav = mm(dAhat, Ki, E=th, gamma=scale_cav * beta)
-        dSucav = mm(Ki, mm(dBhat, Ki), tA=True, E=c['Ecav'], gamma=1.0)
-        _add_outer(dSucav, dmucav, th, beta)
-        dS_cav = _sandwich(self.Suhat, dSucav, self.Suhat, alpha=-1.0)
-        # posterior chain (data independent, from adjoint_constants)
-        deta1 = dops.pack_dR(self.theta_1_R, lincomb(dSucav, beta, dS_cav, 1.0, c['dS_post']))
+        dSucav = mm(Ki, mm(dBhat, Ki), tA=True, E=c['Ecav'], gamma=1.0, outer=(dmucav, th, beta))
+        # with the posterior chain (data independent, from adjoint_constants) for theta1
+        dtheta1 = torch.empty_like(dSucav)
+        dS_cav = mm(self.Suhat, mm(dSucav, self.Suhat), alpha=-1.0, second=(dtheta1, beta, c['dS_post']))
+        deta1 = dops.pack_dR(self.theta_1_R, dtheta1)
         deta2 = mm(self.Suhat, _col(dmucav), alpha=beta, E=_col(self.mu), gamma=scale_post).reshape(D, M)
         # Kuuinv: phi prior, Ahat, Bhat_det, cavity, posterior
-        dKi = mm(dAhat, self.muhat, tA=True, E=c['Kc'], gamma=1.0)
-        mm(c['KiS2'].reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0)
+        dKi = mm(c['KiS2'].reshape(D * M, M), dBhat.reshape(D * M, M), tA=True, E=c['Kc'], gamma=1.0,
+                 outer=(dAhat, self.muhat, 1.0))
         colsum(dS_cav, D, M * M, out=dKi.reshape(-1), beta=1.0)
         M_inner = _sandwich(Ki, dKi, Ki, alpha=-1.0)
-        gsf, gls, gz = dops.dtrace(M_inner, self.zu, self.ls, self.sf)
-        dls, dsf = dops.hyper(self.ls, self.sf, dell, gls, dsf2, sumdv, gsf)
-        lincomb(dzu, 1.0, dzu, 1.0, gz)
+        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': deta2}
 
     def backprop_grads_lvm_mc(self, m, v, dm, dv, kfu, x, alpha=1.0):
@@ -509,15 +508,12 @@ class SGP_Layer(object):
         deta1 = dops.pack_dR(self.theta_1_R, dtheta1)
         dAhat = mm(dm, kfu, tA=True)
         dKi = colsum(dSinv, D, M * M).reshape(M, M)
-        mm(dAhat, self.muhat, dKi, tA=True, beta=1.0)
         dBhat = dops.gram(dv, kfu)
         KiS2 = mm(Ki, self.Suhat, alpha=2.0, E=_eye(M, Ki), gamma=-1.0)
-        mm(KiS2.reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0)
+        mm(KiS2.reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0, outer=(dAhat, self.muhat, 1.0))
         Minner = lincomb(torch.empty_like(dKi), 1.0, c['Mc'], -2.0, dKi)
         M_all = _sandwich(Ki, Minner, Ki, alpha=0.5, E=Ki, gamma=0.5 * D)
-        gsf, gls, gz = dops.dtrace(M_all, self.zu, self.ls, self.sf)
-        dls, dsf = dops.hyper(self.ls, self.sf, dell, gls, dsf2, sumdv, gsf)
-        lincomb(dzu, 1.0, dzu, 1.0, gz)
+        dls, dsf, dzu = dops.kuu_tail(M_all, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': dtheta2}, dx
 
     def backprop_grads_reparam(self, dx, mx, vx, eps):
@@ -591,18 +587,16 @@ class SGP_Layer(object):
         dmcav = mm(dvcav, _col(self.muhat), alpha=2.0).reshape(D, M)
         mm(dAhat, Ki, dmcav, tB=True, beta=1.0)
         _add_outer(dvcav, dmcav, self.theta_2, beta)
-        dvcavinv = _sandwich(self.Suhat, dvcav, self.Suhat, alpha=-1.0)
         c = self._adjoint('mm', alpha)
+        dtheta1 = torch.empty_like(dvcav)
+        dvcavinv = mm(self.Suhat, mm(dvcav, self.Suhat), alpha=-1.0, second=(dtheta1, beta, c['T1']))
         dtheta2 = mm(self.Suhat, _col(dmcav), alpha=beta, E=_col(c['c2']), gamma=1.0).reshape(D, M)
         dKi = colsum(dvcavinv, D, M * M).reshape(M, M)
-        mm(dAhat, self.muhat, dKi, tA=True, beta=1.0)
         # 2 sum_d KiS_d^T dBhat_d - sum_d dBhat_d as one product with KiS2 = 2 KiS - I
-        mm(c['KiS2'].reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0)
-        dtheta1 = lincomb(torch.empty_like(dvcavinv), beta, dvcavinv, 1.0, c['T1'])
+        mm(c['KiS2'].reshape(D * M, M), dBhat.reshape(D * M, M), dKi, tA=True, beta=1.0,
+           outer=(dAhat, self.muhat, 1.0))
         deta1 = dops.pack_dR(self.theta_1_R, dtheta1)
         # M_all = Ki (Mc - 2 dKi) Ki / 2 + (D/2) Ki, with Mc Ki from the adjoint constants
         M_all = mm(Ki, mm(dKi, Ki, alpha=-2.0, E=c['McKi'], gamma=1.0), alpha=0.5, E=Ki, gamma=0.5 * D)
-        gsf, gls, gz = dops.dtrace(M_all, self.zu, self.ls, self.sf)
-        dls, dsf = dops.hyper(self.ls, self.sf, dell, gls, dsf2, sumdv, gsf)
-        dzu = lincomb(torch.empty_like(dzu), 1.0, dzu, 1.0, gz)
+        dls, dsf, dzu = dops.kuu_tail(M_all, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': dtheta2}

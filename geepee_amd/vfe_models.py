@@ -119,8 +119,9 @@ class SGP_Layer(_Layer):
     def compute_KL(self):
         """SGP_Layer.compute_KL (vfe_models.py:309-326) as a device scalar (1,)."""
         out = dops.empty(1, like=self.Kuu)
-        call('gpx_vfe_kl', self.Dout, self.M, P(self.ld_Kuu), P(self._ld_post), float(self._sgn_post),
-             P(self.Kuuinv), P(self.Splusmm), P(out), _lib.S())
+        work = dops.empty(query('gpx_vfe_kl_workspace', self.Dout, self.M), like=self.Kuu)
+        call('gpx_vfe_kl_ws', self.Dout, self.M, P(self.ld_Kuu), P(self._ld_post), float(self._sgn_post),
+             P(self.Kuuinv), P(self.Splusmm), P(out), P(work), _lib.S())
         return out
 
     def forward_post_det(self, x):
@@ -145,9 +146,7 @@ class SGP_Layer(_Layer):
         """Kuu^-1's adjoint through Kuu into the hyper-parameters."""
         Ki = self.Kuuinv
         M_inner = _sandwich(Ki, dKi, Ki, alpha=-1.0)
-        gsf, gls, gz = dops.dtrace(M_inner, self.zu, self.ls, self.sf)
-        dls, dsf = dops.hyper(self.ls, self.sf, dell, gls, dsf2, sumdv, gsf)
-        lincomb(dzu, 1.0, dzu, 1.0, gz)
+        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
         return dsf, dls, dzu
 
     def backprop_grads_reg(self, m, v, dm, dv, kfu, x, want_dx=False):
@@ -170,9 +169,9 @@ class SGP_Layer(_Layer):
         dSu = dops.gram(dv, kfuKi, E=self._C0, gamma=1.0)
         deta1, deta2, dKi_u = self._post_grad_u(dmu, dSu)
         dA = mm(dm, kfu, tA=True)
-        dKi = mm(dA, self.mu, tA=True, E=self._Kc, gamma=1.0)
         dB = dops.gram(dv, kfu)
-        mm(self._kis2('det').reshape(D * M, M), dB.reshape(D * M, M), dKi, tA=True, beta=1.0)
+        dKi = mm(self._kis2('det').reshape(D * M, M), dB.reshape(D * M, M), tA=True, E=self._Kc, gamma=1.0,
+                 outer=(dA, self.mu, 1.0))
         if dKi_u is not None:
             lincomb(dKi, 1.0, dKi, 1.0, dKi_u)
         dsf, dls, dzu = self._kuu_tail(dKi, dsf2, dell, dzu, sumdv)
@@ -201,8 +200,8 @@ class SGP_Layer(_Layer):
         mm(dA, Ki, dmu, tB=True, beta=1.0)
         lincomb(dSu, 1.0, dSu, 1.0, self._C0)
         deta1, deta2, dKi_u = self._post_grad_u(dmu, dSu)
-        dKi = mm(dA, self.mu, tA=True, E=self._Kc, gamma=1.0)
-        mm(self._kis2('mm').reshape(D * M, M), dB.reshape(D * M, M), dKi, tA=True, beta=1.0)
+        dKi = mm(self._kis2('mm').reshape(D * M, M), dB.reshape(D * M, M), tA=True, E=self._Kc, gamma=1.0,
+                 outer=(dA, self.mu, 1.0))
         if dKi_u is not None:
             lincomb(dKi, 1.0, dKi, 1.0, dKi_u)
         dsf, dls, dzu = self._kuu_tail(dKi, dsf2, dell, dzu, sumdv)

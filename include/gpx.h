@@ -52,6 +52,41 @@ int gpx_gemm_batched_ex(int transA, int transB, int m, int n, int k, double alph
                         double gamma, const double *E, int ldE, long strideE, int batch,
                         int splits, double *work, int tile, void *stream);
 
+/* gpx_gemm_batched_ex with outer products and a second output in the same pass: with
+ *   R = alpha op(A[b]) op(B[b]) + beta C[b] + gamma E[b],  S = R + delta sum_t U[b][t] V[b][t]^T
+ * C[b] = S, or with C2: C[b] = R and C2[b] = a2 S + E2[b].  U[b] is terms x m, V[b] terms x n, C2
+ * and E2 (NULL: none) m x n, all contiguous at the given batch strides.  tail NULL: as without. */
+typedef struct GpxGemmTail {
+  double delta;
+  const double *U, *V;
+  int terms;
+  long sU, sV;
+  double *C2;
+  long sC2;
+  double a2;
+  const double *E2;
+  long sE2;
+} GpxGemmTail;
+int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double alpha,
+                          const double *A, int lda, long strideA,
+                          const double *B, int ldb, long strideB,
+                          double beta, double *C, int ldc, long strideC,
+                          double gamma, const double *E, int ldE, long strideE, const GpxGemmTail *tail,
+                          int batch, int splits, double *work, int tile, void *stream);
+
+/* Means and second moments of q(u) from its covariances S (batch x M x M): mu_b = s_b S_b t_b and
+ * P_b = S_b + mu_b mu_b^T, with t_b = theta[b % D] (D x M) and s_b = s0 for b < D, s1 from there on
+ * (posterior and cavity in one launch; geepee/base_models.py:470-476, aep_models.py:528-537). */
+int gpx_moments(int batch, int D, int M, const double *S, const double *theta, double s0, double s1, double *mu,
+                double *P, void *stream);
+
+/* Kuu^-1's adjoint into the hyper-parameters: gpx_dtrace_kzz and gpx_hyper_grads in two launches, and
+ * dZ = dz0 + its z gradient (dZ may be dz0; work: gpx_dtrace_workspace doubles).  Replaces
+ * geepee/aep_models.py:244-247, 296-304. */
+int gpx_kuu_tail(int M, int Q, const double *Mm, const double *z, const double *ls, const double *sf,
+                 const double *dell, const double *dsf2, const double *sumdv, const double *dz0, double *dls,
+                 double *dsf, double *dZ, double *work, void *stream);
+
 /* Batched SPD inverse and log-determinant, one workgroup per matrix (M <= 256):
  * out[b] = inv(A[b]) (out may alias A or be NULL), logdet[b] = log det A[b],
  * info[b] = 0 or k+1 when pivot k is not positive (outputs NaN).  A[b] is read whole and
@@ -303,6 +338,10 @@ int gpx_emission_predict(int Nb, int Dout, int Din, const double *C, const doubl
  * parameterisation).  Replaces SGP_Layer.compute_KL (geepee/vfe_models.py:309-326). */
 int gpx_vfe_kl(int D, int M, const double *ldK, const double *ldS, double sgnS, const double *Kuuinv,
                const double *Splusmm, double *out, void *stream);
+/* The same with gpx_vfe_kl_workspace doubles of scratch: the trace over many workgroups. */
+long gpx_vfe_kl_workspace(int D, int M);
+int gpx_vfe_kl_ws(int D, int M, const double *ldK, const double *ldS, double sgnS, const double *Kuuinv,
+                  const double *Splusmm, double *out, double *work, void *stream);
 
 /* Expected Gaussian log-likelihood E log N(y | f, exp(2 sn)) of (B, D) propagations
  * (three = 0, S = 1) or the mean over S Monte Carlo samples (S, B, D) (three = 1):
