@@ -1,7 +1,7 @@
 // SE kernel matrices, their adjoints, and the small per-layer / likelihood kernels of
 // the AEP objective.  All arrays are row-major FP64 device memory; log
 // hyper-parameters (ls, sf, sn, R) are read from the device so no host sync is needed.
-#include "gpx_common.h"
+#include "gpx_frag.h"
 
 #include <algorithm>
 
@@ -401,50 +401,65 @@ __global__ void eta_to_R_kernel(int D, int M, const double *__restrict__ eta, do
 }
 
 // out[d, triu(i,j)] = (sum_{k>=i} R_ik (G_kj + G_jk)) * (i == j ? R_ii : 1)
-// One wave per upper 16 x 16 output tile (I, J >= I) of one d, four per workgroup: the
-// product R (G + G^T) over the k-blocks K >= I (R is upper triangular) as FP64 MFMAs fed
-// straight from global memory (lane l: A = R[I*16 + l%16][k], B = G[k][J*16 + l%16] +
-// G[J*16 + l%16][k] for k = K*16 + 4s + l/16).  No LDS, no barriers.
+// One workgroup per upper 16 x 16 output tile (I, J >= I) of one d: the product R (G + G^T) over
+// k >= 16 I (R is upper triangular) on the FP64 matrix cores, operands straight from global
+// memory, each wave every fourth group of 8 k and two groups in flight; the waves' sums are added
+// in wave order.  Bound by the load latency of a wave's share (a wave per tile walked all of k:
+// D = 32, M = 128 17 -> 10 us, D = 2, M = 256 18 -> 5.7, D = 1, M = 50 5.2 -> 2.9).
 __global__ __launch_bounds__(256) void pack_dR_kernel(int D, int M, const double *__restrict__ R,
                                                       const double *__restrict__ G, double *__restrict__ out) {
-  const int lane = threadIdx.x & 63, lr = lane >> 4, lc = lane & 15;
-  const int MT = (M + 15) / 16, T = MT * (MT + 1) / 2;
-  int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;
-  int I = 0;
+  __shared__ double red[4][256];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane >> 4,
+            lc = lane & 15;
+  const int MT = (M + 15) / 16;
+  int t = blockIdx.x, I = 0;
   while (t >= MT - I) {
     t -= MT - I;
     ++I;
   }
-  const int J = I + t, d = blockIdx.y;
+  const int J = I + t, d = blockIdx.y, k0 = 16 * I;
   const double *Rd = R + (long)d * M * M, *Gd = G + (long)d * M * M;
-  const int i = I * 16 + lc, j = J * 16 + lc;
+  const GpxOperand<1, true> oa(Rd, M, k0, M, lane), oc(Gd, M, 16 * J, M, lane);
+  const GpxOperand<1, false> ob(Gd, M, 16 * J, M, lane);
   gpx_d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-  for (int K = I; K < MT; ++K) {
-    double av[4], bv[4];
+  GpxFrag<1> a[2], g[2], h[2];
+  auto mul = [&](int u) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      // loads at clamped indices, unconditional (so they issue together), then zeroed
-      // where the padding needs it by a 0/1 weight (a select lets the compiler sink the
-      // load back under a branch); the clamped values are finite
-      const int k = K * 16 + 4 * s + lr;
-      const int ic = min(i, M - 1), jc = min(j, M - 1), kc = min(k, M - 1);
-      const double a = Rd[(long)ic * M + kc], b = Gd[(long)kc * M + jc] + Gd[(long)jc * M + kc];
-      av[s] = a * ((i < M && k < M) ? 1.0 : 0.0);
-      bv[s] = b * ((j < M && k < M) ? 1.0 : 0.0);
+    for (int s = 0; s < 2; ++s) acc = gpx_mfma16(a[u].v[s][0], g[u].v[s][0] + h[u].v[s][0], acc);
+  };
+  const int groups = (M - k0) >> 3, mine = (groups - w + 3) / 4, kr = (M - k0) & 7;
+  if (mine > 0) {
+    auto load = [&](int u, int t) {
+      const int k = k0 + 8 * (w + 4 * min(t, mine - 1));
+      oa.load(a[u], k);
+      ob.load(g[u], k);
+      oc.load(h[u], k);
+    };
+    load(0, 0);
+    int t = 0;
+    for (; t + 2 <= mine; t += 2) {
+      load(1, t + 1);
+      mul(0);
+      load(0, t + 2);
+      mul(1);
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc = gpx_mfma16(av[s], bv[s], acc);
+    if (t < mine) mul(0);
   }
-  const long Kp = (long)M * (M + 1) / 2;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int ii = I * 16 + lr + 4 * r, jj = J * 16 + lc;
-    if (ii >= M || jj >= M || jj < ii) continue;
-    const long rowoff = (long)ii * M - (long)ii * (ii - 1) / 2;
-    out[(long)d * Kp + rowoff + (jj - ii)] = (ii == jj) ? acc[r] * Rd[(long)ii * M + ii] : acc[r];
+  if (kr && w == groups % 4) {
+    oa.load_tail(a[0], k0 + 8 * groups, kr, lane);
+    ob.load_tail(g[0], k0 + 8 * groups, kr, lane);
+    oc.load_tail(h[0], k0 + 8 * groups, kr, lane);
+    mul(0);
   }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[w][r * 64 + lane] = acc[r];
+  __syncthreads();
+  const int ii = k0 + lr + 4 * w, jj = J * 16 + lc;  // wave w finishes register w
+  if (ii >= M || jj >= M || jj < ii) return;
+  const int e = w * 64 + lane;
+  const double v = red[0][e] + red[1][e] + red[2][e] + red[3][e];
+  const long rowoff = (long)ii * M - (long)ii * (ii - 1) / 2;
+  out[(long)d * ((long)M * (M + 1) / 2) + rowoff + (jj - ii)] = ii == jj ? v * Rd[(long)ii * M + ii] : v;
 }
 
 __global__ void lincomb_kernel(long n, double a, const double *__restrict__ x, long nx, double b,
@@ -1150,8 +1165,8 @@ int gpx_pack_dR(int D, int M, const double *R, const double *G, double *out, voi
   if (n == 0) return GPX_OK;
   if (D > 65535) return GPX_EINVAL;
   const int MT = (M + 15) / 16;
-  hipLaunchKernelGGL(pack_dR_kernel, dim3(gpx_cdiv(MT * (MT + 1) / 2, 4), D), dim3(256), 0, (hipStream_t)stream,
-                     D, M, R, G, out);
+  hipLaunchKernelGGL(pack_dR_kernel, dim3(MT * (MT + 1) / 2, D), dim3(256), 0, (hipStream_t)stream, D, M, R, G,
+                     out);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }
