@@ -125,3 +125,11 @@ typedef double gpx_d4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ gpx_d4 gpx_mfma16(double a, double b, gpx_d4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
+
+// Four 4 x 4 x 4 products of the FP64 MFMA (16 cycles, the same rate): lane l supplies A[l % 16][l / 16] of
+// sixteen rows, four to a product, and B[l / 16][l % 16] of sixteen columns, four to a product.
+// With one B for all products (lane: B[l / 16][l % 4]) lane l holds the sum over k at row
+// 4 ((l / 4) % 4) + l / 16, column l % 4; with one A (lane: A[l % 4][l / 16]) row l / 16, column l % 16.
+__device__ __forceinline__ double gpx_mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}

@@ -357,30 +357,43 @@ __device__ __forceinline__ void wave_lds_sync() {
 // 8-wave sums of the column sums and V go through LDS in wave order (double-buffered
 // by block parity, so one barrier per block serves the staging and both sums); a block's
 // sums are read and written out during the next block, beside its first MFMAs.
-// DB, DS: the 16-row and 4-row slices of the D contraction (2, 8 for D <= 32; 1, DS for
-// D <= 16); KS = ceil(Q / 4).
+// DS = ceil(D / 4) for D <= 16, 8 up to 32; KS = ceil(Q / 4); G = ceil((Q + 1) / 4).
 // ---------------------------------------------------------------------------
 //
-// What bounds it: per row and block KS + DS + 4 (DB + 2) MFMAs of 64 cycles and the exps and other FP64
-// vector work of the same SIMD, which add up (26 MFMAs and about 320 cycles at Q = 8,
-// D = 32), on two waves per SIMD (LDS and registers hold one workgroup per CU).  Adjoint
-// entry, microseconds, expanded-square exponent -> this one: N = 4096, M = 128, Q = 8, D = 32
-// 300 -> 260; 9999, 200, 4, 4 927 -> 850; 3001, 190, 10, 12 421 -> 365; below N = 1000 (a
-// per-point and a per-pair kernel before) 500, 200, 8, 16 200 -> 138, 300, 100, 5, 8 96 -> 67.
+// What bounds it: per row and block 64 (KS + 2 DS + 2 G) cycles of MFMAs (the dB-hat, LW and U products
+// as 4 x 4 x 4 forms of only the rows and columns there are, where 16 x 16 tiles were up to three
+// quarters padding; not at D > 16, whose registers hold no operands for them) and about 230 of
+// exps and other FP64 vector work on the same SIMD, which add up, and the LDS reads of operands;
+// two waves per SIMD (LDS and registers hold one workgroup per CU; four at 128 registers spilled
+// and took 1882 us in place of 711).  Adjoint entry, microseconds, expanded-square exponent ->
+// now: N = 4096, M = 128, Q = 8, D = 32 300 -> 255; 9999, 200, 4, 4 927 -> 610; 3001, 190, 10, 12
+// 421 -> 305; 500, 200, 8, 16 200 -> 118.
 constexpr int MG_NW = 8;
-template <int DB, int DS, int KS>
+
+// D += A B of the 16 x 16 x 4 MFMA on four doubles in place.
+__device__ __forceinline__ void mfma16_at(double a, double b, double *d) {
+  const gpx_d4 t = gpx_mfma16(a, b, gpx_d4{d[0], d[1], d[2], d[3]});
+#pragma unroll
+  for (int r = 0; r < 4; ++r) d[r] = t[r];
+}
+
+template <int DS, int KS, int G>
 __global__ __launch_bounds__(64 * MG_NW) void fused_bwd_merged_kernel(
     int N, int M, int Q, int D, const double *__restrict__ z, const double *__restrict__ sf,
     const double *__restrict__ Bp, const double *__restrict__ dv, const double *__restrict__ pf,
     const double *__restrict__ un, int nsplit, int nchunk, double *__restrict__ dBpart,
     double *__restrict__ LWpart, double *__restrict__ Tpart, double *__restrict__ Vpart) {
   constexpr int NR = 2;
+  // 4 x 4 MFMA forms where they need fewer than a 16-row tile's rows: of U and LW (G groups of
+  // four columns q'), of dB-hat (DS groups of four rows d)
+  constexpr bool U4 = G < 4 && DS < 8, D4 = DS < 4;
+  constexpr int DB = DS > 4 ? 2 : 1, UC = U4 ? G : 4, LR = U4 ? G : 4, DR = D4 ? DS : 4 * DB;
   __shared__ double pfs[2][16][PF_W + 2];      // point features
   __shared__ double lus[2][16][PF_W + 1];      // u at the tile's rows (16) and columns (16)
   __shared__ double dvs[2][16][32];
-  __shared__ double trn[MG_NW][16][17];        // per-wave transpose of L
+  __shared__ double trn[MG_NW][NR][16][17];    // per-wave transposes of L
   __shared__ double csum[2][MG_NW][16][17];    // per-wave column sums  [n][b]
-  __shared__ double vsum[2][MG_NW][16][17];    // per-wave V terms      [n][q']
+  __shared__ double vsum[2][MG_NW][16][(DS < 8 ? 4 * G : 16) + 1];  // per-wave V terms   [n][q']
   // the exponent's pair operands of the wave's rows, in LDS where D > 16 leaves no registers
   constexpr bool AF_LDS = DB == 2;
   __shared__ double afs[AF_LDS ? MG_NW : 1][NR][KS][AF_LDS ? 64 : 1];
@@ -405,7 +418,8 @@ __global__ __launch_bounds__(64 * MG_NW) void fused_bwd_merged_kernel(
     act[u] = a[u] < M;
   }
   // pair operands of the wave's rows: -(z_a - z_b)^2 (k = kq + 4s), sf4 B-hat, the V weight
-  double af[AF_LDS ? 1 : NR][KS], bs[NR][DS], zw[NR];
+  double af[AF_LDS ? 1 : NR][KS], bs[NR][DS], zw[NR][U4 ? G : 1];
+  const int k4 = lane & 3, n4 = 4 * ((lane >> 2) & 3) + kq;  // 4 x 4 results: column k4, row n4
 #pragma unroll
   for (int u = 0; u < NR; ++u) {
     const bool bv = jb < M && act[u];
@@ -420,36 +434,31 @@ __global__ __launch_bounds__(64 * MG_NW) void fused_bwd_merged_kernel(
       const int d = kq + 4 * s;
       bs[u][s] = (bv && d < D) ? sf4 * Bp[((long)a[u] * M + jb) * D + d] : 0.0;
     }
-    // V weight of this lane's column q' = ka of U: w z_a[q'-1]
-    zw[u] = (act[u] && ka >= 1 && ka <= Q) ? (off ? 2.0 : 1.0) * z[a[u] * Q + ka - 1] : 0.0;
+    // V weight of this lane's columns q' of U: w z_a[q'-1]
+#pragma unroll
+    for (int g = 0; g < (U4 ? G : 1); ++g) {
+      const int q = U4 ? 4 * g + k4 : ka;
+      zw[u][g] = (act[u] && q >= 1 && q <= Q) ? (off ? 2.0 : 1.0) * z[a[u] * Q + q - 1] : 0.0;
+    }
   }
-  // B operand of U: [1 | z_b] for b = 16B + kq + 4s (rows), q' = ka (columns); padding
+  // B operand of U: [1 | z_b] for b = 16B + kq + 4s (rows), q' (columns); padding
   // columns b >= M give zeros (their L is 0 as well)
-  double zx[4];
+  double zx[4][U4 ? G : 1];
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const int b = 16 * B + kq + 4 * s;
-    zx[s] = (b < M && ka <= Q) ? (ka == 0 ? 1.0 : z[b * Q + ka - 1]) : 0.0;
-  }
-  // D <= 4 with Q <= 8: the dB-hat and LW contractions as per-lane FMAs over the lane's four
-  // points (summed over the four lane rows once, at the end), where the MFMA forms would fill
-  // 4 and at most 9 of their 16 output rows
-  constexpr bool VSM = DB == 1 && DS == 1 && KS <= 2;
-  constexpr int VQ = 4 * KS + 1;  // Q + 1 <= VQ
-  gpx_d4 dacc[VSM ? 1 : NR][DB], lacc[VSM ? 1 : NR];
+  for (int s = 0; s < 4; ++s)
 #pragma unroll
-  for (int u = 0; u < (VSM ? 1 : NR); ++u) {
-    lacc[u] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+    for (int g = 0; g < (U4 ? G : 1); ++g) {
+      const int b = 16 * B + kq + 4 * s, q = U4 ? 4 * g + k4 : ka;
+      zx[s][g] = (b < M && q <= Q) ? (q == 0 ? 1.0 : z[b * Q + q - 1]) : 0.0;
+    }
+  // rows d = 4 i + kq of dacc[i], q' = 4 i + kq of lacc[i], column b = ka
+  double dacc[NR][DR], lacc[NR][LR];
 #pragma unroll
-    for (int db = 0; db < DB; ++db) dacc[u][db] = gpx_d4{0.0, 0.0, 0.0, 0.0};
-  }
-  double vd[VSM ? NR : 1][4], vl[VSM ? NR : 1][VQ];
+  for (int u = 0; u < NR; ++u) {
 #pragma unroll
-  for (int u = 0; u < (VSM ? NR : 1); ++u) {
+    for (int i = 0; i < LR; ++i) lacc[u][i] = 0.0;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) vd[u][d] = 0.0;
-#pragma unroll
-    for (int q = 0; q < VQ; ++q) vl[u][q] = 0.0;
+    for (int i = 0; i < DR; ++i) dacc[u][i] = 0.0;
   }
   // staging: thread (row sk < 16, column sc < 32) of each of the three arrays
   const int sk = tid >> 5, sc = tid & 31;
@@ -495,109 +504,126 @@ __global__ __launch_bounds__(64 * MG_NW) void fused_bwd_merged_kernel(
   for (int n0 = nbeg; n0 < nend; n0 += 16) {
     const bool more = n0 + 16 < nend;  // uniform over the workgroup
     if (more) fetch(n0 + 16);
-    double pa[KS], da[DS], dvv[4][DB], dq[4], ub[4];
+    double pa[KS], da[DS], dvv[4][D4 ? DS : DB], dq[4][U4 ? G : 1], ub[4];
 #pragma unroll
     for (int s = 0; s < KS; ++s) pa[s] = pfs[buf][ka][kq + 4 * s];
 #pragma unroll
     for (int r = 0; r < 4; ++r) ub[r] = lus[buf][kq + 4 * r][16 + ka];
 #pragma unroll
     for (int s = 0; s < DS; ++s) da[s] = dvs[buf][ka][(kq + 4 * s) ^ swa];
-    if constexpr (!VSM) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = kq + 4 * r;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) dvv[r][db] = dvs[buf][k][(16 * db + ka) ^ dv_swizzle(k)];
-        dq[r] = pfs[buf][k][16 + ka];
-      }
-    }
-    double cs[4] = {0.0, 0.0, 0.0, 0.0}, vw[4] = {0.0, 0.0, 0.0, 0.0};
-    double pp[VSM ? NR : 1][4], LL[VSM ? NR : 1][4];
-#pragma unroll
-    for (int u = 0; u < NR; ++u) {
-      gpx_d4 e, g = gpx_d4{0.0, 0.0, 0.0, 0.0};
-      if (act[u]) {  // wave-uniform
-#pragma unroll
-        for (int r = 0; r < 4; ++r) e[r] = ub[r] + lus[buf][kq + 4 * r][wave + 8 * u];
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          double f;
-          if constexpr (AF_LDS) f = afs[wave][u][s][lane]; else f = af[u][s];
-          e = gpx_mfma16(pa[s], f, e);
-        }
-#pragma unroll
-        for (int s = 0; s < DS; ++s) g = gpx_mfma16(da[s], bs[u][s], g);
-      }
-      // the previous block's 8-wave sums, while this block's first MFMAs run (its buffer
-      // half is not written again before the next barrier)
-      if (u == 0 && n0 > nbeg) reduce(n0 - 16, buf ^ 1);
-      if (!act[u]) continue;
-      double p[4], L[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        p[r] = gpx_exp_tab(e[r], etab);
-        L[r] = g[r] * p[r];
-      }
-      if constexpr (VSM) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          pp[u][r] = p[r];
-          LL[u][r] = L[r];
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-#pragma unroll
-          for (int db = 0; db < DB; ++db) dacc[VSM ? 0 : u][db] = gpx_mfma16(dvv[r][db], p[r], dacc[VSM ? 0 : u][db]);
-          lacc[VSM ? 0 : u] = gpx_mfma16(dq[r], L[r], lacc[VSM ? 0 : u]);
-        }
-      }
-      // U = L [1 | z_b]: L (lane: n = kq + 4r, b = ka) transposed to the A-operand
-      // layout (lane: n = ka, b = kq + 4s) through the wave's LDS
-#pragma unroll
-      for (int r = 0; r < 4; ++r) trn[wave][kq + 4 * r][ka] = L[r];
-      wave_lds_sync();
-      double lt[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) lt[s] = trn[wave][ka][kq + 4 * s];
-      wave_lds_sync();
-      gpx_d4 U = gpx_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) U = gpx_mfma16(lt[s], zx[s], U);
-      // lane holds U[n = kq + 4r][q' = ka]
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + kq + 4 * r;
-        if (ka == 0 && n < nend) Tpart[((long)B * N + n) * M + a[u]] = U[r];
-        vw[r] += zw[u] * U[r];
-        cs[r] += L[r];
-      }
-    }
-    if constexpr (VSM) {
-      // lane: pair column b = ka, points n = kq + 4r (r < 4): dBhat[d][b] += dv[n][d] p[n][b],
-      // LW[b][q'] += [1 | d_n][q'] L[n][b]
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = kq + 4 * r;
-        double dvl[4], dql[VQ];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) dvl[d] = dvs[buf][k][d ^ dv_swizzle(k)];
-#pragma unroll
-        for (int q = 0; q < VQ; ++q) dql[q] = pfs[buf][k][16 + q];
-#pragma unroll
-        for (int u = 0; u < NR; ++u) {
-          if (!act[u]) continue;
-#pragma unroll
-          for (int d = 0; d < 4; ++d) vd[u][d] = fma(dvl[d], pp[u][r], vd[u][d]);
-#pragma unroll
-          for (int q = 0; q < VQ; ++q) vl[u][q] = fma(dql[q], LL[u][r], vl[u][q]);
-        }
-      }
-    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      csum[buf][wave][kq + 4 * r][ka] = cs[r];
-      vsum[buf][wave][kq + 4 * r][ka] = vw[r];
+      const int k = kq + 4 * r;
+#pragma unroll
+      for (int i = 0; i < (D4 ? DS : DB); ++i)
+        dvv[r][i] = dvs[buf][k][(D4 ? 4 * i + k4 : 16 * i + ka) ^ dv_swizzle(k)];
+#pragma unroll
+      for (int i = 0; i < (U4 ? G : 1); ++i) dq[r][i] = pfs[buf][k][16 + (U4 ? 4 * i + k4 : ka)];
+    }
+    double cs[4] = {0.0, 0.0, 0.0, 0.0}, vw[UC];
+#pragma unroll
+    for (int i = 0; i < UC; ++i) vw[i] = 0.0;
+    // both rows in step, without a branch (rows past M carry zeros), so that one's latencies
+    // hide behind the other's work
+    gpx_d4 e[NR], g[NR];
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) e[u][r] = ub[r] + lus[buf][kq + 4 * r][wave + 8 * u];
+      g[u] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+    }
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        double f;
+        if constexpr (AF_LDS) f = afs[wave][u][s][lane]; else f = af[u][s];
+        e[u] = gpx_mfma16(pa[s], f, e[u]);
+      }
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int u = 0; u < NR; ++u) g[u] = gpx_mfma16(da[s], bs[u][s], g[u]);
+    // the previous block's 8-wave sums, while this block's first MFMAs run (its buffer
+    // half is not written again before the next barrier)
+    if (n0 > nbeg) reduce(n0 - 16, buf ^ 1);
+    double p[NR][4], L[NR][4];
+#pragma unroll
+    for (int u = 0; u < NR; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[u][r] = gpx_exp_tab(e[u][r], etab);
+        L[u][r] = g[u][r] * p[u][r];
+        cs[r] += L[u][r];
+        // L (lane: n = kq + 4r, b = ka) to the A-operand layout (lane: n = ka, b = kq + 4s)
+        // through the wave's LDS
+        trn[wave][u][kq + 4 * r][ka] = L[u][r];
+      }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        if constexpr (D4) {
+#pragma unroll
+          for (int i = 0; i < DS; ++i) dacc[u][i] = gpx_mfma4(dvv[r][i], p[u][r], dacc[u][i]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < DB; ++i) mfma16_at(dvv[r][i], p[u][r], dacc[u] + 4 * i);
+        }
+        if constexpr (U4) {
+#pragma unroll
+          for (int i = 0; i < G; ++i) lacc[u][i] = gpx_mfma4(dq[r][i], L[u][r], lacc[u][i]);
+        } else {
+          mfma16_at(dq[r][0], L[u][r], lacc[u]);
+        }
+      }
+    // U = L [1 | z_b]
+    double lt[NR][4];
+#pragma unroll
+    for (int u = 0; u < NR; ++u)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) lt[u][s] = trn[wave][u][ka][kq + 4 * s];
+    if constexpr (U4) {  // lane holds U[n = n4][q' = 4 i + k4]
+      double U[NR][G];
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+#pragma unroll
+        for (int i = 0; i < G; ++i) U[u][i] = 0.0;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < NR; ++u)
+#pragma unroll
+          for (int i = 0; i < G; ++i) U[u][i] = gpx_mfma4(lt[u][s], zx[s][i], U[u][i]);
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        if (k4 == 0 && act[u] && n0 + n4 < nend) Tpart[((long)B * N + n0 + n4) * M + a[u]] = U[u][0];
+#pragma unroll
+        for (int i = 0; i < G; ++i) vw[i] += zw[u][i] * U[u][i];
+      }
+    } else {  // U[n = kq + 4r][q' = ka]
+      gpx_d4 U[NR];
+#pragma unroll
+      for (int u = 0; u < NR; ++u) U[u] = gpx_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < NR; ++u) U[u] = gpx_mfma16(lt[u][s], zx[s][0], U[u]);
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int n = n0 + kq + 4 * r;
+          if (ka == 0 && act[u] && n < nend) Tpart[((long)B * N + n) * M + a[u]] = U[u][r];
+          vw[r] += zw[u][0] * U[u][r];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) csum[buf][wave][kq + 4 * r][ka] = cs[r];
+#pragma unroll
+    for (int i = 0; i < UC; ++i) {
+      if constexpr (U4) vsum[buf][wave][n4][4 * i + k4] = vw[i]; else vsum[buf][wave][kq + 4 * i][ka] = vw[i];
     }
     if (more) stage(buf ^ 1);
     __syncthreads();
@@ -607,31 +633,15 @@ __global__ __launch_bounds__(64 * MG_NW) void fused_bwd_merged_kernel(
 #pragma unroll
   for (int u = 0; u < NR; ++u) {
     if (!act[u]) continue;
-    if constexpr (VSM) {
-      // sum over the four lane rows (lanes ka + 16 kq), in a fixed order
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const double t = gpx_swap_add<16>(gpx_swap_add<32>(vd[u][d]));
-        if (kq == 0 && d < D && jb < M) dBpart[(((long)ns * D + d) * M + a[u]) * M + jb] = sf4 * t;
-      }
-#pragma unroll
-      for (int q = 0; q < VQ; ++q) {
-        const double t = gpx_swap_add<16>(gpx_swap_add<32>(vl[u][q]));
-        if (kq == 0 && q <= Q && jb < M) LWpart[(((long)ns * M + a[u]) * M + jb) * (Q + 1) + q] = t;
-      }
-      continue;
+    for (int i = 0; i < DR; ++i) {
+      const int d = 4 * i + kq;
+      if (d < D && jb < M) dBpart[(((long)ns * D + d) * M + a[u]) * M + jb] = sf4 * dacc[u][i];
     }
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int d = 16 * db + kq + 4 * r;
-        if (d < D && jb < M) dBpart[(((long)ns * D + d) * M + a[u]) * M + jb] = sf4 * dacc[VSM ? 0 : u][db][r];
-      }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qq = kq + 4 * r;
-      if (qq <= Q && jb < M) LWpart[(((long)ns * M + a[u]) * M + jb) * (Q + 1) + qq] = lacc[VSM ? 0 : u][r];
+    for (int i = 0; i < LR; ++i) {
+      const int qq = 4 * i + kq;
+      if (qq <= Q && jb < M) LWpart[(((long)ns * M + a[u]) * M + jb) * (Q + 1) + qq] = lacc[u][i];
     }
   }
 }
@@ -982,16 +992,23 @@ int gpx_fused_mm_bwd_points(int N, int M, int Q, int D, const double *mx, const 
   const int T = (M + 15) / 16, ntiles = T * (T + 1) / 2;
   const int nchunk = ((N + nsplit - 1) / nsplit + 15) / 16 * 16;
   dim3 gm(ntiles, nsplit);
-#define GPX_MERGED(DBV, DSV, KSV)                                                                               \
-  hipLaunchKernelGGL((fused_bwd_merged_kernel<DBV, DSV, KSV>), gm, dim3(64 * MG_NW), 0, st, N, M, Q, D, z, sf, Bp, \
+#define GPX_MERGED(DSV, KSV, GV)                                                                                \
+  hipLaunchKernelGGL((fused_bwd_merged_kernel<DSV, KSV, GV>), gm, dim3(64 * MG_NW), 0, st, N, M, Q, D, z, sf, Bp, \
                      dv, (const double *)W.pf, (const double *)W.un, nsplit, nchunk, W.dBpart, W.LWpart, W.Tpart, W.Vpart)
-#define GPX_MERGED_KS(DBV, DSV) \
-  if (Q <= 4) GPX_MERGED(DBV, DSV, 1); else if (Q <= 8) GPX_MERGED(DBV, DSV, 2); \
-  else if (Q <= 12) GPX_MERGED(DBV, DSV, 3); else GPX_MERGED(DBV, DSV, 4);
-  if (D <= 4) { GPX_MERGED_KS(1, 1) }
-  else if (D <= 8) { GPX_MERGED_KS(1, 2) }
-  else if (D <= 16) { GPX_MERGED_KS(1, 4) }
-  else { GPX_MERGED_KS(2, 8) }
+  // KS = ceil(Q / 4) slices of the exponent, G = ceil((Q + 1) / 4) groups of [1 | z]
+#define GPX_MERGED_KS(DSV)                            \
+  if (Q <= 3) GPX_MERGED(DSV, 1, 1);                  \
+  else if (Q == 4) GPX_MERGED(DSV, 1, 2);             \
+  else if (Q <= 7) GPX_MERGED(DSV, 2, 2);             \
+  else if (Q == 8) GPX_MERGED(DSV, 2, 3);             \
+  else if (Q <= 11) GPX_MERGED(DSV, 3, 3);            \
+  else if (Q == 12) GPX_MERGED(DSV, 3, 4);            \
+  else GPX_MERGED(DSV, 4, 4);
+  if (D <= 4) { GPX_MERGED_KS(1) }
+  else if (D <= 8) { GPX_MERGED_KS(2) }
+  else if (D <= 12) { GPX_MERGED_KS(3) }
+  else if (D <= 16) { GPX_MERGED_KS(4) }
+  else { GPX_MERGED_KS(8) }
 #undef GPX_MERGED_KS
 #undef GPX_MERGED
   GPX_CHECK_LAUNCH();
