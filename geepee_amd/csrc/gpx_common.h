@@ -60,6 +60,14 @@ __device__ __forceinline__ double gpx_wave_sum(double v) {
   return gpx_dpp_add<0xB1>(v);
 }
 
+// Sum over the 16 lanes of a row (every lane of the row gets it).
+__device__ __forceinline__ double gpx_row_sum(double v) {
+  v = gpx_dpp_add<0x140>(v);
+  v = gpx_dpp_add<0x141>(v);
+  v = gpx_dpp_add<0x4E>(v);
+  return gpx_dpp_add<0xB1>(v);
+}
+
 // Block-wide sum for blockDim.x a multiple of 64 (<= 1024).  `red` is LDS scratch of
 // at least 16 doubles.  Every thread gets the total.
 __device__ __forceinline__ double gpx_block_sum(double v, double *red) {

@@ -21,6 +21,8 @@
 // dpsi2_n = sum_d dv_nd Bsym[d].
 #include "gpx_common.h"
 
+#include <algorithm>
+
 #include <mutex>
 
 #define FQ_MAX 16
@@ -691,132 +693,209 @@ __global__ __launch_bounds__(256) void fused_pairs_finish(int M, int Q, int D, i
 }
 
 
-// Per-point finish of the fused adjoint: T = sum of the S slots of Tpart, V = sum of the
-// SV slots of Vpart, Lp = dpsi1 psi1,
-// then the same per-point formulas (and outputs) as the materialising path's row pass.
-// One wave per point: its lanes stride over the M columns and the sums are wave
-// reductions, so no workgroup barrier is needed.
-// QC: Q fixed at compile time for the common shapes (0: read at run time).
-template <int QC>
-__global__ __launch_bounds__(256) void fused_rows_finish(
+// Per-point finish of the fused adjoint, a workgroup per point, point after point: T = the sum of
+// the S slots of Tpart, V of the SV slots of Vpart, Lp = dpsi1 psi1, then dmx, dvx and the point's
+// share of dell, and, in registers over the workgroup's points, what T and Lp give to dZ:
+//   dZ_aq += T (2 d mu - z (d + 1/l)) - Lp e (z - mu),  d = 1/(2v+l), e = 1/(v+l)
+// (the rest of dZ comes from the pair sums LW).  Lane (g, c) of wave w owns q = g + 4 r (r < KR) and
+// the columns a = 16 (w + 4 j) + c; the lane groups share the slots, sums over a run across the 16
+// lanes of a row, then over the waves through LDS.  Bound by reading the slots (13 N M doubles at
+// M = 200).  With the tail below, in place of a wave per point that stored T and Lp for two
+// products, two column sums and an assembly: whole adjoint, us, N = 3001, M = 190, Q = 10, D = 12
+// 321 -> 299, 4096, 128, 8, 32 271 -> 266, 300, 100, 5, 8 58 -> 49, 150, 20, 4, 8 40 -> 30.
+// part[block]: [dZ (M x Q) | sum of H (Q) | S0, A1].
+constexpr int RF_RED = 5 * FQ_MAX + 2;
+
+template <int KR, int MJ>  // MJ: column tiles of a wave, ceil(M / 64)
+__global__ __launch_bounds__(256, 3) void fused_rows_finish(
     int N, int M, int Q, int S, int SV, const double *__restrict__ mx, const double *__restrict__ vx,
     const double *__restrict__ z, const double *__restrict__ ls, const double *__restrict__ Tpart,
     const double *__restrict__ Vpart, const double *__restrict__ dpsi1, const double *__restrict__ psi1,
-    double *__restrict__ dmx, double *__restrict__ dvx, double *__restrict__ Tout,
-    double *__restrict__ Lpout, double *__restrict__ Hout, double *__restrict__ s0out,
-    double *__restrict__ Dn, double *__restrict__ Pn, double *__restrict__ En) {
-  constexpr int QN = QC ? QC : FQ_MAX, FRED = 4 * QN + 2;
-  if (QC) Q = QC;
-  const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  double mu[QN];
+    double *__restrict__ dmx, double *__restrict__ dvx, double *__restrict__ part) {
+  constexpr int ZLD = 4 * KR + 1;
+  extern __shared__ double rf_lds[];  // z, rows of ZLD
+  __shared__ double red[2][4][RF_RED];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15, MT = (M + 15) >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int e = tid; e < M * ZLD; e += 256) rf_lds[e] = e % ZLD < Q ? z[e / ZLD * Q + e % ZLD] : 0.0;
+  __syncthreads();
+  double l[KR], il[KR], dz[MJ][KR], hsum = 0.0, s0sum = 0.0, a1sum = 0.0;
+  int col[MJ];
+  bool on[MJ];
 #pragma unroll
-  for (int q = 0; q < QN; ++q) mu[q] = (q < Q) ? mx[(long)n * Q + q] : 0.0;
-  // [0] S0, [1] sum Lp, [2+q] S1, [2+Q+q] sum T z^2, [2+2Q+q] B1, [2+3Q+q] C1
-  double c[FRED];
-#pragma unroll
-  for (int i = 0; i < FRED; ++i) c[i] = 0.0;
-  // T = sum of the S slots of Tpart for this lane's columns m = lane + 64 j (j < 4, M <= 256),
-  // each column summed in slot order; the loads of four slots at clamped (always valid)
-  // indices issue together, and the clamped lanes' sums are never read
-  constexpr int MJ = (FM_MAX + 63) / 64;
-  const int nj = (M + 63) >> 6;
-  double Tm[MJ];
-#pragma unroll
-  for (int j = 0; j < MJ; ++j) Tm[j] = 0.0;
-  for (int s0 = 0; s0 < S; s0 += 4) {
-    double tv[4][MJ];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const double *row = Tpart + ((long)min(s0 + u, S - 1) * N + n) * M;
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) tv[u][j] = j < nj ? row[min(lane + 64 * j, M - 1)] : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (s0 + u < S) {
-#pragma unroll
-        for (int j = 0; j < MJ; ++j) Tm[j] += tv[u][j];
-      }
+  for (int r = 0; r < KR; ++r) {
+    l[r] = g + 4 * r < Q ? exp(2.0 * ls[g + 4 * r]) : 1.0;
+    il[r] = 1.0 / l[r];
   }
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
-    const int m = lane + 64 * j;
-    if (m >= M) break;
-    const double T = Tm[j];
-    const double Lp = dpsi1[(long)n * M + m] * psi1[(long)n * M + m];
-    Tout[(long)n * M + m] = T;
-    Lpout[(long)n * M + m] = Lp;
-    c[0] += T;
-    c[1] += Lp;
+    const int a = 16 * (w + 4 * j) + c;
+    on[j] = a < M;
+    col[j] = min(a, M - 1);
 #pragma unroll
-    for (int q = 0; q < QN; ++q)
-      if (q < Q) {
-        const double zq = z[m * Q + q], zm = zq - mu[q];
-        c[2 + q] += T * zq;
-        c[2 + QN + q] += T * zq * zq;
-        c[2 + 2 * QN + q] += Lp * zm;
-        c[2 + 3 * QN + q] += Lp * zm * zm;
-      }
+    for (int r = 0; r < KR; ++r) dz[j][r] = 0.0;
   }
+  const int tn = (MT - w + 3) >> 2;  // this wave's column tiles (may be 0)
+  const int tq = min(tid, Q - 1);
+  const double ell = exp(ls[tq]), lq = exp(2.0 * ls[tq]), ilq = 1.0 / lq;
+  int par = 0;
+  for (int n = blockIdx.x; n < N; n += gridDim.x, par ^= 1) {
+    // every load at a clamped (valid) index, issued together; S <= 16, SV <= 136
+    double tv[4][MJ], vv[3][KR], T[MJ], Lp[MJ], V[KR];
 #pragma unroll
-  for (int i = 0; i < FRED; ++i) {
-    if (i >= 2 && (i - 2) % QN >= Q) continue;
-    c[i] = gpx_wave_sum(c[i]);
-  }
-  double out_S1 = 0.0, out_TZ2 = 0.0, out_B1 = 0.0, out_C1 = 0.0;
+    for (int i = 0; i < 4; ++i) {
+      const double *row = Tpart + ((long)min(g + 4 * i, S - 1) * N + n) * M;
 #pragma unroll
-  for (int q = 0; q < QN; ++q)
-    if (q == lane) {
-      out_S1 = c[2 + q];
-      out_TZ2 = c[2 + QN + q];
-      out_B1 = c[2 + 2 * QN + q];
-      out_C1 = c[2 + 3 * QN + q];
+      for (int j = 0; j < MJ; ++j) tv[i][j] = 4 * i < S && j < tn ? row[col[j]] : 0.0;
     }
-  // V = sum of the SV slots of Vpart: lane l sums the Q values of slots l, l + 64, ...
-  // (one row of Q contiguous values each), then a wave sum per q
-  double Vq[QN];
 #pragma unroll
-  for (int q = 0; q < QN; ++q) Vq[q] = 0.0;
-  for (int s = lane; s < SV; s += 64) {
-    const double *row = Vpart + ((long)s * N + n) * Q;
+    for (int i = 0; i < 3; ++i) {
+      const double *row = Vpart + ((long)min(16 * w + c + 64 * i, SV - 1) * N + n) * Q;
 #pragma unroll
-    for (int q = 0; q < QN; ++q)
-      if (q < Q) Vq[q] += row[q];
-  }
-  double Vsel = 0.0;
+      for (int r = 0; r < KR; ++r) vv[i][r] = 64 * i < SV ? row[min(g + 4 * r, Q - 1)] : 0.0;
+    }
 #pragma unroll
-  for (int q = 0; q < QN; ++q) {
-    if (q >= Q) continue;
-    const double t = gpx_wave_sum(Vq[q]);
-    if (q == lane) Vsel = t;
+    for (int j = 0; j < MJ; ++j) {
+      const double x = dpsi1[(long)n * M + col[j]] * psi1[(long)n * M + col[j]];
+      Lp[j] = on[j] ? x : 0.0;
+      T[j] = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (g + 4 * i < S) T[j] += tv[i][j];
+    }
+#pragma unroll
+    for (int r = 0; r < KR; ++r) {
+      V[r] = 0.0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        if (16 * w + c + 64 * i < SV) V[r] += vv[i][r];
+    }
+    double S0 = 0.0, A1 = 0.0;
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) {
+      if (j < tn) T[j] = gpx_swap_add<16>(gpx_swap_add<32>(T[j]));
+      T[j] = on[j] ? T[j] : 0.0;
+      S0 += T[j];
+      A1 += Lp[j];
+    }
+    S0 = gpx_row_sum(S0);
+    A1 = gpx_row_sum(A1);
+    double *rw = red[par][w];
+#pragma unroll
+    for (int r = 0; r < KR; ++r) {
+      const int q = g + 4 * r, qc = min(q, Q - 1);
+      const double mu = mx[(long)n * Q + qc], v = vx[(long)n * Q + qc];
+      const double d = gpx_recip(2.0 * v + l[r]), e = gpx_recip(v + l[r]);
+      double S1 = 0.0, Z2 = 0.0, B1 = 0.0, C1 = 0.0;
+#pragma unroll
+      for (int j = 0; j < MJ; ++j) {
+        if (j >= tn) break;
+        const double zz = rf_lds[col[j] * ZLD + q], zm = zz - mu, tz = T[j] * zz, lz = Lp[j] * zm;
+        S1 += tz;
+        Z2 = fma(tz, zz, Z2);
+        B1 += lz;
+        C1 = fma(lz, zm, C1);
+        dz[j][r] += d * (2.0 * mu * T[j] - tz) - il[r] * tz - e * lz;
+      }
+      S1 = gpx_row_sum(S1);
+      Z2 = gpx_row_sum(Z2);
+      B1 = gpx_row_sum(B1);
+      C1 = gpx_row_sum(C1);
+      const double Vq = gpx_row_sum(V[r]);
+      if (c == 0) {
+        rw[2 + q] = S1;
+        rw[2 + FQ_MAX + q] = Z2;
+        rw[2 + 2 * FQ_MAX + q] = Vq;
+        rw[2 + 3 * FQ_MAX + q] = B1;
+        rw[2 + 4 * FQ_MAX + q] = C1;
+      }
+    }
+    if (lane == 0) {
+      rw[0] = S0;
+      rw[1] = A1;
+    }
+    __syncthreads();  // red[par] is next written two points on, behind the next point's barrier
+    if (tid < Q) {
+      const int q = tid;
+      auto sum = [&](int i) { return red[par][0][i] + red[par][1][i] + red[par][2][i] + red[par][3][i]; };
+      const double s0 = sum(0), a1 = sum(1), s1 = sum(2 + q), tz2 = sum(2 + FQ_MAX + q), vs = sum(2 + 2 * FQ_MAX + q),
+                   b1 = sum(2 + 3 * FQ_MAX + q), c1 = sum(2 + 4 * FQ_MAX + q);
+      const double m = mx[(long)n * Q + q], v = vx[(long)n * Q + q];
+      const double d = 1.0 / (2.0 * v + lq), e = 1.0 / (v + lq);
+      const double quad = m * m * s0 - 2.0 * m * s1 + 0.5 * (tz2 + vs);
+      dmx[(long)n * Q + q] = -2.0 * d * (m * s0 - s1) + e * b1;
+      dvx[(long)n * Q + q] = 2.0 * d * d * quad - d * s0 + 0.5 * e * (e * c1 - a1);
+      hsum += 2.0 * ell * (v * ilq * d * s0 + d * d * quad + (tz2 - vs) * (0.5 * ilq * ilq));
+      hsum += e * ell * (e * c1 + v * ilq * a1);
+      s0sum += s0;
+      a1sum += a1;
+    }
   }
-  if (lane < Q) {
-    const int q = lane;
-    const double V = Vsel;
-    const double S0 = c[0], A1 = c[1];
-    const double S1 = out_S1, TZ2 = out_TZ2, B1 = out_B1, C1 = out_C1;
-    const double l = exp(2.0 * ls[q]);
-    const double m = mx[(long)n * Q + q], vv = vx[(long)n * Q + q];
-    const double ell = exp(ls[q]);
-    const double d = 1.0 / (2.0 * vv + l), e = 1.0 / (vv + l);
-    const double S2 = 0.5 * (TZ2 + V);
-    const double quad = m * m * S0 - 2.0 * m * S1 + S2;
-    dmx[(long)n * Q + q] = -2.0 * d * (m * S0 - S1) + e * B1;
-    dvx[(long)n * Q + q] = 2.0 * d * d * quad - d * S0 + 0.5 * e * (e * C1 - A1);
-    Hout[(long)n * Q + q] = e * ell * (e * C1 + (vv / l) * A1) +
-                            2.0 * ell * ((vv / l) * d * S0 + d * d * quad + (TZ2 - V) / (2.0 * l * l));
-    Dn[(long)n * (Q + 1) + 1 + q] = d;
-    Pn[(long)n * 2 * Q + q] = d * m;
-    Pn[(long)n * 2 * Q + Q + q] = d;
-    En[(long)n * 2 * Q + q] = e;
-    En[(long)n * 2 * Q + Q + q] = e * m;
+  double *po = part + (long)blockIdx.x * (M * Q + Q + 2);
+#pragma unroll
+  for (int j = 0; j < MJ; ++j)
+#pragma unroll
+    for (int r = 0; r < KR; ++r)
+      if (on[j] && g + 4 * r < Q) po[col[j] * Q + g + 4 * r] = dz[j][r];
+  if (tid < Q) po[M * Q + tid] = hsum;
+  if (tid == 0) {
+    po[M * Q + Q] = s0sum;
+    po[M * Q + Q + 1] = a1sum;
   }
-  if (lane == 0) {
-    Dn[(long)n * (Q + 1)] = 1.0;
-    s0out[2 * n] = c[0];
-    s0out[2 * n + 1] = c[1];
+}
+
+// The tail: dZ_a = the blocks' partials + sum_b (Lsum_ab / l - W_ab) z_b (one workgroup per a; LW
+// ((M*M) x (Q+1)) = [Lsum | W]), and a last workgroup for dell and dsf2 = (A1 + 2 S0) / sf2.
+__global__ __launch_bounds__(256) void fused_tail_kernel(int M, int Q, int blocks, const double *__restrict__ z,
+                                                         const double *__restrict__ ls,
+                                                         const double *__restrict__ sf,
+                                                         const double *__restrict__ LW,
+                                                         const double *__restrict__ part, double *__restrict__ dsf2,
+                                                         double *__restrict__ dell, double *__restrict__ dZ) {
+  __shared__ double red[16][17];
+  const int a = blockIdx.x, tid = threadIdx.x, q = tid & 15, h = tid >> 4, width = M * Q + Q + 2;
+  double s = 0.0;
+  if (a < M && q < Q) {
+    const double il = 1.0 / exp(2.0 * ls[q]);
+    for (int b = h; b < M; b += 16) {
+      const double *row = LW + ((long)a * M + b) * (Q + 1);
+      s += (il * row[0] - row[1 + q]) * z[b * Q + q];
+    }
   }
+  // columns of the partials: dZ's row a, or [H | S0 | A1]
+  const int cols = a < M ? Q : Q + 2;
+  double t = 0.0, x = 0.0;
+  if (q < cols) {
+#pragma unroll 4
+    for (int k = h; k < blocks; k += 16) t += part[(long)k * width + a * Q + q];
+  }
+  if (a == M && q == 0 && Q + 1 == 16) {  // the 17th column, A1 at Q = 15
+    for (int k = h; k < blocks; k += 16) x += part[(long)k * width + M * Q + 16];
+  }
+  red[h][q] = s + t;
+  if (q == 0) red[h][16] = x;
+  __syncthreads();
+  if (tid > 16) return;
+  double v = red[0][tid];
+#pragma unroll
+  for (int k = 1; k < 16; ++k) v += red[k][tid];
+  if (a < M) {
+    if (tid < Q) dZ[a * Q + tid] = v;
+    return;
+  }
+  if (tid < Q) dell[tid] = v;
+  red[0][tid] = v;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (tid == 0) dsf2[0] = (red[0][Q + 1] + 2.0 * red[0][Q]) / exp(2.0 * sf[0]);
+}
+
+// Workgroups of the row finish: as many as the registers let a CU hold (four where KR and MJ are
+// small, else three), each with as many points as the others.
+int rows_finish_blocks(int N, int M, int Q) {
+  const int per = Q <= 4 || M <= 64 || (Q <= 8 && M <= 128) ? 1024 : 768;
+  return (int)gpx_cdiv(N, gpx_cdiv(N, per));
 }
 
 // psi1, m = psi1 Ahat^T and v = sf2 + sum_s part - m^2 for FIN_PTS points per block.
@@ -900,27 +979,18 @@ __global__ __launch_bounds__(256) void fused_fwd_finish(int N, int M, int Q, int
 
 }  // namespace
 
-extern "C" long gpx_psi_tail_workspace(int N, int M, int Q);
 extern "C" int gpx_gemm_batched(int transA, int transB, int m, int n, int k, double alpha,
                                 const double *A, int lda, long strideA, const double *B, int ldb,
                                 long strideB, double beta, double *C, int ldc, long strideC,
                                 int batch, int splits, double *work, int tile, void *stream);
-extern "C" int gpx_psi_bwd_tail(int N, int M, int Q, const double *z, const double *ls, const double *sf,
-                                const double *T, const double *Lp, const double *H, const double *s0,
-                                const double *Dn, const double *Pn, const double *En, const double *LW,
-                                double *TP, double *LE, double *cols0, double *dsf2, double *dell, double *dZ, double *kwork,
-                                void *stream);
-
 extern "C" {
 
 long gpx_fused_bwd_workspace(int N, int M, int Q, int D, int splits, int nsplit) {
   const long MM = (long)M * M;
   long s = (long)nsplit * D * MM + (long)nsplit * MM * (Q + 1) + MM * (Q + 1);  // dBpart, LWpart, LW
   s += (long)fused_t_slots(M) * N * M + (long)fused_v_slots(M) * N * Q;  // Tpart, Vpart
-  s += 3L * N * M + (long)N * Q + 2L * N;                                     // dpsi1, T, Lp, H, s0
-  s += (long)N * (Q + 1) + 4L * N * Q + 4L * M * Q + 2;                       // Dn, Pn, En, TP, LE, cols0
+  s += (long)N * M + (long)rows_finish_blocks(N, M, Q) * (M * Q + Q + 2);           // dpsi1, row finish's partials
   s += (long)N * PF_W + (long)N * M;                                          // point features, u
-  s += gpx_psi_tail_workspace(N, M, Q);                                       // tail split-K partials
   return s;
 }
 
@@ -930,8 +1000,7 @@ namespace {
 
 // Workspace of the fused adjoint (gpx_fused_bwd_workspace doubles), carved in order.
 struct FusedBwdWork {
-  double *dBpart, *LWpart, *LW, *Tpart, *Vpart, *dpsi1, *Tn, *Lp, *H, *s0, *Dn, *Pn, *En, *TP, *LE, *cols0, *un,
-      *pf;
+  double *dBpart, *LWpart, *LW, *Tpart, *Vpart, *dpsi1, *rows, *un, *pf;
   FusedBwdWork(double *work, int N, int M, int Q, int D, int splits, int nsplit) {
     const long MM = (long)M * M;
     dBpart = work;
@@ -940,18 +1009,9 @@ struct FusedBwdWork {
     Tpart = LW + MM * (Q + 1);
     Vpart = Tpart + (long)fused_t_slots(M) * N * M;
     dpsi1 = Vpart + (long)fused_v_slots(M) * N * Q;
-    Tn = dpsi1 + (long)N * M;
-    Lp = Tn + (long)N * M;
-    H = Lp + (long)N * M;
-    s0 = H + (long)N * Q;
-    Dn = s0 + 2L * N;
-    Pn = Dn + (long)N * (Q + 1);
-    En = Pn + 2L * N * Q;
-    TP = En + 2L * N * Q;
-    LE = TP + 2L * M * Q;
-    cols0 = LE + 2L * M * Q;
-    un = cols0 + 2;
-    pf = un + (long)N * M;  // the tail's partials follow
+    rows = dpsi1 + (long)N * M;
+    un = rows + (long)rows_finish_blocks(N, M, Q) * (M * Q + Q + 2);
+    pf = un + (long)N * M;
   }
 };
 
@@ -1016,12 +1076,19 @@ int gpx_fused_mm_bwd_points(int N, int M, int Q, int D, const double *mx, const 
   int rc = gpx_gemm_batched(0, 0, N, M, D, 1.0, dm_all, D, 0, Ahat, M, 0, 0.0, W.dpsi1, M, 0, 1, 1, nullptr, 0,
                             stream);
   if (rc) return rc;
-#define GPX_ROWS(QV)                                                                                           \
-  hipLaunchKernelGGL((fused_rows_finish<QV>), dim3(gpx_cdiv(N, 4)), dim3(256), 0, st, N, M, Q,                 \
-                     fused_t_slots(M), fused_v_slots(M), mx, vx, z, ls,              \
-                     (const double *)W.Tpart, (const double *)W.Vpart, (const double *)W.dpsi1, psi1, dmx, dvx,   \
-                     W.Tn, W.Lp, W.H, W.s0, W.Dn, W.Pn, W.En)
-  if (Q == 4) GPX_ROWS(4); else if (Q == 5) GPX_ROWS(5); else if (Q == 8) GPX_ROWS(8); else GPX_ROWS(0);
+  const int kr = (Q + 3) / 4, rows_lds = (int)sizeof(double) * M * (4 * kr + 1);
+#define GPX_ROWS(KRV, MJV)                                                                                    \
+  hipLaunchKernelGGL((fused_rows_finish<KRV, MJV>), dim3(rows_finish_blocks(N, M, Q)), dim3(256), rows_lds, st, N, M, Q, \
+                     fused_t_slots(M), fused_v_slots(M), mx, vx, z, ls, (const double *)W.Tpart,              \
+                     (const double *)W.Vpart, (const double *)W.dpsi1, psi1, dmx, dvx, W.rows)
+#define GPX_ROWS_MJ(KRV) \
+  if (M <= 64) GPX_ROWS(KRV, 1); else if (M <= 128) GPX_ROWS(KRV, 2); else if (M <= 192) GPX_ROWS(KRV, 3); \
+  else GPX_ROWS(KRV, 4);
+  if (kr == 1) { GPX_ROWS_MJ(1) }
+  else if (kr == 2) { GPX_ROWS_MJ(2) }
+  else if (kr == 3) { GPX_ROWS_MJ(3) }
+  else { GPX_ROWS_MJ(4) }
+#undef GPX_ROWS_MJ
 #undef GPX_ROWS
   GPX_CHECK_LAUNCH();
   return GPX_OK;
@@ -1059,8 +1126,10 @@ int gpx_fused_mm_bwd_tail(int N, int M, int Q, int D, const double *z, const dou
   if (!fused_bwd_args_ok(N, M, Q, D, splits, nsplit)) return GPX_EINVAL;
   if (!z || !ls || !sf || !dsf2 || !dell || !dZ || !work) return GPX_EINVAL;
   FusedBwdWork W(work, N, M, Q, D, splits, nsplit);
-  return gpx_psi_bwd_tail(N, M, Q, z, ls, sf, W.Tn, W.Lp, W.H, W.s0, W.Dn, W.Pn, W.En, W.LW, W.TP, W.LE, W.cols0,
-                          dsf2, dell, dZ, W.pf + (long)N * PF_W, stream);
+  hipLaunchKernelGGL(fused_tail_kernel, dim3(M + 1), dim3(256), 0, (hipStream_t)stream, M, Q, rows_finish_blocks(N, M, Q),
+                     z, ls, sf, (const double *)W.LW, (const double *)W.rows, dsf2, dell, dZ);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
 }
 
 int gpx_fused_mm_bwd(int N, int M, int Q, int D, const double *mx, const double *vx, const double *z,

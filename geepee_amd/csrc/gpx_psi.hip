@@ -233,13 +233,6 @@ __global__ __launch_bounds__(256) void psi2_kernel(int N, int M, int Q, const do
 constexpr int PSI_NRED = 5 * GPX_QMAX + 2;
 constexpr int PSI_ZLD = GPX_QMAX + 1;
 
-__device__ __forceinline__ double psi_row_sum(double v) {  // over the 16 lanes of a row
-  v = gpx_dpp_add<0x140>(v);
-  v = gpx_dpp_add<0x141>(v);
-  v = gpx_dpp_add<0x4E>(v);
-  return gpx_dpp_add<0xB1>(v);
-}
-
 template <int TN, int W, bool SYM>
 __global__ __launch_bounds__(64 * W, 3) void psi_bwd_points_kernel(
     int N, int M, int Q, const double *__restrict__ mx, const double *__restrict__ vx,
@@ -342,8 +335,8 @@ __global__ __launch_bounds__(64 * W, 3) void psi_bwd_points_kernel(
     double *rw = red[par][w];
     int zo = first + c;  // opaque: z is re-read from LDS for each point, not kept in registers
     asm volatile("" : "+v"(zo));
-    S0 = psi_row_sum(S0);
-    A1 = psi_row_sum(A1);
+    S0 = gpx_row_sum(S0);
+    A1 = gpx_row_sum(A1);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       if (4 * r >= Q) break;
@@ -362,11 +355,11 @@ __global__ __launch_bounds__(64 * W, 3) void psi_bwd_points_kernel(
         C1 = fma(lz, zm, C1);
         dz[j][r] += fma(u - tz, il[r], d * (2.0 * mu * T[j] - tz - u)) - e * lz;
       }
-      V = psi_row_sum(V);
-      S1 = psi_row_sum(S1);
-      Z2 = psi_row_sum(Z2);
-      B1 = psi_row_sum(B1);
-      C1 = psi_row_sum(C1);
+      V = gpx_row_sum(V);
+      S1 = gpx_row_sum(S1);
+      Z2 = gpx_row_sum(Z2);
+      B1 = gpx_row_sum(B1);
+      C1 = gpx_row_sum(C1);
       if (c == 0) {
         rw[2 + q] = S1;
         rw[2 + GPX_QMAX + q] = Z2;
@@ -463,7 +456,7 @@ int psi_bwd_launch(int blocks, int N, int M, int Q, int sym, const double *mx, c
   return GPX_OK;
 }
 
-// Final assembly for the hyper-parameter adjoints of the fused path.  One block per inducing point a
+// Final assembly for the hyper-parameter adjoints from pair sums (gpx_psi_bwd_tail).  One block per inducing point a
 // (threads over b), plus block M which finishes the scalar / per-q sums.
 //   LW:  M^2 x (Q+1)  [Lsum | W]          (sum_n L_nab [1 | d_nq])
 //   TP:  M x 2Q       [P | R']            (sum_n T_na [d mu | d])
@@ -543,7 +536,7 @@ extern "C" int gpx_gemm_batched(int transA, int transB, int m, int n, int k, dou
 
 extern "C" {
 
-// Tail of the fused psi adjoint: from the per-point
+// Tail of a psi adjoint whose caller holds its sums: from the per-point
 // outputs T, Lp (N x M), H (N x Q), s0 (N x 2), Dn, Pn, En and the pair sums LW
 // ((M*M) x (Q+1)) finish dsf2, dell (w.r.t. ell) and dZ.  TP, LE (M x 2Q) and cols0 (2)
 // are workspace.
