@@ -34,6 +34,8 @@ SIGNATURES = {
     'gpx_se_kernel': (_i, [_i, _i, _i, _p, _i, _p, _p, _p, _d, _p, _p]),
     'gpx_kfu_bwd_workspace': (_l, [_i, _i, _i]),
     'gpx_kfu_bwd': (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
+    'gpx_kfu_bwd_reg_workspace': (_l, [_i, _i, _i]),
+    'gpx_kfu_bwd_reg': (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     'gpx_dtrace_workspace': (_l, [_i, _i]),
     'gpx_dtrace_kzz': (_i, [_i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p]),
     'gpx_colsum': (_i, [_i, _i, _p, _d, _d, _p, _p]),

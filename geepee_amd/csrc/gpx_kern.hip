@@ -71,17 +71,26 @@ __global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const doub
 // sums go to part[b][w][m].  Bound by reading dK and K once; partials of 16-row slabs summed
 // by 14 workgroups were most of the adjoint before (three passes at N = 20000, M = 200, Q = 8
 // 104 -> 38 us; N = 1000, M = 100, Q = 10 17 -> 18 us).
-template <int QC>
+// REG: dK is formed here, dK_nm = sum_d dm_nd A_dm + 2 dv_nd T_dnm (the propagation's adjoint at
+// deterministic inputs), which a product, a weighted sum over T and this pass wrote and read three
+// times; and sum_nd dv, one value per block, goes to part[b][2Q + 1][0].
+struct KfuReg {
+  int D;
+  const double *dm, *dv, *A, *T;
+};
+
+template <int QC, bool REG>
 __global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, int MP, const double *__restrict__ dK,
-                                                       const double *__restrict__ K,
+                                                       KfuReg reg, const double *__restrict__ K,
                                                        const double *__restrict__ x,
                                                        const double *__restrict__ z,
                                                        double *__restrict__ part) {
   __shared__ double red[2 * QC + 1][256];
+  __shared__ double sdv[4];
   // g is uniform over a wave (MP a multiple of 64): its x rows are scalar loads
   const int tid = threadIdx.x, m = tid % MP, g = __builtin_amdgcn_readfirstlane(tid / MP), G = 256 / MP,
             mc = min(m, M - 1);
-  double zr[QC], lx[QC], ld2[QC], cs = 0.0;
+  double zr[QC], lx[QC], ld2[QC], cs = 0.0, vsum = 0.0;
 #pragma unroll
   for (int q = 0; q < QC; ++q) {
     zr[q] = q < Q ? z[mc * Q + q] : 0.0;
@@ -94,7 +103,23 @@ __global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, int 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const long o = (long)min((long)n + (long)u * step, N - 1L) * M + mc;
-      L[u] = dK[o] * K[o];
+      if constexpr (REG) L[u] = 0.0; else L[u] = dK[o] * K[o];
+    }
+    if constexpr (REG) {
+      const int D = reg.D;
+#pragma unroll 2
+      for (int d = 0; d < D; ++d) {
+        const double a = reg.A[(long)d * M + mc];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const long rr = (long)n + (long)u * step, r = min(rr, N - 1L);
+          const double vv = reg.dv[r * D + d];
+          L[u] = fma(2.0 * vv, reg.T[((long)d * N + r) * M + mc], fma(reg.dm[r * D + d], a, L[u]));
+          if (rr < N) vsum += vv;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) L[u] *= K[(long)min((long)n + (long)u * step, N - 1L) * M + mc];
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -116,13 +141,19 @@ __global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, int 
     red[1 + q][tid] = lx[q];
     red[1 + QC + q][tid] = ld2[q];
   }
+  if (REG && m == 0) sdv[g] = vsum;  // the same in every column of the group
   __syncthreads();
-  const int W = 2 * Q + 1;
+  const int W = 2 * Q + 1, rows = REG ? W + 1 : W;
   for (int e = tid; e < W * M; e += 256) {
     const int w = e / M, c = e % M, r = w <= Q ? w : w - Q + QC;
     double s = red[r][c];
     for (int h = 1; h < G; ++h) s += red[r][h * MP + c];
-    part[((long)blockIdx.x * W + w) * M + c] = s;
+    part[((long)blockIdx.x * rows + w) * M + c] = s;
+  }
+  if (REG && tid == 0) {
+    double s = sdv[0];
+    for (int h = 1; h < G; ++h) s += sdv[h];
+    part[((long)blockIdx.x * rows + W) * M] = s;
   }
 }
 
@@ -173,8 +204,9 @@ __global__ __launch_bounds__(1024) void kfu_bwd_final(int nblk, int M, int W, co
 
 // Pass 3, one wave per output j <= Q, lanes over m and a fixed-order wave reduction:
 // dsf2 = sum_m colsum_m / sf2, dell_q = sum_m Ld2_mq / ell^3, and
-// dZ_mq = -(z_mq colsum_m - Lx_mq) / l_q.
+// dZ_mq = -(z_mq colsum_m - Lx_mq) / l_q.  extra (may be NULL) is added to dsf2.
 __global__ __launch_bounds__(64) void kfu_bwd_scalars(int M, int Q, const double *__restrict__ red,
+                                                      const double *__restrict__ extra,
                                                       const double *__restrict__ z,
                                                       const double *__restrict__ ls,
                                                       const double *__restrict__ sf, double *__restrict__ dsf2,
@@ -190,7 +222,7 @@ __global__ __launch_bounds__(64) void kfu_bwd_scalars(int M, int Q, const double
   s = gpx_wave_sum(s);
   if (lane == 0) {
     if (j == 0)
-      dsf2[0] = s / exp(2.0 * sf[0]);
+      dsf2[0] = extra ? s / exp(2.0 * sf[0]) + extra[0] : s / exp(2.0 * sf[0]);
     else
       dell[j - 1] = s / exp(3.0 * ls[j - 1]);
   }
@@ -281,7 +313,7 @@ __global__ __launch_bounds__(64) void kuu_tail_kernel(int M, int Q, const double
   for (int a = lane; a < M; a += 64) s += part[(long)a * (Q + 1) + j];
   s = gpx_wave_sum(s);
   if (lane != 0) return;
-  if (j == 0) dsf[0] = 2.0 * exp(2.0 * sf[0]) * (dsf2[0] + sumdv[0]) + 2.0 * s;
+  if (j == 0) dsf[0] = 2.0 * exp(2.0 * sf[0]) * (sumdv ? dsf2[0] + sumdv[0] : dsf2[0]) + 2.0 * s;
   else dls[j - 1] = dell[j - 1] * exp(ls[j - 1]) + 2.0 * s;
 }
 
@@ -986,34 +1018,54 @@ static int kfu_blocks(int N, int M) { return (int)std::min<long>(512, gpx_cdiv(N
 
 long gpx_kfu_bwd_workspace(int N, int M, int Q) { return ((long)kfu_blocks(N, M) + 1) * M * (2 * Q + 1); }
 
+static int kfu_bwd_launch(int N, int M, int Q, const double *dK, const KfuReg *reg, const double *K, const double *x,
+                          const double *z, const double *ls, const double *sf, double *dsf2, double *dell, double *dZ,
+                          double *dx, double *work, hipStream_t st) {
+  const int nblk = kfu_blocks(N, M), MP = kfu_cols(M), W = 2 * Q + 1, rows = reg ? W + 1 : W;
+  double *red = work + (long)nblk * M * rows;
+#define GPX_KFU(QV)                                                                                           \
+  if (reg)                                                                                                    \
+    hipLaunchKernelGGL((kfu_bwd_partial<QV, true>), dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, *reg, K, x, z, work); \
+  else                                                                                                        \
+    hipLaunchKernelGGL((kfu_bwd_partial<QV, false>), dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, KfuReg{}, K, x, z, \
+                       work);
+  if (Q <= 4) { GPX_KFU(4) }
+  else if (Q <= 8) { GPX_KFU(8) }
+  else if (Q <= 12) { GPX_KFU(12) }
+  else { GPX_KFU(16) }
+#undef GPX_KFU
+  GPX_CHECK_LAUNCH();
+  if (dx) {
+    hipLaunchKernelGGL(kfu_dx_kernel, dim3(gpx_cdiv(N, 4)), dim3(256), 0, st, N, M, Q, dK, K, x, z, ls, dx);
+    GPX_CHECK_LAUNCH();
+  }
+  hipLaunchKernelGGL(kfu_bwd_final, dim3(gpx_cdiv(M, 64), rows), dim3(1024), 0, st, nblk, M, rows, (const double *)work,
+                     red);
+  GPX_CHECK_LAUNCH();
+  hipLaunchKernelGGL(kfu_bwd_scalars, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)red,
+                     reg ? (const double *)red + (long)W * M : nullptr, z, ls, sf, dsf2, dell, dZ);
+  GPX_CHECK_LAUNCH();
+  return GPX_OK;
+}
+
 // Adjoint of K(x, Z): dsf2 (w.r.t. sf2), dell (w.r.t. ell), dZ (M x Q), dx (N x Q, optional).
 int gpx_kfu_bwd(int N, int M, int Q, const double *dK, const double *K, const double *x,
                 const double *z, const double *ls, const double *sf, double *dsf2, double *dell,
                 double *dZ, double *dx, double *work, void *stream) {
   if (N < 1 || M < 1 || M > 256 || Q < 1 || Q > 16) return GPX_EINVAL;
   if (!dK || !K || !x || !z || !ls || !sf || !dsf2 || !dell || !dZ || !work) return GPX_EINVAL;
-  hipStream_t st = (hipStream_t)stream;
-  const int nblk = kfu_blocks(N, M), MP = kfu_cols(M), W = 2 * Q + 1;
-  double *red = work + (long)nblk * M * W;
-  if (Q <= 4)
-    hipLaunchKernelGGL(kfu_bwd_partial<4>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
-  else if (Q <= 8)
-    hipLaunchKernelGGL(kfu_bwd_partial<8>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
-  else if (Q <= 12)
-    hipLaunchKernelGGL(kfu_bwd_partial<12>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
-  else
-    hipLaunchKernelGGL(kfu_bwd_partial<16>, dim3(nblk), dim3(256), 0, st, N, M, Q, MP, dK, K, x, z, work);
-  GPX_CHECK_LAUNCH();
-  if (dx) {
-    hipLaunchKernelGGL(kfu_dx_kernel, dim3(gpx_cdiv(N, 4)), dim3(256), 0, st, N, M, Q, dK, K, x, z, ls, dx);
-    GPX_CHECK_LAUNCH();
-  }
-  hipLaunchKernelGGL(kfu_bwd_final, dim3(gpx_cdiv(M, 64), W), dim3(1024), 0, st, nblk, M, W, (const double *)work, red);
-  GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(kfu_bwd_scalars, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)red, z, ls, sf, dsf2, dell,
-                     dZ);
-  GPX_CHECK_LAUNCH();
-  return GPX_OK;
+  return kfu_bwd_launch(N, M, Q, dK, nullptr, K, x, z, ls, sf, dsf2, dell, dZ, dx, work, (hipStream_t)stream);
+}
+
+long gpx_kfu_bwd_reg_workspace(int N, int M, int Q) { return ((long)kfu_blocks(N, M) + 1) * M * (2 * Q + 2); }
+
+int gpx_kfu_bwd_reg(int N, int D, int M, int Q, const double *dm, const double *dv, const double *A, const double *T,
+                    const double *K, const double *x, const double *z, const double *ls, const double *sf, double *dsf2,
+                    double *dell, double *dZ, double *work, void *stream) {
+  if (N < 1 || D < 1 || M < 1 || M > 256 || Q < 1 || Q > 16) return GPX_EINVAL;
+  if (!dm || !dv || !A || !T || !K || !x || !z || !ls || !sf || !dsf2 || !dell || !dZ || !work) return GPX_EINVAL;
+  const KfuReg reg{D, dm, dv, A, T};
+  return kfu_bwd_launch(N, M, Q, nullptr, &reg, K, x, z, ls, sf, dsf2, dell, dZ, nullptr, work, (hipStream_t)stream);
 }
 
 long gpx_dtrace_workspace(int M, int Q) { return (long)M * (Q + 1); }
@@ -1050,7 +1102,7 @@ int gpx_dtrace_kzz(int M, int Q, const double *Mm, const double *z, const double
 int gpx_kuu_tail(int M, int Q, const double *Mm, const double *z, const double *ls, const double *sf,
                  const double *dell, const double *dsf2, const double *sumdv, const double *dz0, double *dls,
                  double *dsf, double *dZ, double *work, void *stream) {
-  if (M < 1 || M > 256 || Q < 1 || Q > 16 || !Mm || !z || !ls || !sf || !dell || !dsf2 || !sumdv || !dz0 || !dls ||
+  if (M < 1 || M > 256 || Q < 1 || Q > 16 || !Mm || !z || !ls || !sf || !dell || !dsf2 || !dz0 || !dls ||
       !dsf || !dZ || !work)
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;

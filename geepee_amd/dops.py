@@ -260,6 +260,18 @@ def kfu_bwd(dK, K, x, z, ls, sf, want_dx=False):
     return outs
 
 
+def kfu_bwd_reg(dm, dv, A, T, K, x, z, ls, sf):
+    """(dsf2, dell, dz) of m = K A^T, v = sf2 + (K B_d) . K at inputs x, with T = K B (D, N, M); dsf2
+    includes v's own sf2 term (sum dv)."""
+    N, D = dm.shape
+    M, Q = z.shape
+    outs = [empty(1, like=x), empty(Q, like=x), empty(M, Q, like=x)]
+    work = empty(query('gpx_kfu_bwd_reg_workspace', N, M, Q), like=x)
+    call('gpx_kfu_bwd_reg', N, D, M, Q, P(dm), P(dv), P(A), P(T), P(K), P(x), P(z), P(ls), P(sf),
+         *[P(o) for o in outs], P(work), S())
+    return outs
+
+
 def dtrace(Mm, z, ls, sf):
     M, Q = z.shape
     outs = [empty(1, like=z), empty(Q, like=z), empty(M, Q, like=z)]
@@ -269,7 +281,8 @@ def dtrace(Mm, z, ls, sf):
 
 
 def kuu_tail(Mm, z, ls, sf, dell, dsf2, sumdv, dz):
-    """(dls, dsf, dzu): the hyper-parameter gradients with the trace terms of Kuu's adjoint Mm."""
+    """(dls, dsf, dzu): the hyper-parameter gradients with the trace terms of Kuu's adjoint Mm
+    (sumdv None: already in dsf2)."""
     M, Q = z.shape
     dls, dsf, dzu = torch.empty_like(ls), torch.empty_like(sf), torch.empty_like(dz)
     work = empty(query('gpx_dtrace_workspace', M, Q), like=z)

@@ -393,16 +393,12 @@ class SGP_Layer(object):
             return self._backprop_grads_reg_nat(dm, dv, kfu, x, alpha)
         N = self.N
         D, M = self.Dout, self.M
-        B = kfu.shape[0]
         Ki = self.Kuuinv
         scale_post = N * 1.0 / alpha - 1.0
         scale_cav = -N * 1.0 / alpha
         kfuKi = mm(kfu, Ki)
-        # grads wrt kfu: dm Ahat + 2 sum_d dv_nd (kfu Bhat_det[d])_n
-        dkfu = mm(dm, self.Ahat)
-        dops.wsum(dv, self._T_det, dkfu, alpha=2.0, beta=1.0)
-        dsf2, dell, dzu, _ = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf)
-        sumdv = colsum(dv, B * D, 1)
+        # through kfu: dm Ahat + 2 sum_d dv_nd (kfu Bhat_det[d])_n
+        dsf2, dell, dzu = dops.kfu_bwd_reg(dm, dv, self.Ahat, self._T_det, kfu, x, self.zu, self.ls, self.sf)
         # cavity mean / covariance
         dmucav = mm(dm, kfuKi, tA=True)
         dSucav = dops.gram(dv, kfuKi)
@@ -429,7 +425,7 @@ class SGP_Layer(object):
         if dKi_post is not None:
             lincomb(dKi, 1.0, dKi, 1.0, dKi_post)
         M_inner = _sandwich(Ki, dKi, Ki, alpha=-1.0)
-        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
+        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, None, dzu)
         deta1 = lincomb(deta1_cav, 1.0, deta1_cav, 1.0, deta1_post)
         deta2 = lincomb(deta2_cav, 1.0, deta2_cav, 1.0, deta2_post)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': deta2}
@@ -449,17 +445,13 @@ class SGP_Layer(object):
             Ki^T dBhat Ki (M x M products in place of two contractions over the batch)."""
         N = self.N
         D, M = self.Dout, self.M
-        B = kfu.shape[0]
         Ki = self.Kuuinv
         th = self.theta_2
         beta = self._beta
         scale_post = N * 1.0 / alpha - 1.0
         scale_cav = -N * 1.0 / alpha
-        # grads wrt kfu: dm Ahat + 2 sum_d dv_nd (kfu Bhat_det[d])_n
-        dkfu = mm(dm, self.Ahat)
-        dops.wsum(dv, self._T_det, dkfu, alpha=2.0, beta=1.0)
-        dsf2, dell, dzu, _ = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf)
-        sumdv = colsum(dv, B * D, 1)
+        # through kfu: dm Ahat + 2 sum_d dv_nd (kfu Bhat_det[d])_n
+        dsf2, dell, dzu = dops.kfu_bwd_reg(dm, dv, self.Ahat, self._T_det, kfu, x, self.zu, self.ls, self.sf)
         dAhat = mm(dm, kfu, tA=True)
         dBhat = dops.gram(dv, kfu)
         # cavity: dmu_cav, dSu_cav (+ the normalising factor), then dSuinv_cav
@@ -476,7 +468,7 @@ class SGP_Layer(object):
                  outer=(dAhat, self.muhat, 1.0))
         colsum(dS_cav, D, M * M, out=dKi.reshape(-1), beta=1.0)
         M_inner = _sandwich(Ki, dKi, Ki, alpha=-1.0)
-        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, sumdv, dzu)
+        dls, dsf, dzu = dops.kuu_tail(M_inner, self.zu, self.ls, self.sf, dell, dsf2, None, dzu)
         return {'sf': dsf, 'ls': dls, 'zu': dzu, 'eta1_R': deta1, 'eta2': deta2}
 
     def backprop_grads_lvm_mc(self, m, v, dm, dv, kfu, x, alpha=1.0):

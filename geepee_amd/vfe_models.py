@@ -158,11 +158,15 @@ class SGP_Layer(_Layer):
         Ki = self.Kuuinv
         dm = dm.reshape(B, D)
         dv = dv.reshape(B, D)
-        # grads wrt kfu: dm A + 2 sum_d dv_nd (kfu B_det[d])_n
-        dkfu = mm(dm, self.A)
-        dops.wsum(dv, self._T_post, dkfu, alpha=2.0, beta=1.0)
-        dsf2, dell, dzu, dx = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf, want_dx=want_dx)
-        sumdv = colsum(dv, B * D, 1)
+        # through kfu: dm A + 2 sum_d dv_nd (kfu B_det[d])_n
+        if want_dx:
+            dkfu = mm(dm, self.A)
+            dops.wsum(dv, self._T_post, dkfu, alpha=2.0, beta=1.0)
+            dsf2, dell, dzu, dx = dops.kfu_bwd(dkfu, kfu, x, self.zu, self.ls, self.sf, want_dx=True)
+            sumdv = colsum(dv, B * D, 1)
+        else:
+            dsf2, dell, dzu = dops.kfu_bwd_reg(dm, dv, self.A, self._T_post, kfu, x, self.zu, self.ls, self.sf)
+            sumdv = None
         kfuKi = mm(kfu, Ki)
         # dmu = dm^T kfu Kuu^-1 + Kuu^-1 mu (A = mu Kuu^-1), dSu = sum_n dv kfuKi kfuKi^T + C0
         dmu = mm(dm, kfuKi, tA=True, E=self.A, gamma=1.0)

@@ -81,7 +81,7 @@ int gpx_moments(int batch, int D, int M, const double *S, const double *theta, d
                 double *P, void *stream);
 
 /* Kuu^-1's adjoint into the hyper-parameters: gpx_dtrace_kzz and gpx_hyper_grads in two launches, and
- * dZ = dz0 + its z gradient (dZ may be dz0; work: gpx_dtrace_workspace doubles).  Replaces
+ * dZ = dz0 + its z gradient (dZ may be dz0; sumdv may be NULL; work: gpx_dtrace_workspace doubles).  Replaces
  * geepee/aep_models.py:244-247, 296-304. */
 int gpx_kuu_tail(int M, int Q, const double *Mm, const double *z, const double *ls, const double *sf,
                  const double *dell, const double *dsf2, const double *sumdv, const double *dz0, double *dls,
@@ -153,6 +153,15 @@ long gpx_kfu_bwd_workspace(int N, int M, int Q);
 int gpx_kfu_bwd(int N, int M, int Q, const double *dK, const double *K, const double *x,
                 const double *z, const double *ls, const double *sf, double *dsf2,
                 double *dell, double *dZ, double *dx, double *work, void *stream);
+
+/* The adjoint of m = K A^T, v = sf2 + (K B_d) . K at deterministic inputs w.r.t. K's hyper-parameters,
+ * from dm, dv (N x D), A (D x M) and T_d = K B_d (D x N x M): gpx_kfu_bwd with
+ * dK = dm A + 2 sum_d dv_d T_d formed in its first pass, and sum dv added to dsf2 (the sf2 in v)
+ * (geepee/aep_models.py:456-466, 502-504). */
+long gpx_kfu_bwd_reg_workspace(int N, int M, int Q);
+int gpx_kfu_bwd_reg(int N, int D, int M, int Q, const double *dm, const double *dv, const double *A, const double *T,
+                    const double *K, const double *x, const double *z, const double *ls, const double *sf, double *dsf2,
+                    double *dell, double *dZ, double *work, void *stream);
 
 /* d tr(Mm Kzz) / d(2 sf, 2 ls, z) for Kzz = SE(z, z) without jitter: gsf, gls (Q), gz (M x Q);
  * M <= 256, Q <= 16.
