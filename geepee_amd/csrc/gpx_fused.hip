@@ -19,7 +19,7 @@
 // T_na = sum_b L_nab and V_nq = sum_ab L_nab z_aq z_bq of L = dpsi2 * psi2, and over the
 // points dBhat[d] = sum_n dv_nd psi2_n, Lsum = sum_n L_n, W_q = sum_n L_n d_nq, where
 // dpsi2_n = sum_d dv_nd Bsym[d].
-#include "gpx_common.h"
+#include "gpx_frag.h"
 
 #include <algorithm>
 
@@ -898,10 +898,11 @@ int rows_finish_blocks(int N, int M, int Q) {
   return (int)gpx_cdiv(N, gpx_cdiv(N, per));
 }
 
-// psi1, m = psi1 Ahat^T and v = sf2 + sum_s part - m^2 for FIN_PTS points per block.
-// Points per block of the forward finish (8: twice the blocks of 16, so the latency-bound
-// psi1 and mean loops have two waves per SIMD at N = 4096).  The split partials' loads
-// issue four at a time (summed in split order).
+// psi1, m = psi1 Ahat^T and v = sf2 + sum_s part - m^2 for FIN_PTS points per block (8: two waves
+// per SIMD at N = 4096).  The means are products on the matrix cores, each wave every fourth group
+// of 8 inducing points, added in wave order (a thread per output walked M inducing points with a
+// row of Ahat of its own: N = 4096, M = 128, Q = 8, D = 32 21 -> 10 us, 3001, 190, 10, 12 16 -> 11).
+// The split partials' loads issue four at a time (summed in split order).
 constexpr int FIN_PTS = 8;
 
 __global__ __launch_bounds__(256) void fused_fwd_finish(int N, int M, int Q, int D, const double *__restrict__ mx,
@@ -914,6 +915,7 @@ __global__ __launch_bounds__(256) void fused_fwd_finish(int N, int M, int Q, int
                                                         double *__restrict__ psi1, double *__restrict__ mout,
                                                         double *__restrict__ vout) {
   __shared__ double p1[FIN_PTS][FM_MAX + 1];
+  __shared__ double ms[4][2][FIN_PTS * 16];  // the waves' means
   __shared__ double rden[FIN_PTS][FQ_MAX], mus[FIN_PTS][FQ_MAX], lts[FIN_PTS][FQ_MAX], lcs[FIN_PTS];
   const int n0 = blockIdx.x * FIN_PTS, tid = threadIdx.x;
   const double sf2 = exp(2.0 * sf[0]);
@@ -948,6 +950,31 @@ __global__ __launch_bounds__(256) void fused_fwd_finish(int N, int M, int Q, int
     p1[nn][m] = val;
   }
   __syncthreads();
+  // m: rows are the points (past the last: the last again), columns the outputs
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
+  const double *prow = p1[min(c, FIN_PTS - 1)];
+  const int groups = M >> 3, kr = M & 7;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (16 * t >= D) break;
+    const GpxOperand<1, true> ob(Ahat, M, 16 * t, D, lane);
+    gpx_d4 acc = {0.0, 0.0, 0.0, 0.0};
+    GpxFrag<1> f;
+    for (int k = w; k < groups; k += 4) {
+      ob.load(f, 8 * k);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) acc = gpx_mfma16(prow[8 * k + 2 * g + s], f.v[s][0], acc);
+    }
+    if (kr && w == groups % 4) {
+      ob.load_tail(f, 8 * groups, kr, lane);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        acc = gpx_mfma16(2 * g + s < kr ? prow[8 * groups + 2 * g + s] : 0.0, f.v[s][0], acc);
+    }
+#pragma unroll
+    for (int r = 0; r < FIN_PTS / 4; ++r) ms[w][t][r * 64 + lane] = acc[r];
+  }
+  __syncthreads();
   for (int e = tid; e < FIN_PTS * D; e += 256) {
     const int nn = e / D, d = e % D, n = n0 + nn;
     if (n >= N) continue;
@@ -960,18 +987,8 @@ __global__ __launch_bounds__(256) void fused_fwd_finish(int N, int M, int Q, int
       for (int u = 0; u < 4; ++u)
         if (sp0 + u < S) s += pv[u];
     }
-    // four independent partial sums (k mod 4): a 128-long chain of dependent FMAs was
-    // this loop's latency
-    const double *arow = Ahat + (long)d * M;
-    double m4[4] = {0.0, 0.0, 0.0, 0.0};
-    int k = 0;
-#pragma unroll 2
-    for (; k + 4 <= M; k += 4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) m4[u] += p1[nn][k + u] * arow[k + u];
-    }
-    for (int u = 0; k < M; ++k, ++u) m4[u] += p1[nn][k] * arow[k];
-    const double m = (m4[0] + m4[1]) + (m4[2] + m4[3]);
+    const int i = (nn >> 2) * 64 + (nn & 3) * 16 + (d & 15), t = d >> 4;
+    const double m = ms[0][t][i] + ms[1][t][i] + ms[2][t][i] + ms[3][t][i];
     mout[(long)n * D + d] = m;
     vout[(long)n * D + d] = sf2 + s - m * m;
   }
