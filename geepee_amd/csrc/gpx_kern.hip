@@ -320,6 +320,47 @@ __global__ __launch_bounds__(64) void kuu_tail_kernel(int M, int Q, const double
 // mu_b = s_b S_b t_b and P_b = S_b + mu_b mu_b^T.  Workgroup (b, y) forms all of mu_b (a wave per
 // row, four rows in flight; the matrix comes from the caches the second time) and the rows of
 // P_b of its share y.  In place of a product and an outer product per set: M = 50, 2 sets 11 -> 3 us.
+// M > 128 (the repeated reads outweigh a launch): means first, 16 rows per workgroup, then the
+// outer products (M = 256, 4 matrices 16 -> 10 us; M = 200, 8 15 -> 9).
+__global__ __launch_bounds__(256) void mean_kernel(int D, int M, const double *__restrict__ S,
+                                                   const double *__restrict__ theta, double s0, double s1,
+                                                   double *__restrict__ mu) {
+  const int b = blockIdx.x, lane = threadIdx.x & 63, i0 = blockIdx.y * 16 + (threadIdx.x >> 6) * 4;
+  const double *Sb = S + (long)b * M * M, *t = theta + (long)(b % D) * M;
+  double sv[4][4], acc[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sv[u][j] = Sb[(long)min(i0 + u, M - 1) * M + min(lane + 64 * j, M - 1)];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    acc[u] = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (lane + 64 * j < M) acc[u] = fma(sv[u][j], t[lane + 64 * j], acc[u]);
+    acc[u] = gpx_wave_sum(acc[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (lane == 0 && i0 + u < M) mu[(long)b * M + i0 + u] = (b < D ? s0 : s1) * acc[u];
+}
+
+__global__ __launch_bounds__(256) void second_kernel(int M, const double *__restrict__ S,
+                                                     const double *__restrict__ mu, double *__restrict__ P) {
+  const int b = blockIdx.x, lane = threadIdx.x & 63, i0 = blockIdx.y * 16 + (threadIdx.x >> 6) * 4;
+  const double *Sb = S + (long)b * M * M, *m = mu + (long)b * M;
+  double *Pb = P + (long)b * M * M;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int c = lane + 64 * j;
+    if (c >= M) break;
+    const double mc = m[c];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + u < M) Pb[(long)(i0 + u) * M + c] = m[i0 + u] * mc + Sb[(long)(i0 + u) * M + c];
+  }
+}
+
 __global__ __launch_bounds__(1024) void moments_kernel(int D, int M, const double *__restrict__ S,
                                                        const double *__restrict__ theta, double s0, double s1,
                                                        double *__restrict__ mu, double *__restrict__ P) {
@@ -555,7 +596,9 @@ __global__ void batched_dot_kernel(int batch, int n, const double *__restrict__ 
 // scal[0] = logZ (with the alpha constant), scal[1] = dsn (scaled).
 // dm/dv outputs are scaled by `scale`; dmall = dm - 2 dv m when requested.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void gauss_tilted_kernel(int B, int D, const double *__restrict__ m,
+// Bound by the latency of an element's log and division: as few elements per thread as 64 blocks
+// (their partials) allow (131072 elements 11.6 -> 6.1 us, 1000 7.3 -> 4.4).
+__global__ __launch_bounds__(1024) void gauss_tilted_kernel(int B, int D, const double *__restrict__ m,
                                                            const double *__restrict__ v,
                                                            const double *__restrict__ y,
                                                            const double *__restrict__ sn, double alpha,
@@ -568,11 +611,12 @@ __global__ __launch_bounds__(256) void gauss_tilted_kernel(int B, int D, const d
   const double two_pi = 6.283185307179586;
   double lz = 0.0, sdv = 0.0;
   const long n = (long)B * D;
-  for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
-    const double vt = v[e] + sn2 / alpha;
-    const double r = y[e] - m[e];
-    lz += -0.5 * (log(two_pi * vt) + r * r / vt);
-    const double gm = r / vt, gv = -0.5 / vt + 0.5 * r * r / (vt * vt);
+  const double sa = sn2 / alpha;
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
+    const double vt = v[e] + sa, iv = 1.0 / vt;
+    const double r = y[e] - m[e], gm = r * iv;
+    lz += -0.5 * (log(two_pi * vt) + r * gm);
+    const double gv = 0.5 * (gm * gm - iv);
     sdv += gv;
     dm[e] = scale * gm;
     dv[e] = scale * gv;
@@ -1119,8 +1163,15 @@ int gpx_moments(int batch, int D, int M, const double *S, const double *theta, d
   if (batch < 0 || D < 1 || M < 1 || M > 256) return GPX_EINVAL;
   if (batch == 0) return GPX_OK;
   if (!S || !theta || !mu || !P) return GPX_EINVAL;
-  hipLaunchKernelGGL(moments_kernel, dim3(batch, gpx_cdiv(M, 64)), dim3(1024), 0, (hipStream_t)stream, D, M, S, theta,
-                     s0, s1, mu, P);
+  hipStream_t st = (hipStream_t)stream;
+  if (M <= 128) {
+    hipLaunchKernelGGL(moments_kernel, dim3(batch, gpx_cdiv(M, 64)), dim3(1024), 0, st, D, M, S, theta, s0, s1, mu, P);
+  } else {
+    const dim3 grid(batch, gpx_cdiv(M, 16));
+    hipLaunchKernelGGL(mean_kernel, grid, dim3(256), 0, st, D, M, S, theta, s0, s1, mu);
+    GPX_CHECK_LAUNCH();
+    hipLaunchKernelGGL(second_kernel, grid, dim3(256), 0, st, M, S, (const double *)mu, P);
+  }
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }
@@ -1280,9 +1331,8 @@ int gpx_gauss_tilted(int B, int D, const double *m, const double *v, const doubl
   if (B < 1 || D < 1 || !(alpha > 0) || !m || !v || !y || !sn || !dm || !dv || !scal) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   long n = (long)B * D;
-  int nblk = (int)gpx_cdiv(n, 1024);
-  if (nblk > 64) nblk = 64;
-  hipLaunchKernelGGL(gauss_tilted_kernel, dim3(nblk), dim3(256), 0, st, B, D, m, v, y, sn, alpha, scale, dm, dv,
+  const int threads = n > 64 * 256 ? 1024 : 256, nblk = (int)std::min<long>(64, gpx_cdiv(n, threads));
+  hipLaunchKernelGGL(gauss_tilted_kernel, dim3(nblk), dim3(threads), 0, st, B, D, m, v, y, sn, alpha, scale, dm, dv,
                      dmall, scal + 2);
   GPX_CHECK_LAUNCH();
   hipLaunchKernelGGL(gauss_tilted_finish, dim3(1), dim3(64), 0, st, nblk, B, D, (const double *)(scal + 2), sn,

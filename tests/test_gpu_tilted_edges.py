@@ -1,0 +1,32 @@
+"""The Gaussian tilted likelihood around its block counts and sizes (GPU only).
+
+Tolerance: per-element formulas to a few ulp (1e-13), the two sums of up to 70000 terms of one sign
+or mixed within 1e-12 of the sum of magnitudes.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('B,D', [(1, 1), (256, 1), (257, 1), (5462, 3), (16384, 1), (16385, 1), (17500, 4)])
+@pytest.mark.parametrize('alpha', [1.0, 0.3])
+def test_gauss_tilted(B, D, alpha):
+    from geepee_amd import dops
+    print('tilted', B, D, alpha, flush=True)
+    rs = np.random.RandomState(B + D)
+    m, v, y, sn, scale = rs.randn(B, D), rs.rand(B, D) + 0.1, rs.randn(B, D), np.array([-0.7]), 0.37
+    sn2 = np.exp(2 * sn[0])
+    vt, r = v + sn2 / alpha, y - m
+    gm, gv = r / vt, -0.5 / vt + 0.5 * r * r / vt ** 2
+    terms = -0.5 * (np.log(2 * np.pi * vt) + r * r / vt)
+    const = B * D * (0.5 * np.log(2 * np.pi * sn2 / alpha) - 0.5 * alpha * np.log(2 * np.pi * sn2))
+    t = [torch.as_tensor(a, device='cuda') for a in (m, v, y, sn)]
+    dm, dv, dmall, scal = [a.cpu().numpy() for a in dops.gauss_tilted(*t, alpha, scale, want_dmall=True)]
+    assert np.allclose(dm, scale * gm, rtol=1e-13, atol=1e-15)
+    assert np.allclose(dv, scale * gv, rtol=1e-12, atol=1e-14)
+    assert np.allclose(dmall, scale * gm - 2 * scale * gv * m, rtol=1e-11, atol=1e-13)
+    assert abs(scal[0] - (terms.sum() + const)) < 1e-12 * (np.abs(terms).sum() + abs(const))
+    dsn = (gv.sum() * 2 * sn2 / alpha + B * D * (1 - alpha)) * scale
+    assert abs(scal[1] - dsn) < 1e-12 * (np.abs(gv).sum() * 2 * sn2 / alpha + B * D) * scale
