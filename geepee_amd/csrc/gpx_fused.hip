@@ -289,42 +289,43 @@ __global__ void sym_pairmajor_kernel(int D, int M, const double *__restrict__ B,
 
 
 // Point features of the adjoint, formed once per launch: pf[n] = [w_n (16, zero past Q) | 1 |
-// d_n (15, zero past Q)] and u[n][m].  One workgroup per 16 points.
-constexpr int PF_W = 32;
+// d_n (15, zero past Q)] and u[n][m].  PF_PTS points per workgroup: its set-up (a log and a
+// division per dimension) and M Q multiply-adds per point are latency, hidden by many workgroups
+// (16 points in each: N = 3001, M = 190, Q = 10 12.6 -> 7.3 us).
+constexpr int PF_W = 32, PF_PTS = 4;
 
 __global__ __launch_bounds__(256) void fused_point_feat_kernel(int N, int M, int Q, const double *__restrict__ mx,
                                                                const double *__restrict__ vx,
                                                                const double *__restrict__ z,
                                                                const double *__restrict__ ls,
                                                                double *__restrict__ pf, double *__restrict__ un) {
-  __shared__ double lam[FQ_MAX], mu[16][FQ_MAX + 1], dd[16][FQ_MAX + 1], pc[16];
-  const int tid = threadIdx.x, n0 = blockIdx.x * 16, nn = tid >> 4, q = tid & 15, n = n0 + nn;
-  if (tid < FQ_MAX) lam[tid] = tid < Q ? exp(2.0 * ls[tid]) : 1.0;
-  __syncthreads();
-  const bool in = q < Q && n < N;
-  const double v = in ? vx[(long)n * Q + q] : 0.0, d = 1.0 / (2.0 * v + lam[q]);
-  mu[nn][q] = in ? mx[(long)n * Q + q] : 0.0;
-  dd[nn][q] = d;
-  if (n < N) {
-    double *o = pf + (long)n * PF_W;
-    o[q] = in ? 0.5 * v * d / lam[q] : 0.0;
-    if (q < 15) o[17 + q] = in ? d : 0.0;
-    else o[16] = 1.0;
+  __shared__ double mu[PF_PTS][FQ_MAX], dd[PF_PTS][FQ_MAX], lg[PF_PTS][FQ_MAX];
+  const int tid = threadIdx.x, n0 = blockIdx.x * PF_PTS;
+  if (tid < PF_PTS * 16) {
+    const int nn = tid >> 4, q = tid & 15, n = n0 + nn;
+    const bool in = q < Q && n < N;
+    const double lam = q < Q ? exp(2.0 * ls[q]) : 1.0;
+    const double v = in ? vx[(long)n * Q + q] : 0.0, d = 1.0 / (2.0 * v + lam);
+    mu[nn][q] = in ? mx[(long)n * Q + q] : 0.0;
+    dd[nn][q] = -0.5 * d;
+    lg[nn][q] = in ? 0.25 * log(lam * d) : 0.0;
+    if (n < N) {
+      double *o = pf + (long)n * PF_W;
+      o[q] = in ? 0.5 * v * d / lam : 0.0;
+      if (q < 15) o[17 + q] = in ? d : 0.0;
+      else o[16] = 1.0;
+    }
   }
   __syncthreads();
-  if (tid < 16) {
-    double c = 0.0;
-    for (int k = 0; k < Q; ++k) c += 0.25 * log(lam[k] * dd[tid][k]);
-    pc[tid] = c;
-  }
-  __syncthreads();
-  for (int e = tid; e < 16 * M; e += 256) {
+  for (int e = tid; e < PF_PTS * M; e += 256) {
     const int i = e / M, m = e % M;
     if (n0 + i >= N) break;
-    double u = pc[i];
+    double u = 0.0;
+    for (int k = 0; k < Q; ++k) u += lg[i][k];
+#pragma unroll 4
     for (int k = 0; k < Q; ++k) {
       const double dz = mu[i][k] - z[m * Q + k];
-      u = fma(-0.5 * dd[i][k] * dz, dz, u);
+      u = fma(dd[i][k] * dz, dz, u);
     }
     un[(long)(n0 + i) * M + m] = u;
   }
@@ -866,7 +867,7 @@ __global__ __launch_bounds__(256) void fused_tail_kernel(int M, int Q, int block
   const int cols = a < M ? Q : Q + 2;
   double t = 0.0, x = 0.0;
   if (q < cols) {
-#pragma unroll 4
+#pragma unroll 16
     for (int k = h; k < blocks; k += 16) t += part[(long)k * width + a * Q + q];
   }
   if (a == M && q == 0 && Q + 1 == 16) {  // the 17th column, A1 at Q = 15
@@ -1061,7 +1062,7 @@ int gpx_fused_mm_bwd_points(int N, int M, int Q, int D, const double *mx, const 
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   FusedBwdWork W(work, N, M, Q, D, splits, nsplit);
-  hipLaunchKernelGGL(fused_point_feat_kernel, dim3(gpx_cdiv(N, 16)), dim3(256), 0, st, N, M, Q, mx, vx, z, ls, W.pf,
+  hipLaunchKernelGGL(fused_point_feat_kernel, dim3(gpx_cdiv(N, PF_PTS)), dim3(256), 0, st, N, M, Q, mx, vx, z, ls, W.pf,
                      W.un);
   GPX_CHECK_LAUNCH();
   // both passes in one kernel: the per-pair partials (dBpart, LWpart) are written here too,
