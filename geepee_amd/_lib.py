@@ -207,7 +207,9 @@ def P(t):
 
 
 def S():
-    return torch.cuda.current_stream().cuda_stream
+    """Handle of the current device's current stream.  Every launch asks for it: the raw handle
+    takes 0.4 us, torch.cuda.current_stream(), which builds a Stream object, 2.8."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def require_device():
