@@ -37,8 +37,8 @@ FP64_PEAK_TFLOPS = 78.6     # MI355X dense FP64 (vector and matrix)
 # shapes.  On MI355X a plain copy of 512 MiB reads as FETCH_SIZE 262,200 KiB and
 # WRITE_SIZE 524,288 KiB, so FETCH_SIZE is scaled by 2.0 and WRITE_SIZE by 1.0.
 TRAFFIC = {
-    ('sgplvm', 'gpx_psi_fwd'): 2.0 * 2185 * 1024 + 1.0 * 528384 * 1024,
-    ('sgplvm', 'gpx_fused_mm_bwd'): 2.0 * 59085 * 1024 + 1.0 * 85058 * 1024,
+    ('sgplvm', 'gpx_psi_fwd'): 2.0 * 2189 * 1024 + 1.0 * 528612 * 1024,
+    ('sgplvm', 'gpx_fused_mm_bwd'): 2.0 * 81169 * 1024 + 1.0 * 87074 * 1024,
 }
 
 WORKLOADS = {
@@ -97,7 +97,7 @@ def _blas_info():
 
 def _host_threads():
     """Threads this process may use on the host: the CPU affinity set, capped by
-    OMP_NUM_THREADS when the environment sets it (the GPU box gives each GPU 16)."""
+    OMP_NUM_THREADS when the environment sets it (16 per GPU is typical)."""
     n = len(os.sched_getaffinity(0))
     env = os.environ.get('OMP_NUM_THREADS')
     if env and env.isdigit() and int(env) > 0:
@@ -169,17 +169,16 @@ def roofline_model(entry, name, w):
             # psi1 (N x M) and psi2 (N x M x M) written once; mx, vx (N x Q) and z (M x Q) read once
             tot += 8.0 * (N * M * M + N * M + 2 * N * Q + M * Q)
         elif entry == 'gpx_fused_mm_fwd':
-            # per point and unordered pair: the K=2Q+2 exponent product and the D-long
-            # contraction with Bhat (2 flops per multiply-add); exp counted as one flop
+            # per point and unordered pair: the exponent's Q cross terms and two adds and the
+            # D-long contraction with Bhat (2 flops per multiply-add); exp counted as one flop
             pairs = M * (M + 1) / 2.0
-            tot += N * pairs * (2.0 * (2 * Q + 2) + 1.0 + 2.0 * D)
+            tot += N * pairs * (2.0 * Q + 2.0 + 1.0 + 2.0 * D)
         elif entry == 'gpx_fused_mm_bwd':
-            # per point and unordered pair, each product formed once: the exponent (2K) and
+            # per point and unordered pair, each product formed once: the exponent (2Q + 2) and
             # its exp (1), G = <dv, Bhat> (2D), the dBhat and LW contractions (2D + 2(Q+1)),
             # and the row sums and V terms of the per-point statistics (2 + 2Q)
             pairs = M * (M + 1) / 2.0
-            K = 2 * Q + 2
-            tot += N * pairs * (2.0 * K + 1.0 + 4.0 * D + 2.0 * (Q + 1) + 2.0 + 2.0 * Q)
+            tot += N * pairs * (2.0 * Q + 2.0 + 1.0 + 4.0 * D + 2.0 * (Q + 1) + 2.0 + 2.0 * Q)
     bound = 'hbm' if entry == 'gpx_psi_fwd' else 'mfma'
     return bound, (tot / launches if launches else 0.0)
 
