@@ -648,8 +648,9 @@ __global__ __launch_bounds__(64) void gauss_tilted_finish(int nblk, int B, int D
 
 // SGPSSM.compute_transition_tilted, 2-D branch (aep_models.py:1317-1343).
 // Outputs are already scaled; dmall = dmprop - 2 dvprop mprop for the MM adjoint.
-// Up to 64 blocks; part[2b], part[2b+1] = block b's (logZ, sum dv) partials.
-__global__ __launch_bounds__(256) void transition_kernel(int B, int D, const double *__restrict__ mp,
+// Up to 64 blocks; part[2b], part[2b+1] = block b's (logZ, sum dv) partials.  Bound by the latency of
+// an element's log and divisions, as gauss_tilted_kernel (40000 elements 6.7 -> 5.9 us).
+__global__ __launch_bounds__(1024) void transition_kernel(int B, int D, const double *__restrict__ mp,
                                                           const double *__restrict__ vp,
                                                           const double *__restrict__ mt,
                                                           const double *__restrict__ vt,
@@ -664,7 +665,7 @@ __global__ __launch_bounds__(256) void transition_kernel(int B, int D, const dou
   const double two_pi = 6.283185307179586;
   double lz = 0.0, sdv = 0.0;
   const long n = (long)B * D;
-  for (long e = blockIdx.x * 256L + threadIdx.x; e < n; e += (long)gridDim.x * 256) {
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
     const double vs = vt[e] + vp[e] + sn2 / alpha;
     const double md = mt[e] - mp[e];
     lz += -0.5 * md * md / vs - 0.5 * log(1.0 + alpha * (vt[e] + vp[e]) / sn2) -
@@ -706,7 +707,13 @@ __global__ __launch_bounds__(64) void transition_finish(int nblk, int B, int D, 
 // (unscaled), summed with wave reductions.
 constexpr int EM_T = 64;
 constexpr int EM_DMAX = 8;
-template <int DT>
+// DI: the row length of C kept in LDS, Din rounded up to 4 or 8 with zeros (0: any Din, its
+// loops at run time).  Bound by latency: Nb / 64 waves are less than one per SIMD up to Nb =
+// 65,000.  So a step's mx, vx and y are in registers before the algebra, the loops over Din are
+// unrolled (their sums and the wave sums interleave), the wave sums land in one lane each and
+// are stored together, and dvx reuses dC's product: Nb = 10000, Dout = 8, Din = 4
+// 37 -> 19 us (with the finish 47 -> 23).
+template <int DT, int DI>
 __global__ __launch_bounds__(EM_T) void emission_kernel(int Nb, int Din, const double *__restrict__ C,
                                                         const double *__restrict__ Rp,
                                                         const double *__restrict__ y, int ldy,
@@ -716,16 +723,35 @@ __global__ __launch_bounds__(EM_T) void emission_kernel(int Nb, int Din, const d
                                                         double *__restrict__ dmx, double *__restrict__ dvx,
                                                         double *__restrict__ part) {
   constexpr int NL = DT * (DT + 1) / 2;
+  constexpr int DR = DI ? DI : 1;
   __shared__ double Cs[EM_DMAX * EM_DMAX];
   __shared__ double Rs[EM_DMAX];
   const int tid = threadIdx.x, t = blockIdx.x * EM_T + tid;
-  for (int e = tid; e < DT * Din; e += EM_T) Cs[e] = C[e];
+  const int ldc = DI ? DI : Din;
+  if (DI) {
+    if (tid < DT * DI) Cs[tid] = tid % DR < Din ? C[tid / DR * Din + tid % DR] : 0.0;
+  } else {
+    for (int e = tid; e < DT * Din; e += EM_T) Cs[e] = C[e];
+  }
   if (tid < DT) Rs[tid] = exp(2.0 * Rp[tid]);
-  __syncthreads();
   const bool ok = t < Nb;
   const int tt = ok ? t : Nb - 1;  // padding steps compute a real step's values, weighted 0
   const double wgt = ok ? 1.0 : 0.0;
   const double *vt = vx + (long)tt * ldv, *mt = mx + (long)tt * ldm;
+  double mr[DR], vr[DR], r[DT], u[DT];
+  if (DI) {
+#pragma unroll
+    for (int c = 0; c < DR; ++c) {  // loads at clamped columns, without a branch; zero past Din
+      const double m = mt[c < Din ? c : Din - 1], v = vt[c < Din ? c : Din - 1];
+      mr[c] = c < Din ? m : 0.0;
+      vr[c] = c < Din ? v : 0.0;
+    }
+  }
+#define MT(c) (DI ? mr[DI ? (c) : 0] : mt[c])
+#define VT(c) (DI ? vr[DI ? (c) : 0] : vt[c])
+#pragma unroll
+  for (int a = 0; a < DT; ++a) r[a] = y[(long)tt * ldy + a];
+  __syncthreads();
 #define LI(a, b) ((a) * ((a) + 1) / 2 + (b))
   // Vy = diag(R/alpha) + C diag(vx) C^T (lower triangle)
   double L[NL];
@@ -734,7 +760,8 @@ __global__ __launch_bounds__(EM_T) void emission_kernel(int Nb, int Din, const d
 #pragma unroll
     for (int b = 0; b <= a; ++b) {
       double sum = 0.0;
-      for (int c = 0; c < Din; ++c) sum += Cs[a * Din + c] * vt[c] * Cs[b * Din + c];
+#pragma unroll
+      for (int c = 0; c < ldc; ++c) sum += Cs[a * ldc + c] * VT(c) * Cs[b * ldc + c];
       if (a == b) sum += Rs[a] / alpha;
       L[LI(a, b)] = sum;
     }
@@ -757,13 +784,10 @@ __global__ __launch_bounds__(EM_T) void emission_kernel(int Nb, int Din, const d
     }
   }
   // r = y - C mx;  u = Vy^{-1} r
-  double r[DT], u[DT];
 #pragma unroll
-  for (int a = 0; a < DT; ++a) {
-    double v = y[(long)tt * ldy + a];
-    for (int c = 0; c < Din; ++c) v -= Cs[a * Din + c] * mt[c];
-    r[a] = v;
-  }
+  for (int a = 0; a < DT; ++a)
+#pragma unroll
+    for (int c = 0; c < ldc; ++c) r[a] -= Cs[a * ldc + c] * MT(c);
 #pragma unroll
   for (int a = 0; a < DT; ++a) {  // forward
     double v = r[a];
@@ -809,62 +833,72 @@ __global__ __launch_bounds__(EM_T) void emission_kernel(int Nb, int Din, const d
   // logdet(I + alpha C V C^T / R) = logdet(Vy) + Dout log(alpha) - sum log R
   const double vlog = logdetV + DT * log(alpha) - sumlogR;
   double part0 = -0.5 * quad - 0.5 * vlog - 0.5 * DT * alpha * log(6.283185307179586) - 0.5 * alpha * sumlogR;
-  part0 = gpx_wave_sum(wgt * part0);
-  if (tid == 0) part[(long)blockIdx.x * (DT * Din + DT + 1)] = part0;
-  // dSigma = -Vinv/2 + u u^T / 2
-  const long pb = (long)blockIdx.x * (DT * Din + DT + 1);
+  // the block's sums: lane e keeps sum e (and e + 64)
+  double keep[2] = {gpx_wave_sum(wgt * part0), 0.0};
+  // dSigma = S = -Vinv/2 + u u^T / 2
+#define SG(a, b) (-0.5 * VI(a, b) + 0.5 * u[a] * u[b])
 #pragma unroll
   for (int a = 0; a < DT; ++a) {
-    const double dr = gpx_wave_sum(wgt * (-0.5 * VI(a, a) + 0.5 * u[a] * u[a]));
-    if (tid == 0) part[pb + 1 + DT * Din + a] = dr;
-    for (int c = 0; c < Din; ++c) {
-      double v = 0.0;
-#pragma unroll
-      for (int b = 0; b < DT; ++b) v += (-0.5 * VI(a, b) + 0.5 * u[a] * u[b]) * Cs[b * Din + c];
-      const double dc = gpx_wave_sum(wgt * (u[a] * mt[c] + 2.0 * v * vt[c]));
-      if (tid == 0) part[pb + 1 + a * Din + c] = dc;
-    }
+    const double dr = gpx_wave_sum(wgt * SG(a, a));
+    const int e = 1 + DT * Din + a;
+    keep[0] = tid == e ? dr : keep[0];
+    keep[1] = tid + EM_T == e ? dr : keep[1];
   }
-  if (ok) {
-    for (int c = 0; c < Din; ++c) {
-      double gm = 0.0, gv = 0.0;
 #pragma unroll
-      for (int a = 0; a < DT; ++a) {
-        gm += u[a] * Cs[a * Din + c];
+  for (int c = 0; c < ldc; ++c) {
+    double gm = 0.0, gv = 0.0;
 #pragma unroll
-        for (int b = 0; b < DT; ++b)
-          gv += (-0.5 * VI(a, b) + 0.5 * u[a] * u[b]) * Cs[a * Din + c] * Cs[b * Din + c];
-      }
+    for (int a = 0; a < DT; ++a) {
+      double v = 0.0;  // (S C)[a][c]
+#pragma unroll
+      for (int b = 0; b < DT; ++b) v += SG(a, b) * Cs[b * ldc + c];
+      gm += u[a] * Cs[a * ldc + c];
+      gv += v * Cs[a * ldc + c];
+      const double dc = gpx_wave_sum(wgt * (u[a] * MT(c) + 2.0 * v * VT(c)));
+      const int e = 1 + a * Din + c;
+      keep[0] = tid == e && c < Din ? dc : keep[0];
+      keep[1] = tid + EM_T == e && c < Din ? dc : keep[1];
+    }
+    if (ok && c < Din) {
       dmx[(long)t * Din + c] = gm * scale;
       dvx[(long)t * Din + c] = gv * scale;
     }
   }
+  const int W = DT * Din + DT + 1;
+  double *pb = part + (long)blockIdx.x * W;
+  if (tid < W) pb[tid] = keep[0];
+  if (tid + EM_T < W) pb[tid + EM_T] = keep[1];
+#undef SG
+#undef MT
+#undef VT
 #undef VI
 #undef LI
 }
 
-// logZ, dC, dR from the block partials (the dR chain of lik_layers.py:610-613).
-__global__ void emission_final(int nblk, int Nb, int Dout, int Din, const double *__restrict__ part,
-                               const double *__restrict__ Rp, double alpha, double scale,
-                               double *__restrict__ dC, double *__restrict__ dR, double *__restrict__ scal) {
-  const int W = Dout * Din + Dout + 1;
-  for (int i = threadIdx.x; i < W; i += blockDim.x) {
-    double s = 0.0;
-#pragma unroll 8
-    for (int b = 0; b < nblk; ++b) s += part[(long)b * W + i];
-    if (i == 0) {
-      scal[0] = s * scale;
-    } else if (i <= Dout * Din) {
-      dC[i - 1] = s * scale;
-    } else {
-      const int a = i - 1 - Dout * Din;
-      const double R = exp(2.0 * Rp[a]);
-      const double g = s / alpha + 0.5 * Nb * (1.0 - alpha) / R;
-      dR[a] = g * 2.0 * R * scale;
-    }
+// logZ, dC, dR from the block partials (the dR chain of lik_layers.py:610-613), a wave per
+// sum: lane l adds blocks l, l + 64, ... in order, then the wave's lanes.
+__global__ __launch_bounds__(64) void emission_final(int nblk, int Nb, int Dout, int Din,
+                                                     const double *__restrict__ part,
+                                                     const double *__restrict__ Rp, double alpha, double scale,
+                                                     double *__restrict__ dC, double *__restrict__ dR,
+                                                     double *__restrict__ scal) {
+  const int W = Dout * Din + Dout + 1, i = blockIdx.x;
+  double s = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nblk; b += 64) s += part[(long)b * W + i];
+  s = gpx_wave_sum(s);
+  if (threadIdx.x != 0) return;
+  if (i == 0) {
+    scal[0] = s * scale;
+  } else if (i <= Dout * Din) {
+    dC[i - 1] = s * scale;
+  } else {
+    const int a = i - 1 - Dout * Din;
+    const double R = exp(2.0 * Rp[a]);
+    const double g = s / alpha + 0.5 * Nb * (1.0 - alpha) / R;
+    dR[a] = g * 2.0 * R * scale;
   }
 }
-
 
 // out[d][n][m] = w[n, d] * X[n][m]   (the dv-weighted rows of aep_models.py:464, 490)
 __global__ void rowscale_kernel(int N, int D, int M, const double *__restrict__ w,
@@ -1350,9 +1384,10 @@ int gpx_transition_tilted(int B, int D, const double *mp, const double *vp, cons
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   long n = (long)B * D;
-  int nblk = (int)gpx_cdiv(n, 1024);
+  const int nt = n > 64 * 256 ? 1024 : 256;
+  int nblk = (int)gpx_cdiv(n, nt);
   if (nblk > 64) nblk = 64;
-  hipLaunchKernelGGL(transition_kernel, dim3(nblk), dim3(256), 0, st, B, D, mp, vp, mt, vt, sn, alpha, scale, dmall,
+  hipLaunchKernelGGL(transition_kernel, dim3(nblk), dim3(nt), 0, st, B, D, mp, vp, mt, vt, sn, alpha, scale, dmall,
                      dvp, dmt, dvt, scal + 2);
   GPX_CHECK_LAUNCH();
   hipLaunchKernelGGL(transition_finish, dim3(1), dim3(64), 0, st, nblk, B, D, (const double *)(scal + 2), sn,
@@ -1375,9 +1410,18 @@ int gpx_emission_tilted(int Nb, int Dout, int Din, const double *C, const double
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   const unsigned nblk = gpx_cdiv(Nb, EM_T);
-#define GPX_EMIS(DTV)                                                                                         \
-  hipLaunchKernelGGL((emission_kernel<DTV>), dim3(nblk), dim3(EM_T), 0, st, Nb, Din, C, Rp, y, ldy, mx, ldm, vx, \
-                     ldv, alpha, scale, dmx, dvx, work)
+#define GPX_EMIS1(DTV, DIV)                                                                                        \
+  hipLaunchKernelGGL((emission_kernel<DTV, DIV>), dim3(nblk), dim3(EM_T), 0, st, Nb, Din, C, Rp, y, ldy, mx, ldm, \
+                     vx, ldv, alpha, scale, dmx, dvx, work)
+#define GPX_EMIS(DTV)          \
+  do {                         \
+    if (Din <= 4)              \
+      GPX_EMIS1(DTV, 4);       \
+    else if (Din <= 8)         \
+      GPX_EMIS1(DTV, 8);       \
+    else                       \
+      GPX_EMIS1(DTV, 0);       \
+  } while (0)
   switch (Dout) {
     case 1: GPX_EMIS(1); break;
     case 2: GPX_EMIS(2); break;
@@ -1386,11 +1430,16 @@ int gpx_emission_tilted(int Nb, int Dout, int Din, const double *C, const double
     case 5: GPX_EMIS(5); break;
     case 6: GPX_EMIS(6); break;
     case 7: GPX_EMIS(7); break;
-    default: GPX_EMIS(8); break;
+    default:  // Dout Din <= 64
+      if (Din <= 4)
+        GPX_EMIS1(8, 4);
+      else
+        GPX_EMIS1(8, 8);
   }
 #undef GPX_EMIS
+#undef GPX_EMIS1
   GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(emission_final, dim3(1), dim3(256), 0, st, (int)nblk, Nb, Dout, Din, (const double *)work,
+  hipLaunchKernelGGL(emission_final, dim3(Dout * Din + Dout + 1), dim3(64), 0, st, (int)nblk, Nb, Dout, Din, (const double *)work,
                      Rp, alpha, scale, dC, dR, scal);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
