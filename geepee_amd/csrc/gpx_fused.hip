@@ -29,6 +29,15 @@
 #define FM_MAX 256
 #define U_PAD -1.0e4  // u of a padding point or column: its exp is an exact 0
 
+// u no lower than U_PAD (a NaN stays): psi2 of a point so far out is an exact 0 either way, and
+// the exponent of an infinite or huge mean or variance stays within what gpx_exp_tab reduces.
+__device__ __forceinline__ double u_floor(double u) { return u < U_PAD ? U_PAD : u; }
+
+// w = (1/l - d)/4 = v d / (2 l), with its limit at an infinite v (where v d is inf * 0).
+__device__ __forceinline__ double cross_weight(double v, double d, double l) {
+  return isinf(v) ? 0.25 / l : 0.5 * v * d / l;
+}
+
 namespace {
 
 __device__ __forceinline__ void decode_tile(int t, int T, int &A, int &B) {
@@ -131,7 +140,7 @@ __global__ __launch_bounds__(256) void fused_fwd_kernel(int N, int M, int Q, int
     const double v = q < Q ? vx[(long)n * Q + q] : 0.0, l = lam[q], dd = 1.0 / (2.0 * v + l);
     pmu[e] = q < Q ? mx[(long)n * Q + q] : 0.0;
     pd[e] = dd;
-    pw[e] = 0.5 * v * dd / l;
+    pw[e] = cross_weight(v, dd, l);
     pl[e] = 0.25 * log(l * dd);  // columns past Q: log 1
   }
   __syncthreads();
@@ -154,6 +163,7 @@ __global__ __launch_bounds__(256) void fused_fwd_kernel(int N, int M, int Q, int
           const double dz = mu[q] - zs[m * ZS + q];  // columns past Q: both zero
           u = fma(hd[q] * dz, dz, u);
         }
+        u = u_floor(u);
       }
       us[m * PTS + pt] = u;
     }
@@ -311,7 +321,7 @@ __global__ __launch_bounds__(256) void fused_point_feat_kernel(int N, int M, int
     lg[nn][q] = in ? 0.25 * log(lam * d) : 0.0;
     if (n < N) {
       double *o = pf + (long)n * PF_W;
-      o[q] = in ? 0.5 * v * d / lam : 0.0;
+      o[q] = in ? cross_weight(v, d, lam) : 0.0;
       if (q < 15) o[17 + q] = in ? d : 0.0;
       else o[16] = 1.0;
     }
@@ -327,7 +337,7 @@ __global__ __launch_bounds__(256) void fused_point_feat_kernel(int N, int M, int
       const double dz = mu[i][k] - z[m * Q + k];
       u = fma(dd[i][k] * dz, dz, u);
     }
-    un[(long)(n0 + i) * M + m] = u;
+    un[(long)(n0 + i) * M + m] = u_floor(u);
   }
 }
 

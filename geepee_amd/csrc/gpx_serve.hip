@@ -291,7 +291,9 @@ __global__ __launch_bounds__(SV_NT, 4) void serve_kernel(const GpxServeModel *__
           const double dz = sm.hm[p][q] - zm[q];
           u = fma(-0.5 * sm.pd[p][q] * dz, dz, u);
         }
-        sm.ft[m * SERVE_TILE + p] = m < M ? u : -1.0e4;
+        // no lower than the padding's: psi2 is an exact 0 there, and an exponent of any size stays
+        // within what gpx_exp_tab reduces (a NaN stays)
+        sm.ft[m * SERVE_TILE + p] = m < M && !(u < -1.0e4) ? u : -1.0e4;
       }
       __syncthreads();
       gpx_d4 acc;

@@ -106,3 +106,57 @@ def test_posterior_propagation_without_psi2(N, M, Q, D):
     for got in ((m, v), (m2, v2)):
         for x, y in zip(got, _reference(*P)):
             _close(x, y)
+
+
+def _far_rows(mx, vx):
+    """Rows whose psi2 is an exact 0: infinite and huge means and variances."""
+    inf = float('inf')
+    mx[0, 0], mx[1, -1], mx[2, 0], mx[3, -1] = inf, -inf, 1e40, -1e60
+    vx[4, 0], vx[5, -1] = inf, 1e308
+    mx[6, 0], vx[6, -1] = 1e35, inf if mx.shape[1] > 1 else 0.5
+
+
+@pytest.mark.parametrize('Q,D', [(1, 1), (2, 3), (5, 6), (8, 17)])
+@pytest.mark.parametrize('N,M', [(7, 3), (40, 33), (70, 130)])
+def test_posterior_propagation_infinite_inputs(N, M, Q, D):
+    """An infinite or huge mean or variance gives psi2 = 0, so mean 0 and variance sf2; the other
+    rows are those of the call without it, and a NaN stays in its row."""
+    from geepee_amd.layers import SGP_Layer
+    print('far inputs', N, M, Q, D, flush=True)
+    P = _problem(N, M, Q, D)
+    L = SGP_Layer(100, Q, D, M)
+    mx, vx, L.zu, L.ls, L.sf, L.A, L.B_sto = [p.cuda().contiguous() for p in P]
+    L._pred_ready, L._Bp_post = True, None
+    m0, v0 = L.forward_prop_thru_post(mx, vx)
+    _far_rows(mx, vx)
+    m, v = L.forward_prop_thru_post(mx, vx)
+    assert m[:7].abs().max() < 1e-140, m[:7]
+    torch.testing.assert_close(v[:7], torch.exp(2 * L.sf).expand(7, D), rtol=1e-15, atol=0.0)
+    assert torch.equal(m[7:], m0[7:]) and torch.equal(v[7:], v0[7:])
+    m2, v2, psi1, psi2 = L.forward_prop_thru_post(mx, vx, return_info=True)
+    assert torch.equal(psi2[:7], torch.zeros_like(psi2[:7]))
+    mx[0, 0], vx[1, 0] = float('nan'), float('nan')
+    m, v = L.forward_prop_thru_post(mx, vx)
+    assert torch.isnan(m[:2]).all() and torch.isnan(v[:2]).all()
+    assert torch.isfinite(m[2:]).all() and torch.isfinite(v[2:]).all()
+
+
+@pytest.mark.parametrize('N,M,Q,D', [(40, 33, 2, 3), (40, 20, 5, 6), (1003, 33, 3, 2)])
+def test_fused_adjoint_huge_inputs(N, M, Q, D):
+    """Points so far out that psi1 and psi2 are exact zeros contribute nothing to any gradient."""
+    from geepee_amd import dops
+    print('far adjoint', N, M, Q, D, flush=True)
+    P = _problem(N, M, Q, D)
+    rs = np.random.RandomState(6)
+    dm, dv = (torch.as_tensor(rs.randn(N, D)).cuda() for _ in range(2))
+    mx, vx, z, ls, sf, A, B = [p.cuda() for p in P]
+    Bp = dops.sym_pairmajor(B)
+    mx[0, 0], mx[N - 1, -1] = 1e40, -1e50
+    psi1, _, _ = dops.fused_mm_fwd(mx, vx, z, ls, sf, A, Bp)
+    got = dops.fused_mm_bwd(mx, vx, z, ls, sf, A, Bp, psi1, dm, dv)
+    for x in got[4:]:
+        assert torch.equal(x[0], torch.zeros_like(x[0])) and torch.equal(x[-1], torch.zeros_like(x[-1])), x[[0, -1]]
+    cut = lambda x: x[1:-1].contiguous()
+    want = dops.fused_mm_bwd(cut(mx), cut(vx), z, ls, sf, A, Bp, cut(psi1), cut(dm), cut(dv))
+    for x, y in zip(got[:4], want[:4]):
+        _close(x, y.cpu())

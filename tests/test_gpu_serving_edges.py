@@ -96,3 +96,17 @@ def test_serving_edges():
             assert g.shape == w.shape and _nrel(g, w) < bar, (MODELS[i], len(X), _nrel(g, w), bar)
     alone = store.predict_many([reqs[14]], noisy=True)[0]
     assert all(np.array_equal(a, b) for a, b in zip(alone, outs[14]))
+
+
+@pytest.mark.parametrize('M,H,Dout', [(20, 2, 1), (33, 5, 3)])
+def test_serving_far_hidden_values(M, H, Dout):
+    """Hidden means so large that psi1 and psi2 are exact zeros: mean 0, variance sf2 + sn2."""
+    from geepee_amd.serving import ModelStore
+    rs = np.random.RandomState(M)
+    sp = _spec(rs, M, 4, H, Dout)
+    sp['params']['eta2_0'] = 1e45 * sp['params']['eta2_0']
+    print('serving far', M, H, Dout, flush=True)
+    m, v = ModelStore([sp]).predict_many([(0, rs.randn(19, 4))], noisy=True)[0]
+    assert np.array_equal(m, np.zeros((19, Dout)))
+    want = np.exp(2 * sp['params']['sf_1'][0]) + np.exp(2 * sp['params']['sn'][0])
+    assert np.allclose(v, want, rtol=1e-14, atol=0.0), v
