@@ -407,6 +407,8 @@ class SDGPR(Base_Model):
         self.lik_layer = _make_lik(lik, self.N, self.Dout)
         self.sgp_layers = [SGP_Layer(self.N, self.size[i], self.size[i + 1], self.Ms[i])
                            for i in range(self.L)]
+        for layer in self.sgp_layers[1:]:
+            layer.gaussian_inputs = True
 
     def init_hypers(self, y_train=None):
         """base_models.py:1290-1312: layer 0 on the training inputs, the hidden layers
@@ -785,8 +787,10 @@ class SGPSSM(Base_Model):
             self.x_control = None
             self.Dcon_dyn = self.Dcon_emi = 0
         self.dyn_layer = SGP_Layer(self.N - 1, self.Din + self.Dcon_dyn, self.Din, self.M)
+        self.dyn_layer.gaussian_inputs = True
         if gp_emi:
             self.emi_layer = SGP_Layer(self.N, self.Din + self.Dcon_emi, self.Dout, self.M)
+            self.emi_layer.gaussian_inputs = True
             self.lik_layer = _make_lik(lik, self.N, self.Dout)
         else:
             self.emi_layer = Gauss_Emis(self.y_dev, self.Dout, self.Din + self.Dcon_emi)

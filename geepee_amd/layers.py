@@ -58,6 +58,8 @@ class SGP_Layer(object):
         self.M = no_pseudo
         self.nat_param = nat_param
         self._pred_ready = False
+        # whether predictions propagate Gaussian inputs through this layer beside deterministic ones
+        self.gaussian_inputs = False
         # fused=True: moment-matched propagation never writes psi2 to HBM; the forward
         # returns None in psi2's slot and the adjoint recomputes it.
         self.fused = False
@@ -159,15 +161,18 @@ class SGP_Layer(object):
             self.Splusmm = _plus_outer(self.Su, self.mu, self.mu)
         self._pred_ready = False
 
-    def _posterior_predictive(self):
-        """A, B_sto, B_det of update_posterior (base_models.py:477-488)."""
+    def _posterior_predictive(self, gaussian=False):
+        """A, B_sto, B_det of update_posterior (base_models.py:477-488), and with gaussian also
+        B_sto in the fused kernels' layout: a caller that makes the posterior safe to use from
+        other streams (by waiting for it) covers that operand too."""
         if self._pred_ready:
             return
         Ki = self.Kuuinv
         self.A = mm(self.mu, Ki, tB=True)
         self.B_sto = _sandwich(Ki, self.Splusmm, Ki, E=Ki, gamma=-1.0)
         self.B_det = _sandwich(Ki, self.Su, Ki, E=Ki, gamma=-1.0)
-        self._Bp_post = None
+        fused = gaussian and dops.fused_fits(self.M, self.zu.shape[1], self.Dout)
+        self._Bp_post = dops.sym_pairmajor(self.B_sto) if fused else None
         self._pred_ready = True
 
     # ------------------------------------------------------------------
@@ -323,7 +328,7 @@ class SGP_Layer(object):
         return m.reshape(S, B, self.Dout), v.reshape(S, B, self.Dout)
 
     def forward_prop_thru_post(self, mx, vx=None, mode=PROP_MM, return_info=False):
-        self._posterior_predictive()
+        self._posterior_predictive(gaussian=not return_info and (vx is not None or self.gaussian_inputs))
         if vx is None:
             kfu = dops.se(mx, self.zu, self.ls, self.sf)
             mout = mm(kfu, self.A, tB=True)
@@ -338,9 +343,10 @@ class SGP_Layer(object):
             # psi2 itself is not asked for: fold it into the contraction with B_sto instead of
             # storing N M^2 of it (M = 100, Q = 4, one output, us: 1 point 53 -> 21, 1000 93 -> 30,
             # 5000 447 -> 63; M = 256, Q = 10, D = 2: 1 point 57 -> 56, 5000 2245 -> 354)
-            if self._Bp_post is None:
-                self._Bp_post = dops.sym_pairmajor(self.B_sto)
-            _, mout, vout = dops.fused_mm_fwd(mx, vx, self.zu, self.ls, self.sf, self.A, self._Bp_post)
+            # (a posterior formed without the operand: formed here and not kept, since another
+            # stream, or work after a capture of this call, could not tell when it is there)
+            Bp = self._Bp_post if self._Bp_post is not None else dops.sym_pairmajor(self.B_sto)
+            _, mout, vout = dops.fused_mm_fwd(mx, vx, self.zu, self.ls, self.sf, self.A, Bp)
             return mout, vout
         psi1, psi2 = dops.psi_fwd(mx, vx, self.zu, self.ls, self.sf)
         mout = mm(psi1, self.A, tB=True)

@@ -80,7 +80,7 @@ class ModelStore(object):
                 sfx = '' if sp['kind'] == 'sgpr' else '_%d' % l
                 L = SGP_Layer(sp['N'], sizes[l], sizes[l + 1], sp['Ms'][l])
                 L.update_hypers(dp.views, key_suffix=sfx)
-                L._posterior_predictive()
+                L._posterior_predictive(gaussian=l > 0)
                 lay.append(L)
                 d = descs[i].layer[l]
                 d.type, d.M, d.Din, d.Dout = (0 if l == 0 else 1), L.M, L.Din, L.Dout

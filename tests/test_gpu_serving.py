@@ -115,3 +115,35 @@ def test_server_continuous_batching_matches_alone():
     lat_p, outs_p, _ = server.run_plain(reqs[:10])
     for (t, mid, X), (m, v), (pm, pv) in zip(reqs[:10], outs[:10], outs_p):
         assert nrel(pm, m) < 1e-9 and nrel(pv, v) < 1e-9
+
+
+def test_first_gaussian_call_on_any_stream():
+    """The resident layers are ready when the store is built: the first call of a two-layer model on
+    each of two streams, and one inside a capture that is never replayed, agree with later ones."""
+    import torch
+    from geepee_amd.serving import ModelStore
+    say('first gaussian call on any stream')
+    specs = [sp for sp in _specs() if sp['kind'] != 'sgpr'][:1]
+    X = np.random.RandomState(4).randn(37, specs[0]['Din'])
+    want = ModelStore(specs).predict_plain(0, X)
+    store = ModelStore(specs)
+    got = []
+    for st in (torch.cuda.Stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(st):
+            got.append(store.predict_plain(0, X))
+    assert all(np.array_equal(g, w) for o in got for g, w in zip(o, want))
+    store = ModelStore(specs)
+    L = store.layers[0][1]
+    m = torch.zeros(5, L.Din, dtype=torch.float64, device='cuda')
+    v = torch.ones_like(m)
+    first = [t.clone() for t in ModelStore(specs).layers[0][1].forward_prop_thru_post(m, v)]
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        held = L.forward_prop_thru_post(m, v)
+    eager = L.forward_prop_thru_post(m, v)
+    assert all(torch.equal(a, b) for a, b in zip(eager, first))
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(held, first))

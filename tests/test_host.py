@@ -186,3 +186,50 @@ def test_spd_status_raises_linalg_error():
     Base_Model.check_status(m)
     with pytest.raises(np.linalg.LinAlgError, match='during optimisation'):
         Base_Model.check_status(m, sticky=True)
+
+
+def _stub_layer(monkeypatch, M=20, Q=3, D=2):
+    """A layer on the CPU whose kernels are stand-ins that count the operand's formations."""
+    import torch
+    from geepee_amd import layers
+    formed = []
+    monkeypatch.setattr(layers.dops, 'sym_pairmajor', lambda B: formed.append(B) or B.permute(1, 2, 0))
+    monkeypatch.setattr(layers.dops, 'fused_mm_fwd', lambda *a, **k: (None, a[6], a[6]))
+    monkeypatch.setattr(layers, 'mm', lambda A, B, *a, **k: A)
+    monkeypatch.setattr(layers, '_sandwich', lambda A, B, C, **k: B)
+    L = layers.SGP_Layer(100, Q, D, M)
+    L.zu, L.ls, L.sf = torch.zeros(M, Q), torch.zeros(Q), torch.zeros(1)
+    L.Kuuinv, L.mu, L.Su, L.Splusmm = torch.zeros(M, M), torch.zeros(D, M), *torch.zeros(2, D, M, M)
+    return L, formed
+
+
+def test_gaussian_operand_comes_with_the_posterior(monkeypatch):
+    """The fused layout of B_sto is formed together with A, B_sto and B_det, so whatever orders
+    those for another stream orders it as well."""
+    import torch
+    x = torch.zeros(5, 3)
+    L, formed = _stub_layer(monkeypatch)
+    L.forward_prop_thru_post(x, x)
+    L.forward_prop_thru_post(x, x)
+    assert len(formed) == 1 and L._Bp_post is not None
+    L, formed = _stub_layer(monkeypatch)
+    L._posterior_predictive(gaussian=False)
+    assert not formed and L._Bp_post is None
+    L._pred_ready = False
+    L._posterior_predictive(gaussian=True)
+    assert len(formed) == 1 and L._Bp_post is not None
+    L, formed = _stub_layer(monkeypatch, Q=16)     # outside the fused kernels
+    L._posterior_predictive(gaussian=True)
+    assert not formed and L._Bp_post is None
+
+
+def test_gaussian_operand_formed_by_a_call_is_not_kept(monkeypatch):
+    """On a posterior formed without it (by a deterministic call, say on another stream), a call
+    forms its own operand and leaves nothing behind for callers that could not wait for it."""
+    import torch
+    x = torch.zeros(5, 3)
+    L, formed = _stub_layer(monkeypatch)
+    L._posterior_predictive()
+    L.forward_prop_thru_post(x, x)
+    L.forward_prop_thru_post(x, x)
+    assert len(formed) == 2 and L._Bp_post is None
