@@ -470,11 +470,16 @@ def fused_mm_fwd(mx, vx, z, ls, sf, Ahat, Bp, plan=None):
 def fused_mm_fwd_noalloc(mx, vx, z, ls, sf, Ahat, Bp, psi1, mout, vout, plan=None):
     """fused_mm_fwd into caller-provided outputs through the allocation-free entry point
     (its workspace is the library's fixed per-GPU scratch; overlapping calls on one GPU
-    race)."""
+    race).  Without a plan of the caller's, the splits are as many as the scratch holds: any N with
+    N D + M^2 <= gpx_fused_fwd_noalloc_max() is taken."""
     N, Q = mx.shape
     M = z.shape[0]
     D = Ahat.shape[0]
-    plan = plan or fused_plan(N, M, Q, D)
+    if plan is None:
+        plan = dict(fused_plan(N, M, Q, D))
+        most = query('gpx_fused_fwd_noalloc_max')
+        while plan['splits_f'] > 1 and query('gpx_fused_fwd_workspace', N, M, D, plan['splits_f']) > most:
+            plan['splits_f'] = -(-plan['splits_f'] // 2)
     call('gpx_fused_mm_fwd_noalloc', N, M, Q, D, P(mx), P(vx), P(z), P(ls), P(sf), P(Ahat), P(Bp),
          plan['splits_f'], plan['nsub'], P(psi1), P(mout), P(vout), S())
     return psi1, mout, vout

@@ -233,3 +233,23 @@ def test_gaussian_operand_formed_by_a_call_is_not_kept(monkeypatch):
     L.forward_prop_thru_post(x, x)
     L.forward_prop_thru_post(x, x)
     assert len(formed) == 2 and L._Bp_post is None
+
+
+@pytest.mark.parametrize('N,M,D', [(20000, 128, 32), (50000, 100, 32), (100000, 256, 32), (130000, 16, 32),
+                                   (1000000, 64, 4), (4096, 128, 32)])
+def test_noalloc_plan_fits_the_scratch(N, M, D, monkeypatch, tmp_path):
+    """The allocation-free forward takes every shape whose partial sums fit the scratch at one
+    split, however many splits the plan would like."""
+    from geepee_amd import _lib
+    monkeypatch.setenv('GEEPEE_AMD_TUNE_CACHE', str(tmp_path / 'none.json'))
+    autotune.clear()
+    seen = []
+    monkeypatch.setattr(dops, 'call', lambda name, *a: seen.append((name,) + a))
+    monkeypatch.setattr(dops, 'P', lambda t: t)
+    monkeypatch.setattr(dops, 'S', lambda: 0)
+    shape = lambda *s: type('T', (), {'shape': s})()
+    dops.fused_mm_fwd_noalloc(shape(N, 3), shape(N, 3), shape(M, 3), None, None, shape(D, M), None, None, None, None)
+    (name, splits), = [(c[0], c[12]) for c in seen]
+    assert name == 'gpx_fused_mm_fwd_noalloc' and splits >= 1
+    assert _lib.query('gpx_fused_fwd_workspace', N, M, D, splits) <= _lib.query('gpx_fused_fwd_noalloc_max')
+    autotune.clear()
