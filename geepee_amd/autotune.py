@@ -60,8 +60,14 @@ def _load():
     return _cache
 
 
+# What a stored plan was timed on: raised whenever a kernel or the meaning of one of its knobs
+# changes (gemm: tile became a wave's, not a workgroup's; fused: splits_b no longer splits the
+# adjoint).  Plans of another revision stay in the file and are not read.
+REVISION = {'fused': 2, 'gemm': 2}
+
+
 def _key(kind, shape):
-    return '%s|%s|%s' % (_device_tag(), kind, ','.join(str(int(s)) for s in shape))
+    return '%s|%s.%d|%s' % (_device_tag(), kind, REVISION[kind], ','.join(str(int(s)) for s in shape))
 
 
 def lookup(kind, shape):

@@ -253,3 +253,25 @@ def test_noalloc_plan_fits_the_scratch(N, M, D, monkeypatch, tmp_path):
     assert name == 'gpx_fused_mm_fwd_noalloc' and splits >= 1
     assert _lib.query('gpx_fused_fwd_workspace', N, M, D, splits) <= _lib.query('gpx_fused_fwd_noalloc_max')
     autotune.clear()
+
+
+@pytest.mark.parametrize('kind,shape,plan', [
+    ('fused', (500, 40, 3, 4), {'nsub': 4, 'splits_f': 6, 'splits_b': 3, 'nsplit': 1}),
+    ('gemm', (128, 128, 4096, 1, 1, 0), {'splits': 64, 'tile': 64})])
+def test_plans_of_other_kernels_are_not_read(kind, shape, plan, monkeypatch, tmp_path):
+    """A cache file from before the kernels' knobs changed (keys without a revision) leaves the rules
+    in place; it is kept when a new plan is stored beside it."""
+    path = tmp_path / 'tune.json'
+    old = 'gfx950|%s|%s' % (kind, ','.join(str(s) for s in shape))
+    path.write_text(json.dumps({old: plan}))
+    monkeypatch.setenv('GEEPEE_AMD_TUNE_CACHE', str(path))
+    monkeypatch.setattr(autotune, '_tag', 'gfx950')
+    autotune.clear()
+    assert autotune.lookup(kind, shape) is None
+    if kind == 'fused':
+        assert dops.fused_plan(*shape) == dops.fused_plan(*shape, tuned=False)
+    autotune.store(kind, shape, dict(plan, ms=1.0))
+    autotune.clear()
+    assert autotune.lookup(kind, shape) == dict(plan, ms=1.0)
+    assert json.loads(path.read_text())[old] == plan
+    autotune.clear()
