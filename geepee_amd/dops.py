@@ -20,7 +20,8 @@ def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=Non
     """C = alpha op(A) op(B) + beta C + gamma E (2-D or batched 3-D; 2-D operands
     broadcast; E, and outer and second as in _lib.mm, ride in the product's own epilogue).
     Picks a split-K factor when the output has few tiles and K is long (a tuned plan
-    for the shape, if the autotuner stored one, wins)."""
+    for the shape, if the autotuner stored one, wins; plans are timed without outer and second,
+    whose kernels differ, and are not used with them)."""
     if C is None:
         batch = max(t.shape[0] if t.dim() == 3 else 1 for t in (A, B))
         m = A.shape[-1] if tA else A.shape[-2]
@@ -33,7 +34,9 @@ def mm(A, B, C=None, tA=False, tB=False, alpha=1.0, beta=0.0, splits=None, E=Non
         k = A.shape[-2] if tA else A.shape[-1]
         batch = C.shape[0] if C.dim() == 3 else 1
         from . import autotune
-        hit = autotune.lookup('gemm', (m, n, k, batch, int(tA), int(tB)))
+        hit = None
+        if outer is None and second is None:
+            hit = autotune.lookup('gemm', (m, n, k, batch, int(tA), int(tB)))
         if hit:
             splits, tile = hit['splits'], hit['tile']
         else:

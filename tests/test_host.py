@@ -275,3 +275,20 @@ def test_plans_of_other_kernels_are_not_read(kind, shape, plan, monkeypatch, tmp
     assert autotune.lookup(kind, shape) == dict(plan, ms=1.0)
     assert json.loads(path.read_text())[old] == plan
     autotune.clear()
+
+
+def test_tuned_product_plan_not_used_with_a_tail(monkeypatch, tmp_path):
+    """A plan is timed without the outer product and the second output; a product with either keeps
+    the rule's split count and tile."""
+    import torch
+    monkeypatch.setenv('GEEPEE_AMD_TUNE_CACHE', str(tmp_path / 'tune.json'))
+    autotune.clear()
+    autotune.store('gemm', (20, 20, 2048, 1, 0, 0), {'splits': 3, 'tile': 64})
+    seen = []
+    monkeypatch.setattr(dops._lib, 'mm', lambda *a, **k: seen.append((k['splits'], k['tile'])))
+    A, B, C, U = torch.zeros(20, 2048), torch.zeros(2048, 20), torch.zeros(20, 20), torch.zeros(1, 20)
+    dops.mm(A, B, C)
+    dops.mm(A, B, C, outer=(U, U, 1.0))
+    dops.mm(A, B, C, second=(C, 1.0, None))
+    assert seen == [(3, 64), (4, 0), (4, 0)]
+    autotune.clear()
