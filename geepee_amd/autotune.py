@@ -124,15 +124,15 @@ def _pow2_upto(lo, hi):
 def fused_candidates(N, M):
     T = (M + 15) // 16
     ntiles = T * (T + 1) // 2
-    fwd = [{'nsub': ns, 'splits_f': s} for ns in (1, 2, 4) for s in _pow2_upto(1, min(ntiles, 64))
+    fwd = [{'nsub': ns, 'splits_f': s} for ns in (1, 2, 4) for s in _pow2_upto(1, ntiles)
            if -(-N // (16 * ns)) * s >= 64]
-    bwd = [s for s in _pow2_upto(1, min(-(-N // 16), 64)) if ntiles * 4 * s >= 64]
+    most = min(-(-N // 16), 256)
+    bwd = [s for s in _pow2_upto(1, most) if 64 <= ntiles * 4 * s <= 8192]
     # point-range counts that fill whole rounds of 256 workgroups over the tiles (the
     # adjoint kernel runs one workgroup per CU)
-    bwd = sorted(set(bwd) | {k * 256 // ntiles for k in (1, 2, 3, 4)
-                             if 1 <= k * 256 // ntiles <= min(-(-N // 16), 64)})
+    bwd = sorted(set(bwd) | {k * 256 // ntiles for k in (1, 2, 3, 4) if 1 <= k * 256 // ntiles <= most})
     # (the middle list: the adjoint's splits_b, which no longer splits anything)
-    return fwd or [{'nsub': 1, 'splits_f': min(ntiles, 64)}], [1], bwd or [min(-(-N // 16), 64)]
+    return fwd or [{'nsub': 1, 'splits_f': ntiles}], [1], bwd or [most]
 
 
 def tune_fused(N, M, Q, D, reps=5, seed=0, save=True, verbose=False):

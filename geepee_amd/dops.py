@@ -1,6 +1,8 @@
 """Device operations: typed wrappers that allocate outputs (torch, as plain device
 memory) and launch the libgpx kernels on the current stream.  Nothing here computes
 on the host or falls back to torch arithmetic."""
+import math
+
 import torch
 
 from . import _lib
@@ -427,12 +429,17 @@ def fused_plan(N, M, Q=None, D=None, tuned=True):
 
     Forward: two point tiles per workgroup (one B-hat load for both) once they leave two
     workgroups per CU, and 4 splits, whose share of B-hat one XCD's L2 keeps; 8 where fewer
-    than 400 workgroups would hold many tiles each.  (Microseconds at (N, M, Q, D), plan
-    nsub/splits: (3001, 190, 10, 12) 1/4 133, 1/8 137, 2/8 146, 2/11 180; (500, 200, 8, 16) 1/8
-    49, 1/16 50, 1/32 60; (9999, 200, 4, 4) 2/4 285, 2/3 295, 4/8 328.)
+    than 400 workgroups would hold many tiles each, and from there twice as many while that
+    makes at most 400 workgroups.  (Microseconds at (N, M, Q, D), plan nsub/splits: (3001, 190, 10,
+    12) 1/4 126, 1/8 130, 2/8 139; (9999, 200, 4, 4) 2/4 280, 2/2 332, 4/8 300; (900, 256, 10, 12) 1/8
+    85, 1/16 94; (400, 200, 4, 4) 1/8 44, 1/16 40; (100, 256, 8, 8) 1/8 55, 1/32 32, 1/64 35; (1, 256, 10,
+    2) 1/8 56, 1/64 29, 1/136 30; (1, 100, 4, 1) 1/8 21, 1/28 15.5.)
     Adjoint: one workgroup per CU takes ceil(blocks / k) 16-point blocks plus about two
-    blocks' worth of set-up and stores, in ceil(tiles k / 256) rounds; the k with the least
-    product.  ((900, 256, 10, 12): k = 2 316, 3 246, 4 256, 8 244.)"""
+    blocks' worth of set-up and stores, in ceil(tiles k / 256) rounds, and each of the k
+    ranges costs the sum of the partials about 1/16 of a block; the k with the least total
+    among the fullest of 1 to 8 rounds, at most 32 or 4 sqrt(blocks), where the sum outweighs
+    shorter ranges.  ((8000, 16, 4, 4): k = 32 84, 85 69, 128 69, 256 80; (50000, 32, 8, 16): 32 543, 85 366, 170
+    389; (8000, 48, 4, 4): 32 93, 42 87, 85 94; (900, 256, 10, 12): 2 247, 3 194, 8 197.)"""
     if tuned and Q is not None:
         from . import autotune
         hit = autotune.lookup('fused', (N, M, Q, D))
@@ -443,9 +450,18 @@ def fused_plan(N, M, Q=None, D=None, tuned=True):
     nsub = 2 if N >= 4096 else 1
     blocks = -(-N // (16 * nsub))
     splits_f = 8 if 4 * blocks < 400 and (ntiles >= 56 or blocks < 32) else 4
+    while splits_f >= 8 and splits_f < ntiles and 2 * splits_f * blocks <= 400:
+        splits_f *= 2
     splits_f = min(ntiles, splits_f)
     nb = -(-N // 16)
-    nsplit = min(range(1, min(nb, 32) + 1), key=lambda k: (-(-ntiles * k // 256) * (-(-nb // k) + 2), k))
+    most = min(nb, max(32, 4 * math.isqrt(nb)))
+    nsplit, least = 1, float('inf')
+    for rounds in range(1, 9):
+        each = -(-nb // max(1, min(most, 256 * rounds // ntiles)))  # blocks per range
+        k = -(-nb // each)
+        cost = -(-ntiles * k // 256) * (each + 2) + k / 16
+        if cost < least:
+            nsplit, least = k, cost
     return {'nsub': nsub, 'splits_f': splits_f, 'splits_b': 1, 'nsplit': nsplit}
 
 

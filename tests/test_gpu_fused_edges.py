@@ -160,3 +160,28 @@ def test_fused_adjoint_huge_inputs(N, M, Q, D):
     want = dops.fused_mm_bwd(cut(mx), cut(vx), z, ls, sf, A, Bp, cut(psi1), cut(dm), cut(dv))
     for x, y in zip(got[:4], want[:4]):
         _close(x, y.cpu())
+
+
+@pytest.mark.parametrize('N,M,Q,D', [(1, 250, 4, 2), (37, 256, 3, 5), (90, 200, 2, 17), (5, 70, 5, 1), (3000, 9, 2, 3),
+                                     (2500, 16, 3, 20), (1500, 48, 2, 4)])
+def test_fused_default_plan_extremes(N, M, Q, D):
+    """The rule's own plan where it asks for the most splits (few points, many tiles) and the most
+    point ranges (many points, few tiles)."""
+    from geepee_amd import dops
+    plan = dops.fused_plan(N, M, Q, D, tuned=False)
+    print('default plan', N, M, Q, D, plan, flush=True)
+    assert plan['splits_f'] > 8 or plan['nsplit'] >= 32
+    P = _problem(N, M, Q, D)
+    rs = np.random.RandomState(7)
+    gm, gv = (torch.as_tensor(rs.randn(N, D)) for _ in range(2))
+    ins = [p.clone().requires_grad_(True) for p in P]
+    m, v = _reference(*ins)
+    dmx, dvx, dz, _, _, _, dB = torch.autograd.grad([m, v], ins, [gm, gv])
+    mx, vx, z, ls, sf, A, B = [p.cuda() for p in P]
+    Bp = dops.sym_pairmajor(B)
+    psi1, mo, vo = dops.fused_mm_fwd(mx, vx, z, ls, sf, A, Bp, plan=plan)
+    _close(mo, m)
+    _close(vo, v)
+    out = dops.fused_mm_bwd(mx, vx, z, ls, sf, A, Bp, psi1, gm.cuda() - 2 * gv.cuda() * mo, gv.cuda(), plan=plan)
+    for got, want in zip((out[0], out[3], out[4], out[5]), (dB, dz, dmx, dvx)):
+        _close(got, want)

@@ -292,3 +292,19 @@ def test_tuned_product_plan_not_used_with_a_tail(monkeypatch, tmp_path):
     dops.mm(A, B, C, second=(C, 1.0, None))
     assert seen == [(3, 64), (4, 0), (4, 0)]
     autotune.clear()
+
+
+@pytest.mark.parametrize('N', [1, 10, 50, 100, 200, 600, 1000, 3001, 4096, 8000, 9999, 50000, 200000])
+@pytest.mark.parametrize('M', [5, 16, 32, 48, 64, 100, 128, 200, 256])
+def test_fused_plan_leaves_no_cu_idle(N, M):
+    """Workgroups are not held back below the 256 CUs while there is work to split: the forward's
+    tiles for few points, the adjoint's point ranges for few tiles (down to two blocks a range, or
+    the 4 sqrt(blocks) at which summing the ranges' partials costs more than shorter ranges give)."""
+    p = dops.fused_plan(N, M, 4, 8, tuned=False)
+    nt, nb = _ntiles(M), -(-N // 16)
+    blocks = -(-N // (16 * p['nsub']))
+    if blocks <= 25 and nt > 8:
+        assert blocks * p['splits_f'] >= 128 or p['splits_f'] == nt
+    each = -(-nb // p['nsplit'])
+    assert nt * p['nsplit'] >= 128 or each <= 3 or p['nsplit'] >= 0.8 * 4 * nb ** 0.5
+    assert p['nsplit'] <= max(32, 4 * nb ** 0.5)
