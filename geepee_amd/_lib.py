@@ -109,8 +109,6 @@ SIGNATURES = {
                                      _p, _p]),
     'gpx_fused_mm_bwd_pairs': (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p]),
     'gpx_fused_mm_bwd_tail': (_i, [_i, _i, _i, _i, _p, _p, _p, _i, _i, _p, _p, _p, _p, _p]),
-    'gpx_psi_bwd_tail': (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p,
-                              _p, _p]),
     'gpx_psi_qmax': (_i, []),
     'gpx_psi_fwd': (_i, [_i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _p]),
     'gpx_psi_bwd_gen_workspace': (_l, [_i, _i, _i]),

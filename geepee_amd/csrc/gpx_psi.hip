@@ -19,8 +19,6 @@
 // A dpsi2 that is not symmetric enters as its symmetric part.
 #include "gpx_frag.h"
 
-#include <cstdint>
-
 #define GPX_QMAX 16
 
 namespace {
@@ -456,124 +454,9 @@ int psi_bwd_launch(int blocks, int N, int M, int Q, int sym, const double *mx, c
   return GPX_OK;
 }
 
-// Final assembly for the hyper-parameter adjoints from pair sums (gpx_psi_bwd_tail).  One block per inducing point a
-// (threads over b), plus block M which finishes the scalar / per-q sums.
-//   LW:  M^2 x (Q+1)  [Lsum | W]          (sum_n L_nab [1 | d_nq])
-//   TP:  M x 2Q       [P | R']            (sum_n T_na [d mu | d])
-//   LE:  M x 2Q       [sum Lp e | sum Lp e mu]
-//   colH: Q (sum_n H), cols0: 2 (sum_n S0, sum_n Lp)
-__global__ __launch_bounds__(256) void psi_bwd_final_kernel(
-    int M, int Q, const double *__restrict__ z, const double *__restrict__ ls,
-    const double *__restrict__ sf, const double *__restrict__ LW,
-    const double *__restrict__ TP, const double *__restrict__ LE,
-    const double *__restrict__ colH, const double *__restrict__ cols0,
-    double *__restrict__ dsf2, double *__restrict__ dell, double *__restrict__ dZ) {
-  const int a = blockIdx.x, b = threadIdx.x, lane = b & 63, w = b >> 6;
-  if (a == M) {
-    if (b == 0) {
-      const double sf2 = exp(2.0 * sf[0]);
-      dsf2[0] = (cols0[1] + 2.0 * cols0[0]) / sf2;
-    }
-    return;
-  }
-  // per-a sums over b: R_a, (Lsum z)_aq, sum_b W_abq z_bq
-  double c[2 * GPX_QMAX + 1];
-#pragma unroll
-  for (int i = 0; i < 2 * GPX_QMAX + 1; ++i) c[i] = 0.0;
-  for (int bb = b; bb < M; bb += 256) {
-    const double *row = LW + ((long)a * M + bb) * (Q + 1);
-    const double ls_ab = row[0];
-    c[0] += ls_ab;
-#pragma unroll
-    for (int q = 0; q < GPX_QMAX; ++q)
-      if (q < Q) {
-        const double zb = z[bb * Q + q];
-        c[1 + q] += ls_ab * zb;
-        c[1 + GPX_QMAX + q] += row[1 + q] * zb;
-      }
-  }
-  __shared__ double tot[2 * GPX_QMAX + 1];
-  __shared__ double red2[4][2 * GPX_QMAX + 1];
-#pragma unroll
-  for (int i = 0; i < 2 * GPX_QMAX + 1; ++i) {
-    const double s = gpx_wave_sum(c[i]);
-    if (lane == 0) red2[w][i] = s;
-  }
-  __syncthreads();
-  for (int i = b; i < 2 * GPX_QMAX + 1; i += 256)
-    tot[i] = red2[0][i] + red2[1][i] + red2[2][i] + red2[3][i];
-  __syncthreads();
-  if (b < Q) {
-    const int q = b;
-    const double l = exp(2.0 * ls[q]);
-    const double zaq = z[a * Q + q];
-    const double Ra = tot[0], LZ = tot[1 + q], WZ = tot[1 + GPX_QMAX + q];
-    const double P = TP[a * 2 * Q + q], Rp = TP[a * 2 * Q + Q + q];
-    const double g2 = -(zaq * Ra - LZ) / l + 2.0 * P - zaq * Rp - WZ;
-    const double g1 = -(zaq * LE[a * 2 * Q + q] - LE[a * 2 * Q + Q + q]);
-    dZ[a * Q + q] = g1 + g2;
-  }
-}
-
-// out[j] = sum_i P[i*cols + j] over `rows`: one block per column, fixed-order reduction.
-__global__ __launch_bounds__(256) void colsum_kernel(int rows, int cols, const double *__restrict__ P,
-                                                     double *__restrict__ out) {
-  __shared__ double red[16];
-  const int j = blockIdx.x;
-  double s = 0.0;
-#pragma unroll 8
-  for (long i = threadIdx.x; i < rows; i += 256) s += P[i * cols + j];
-  s = gpx_block_sum(s, red);
-  if (threadIdx.x == 0) out[j] = s;
-}
-
 }  // namespace
 
-extern "C" int gpx_gemm_batched(int transA, int transB, int m, int n, int k, double alpha,
-                                const double *A, int lda, long strideA, const double *B, int ldb,
-                                long strideB, double beta, double *C, int ldc, long strideC,
-                                int batch, int splits, double *work, int tile, void *stream);
-
 extern "C" {
-
-// Tail of a psi adjoint whose caller holds its sums: from the per-point
-// outputs T, Lp (N x M), H (N x Q), s0 (N x 2), Dn, Pn, En and the pair sums LW
-// ((M*M) x (Q+1)) finish dsf2, dell (w.r.t. ell) and dZ.  TP, LE (M x 2Q) and cols0 (2)
-// are workspace.
-// Split-K factor of the two N-long reductions TP = T^T Pn, LE = Lp^T En (M x 2Q outputs,
-// few tiles) and the doubles of partials they need.
-static int tail_splits(int N) {
-  int s = N / 128;
-  return s < 1 ? 1 : (s > 64 ? 64 : s);
-}
-
-long gpx_psi_tail_workspace(int N, int M, int Q) { return 2L * tail_splits(N) * M * 2 * Q; }
-
-int gpx_psi_bwd_tail(int N, int M, int Q, const double *z, const double *ls, const double *sf,
-                     const double *T, const double *Lp, const double *H, const double *s0,
-                     const double *Dn, const double *Pn, const double *En, const double *LW,
-                     double *TP, double *LE, double *cols0, double *dsf2, double *dell, double *dZ,
-                     double *kwork, void *stream) {
-  if (N < 1 || M < 1 || M > 256 || Q < 1 || Q > GPX_QMAX || !kwork) return GPX_EINVAL;
-  hipStream_t st = (hipStream_t)stream;
-  const int ks = tail_splits(N);
-  // TP = T^T Pn and LE = Lp^T En as one batch of two split-K products: member 1's operands
-  // are addressed from member 0's at the element distances between the buffers
-  const long sA = ((intptr_t)Lp - (intptr_t)T) / (long)sizeof(double);
-  const long sB = ((intptr_t)En - (intptr_t)Pn) / (long)sizeof(double);
-  const long sC = ((intptr_t)LE - (intptr_t)TP) / (long)sizeof(double);
-  int rc = gpx_gemm_batched(1, 0, M, 2 * Q, N, 1.0, T, M, sA, Pn, 2 * Q, sB, 0.0, TP, 2 * Q, sC, 2, ks, kwork, 0,
-                            stream);
-  if (rc) return rc;
-  hipLaunchKernelGGL(colsum_kernel, dim3(Q), dim3(256), 0, st, N, Q, H, dell);
-  GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(colsum_kernel, dim3(2), dim3(256), 0, st, N, 2, s0, cols0);
-  GPX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(psi_bwd_final_kernel, dim3(M + 1), dim3(256), 0, st, M, Q, z, ls, sf, LW, TP, LE,
-                     (const double *)nullptr, (const double *)cols0, dsf2, dell, dZ);
-  GPX_CHECK_LAUNCH();
-  return GPX_OK;
-}
 
 int gpx_psi_qmax(void) { return GPX_QMAX; }
 

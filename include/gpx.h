@@ -473,14 +473,6 @@ int gpx_fused_mm_bwd_tail(int N, int M, int Q, int D, const double *z, const dou
                           int splits, int nsplit, double *dsf2, double *dell, double *dZ, double *work,
                           void *stream);
 
-/* Final stage of a psi adjoint whose caller holds its sums (pair sums LW and per-point statistics in, dsf2,
- * dell, dZ out); the tail of compute_psi_derivatives (geepee/kernels.py:430-442, 371-376). */
-int gpx_psi_bwd_tail(int N, int M, int Q, const double *z, const double *ls, const double *sf,
-                     const double *T, const double *Lp, const double *H, const double *s0,
-                     const double *Dn, const double *Pn, const double *En, const double *LW,
-                     double *TP, double *LE, double *cols0, double *dsf2, double *dell, double *dZ,
-                     void *stream);
-
 /* ---- serving ------------------------------------------------------------------ */
 
 /* One launch of predictive mean / variance for many (request, model) work items of at

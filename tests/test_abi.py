@@ -74,3 +74,26 @@ def test_noalloc_rejects_oversize_before_any_launch():
     assert L.gpx_fused_mm_fwd_noalloc(N, M, Q, D, 1, 1, 1, 1, 1, 1, 1, splits, 1, 1, 1, 1, None) == -3
     # invalid arguments are still GPX_EINVAL
     assert L.gpx_fused_mm_fwd_noalloc(N, M, 99, D, 1, 1, 1, 1, 1, 1, 1, splits, 1, 1, 1, 1, None) == -1
+
+
+def _arg_counts(text):
+    """{entry point: number of arguments} of the prototypes or definitions in C source."""
+    text = re.sub(r'/\*.*?\*/|//[^\n]*', '', text, flags=re.S)
+    out = {}
+    for name, args in re.findall(r'^\s*(?:extern "C"\s+)?(?:long|int)\s+(gpx_\w+)\s*\(([^)]*)\)', text, flags=re.M):
+        args = args.strip()
+        out.setdefault(name, set()).add(0 if args in ('', 'void') else args.count(',') + 1)
+    return out
+
+
+def test_header_definitions_and_bindings_agree():
+    """The header, the sources and the ctypes table give every entry point the same arguments."""
+    import glob
+    head = _arg_counts(open(os.path.join(ROOT, 'include', 'gpx.h')).read())
+    src = {}
+    for f in glob.glob(os.path.join(ROOT, 'geepee_amd', 'csrc', '*.hip')):
+        for name, n in _arg_counts(open(f).read()).items():
+            src.setdefault(name, set()).update(n)
+    for name in _declared():
+        counts = head[name] | src[name] | {len(_lib.SIGNATURES[name][1])}
+        assert len(counts) == 1, (name, head[name], src[name], len(_lib.SIGNATURES[name][1]))
