@@ -530,11 +530,19 @@ int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double al
   // against 32 x 32: n = 256 172 : 228, 200 125 : 133, 128 (2504 tiles) 63 : 65; 5000 x 100 x 100, 4
   // (632 tiles) 24 : 18).  16 x 16 per workgroup, its waves sharing k, where those are at most three
   // per CU (against 32 x 32: 128^3 4.4 : 5.5, 200^3, 4 (676 tiles) 5.8 : 6.0, 128^3, 32 (2048) 13 : 7.8).
-  // Else 32 x 32, a tile per wave if that makes a wave per SIMD (4001 x 256 x 256 (1008) 17.4 : 18.3;
-  // 128^3, 32 (512) 10.5 : 8.8) or if k leaves four waves nothing to share.
+  // Else 32 x 32: a tile per wave takes whole rounds of 1024 (a wave per SIMD), four waves sharing
+  // a tile's k take rounds of 256 at a quarter of the time and 3% more, and four more waves' loads in
+  // flight.  So a tile per wave where its rounds are at least 7/8 full (us against shared k, 256 x 256
+  // x 256 or x 256 x 256 (tiles): (768) 16.4 : 14.1, (896) 16.7 : 17.3, (1008) 16.9 : 17.4, (1256) 27.8 : 20.4,
+  // (1504) 28.3 : 23.9, (2000) 29.3 : 30.0, (4000) 51.8 : 54.2; n = k = 100: (1252) 13.6 : 11.3, (1920) 14.1 :
+  // 15.2), 3/4 where k is short (64^3 (800) 8.6 : 9.1, (1600) 13.1 : 13.9; 50^3 (1200) 10.2 : 9.3, (1600) 10.6 : 11.5),
+  // and k is not so long that the loads decide (200 x 1000 (882) 48 : 41, (2625) 113 : 100).  Up to
+  // k = 16 most of four waves have nothing to share, and only few tiles gain from them (k = 8 (658) 5.9 :
+  // 6.0, (1256) 7.0 : 7.8; k = 12 (504) 6.1 : 5.7, (752) 6.4 : 6.4; k = 32 (512) 7.0 : 6.0, (1256) 9.4 : 8.6).
+  const bool full = t2 >= 4096 || 8 * t2 > (k <= 64 ? 6 : 7) * 1024 * (long)gpx_cdiv(t2, 1024);
   if (!tail && (tile == 64 || (tile != 32 && t4 >= 2048 && k >= 64))) rc = GEMM_DIRECT(4, 1);
   else if (tile != 32 && t1 <= 768) rc = GEMM_DIRECT(1, 4);
-  else if (t2 >= 1024 || k <= 32) rc = GEMM_DIRECT(2, 1);
+  else if (k <= 16 ? t2 > 576 : k <= 256 && full) rc = GEMM_DIRECT(2, 1);
   else rc = GEMM_DIRECT(2, 4);
 #undef GEMM_DIRECT
   if (rc != GPX_OK) return rc;

@@ -53,3 +53,16 @@ def test_gram_edges(N, D, M):
     assert _nrel(dops.gram(dw, dX, E=dE, gamma=-0.5).cpu().numpy(), ref - 0.5 * E) < 1e-12
     assert _nrel(dops.gram(dw, dX, E=dE[0].contiguous(), gamma=1.0).cpu().numpy(), ref + E[:1]) < 1e-12
     assert not dops.gram(dw[:0], dX[:0]).any()
+
+
+# (tiles of 32 x 32, k) on both sides of each line of the rule that gives a tile to a wave or to four
+@pytest.mark.parametrize('k', [16, 17, 64, 65, 256, 257])
+@pytest.mark.parametrize('tiles', [576, 577, 768, 769, 896, 897, 1024, 1025, 1536, 1537, 1792, 1793, 4095, 4096])
+def test_gemm_wave_rule(tiles, k):
+    from geepee_amd import _lib as L
+    rs = np.random.RandomState(tiles + k)
+    print('gemm rule', tiles, k, flush=True)
+    A, B = rs.randn(32 * tiles - 5, k), rs.randn(k, 27)
+    C = torch.full((A.shape[0], 27), float('nan'), dtype=torch.float64, device='cuda')
+    L.mm(torch.as_tensor(A, device='cuda'), torch.as_tensor(B, device='cuda'), C, tile=32)
+    assert _nrel(C.cpu().numpy(), A @ B) < 1e-12
