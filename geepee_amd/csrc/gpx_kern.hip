@@ -27,21 +27,23 @@ __global__ void se_any_kernel(int N, int M, int Q, const double *__restrict__ x,
   K[e] = k;
 }
 
-// Q <= QC: a block takes SE_ROWS rows by 64 columns, each wave every fourth row.  x, 1/l and
+// Q <= QC: a block takes ROWS rows by 64 columns, each wave every fourth row.  x, 1/l and
 // sf2 are formed once per block, a thread's z row stays in registers.  Bound by its exps and
 // its writes (N = 20000, M = 200, Q = 8: 58 -> 22 us; with the lengthscales' exps and divisions
-// per entry it was bound by those).
-constexpr int SE_ROWS = 16;
-template <int QC>
+// per entry it was bound by those).  16 rows; 4 where 16 would make at most 128 blocks: such a launch
+// is as long as one thread's entries (us, 4 rows : 16: 50 x 50, Q = 2 3.2 : 3.8; 256 x 256, Q = 10 3.4 :
+// 4.5; 1000 x 100, Q = 10 (126 blocks) 3.7 : 4.5; 3000 x 64, Q = 16 (188) 7.7 : 5.6).
+constexpr int SE_ROWS = 16, SE_ROWS_FEW = 4, SE_FEW = 128;
+template <int QC, int ROWS>
 __global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const double *__restrict__ x, int ldx,
                                                  const double *__restrict__ z, const double *__restrict__ ls,
                                                  const double *__restrict__ sf, double jitter,
                                                  double *__restrict__ K) {
-  __shared__ double xs[SE_ROWS][QC], il[QC], s2;
-  const int tid = threadIdx.x, n0 = blockIdx.x * SE_ROWS, m = blockIdx.y * 64 + (tid & 63);
+  __shared__ double xs[ROWS][QC], il[QC], s2;
+  const int tid = threadIdx.x, n0 = blockIdx.x * ROWS, m = blockIdx.y * 64 + (tid & 63);
   if (tid < QC) il[tid] = tid < Q ? exp(-2.0 * ls[tid]) : 0.0;
   if (tid == 255) s2 = exp(2.0 * sf[0]);
-  for (int e = tid; e < SE_ROWS * QC; e += 256) {
+  for (int e = tid; e < ROWS * QC; e += 256) {
     const int i = e / QC, q = e % QC;
     xs[i][q] = q < Q ? x[(long)min(n0 + i, N - 1) * ldx + q] : 0.0;
   }
@@ -50,7 +52,7 @@ __global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const doub
   for (int q = 0; q < QC; ++q) zr[q] = q < Q ? z[min(m, M - 1) * Q + q] : 0.0;
   __syncthreads();
 #pragma unroll
-  for (int u = 0; u < SE_ROWS / 4; ++u) {
+  for (int u = 0; u < ROWS / 4; ++u) {
     const int i = (tid >> 6) + 4 * u, n = n0 + i;
     double r2 = 0.0;
 #pragma unroll
@@ -1077,13 +1079,17 @@ int gpx_se_kernel(int N, int M, int Q, const double *x, int ldx, const double *z
     hipLaunchKernelGGL(se_any_kernel, dim3(gpx_cdiv((long)N * M, 256)), dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf,
                        jitter, K);
   } else {
-    const dim3 grid(gpx_cdiv(N, SE_ROWS), gpx_cdiv(M, 64));
-    if (Q <= 4)
-      hipLaunchKernelGGL(se_kernel<4>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
-    else if (Q <= 8)
-      hipLaunchKernelGGL(se_kernel<8>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
-    else
-      hipLaunchKernelGGL(se_kernel<16>, grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+    const bool few = (long)gpx_cdiv(N, SE_ROWS) * gpx_cdiv(M, 64) <= SE_FEW;
+    const dim3 grid(gpx_cdiv(N, few ? SE_ROWS_FEW : SE_ROWS), gpx_cdiv(M, 64));
+#define GPX_SE(QV)                                                                                              \
+  if (few)                                                                                                      \
+    hipLaunchKernelGGL((se_kernel<QV, SE_ROWS_FEW>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K); \
+  else                                                                                                          \
+    hipLaunchKernelGGL((se_kernel<QV, SE_ROWS>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+    if (Q <= 4) { GPX_SE(4) }
+    else if (Q <= 8) { GPX_SE(8) }
+    else { GPX_SE(16) }
+#undef GPX_SE
   }
   GPX_CHECK_LAUNCH();
   return GPX_OK;

@@ -45,3 +45,17 @@ def test_se_and_adjoint(N, M, Q):
     assert _nrel(dell.cpu().numpy(), wl) < 1e-10
     assert _nrel(dz.cpu().numpy(), -(z * cs[:, None] - L.T.dot(x)) * il) < 1e-11
     assert _nrel(dx.cpu().numpy(), (L.dot(z) - x * L.sum(1)[:, None]) * il) < 1e-11
+
+
+@pytest.mark.parametrize('Q', [3, 8, 16])
+@pytest.mark.parametrize('N,M', [(2048, 64), (2049, 64), (1024, 65), (1025, 65)])
+def test_se_rows_per_block(N, M, Q):
+    """Entries are the same bits from blocks of 4 and of 16 rows (on both sides of the rule)."""
+    from geepee_amd import dops
+    print('se rows', N, M, Q, flush=True)
+    rs = np.random.RandomState(N + Q)
+    x, z, ls, sf = [torch.as_tensor(a, device='cuda') for a in (rs.randn(N, Q), rs.randn(M, Q), 0.2 * rs.randn(Q),
+                                                                 np.array([0.3]))]
+    K = dops.se(x, z, ls, sf)
+    for r0, r1 in ((0, 1), (3, 40), (N - 17, N)):
+        assert torch.equal(K[r0:r1], dops.se(x[r0:r1].contiguous(), z, ls, sf))
