@@ -159,36 +159,58 @@ __global__ __launch_bounds__(256) void kfu_bwd_partial(int N, int M, int Q, int 
   }
 }
 
-// dx_nq = sum_m L_nm (z_mq - x_nq) / l_q, one wave per row, its lanes over m.
-__global__ __launch_bounds__(256) void kfu_dx_kernel(int N, int M, int Q, const double *__restrict__ dK,
-                                                     const double *__restrict__ K, const double *__restrict__ x,
-                                                     const double *__restrict__ z, const double *__restrict__ ls,
-                                                     double *__restrict__ dx) {
-  const int lane = threadIdx.x & 63;
-  const long n = blockIdx.x * 4L + (threadIdx.x >> 6);
-  if (n >= N) return;  // whole wave, no barriers
-  double L[4];
+// dx_nq = sum_m L_nm (z_mq - x_nq) / l_q of row n by one wave: lane (g, c) takes q = g + 4 k (k < KR) and
+// m = c, c + 16, ..., so the row's Q sums are KR sums over 16 lanes.  z: LDS, rows of zld.
+template <int KR>
+__device__ __forceinline__ void kfu_dx_row(long n, int lane, int M, int Q, const double *dK, const double *K,
+                                           const double *x, const double *z, int zld, const double *ls, double *dx) {
+  const int g = lane >> 4, c = lane & 15;
+  double xv[KR], s[KR];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int m = min(lane + 64 * j, M - 1);
-    L[j] = dK[n * M + m] * K[n * M + m] * (lane + 64 * j < M ? 1.0 : 0.0);
+  for (int k = 0; k < KR; ++k) {
+    xv[k] = x[n * Q + min(g + 4 * k, Q - 1)];
+    s[k] = 0.0;
   }
-  for (int q = 0; q < Q; ++q) {
-    const double xv = x[n * Q + q];
-    double s = 0.0;
+#pragma unroll 2
+  for (int m0 = 0; m0 < M; m0 += 16) {
+    const int mc = min(m0 + c, M - 1);
+    const double L = dK[n * M + mc] * K[n * M + mc] * (m0 + c < M ? 1.0 : 0.0);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) s = fma(L[j], z[min(lane + 64 * j, M - 1) * Q + q] - xv, s);
-    s = gpx_wave_sum(s);
-    if (lane == 0) dx[n * Q + q] = s / exp(2.0 * ls[q]);
+    for (int k = 0; k < KR; ++k) s[k] = fma(L, z[mc * zld + min(g + 4 * k, Q - 1)] - xv[k], s[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+    const int q = g + 4 * k;
+    const double t = gpx_row_sum(s[k]);
+    if (c == 0 && q < Q) dx[n * Q + q] = t / exp(2.0 * ls[q]);
   }
 }
 
 // Pass 2: red[w][m] = sum over the blocks of part[b][w][m]: 64 columns by 16 groups of blocks
-// (loads eight at a time), the groups added in order.
-__global__ __launch_bounds__(1024) void kfu_bwd_final(int nblk, int M, int W, const double *__restrict__ part,
-                                                      double *__restrict__ red) {
+// (loads eight at a time), the groups added in order.  KR > 0: the workgroups past the first `sums`
+// form dx, a wave to a row, with z in LDS (M rows of Q | 1).  Whole adjoint with dx, us: N = 1000, M = 100,
+// Q = 10 16.4 (18.3 with dx in the first pass, 19.5 in a launch of its own with a wave sum over m for
+// each q), 20000, 200, 16 88 (135, 195; 97 with two rows a wave).
+template <int KR>
+__global__ __launch_bounds__(1024) void kfu_bwd_final(int nblk, int M, int W, int sums, const double *__restrict__ part,
+                                                      double *__restrict__ red, int N, int Q,
+                                                      const double *__restrict__ dK, const double *__restrict__ K,
+                                                      const double *__restrict__ x, const double *__restrict__ z,
+                                                      const double *__restrict__ ls, double *__restrict__ dx) {
   __shared__ double sm[16][64];
-  const int c = threadIdx.x & 63, g = threadIdx.x >> 6, m = blockIdx.x * 64 + c, w = blockIdx.y;
+  extern __shared__ double zs[];
+  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+  if constexpr (KR > 0) {
+    if ((int)blockIdx.x >= sums) {  // uniform over the workgroup
+      const int zld = Q | 1;
+      const long n = ((long)blockIdx.x - sums) * 16 + g;
+      for (int e = threadIdx.x; e < M * Q; e += 1024) zs[e / Q * zld + e % Q] = z[e];
+      __syncthreads();
+      if (n < N) kfu_dx_row<KR>(n, c, M, Q, dK, K, x, zs, zld, ls, dx);
+      return;
+    }
+  }
+  const int cb = (M + 63) >> 6, m = (int)blockIdx.x % cb * 64 + c, w = (int)blockIdx.x / cb;
   const double *P = part + (long)w * M + min(m, M - 1);
   const long bs = (long)W * M;
   double s = 0.0;
@@ -1119,12 +1141,17 @@ static int kfu_bwd_launch(int N, int M, int Q, const double *dK, const KfuReg *r
   else { GPX_KFU(16) }
 #undef GPX_KFU
   GPX_CHECK_LAUNCH();
-  if (dx) {
-    hipLaunchKernelGGL(kfu_dx_kernel, dim3(gpx_cdiv(N, 4)), dim3(256), 0, st, N, M, Q, dK, K, x, z, ls, dx);
-    GPX_CHECK_LAUNCH();
-  }
-  hipLaunchKernelGGL(kfu_bwd_final, dim3(gpx_cdiv(M, 64), rows), dim3(1024), 0, st, nblk, M, rows, (const double *)work,
-                     red);
+  const int sums = (int)gpx_cdiv(M, 64) * rows;
+#define GPX_KFU_FINAL(KR)                                                                                         \
+  hipLaunchKernelGGL(kfu_bwd_final<KR>, dim3(sums + (KR ? gpx_cdiv(N, 16) : 0)), dim3(1024),                          \
+                     KR ? M * (Q | 1) * sizeof(double) : 0, st, nblk, M, rows, sums, (const double *)work, red, N, Q, \
+                     dK, K, x, z, ls, dx)
+  if (!dx) GPX_KFU_FINAL(0);
+  else if (Q <= 4) GPX_KFU_FINAL(1);
+  else if (Q <= 8) GPX_KFU_FINAL(2);
+  else if (Q <= 12) GPX_KFU_FINAL(3);
+  else GPX_KFU_FINAL(4);
+#undef GPX_KFU_FINAL
   GPX_CHECK_LAUNCH();
   hipLaunchKernelGGL(kfu_bwd_scalars, dim3(Q + 1), dim3(64), 0, st, M, Q, (const double *)red,
                      reg ? (const double *)red + (long)W * M : nullptr, z, ls, sf, dsf2, dell, dZ);
