@@ -748,7 +748,7 @@ __global__ __launch_bounds__(256, 3) void fused_rows_finish(
   }
   const int tn = (MT - w + 3) >> 2;  // this wave's column tiles (may be 0)
   const int tq = min(tid, Q - 1);
-  const double ell = exp(ls[tq]), lq = exp(2.0 * ls[tq]), ilq = 1.0 / lq;
+  const double ell = exp(ls[tq]), lq = exp(2.0 * ls[tq]);
   int par = 0;
   for (int n = blockIdx.x; n < N; n += gridDim.x, par ^= 1) {
     // every load at a clamped (valid) index, issued together; S <= 16, SV <= 136
@@ -836,8 +836,8 @@ __global__ __launch_bounds__(256, 3) void fused_rows_finish(
       const double quad = m * m * s0 - 2.0 * m * s1 + 0.5 * (tz2 + vs);
       dmx[(long)n * Q + q] = -2.0 * d * (m * s0 - s1) + e * b1;
       dvx[(long)n * Q + q] = 2.0 * d * d * quad - d * s0 + 0.5 * e * (e * c1 - a1);
-      hsum += 2.0 * ell * (v * ilq * d * s0 + d * d * quad + (tz2 - vs) * (0.5 * ilq * ilq));
-      hsum += e * ell * (e * c1 + v * ilq * a1);
+      hsum += 2.0 * ell * (v / lq * d * s0 + d * d * quad + (tz2 - vs) / (2.0 * lq * lq));
+      hsum += e * ell * (e * c1 + v / lq * a1);
       s0sum += s0;
       a1sum += a1;
     }
@@ -875,11 +875,18 @@ __global__ __launch_bounds__(256) void fused_tail_kernel(int M, int Q, int block
   }
   // columns of the partials: dZ's row a, or [H | S0 | A1]
   const int cols = a < M ? Q : Q + 2;
-  double t = 0.0, x = 0.0;
+  // (four running sums a thread: over up to 1024 blocks a single one let dell's error grow)
+  double t4[4] = {0.0, 0.0, 0.0, 0.0}, x = 0.0;
   if (q < cols) {
-#pragma unroll 16
-    for (int k = h; k < blocks; k += 16) t += part[(long)k * width + a * Q + q];
+#pragma unroll 4
+    for (int k = h; k < blocks; k += 64)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double p = part[(long)min(k + 16 * u, blocks - 1) * width + a * Q + q];
+        t4[u] += k + 16 * u < blocks ? p : 0.0;
+      }
   }
+  const double t = (t4[0] + t4[1]) + (t4[2] + t4[3]);
   if (a == M && q == 0 && Q + 1 == 16) {  // the 17th column, A1 at Q = 15
     for (int k = h; k < blocks; k += 16) x += part[(long)k * width + M * Q + 16];
   }
