@@ -637,8 +637,9 @@ __global__ __launch_bounds__(1024) void gauss_tilted_kernel(int B, int D, const 
   const long n = (long)B * D;
   const double sa = sn2 / alpha;
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
+    // two divisions: r (1/vt) would be off by half an ulp more than r / vt
     const double vt = v[e] + sa, iv = 1.0 / vt;
-    const double r = y[e] - m[e], gm = r * iv;
+    const double r = y[e] - m[e], gm = r / vt;
     lz += -0.5 * (log(two_pi * vt) + r * gm);
     const double gv = 0.5 * (gm * gm - iv);
     sdv += gv;

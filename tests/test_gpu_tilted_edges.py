@@ -30,3 +30,13 @@ def test_gauss_tilted(B, D, alpha):
     assert abs(scal[0] - (terms.sum() + const)) < 1e-12 * (np.abs(terms).sum() + abs(const))
     dsn = (gv.sum() * 2 * sn2 / alpha + B * D * (1 - alpha)) * scale
     assert abs(scal[1] - dsn) < 1e-12 * (np.abs(gv).sum() * 2 * sn2 / alpha + B * D) * scale
+
+
+def test_gauss_tilted_mean_gradient_is_one_division():
+    """With unit noise and alpha = 1 the mean's gradient is (y - m) / (v + 1), correctly rounded."""
+    from geepee_amd import dops
+    rs = np.random.RandomState(3)
+    m, v, y = rs.randn(3000, 3), rs.rand(3000, 3) + 0.01, rs.randn(3000, 3)
+    t = [torch.as_tensor(a, device='cuda') for a in (m, v, y, np.zeros(1))]
+    dm = dops.gauss_tilted(*t, 1.0, 1.0)[0].cpu().numpy()
+    assert np.array_equal(dm, (y - m) / (v + 1.0))
