@@ -16,6 +16,16 @@
 
 static inline unsigned gpx_cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
 
+// Threads per block for n independent elements over at most 64 blocks (whose partial sums have
+// fixed room): 256, and past 64 x 256 elements as many as give every thread one element, or the
+// same number of them.  The kernels are bound by the latency of an element's logs and divisions
+// (us with 256 : 1024 : these threads, launch and finish included: SSM x gradients 32000 elements 8.2 : 9.2 :
+// 7.4, 40000 9.8 : 9.1 : 8.1, 75052 12.7 : 13.2 : 11.4, 132000 18.6 : 16.6 : 14.4; LVM 75052 11.7 : 13.7 : 11.6).
+static inline unsigned gpx_even_threads(long n) {
+  const long per = gpx_cdiv(n, 64);
+  return per <= 256 ? 256 : gpx_cdiv(gpx_cdiv(per, gpx_cdiv(per, 1024)), 64) * 64;
+}
+
 // v + v[lane ^ O] for O = 32 or 16, with gfx950's cross-row lane swaps on the vector ALU:
 // permlane32_swap(x, x) gives x[l % 32] and x[l % 32 + 32], permlane16_swap(x, x) gives
 // x[l & ~16] and x[l | 16], so their sum is the xor-shuffle step's sum (the two operands

@@ -1399,7 +1399,7 @@ int gpx_gauss_tilted(int B, int D, const double *m, const double *v, const doubl
   if (B < 1 || D < 1 || !(alpha > 0) || !m || !v || !y || !sn || !dm || !dv || !scal) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   long n = (long)B * D;
-  const int threads = n > 64 * 256 ? 1024 : 256, nblk = (int)std::min<long>(64, gpx_cdiv(n, threads));
+  const int threads = gpx_even_threads(n), nblk = (int)std::min<long>(64, gpx_cdiv(n, threads));
   hipLaunchKernelGGL(gauss_tilted_kernel, dim3(nblk), dim3(threads), 0, st, B, D, m, v, y, sn, alpha, scale, dm, dv,
                      dmall, scal + 2);
   GPX_CHECK_LAUNCH();
@@ -1418,7 +1418,7 @@ int gpx_transition_tilted(int B, int D, const double *mp, const double *vp, cons
     return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
   long n = (long)B * D;
-  const int nt = n > 64 * 256 ? 1024 : 256;
+  const int nt = gpx_even_threads(n);
   int nblk = (int)gpx_cdiv(n, nt);
   if (nblk > 64) nblk = 64;
   hipLaunchKernelGGL(transition_kernel, dim3(nblk), dim3(nt), 0, st, B, D, mp, vp, mt, vt, sn, alpha, scale, dmall,

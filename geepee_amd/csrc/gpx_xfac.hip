@@ -5,10 +5,6 @@
 
 // Workgroups of the x-gradient kernels; scal holds 2 + 2 * GPX_XF_BLOCKS doubles.
 #define GPX_XF_BLOCKS 64
-// Their threads: bound by the latency of an element's logs and divisions, so as few elements per
-// thread as those workgroups allow (40000 elements of ssm_grad_kernel 13.4 -> 8.9 us; 32768
-// of lvm_grad_kernel 7.5 either way).
-static unsigned xf_threads(long n) { return n > GPX_XF_BLOCKS * 256L ? 1024 : 256; }
 
 namespace {
 
@@ -324,7 +320,7 @@ int gpx_lvm_x_grads(int N, int B, int Q, const long *idx, const double *x1, cons
   if (N < 1 || B < 1 || Q < 1 || !x1 || !x2 || !gmx || !gvx || !g1 || !g2 || !scal) return GPX_EINVAL;
   const double sc_cav = -(double)N / B / alpha;
   const double sc_post = -(double)N / B * (1.0 - 1.0 / alpha);
-  const unsigned nt = xf_threads((long)B * Q);
+  const unsigned nt = gpx_even_threads((long)B * Q);
   unsigned nblk = gpx_cdiv((long)B * Q, nt);
   if (nblk > GPX_XF_BLOCKS) nblk = GPX_XF_BLOCKS;
   hipLaunchKernelGGL(lvm_grad_kernel, dim3(nblk), dim3(nt), 0, (hipStream_t)stream, N, B, Q, idx, x1, x2, gmx,
@@ -354,7 +350,7 @@ int gpx_ssm_x_grads(int N, int Q, int s, int e, const double *xf1, const double 
   if (N < 2 || Q < 1 || s < 0 || e > N || e - s < 2 || !xf1 || !x2 || !dup || !vup || !dmt || !dvt ||
       !dmn || !dvn || !g1 || !g2 || !scal || ldu < Q || ldn < Q)
     return GPX_EINVAL;
-  const unsigned nt = xf_threads((long)N * Q);
+  const unsigned nt = gpx_even_threads((long)N * Q);
   unsigned nblk = gpx_cdiv((long)N * Q, nt);
   if (nblk > GPX_XF_BLOCKS) nblk = GPX_XF_BLOCKS;
   hipLaunchKernelGGL(ssm_grad_kernel, dim3(nblk), dim3(nt), 0, (hipStream_t)stream, N, Q, s, e, xf1, x2, alpha,

@@ -40,3 +40,34 @@ def test_gauss_tilted_mean_gradient_is_one_division():
     t = [torch.as_tensor(a, device='cuda') for a in (m, v, y, np.zeros(1))]
     dm = dops.gauss_tilted(*t, 1.0, 1.0)[0].cpu().numpy()
     assert np.array_equal(dm, (y - m) / (v + 1.0))
+
+
+@pytest.mark.parametrize('n', [16384, 16385, 20001, 65536, 65537, 75052, 131072, 131073])
+def test_x_gradients_over_thread_counts(n):
+    """Each latent element's gradient is the same bits whatever the launch shape (a slice of the rows
+    gives the slice's), and the sum of log-normalisers is that of the slices; the same for the
+    transition terms."""
+    from geepee_amd import dops, xfactors as X
+    print('x gradients', n, flush=True)
+    rs = np.random.RandomState(n)
+    dev = lambda *s: torch.as_tensor(rs.randn(*s), device='cuda')
+    x1, x2, gm, gv = dev(n, 1), 0.3 * dev(n, 1), dev(n, 1), dev(n, 1)
+    args = (0.6, 0.2, 1.5)
+
+    def lvm(a, b):
+        xs = X.lvm_x_state(x1[a:b].contiguous(), x2[a:b].contiguous(), None, *args, False)
+        g1, g2, s = X.lvm_x_grads(xs, gm[a:b], gv[a:b], b - a, b - a, *args, 1, False)
+        return g1, g2, float(s[0])
+
+    cuts = list(range(0, n, 9001)) + [n]
+    whole, parts = lvm(0, n), [lvm(a, b) for a, b in zip(cuts, cuts[1:])]
+    for k in (0, 1):
+        assert torch.equal(whole[k], torch.cat([p[k] for p in parts]))
+    assert abs(whole[2] - sum(p[2] for p in parts)) < 1e-12 * n
+    t = [dev(n, 1), dev(n, 1).abs() + 0.1, dev(n, 1), dev(n, 1).abs() + 0.1]
+    sn = torch.zeros(1, dtype=torch.float64, device='cuda')
+    full = dops.transition(*t, sn, 0.6, 1.0)
+    part = [dops.transition(*[u[a:b].contiguous() for u in t], sn, 0.6, 1.0) for a, b in zip(cuts, cuts[1:])]
+    for k in range(4):
+        assert torch.equal(full[k], torch.cat([p[k] for p in part]))
+    assert abs(float(full[4][0]) - sum(float(p[4][0]) for p in part)) < 1e-12 * n
