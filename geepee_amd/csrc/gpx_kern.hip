@@ -341,98 +341,34 @@ __global__ __launch_bounds__(64) void kuu_tail_kernel(int M, int Q, const double
   else dls[j - 1] = dell[j - 1] * exp(ls[j - 1]) + 2.0 * s;
 }
 
-// mu_b = s_b S_b t_b and P_b = S_b + mu_b mu_b^T.  Workgroup (b, y) forms all of mu_b (a wave per
-// row, four rows in flight; the matrix comes from the caches the second time) and the rows of
-// P_b of its share y.  In place of a product and an outer product per set: M = 50, 2 sets 11 -> 3 us.
-// M > 128 (the repeated reads outweigh a launch): means first, 16 rows per workgroup, then the
-// outer products (M = 256, 4 matrices 16 -> 10 us; M = 200, 8 15 -> 9).
+// mu_b = s_b S_b t_b (a wave per row), then P_b = S_b + mu_b mu_b^T (a thread per element).  Both launches
+// are latency, so their chains are as short as they get: us, M = 50, 2 matrices 5.7, 128, 10 6.2, 256, 4
+// 6.0, 256, 64 19; one launch that formed the means again in each workgroup 5.8, 8.8, -, -; four rows a
+// wave in both 9.6 and 19 at M = 256.
 __global__ __launch_bounds__(256) void mean_kernel(int D, int M, const double *__restrict__ S,
                                                    const double *__restrict__ theta, double s0, double s1,
                                                    double *__restrict__ mu) {
-  const int b = blockIdx.x, lane = threadIdx.x & 63, i0 = blockIdx.y * 16 + (threadIdx.x >> 6) * 4;
-  const double *Sb = S + (long)b * M * M, *t = theta + (long)(b % D) * M;
-  double sv[4][4], acc[4];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, i = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (i >= M) return;  // whole waves, no barriers
+  const double *row = S + ((long)b * M + i) * M, *t = theta + (long)(b % D) * M;
+  double acc = 0.0;
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sv[u][j] = Sb[(long)min(i0 + u, M - 1) * M + min(lane + 64 * j, M - 1)];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    acc[u] = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (lane + 64 * j < M) acc[u] = fma(sv[u][j], t[lane + 64 * j], acc[u]);
-    acc[u] = gpx_wave_sum(acc[u]);
+  for (int j = 0; j < 4; ++j) {
+    const int c = lane + 64 * j;
+    const double v = row[min(c, M - 1)] * t[min(c, M - 1)];
+    acc += c < M ? v : 0.0;
   }
-#pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (lane == 0 && i0 + u < M) mu[(long)b * M + i0 + u] = (b < D ? s0 : s1) * acc[u];
+  acc = gpx_wave_sum(acc);
+  if (lane == 0) mu[(long)b * M + i] = (b < D ? s0 : s1) * acc;
 }
 
 __global__ __launch_bounds__(256) void second_kernel(int M, const double *__restrict__ S,
                                                      const double *__restrict__ mu, double *__restrict__ P) {
-  const int b = blockIdx.x, lane = threadIdx.x & 63, i0 = blockIdx.y * 16 + (threadIdx.x >> 6) * 4;
-  const double *Sb = S + (long)b * M * M, *m = mu + (long)b * M;
-  double *Pb = P + (long)b * M * M;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int c = lane + 64 * j;
-    if (c >= M) break;
-    const double mc = m[c];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (i0 + u < M) Pb[(long)(i0 + u) * M + c] = m[i0 + u] * mc + Sb[(long)(i0 + u) * M + c];
-  }
-}
-
-__global__ __launch_bounds__(1024) void moments_kernel(int D, int M, const double *__restrict__ S,
-                                                       const double *__restrict__ theta, double s0, double s1,
-                                                       double *__restrict__ mu, double *__restrict__ P) {
-  __shared__ double m[256];
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nj = (M + 63) >> 6;
-  const double *Sb = S + (long)b * M * M, *t = theta + (long)(b % D) * M;
-  const double scale = b < D ? s0 : s1;
-  double tv[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) tv[j] = lane + 64 * j < M ? t[lane + 64 * j] : 0.0;
-  for (int i0 = w; i0 < M; i0 += 64) {  // rows i0 + 16 u
-    double sv[4][4], acc[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        sv[u][j] = j < nj ? Sb[(long)min(i0 + 16 * u, M - 1) * M + min(lane + 64 * j, M - 1)] : 0.0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      acc[u] = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (lane + 64 * j < M) acc[u] = fma(sv[u][j], tv[j], acc[u]);
-      acc[u] = gpx_wave_sum(acc[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (lane == 0 && i0 + 16 * u < M) m[i0 + 16 * u] = scale * acc[u];
-  }
-  __syncthreads();
-  if (blockIdx.y == 0 && tid < M) mu[(long)b * M + tid] = m[tid];
-  const int rows = (M + gridDim.y - 1) / gridDim.y, r0 = blockIdx.y * rows, r1 = min(M, r0 + rows);
-  double *Pb = P + (long)b * M * M;
-  for (int i0 = r0 + w; i0 < r1; i0 += 64) {
-    double sv[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        sv[u][j] = j < nj ? Sb[(long)min(i0 + 16 * u, M - 1) * M + min(lane + 64 * j, M - 1)] : 0.0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int i = i0 + 16 * u, c = lane + 64 * j;
-        if (i < r1 && c < M) Pb[(long)i * M + c] = m[i] * m[c] + sv[u][j];
-      }
-  }
+  const int b = blockIdx.x, e = blockIdx.y * 256 + threadIdx.x;
+  if (e >= M * M) return;
+  const double *m = mu + (long)b * M;
+  const long o = (long)b * M * M + e;
+  P[o] = m[e / M] * m[e % M] + S[o];
 }
 
 // One block per column, threads stride over the rows (fixed-order block reduction).
@@ -1232,14 +1168,9 @@ int gpx_moments(int batch, int D, int M, const double *S, const double *theta, d
   if (batch == 0) return GPX_OK;
   if (!S || !theta || !mu || !P) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  if (M <= 128) {
-    hipLaunchKernelGGL(moments_kernel, dim3(batch, gpx_cdiv(M, 64)), dim3(1024), 0, st, D, M, S, theta, s0, s1, mu, P);
-  } else {
-    const dim3 grid(batch, gpx_cdiv(M, 16));
-    hipLaunchKernelGGL(mean_kernel, grid, dim3(256), 0, st, D, M, S, theta, s0, s1, mu);
-    GPX_CHECK_LAUNCH();
-    hipLaunchKernelGGL(second_kernel, grid, dim3(256), 0, st, M, S, (const double *)mu, P);
-  }
+  hipLaunchKernelGGL(mean_kernel, dim3(batch, gpx_cdiv(M, 4)), dim3(256), 0, st, D, M, S, theta, s0, s1, mu);
+  GPX_CHECK_LAUNCH();
+  hipLaunchKernelGGL(second_kernel, dim3(batch, gpx_cdiv(M * M, 256)), dim3(256), 0, st, M, S, (const double *)mu, P);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }

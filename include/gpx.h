@@ -76,7 +76,7 @@ int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double al
 
 /* Means and second moments of q(u) from its covariances S (batch x M x M): mu_b = s_b S_b t_b and
  * P_b = S_b + mu_b mu_b^T, with t_b = theta[b % D] (D x M) and s_b = s0 for b < D, s1 from there on
- * (posterior and cavity in one launch; geepee/base_models.py:470-476, aep_models.py:528-537). */
+ * (posterior and cavity in one call; geepee/base_models.py:470-476, aep_models.py:528-537). */
 int gpx_moments(int batch, int D, int M, const double *S, const double *theta, double s0, double s1, double *mu,
                 double *P, void *stream);
 
