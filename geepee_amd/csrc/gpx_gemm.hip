@@ -93,6 +93,7 @@ __global__ __launch_bounds__(256) void splitk_reduce(int m, int n, int batch, in
 // k == 1: an outer product.  One thread per output over the flattened (batch, row,
 // column) index, with the product and epilogue of the MFMA path, which for k = 1 adds
 // exact zeros to round(a b), so the results are the same bits at a fraction of the latency.
+template <bool EXT>
 __global__ __launch_bounds__(256) void rank1_kernel(int m, int n, int tA, int tB, double alpha,
                                                     const double *__restrict__ A, int lda, long sA,
                                                     const double *__restrict__ B, int ldb, long sB, GemmEpi ep,
@@ -102,11 +103,12 @@ __global__ __launch_bounds__(256) void rank1_kernel(int m, int n, int tA, int tB
   const int b = (int)(e / mn), r = (int)(e - b * mn), i = r / n, j = r - i * n;
   const double a = tA ? A[b * sA + i] : A[b * sA + (long)i * lda];
   const double bb = tB ? B[b * sB + (long)j * ldb] : B[b * sB + j];
-  epi_store<true>(C + b * sC + (long)i * ldc + j, alpha * (a * bb), ep, b, i, j);
+  epi_store<EXT>(C + b * sC + (long)i * ldc + j, alpha * (a * bb), ep, b, i, j);
 }
 
 // n == 1: matrix-vector products.  One wave per output row: lanes stride over k, then a
 // fixed-order wave reduction, so a row's value depends only on its own operands.
+template <bool EXT>
 __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB, double alpha,
                                                    const double *__restrict__ A, int lda, long sA,
                                                    const double *__restrict__ B, int ldb, long sB, GemmEpi ep,
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB,
   for (int kk = lane; kk < k; kk += 64)
     s = fma(tA ? Ab[(long)kk * lda + i] : Ab[(long)i * lda + kk], tB ? Bb[kk] : Bb[(long)kk * ldb], s);
   s = gpx_wave_sum(s);
-  if (lane == 0) epi_store<true>(C + b * sC + (long)i * ldc, alpha * s, ep, b, i, 0);
+  if (lane == 0) epi_store<EXT>(C + b * sC + (long)i * ldc, alpha * s, ep, b, i, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(int m, int k, int tA, int tB,
 // per workgroup), us: 20000 x 200 x 200, 4 products 245 -> 125 (26 -> 51 TF); 4001 x 256 x 256, 2
 // 34 -> 29; 10000 x 6 x 1000 55 -> 17; 256^3, 2 9.6 -> 6.0; 100^3, 5 6.3 -> 4.3; 50^3 5.3 -> 4.1.
 // ---------------------------------------------------------------------------
-template <int TM, int TN, bool TA, bool TB, int KW>
+template <int TM, int TN, bool TA, bool TB, int KW, bool EXT>
 __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int kend, double alpha, const double *A,
                                                  int lda, const double *B, int ldb, const GemmEpi &ep, double *C,
                                                  int ldc, int m0, int n0, int bidx, bool raw, double *red) {
@@ -221,7 +223,7 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
         if (gm < m && gn < n) {
           double *c = C + (long)gm * ldc + gn;
           if (raw) *c = v;
-          else epi_store<(TM < 4)>(c, alpha * v, ep, bidx, gm, gn);
+          else epi_store<EXT>(c, alpha * v, ep, bidx, gm, gn);
         }
       }
     }
@@ -237,7 +239,7 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
         if (gm < m && gn < n) {
           double *c = C + (long)gm * ldc + gn;
           if (raw) *c = acc[i][j][r];
-          else epi_store<(TM < 4)>(c, alpha * acc[i][j][r], ep, bidx, gm, gn);
+          else epi_store<EXT>(c, alpha * acc[i][j][r], ep, bidx, gm, gn);
         }
       }
 }
@@ -247,7 +249,7 @@ __device__ __forceinline__ void gemm_direct_tile(int m, int n, int kbeg, int ken
 // every fourth group of K.  The n columns are cut into bands of ceil- or floor-balanced counts
 // of 16-column tiles (n = 200: 4 + 3 + 3 + 3), so padding is below 16 columns in all.
 // Workgroups are dealt to the XCDs in contiguous runs of tiles, which share operand panels.
-template <int TM, int TX, bool TA, bool TB, int KW>
+template <int TM, int TX, bool TA, bool TB, int KW, bool EXT>
 __global__ __launch_bounds__(256, 2) void gemm_direct_kernel(int m, int n, int k, double alpha, const double *__restrict__ A,
                                                           int lda, long sA, const double *__restrict__ B, int ldb,
                                                           long sB, GemmEpi ep, double *__restrict__ C, int ldc,
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void gemm_direct_kernel(int m, int n, int k
   double *Cb = raw ? part + ((long)q * batch + b) * (long)m * n : C + b * sC;
   if (raw) ldc = n;
 #define GEMM_TILE(TN)                                                                                               \
-  gemm_direct_tile<TM, TN, TA, TB, KW>(m, n, kbeg, kend, alpha, A, lda, B, ldb, ep, Cb, ldc, m0, n0, b, raw, red)
+  gemm_direct_tile<TM, TN, TA, TB, KW, EXT>(m, n, kbeg, kend, alpha, A, lda, B, ldb, ep, Cb, ldc, m0, n0, b, raw, red)
   if constexpr (TX >= 4) {
     if (tn == 4) return GEMM_TILE(4);
     if (tn == 3) return GEMM_TILE(3);
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(256, 2) void gemm_direct_kernel(int m, int n, int k
 #undef GEMM_TILE
 }
 
-template <int TM, int KW>
+template <int TM, int KW, bool EXT>
 int gemm_direct(int tA, int tB, int m, int n, int k, double alpha, const double *A, int lda, long sA, const double *B,
                 int ldb, long sB, const GemmEpi &ep, double *C, int ldc, long sC, int batch, int splits, int kchunk,
                 double *part, hipStream_t st) {
@@ -291,7 +293,7 @@ int gemm_direct(int tA, int tB, int m, int n, int k, double alpha, const double 
   const long blocks = KW > 1 ? tiles : (tiles + 3) / 4;
   const dim3 grid(8 * gpx_cdiv(blocks, 8));
 #define GEMM_GO(TA, TB)                                                                                          \
-  hipLaunchKernelGGL((gemm_direct_kernel<TM, TM, TA, TB, KW>), grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sA, B, \
+  hipLaunchKernelGGL((gemm_direct_kernel<TM, TM, TA, TB, KW, EXT>), grid, dim3(256), 0, st, m, n, k, alpha, A, lda, sA, B, \
                      ldb, sB, ep, C, ldc, sC, batch, splits, kchunk, part)
   if (tA) {
     if (tB) GEMM_GO(true, true); else GEMM_GO(true, false);
@@ -503,13 +505,21 @@ int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double al
   }
   // outer products and matrix-vector products (automatic tile choice only)
   if (tile == 0 && splits == 1 && k == 1) {
-    hipLaunchKernelGGL(rank1_kernel, dim3(gpx_cdiv((long)batch * m * n, 256)), dim3(256), 0, st, m, n, transA,
+    if (tail)
+      hipLaunchKernelGGL(rank1_kernel<true>, dim3(gpx_cdiv((long)batch * m * n, 256)), dim3(256), 0, st, m, n, transA,
+                       transB, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch);
+    else
+      hipLaunchKernelGGL(rank1_kernel<false>, dim3(gpx_cdiv((long)batch * m * n, 256)), dim3(256), 0, st, m, n, transA,
                        transB, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch);
     GPX_CHECK_LAUNCH();
     return GPX_OK;
   }
   if (tile == 0 && splits == 1 && n == 1) {
-    hipLaunchKernelGGL(gemv_kernel, dim3(gpx_cdiv((long)batch * m, 4)), dim3(256), 0, st, m, k, transA, transB,
+    if (tail)
+      hipLaunchKernelGGL(gemv_kernel<true>, dim3(gpx_cdiv((long)batch * m, 4)), dim3(256), 0, st, m, k, transA, transB,
+                       alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch);
+    else
+      hipLaunchKernelGGL(gemv_kernel<false>, dim3(gpx_cdiv((long)batch * m, 4)), dim3(256), 0, st, m, k, transA, transB,
                        alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch);
     GPX_CHECK_LAUNCH();
     return GPX_OK;
@@ -522,9 +532,10 @@ int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double al
   const long z = (long)batch * splits, t4 = z * gpx_cdiv(m, 64) * gpx_cdiv(n, 64),
              t2 = z * gpx_cdiv(m, 32) * gpx_cdiv(n, 32), t1 = z * gpx_cdiv(m, 16) * gpx_cdiv(n, 16);
   int rc;
-#define GEMM_DIRECT(TM, KW)                                                                                       \
-  gemm_direct<TM, KW>(transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, batch, \
-                      splits, kchunk, part, st)
+#define GEMM_DIRECT1(TM, KW, EXT)                                                                                 \
+  gemm_direct<TM, KW, EXT>(transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, ep, C, ldc, strideC, \
+                           batch, splits, kchunk, part, st)
+#define GEMM_DIRECT(TM, KW) tail ? GEMM_DIRECT1(TM, KW, (TM < 4)) : GEMM_DIRECT1(TM, KW, false)
   // (with a tail never 64 x 64 per wave: its 64 stores per lane each carry the epilogue)
   // 64 x 64 per wave once there are two such tiles per SIMD (20000 x n x n, 4 products, us
   // against 32 x 32: n = 256 172 : 228, 200 125 : 133, 128 (2504 tiles) 63 : 65; 5000 x 100 x 100, 4
@@ -545,6 +556,7 @@ int gpx_gemm_batched_tail(int transA, int transB, int m, int n, int k, double al
   else if (k <= 16 ? t2 > 576 : k <= 256 && full) rc = GEMM_DIRECT(2, 1);
   else rc = GEMM_DIRECT(2, 4);
 #undef GEMM_DIRECT
+#undef GEMM_DIRECT1
   if (rc != GPX_OK) return rc;
   if (part) {
     const long total = (long)batch * m * n;
