@@ -27,23 +27,24 @@ __global__ void se_any_kernel(int N, int M, int Q, const double *__restrict__ x,
   K[e] = k;
 }
 
-// Q <= QC: a block takes ROWS rows by 64 columns, each wave every fourth row.  x, 1/l and
-// sf2 are formed once per block, a thread's z row stays in registers.  Bound by its exps and
-// its writes (N = 20000, M = 200, Q = 8: 58 -> 22 us; with the lengthscales' exps and divisions
-// per entry it was bound by those).  16 rows; 4 where 16 would make at most 128 blocks: such a launch
-// is as long as one thread's entries (us, 4 rows : 16: 50 x 50, Q = 2 3.2 : 3.8; 256 x 256, Q = 10 3.4 :
-// 4.5; 1000 x 100, Q = 10 (126 blocks) 3.7 : 4.5; 3000 x 64, Q = 16 (188) 7.7 : 5.6).
-constexpr int SE_ROWS = 16, SE_ROWS_FEW = 4, SE_FEW = 128;
-template <int QC, int ROWS>
+// Q <= QC: a block takes CB columns (16, 32 or 64, as M fills them) by RPT 256 / CB rows, RPT a thread.
+// x, 1/l and sf2 are formed once per block, a thread's z row stays in registers.  Bound by its exps and
+// its writes (N = 20000, M = 200, Q = 8: 58 -> 19 us; with the lengthscales' exps and divisions per
+// entry it was bound by those).  Four rows a thread; one where four would make few blocks: such a
+// launch is as long as one thread's entries (us, one : four, 64 columns: 50 x 50, Q = 2 3.2 : 3.8; 256 x
+// 256, Q = 10 (64 blocks) 3.4 : 4.5; 3000 x 64, Q = 3 (188) 3.9 : 4.2, Q = 8 4.4 : 4.4; 2000 x 128, Q = 8 (250) 5.0 :
+// 4.6; 4000 x 128, Q = 4 (500) 4.7 : 4.7; 4000 x 32, Q = 16 (125) 6.5 : 5.2; 2500 x 64, Q = 16 (157) 8.0 : 5.7).
+template <int QC, int RPT, int CB>
 __global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const double *__restrict__ x, int ldx,
                                                  const double *__restrict__ z, const double *__restrict__ ls,
                                                  const double *__restrict__ sf, double jitter,
                                                  double *__restrict__ K) {
-  __shared__ double xs[ROWS][QC], il[QC], s2;
-  const int tid = threadIdx.x, n0 = blockIdx.x * ROWS, m = blockIdx.y * 64 + (tid & 63);
+  constexpr int step = 256 / CB, rows = RPT * step;
+  __shared__ double xs[rows][QC], il[QC], s2;
+  const int tid = threadIdx.x, n0 = blockIdx.x * rows, m = blockIdx.y * CB + tid % CB, i0 = tid / CB;
   if (tid < QC) il[tid] = tid < Q ? exp(-2.0 * ls[tid]) : 0.0;
   if (tid == 255) s2 = exp(2.0 * sf[0]);
-  for (int e = tid; e < ROWS * QC; e += 256) {
+  for (int e = tid; e < rows * QC; e += 256) {
     const int i = e / QC, q = e % QC;
     xs[i][q] = q < Q ? x[(long)min(n0 + i, N - 1) * ldx + q] : 0.0;
   }
@@ -52,8 +53,8 @@ __global__ __launch_bounds__(256) void se_kernel(int N, int M, int Q, const doub
   for (int q = 0; q < QC; ++q) zr[q] = q < Q ? z[min(m, M - 1) * Q + q] : 0.0;
   __syncthreads();
 #pragma unroll
-  for (int u = 0; u < ROWS / 4; ++u) {
-    const int i = (tid >> 6) + 4 * u, n = n0 + i;
+  for (int u = 0; u < RPT; ++u) {
+    const int i = i0 + step * u, n = n0 + i;
     double r2 = 0.0;
 #pragma unroll
     for (int q = 0; q < QC; ++q) {
@@ -1038,17 +1039,20 @@ int gpx_se_kernel(int N, int M, int Q, const double *x, int ldx, const double *z
     hipLaunchKernelGGL(se_any_kernel, dim3(gpx_cdiv((long)N * M, 256)), dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf,
                        jitter, K);
   } else {
-    const bool few = (long)gpx_cdiv(N, SE_ROWS) * gpx_cdiv(M, 64) <= SE_FEW;
-    const dim3 grid(gpx_cdiv(N, few ? SE_ROWS_FEW : SE_ROWS), gpx_cdiv(M, 64));
-#define GPX_SE(QV)                                                                                              \
-  if (few)                                                                                                      \
-    hipLaunchKernelGGL((se_kernel<QV, SE_ROWS_FEW>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K); \
-  else                                                                                                          \
-    hipLaunchKernelGGL((se_kernel<QV, SE_ROWS>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);
+    const int cb = M <= 16 ? 16 : (M <= 32 ? 32 : 64), step = 256 / cb;
+    const bool few = (long)gpx_cdiv(N, 4 * step) * gpx_cdiv(M, cb) <= (Q <= 4 ? 256 : (Q <= 8 ? 192 : 96));
+    const dim3 grid(gpx_cdiv(N, (few ? 1 : 4) * step), gpx_cdiv(M, cb));
+#define GPX_SE2(QV, CB)                                                                                               \
+  do {                                                                                                                \
+    if (few) hipLaunchKernelGGL((se_kernel<QV, 1, CB>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K); \
+    else hipLaunchKernelGGL((se_kernel<QV, 4, CB>), grid, dim3(256), 0, st, N, M, Q, x, ldx, z, ls, sf, jitter, K);     \
+  } while (0)
+#define GPX_SE(QV) if (cb == 16) GPX_SE2(QV, 16); else if (cb == 32) GPX_SE2(QV, 32); else GPX_SE2(QV, 64);
     if (Q <= 4) { GPX_SE(4) }
     else if (Q <= 8) { GPX_SE(8) }
     else { GPX_SE(16) }
 #undef GPX_SE
+#undef GPX_SE2
   }
   GPX_CHECK_LAUNCH();
   return GPX_OK;

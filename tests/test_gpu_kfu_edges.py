@@ -48,9 +48,11 @@ def test_se_and_adjoint(N, M, Q):
 
 
 @pytest.mark.parametrize('Q', [3, 8, 16])
-@pytest.mark.parametrize('N,M', [(2048, 64), (2049, 64), (1024, 65), (1025, 65)])
+@pytest.mark.parametrize('N,M', [(1536, 64), (1537, 64), (3072, 64), (3073, 64), (4096, 64), (4097, 64), (2049, 65),
+                                 (3073, 32), (8193, 31), (6145, 16), (16385, 15), (70, 17), (70, 33)])
 def test_se_rows_per_block(N, M, Q):
-    """Entries are the same bits from blocks of 4 and of 16 rows (on both sides of the rule)."""
+    """Entries are the same bits from one and from four rows a thread and from 16, 32 and 64 columns a
+    block (on both sides of each line)."""
     from geepee_amd import dops
     print('se rows', N, M, Q, flush=True)
     rs = np.random.RandomState(N + Q)
@@ -59,3 +61,5 @@ def test_se_rows_per_block(N, M, Q):
     K = dops.se(x, z, ls, sf)
     for r0, r1 in ((0, 1), (3, 40), (N - 17, N)):
         assert torch.equal(K[r0:r1], dops.se(x[r0:r1].contiguous(), z, ls, sf))
+    c = min(M, 16)
+    assert torch.equal(K[:, :c], dops.se(x, z[:c].contiguous(), ls, sf))
