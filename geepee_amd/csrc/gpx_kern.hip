@@ -1058,10 +1058,15 @@ int gpx_se_kernel(int N, int M, int Q, const double *x, int ldx, const double *z
   return GPX_OK;
 }
 
-// Columns of the adjoint's thread layout, and its number of blocks: at least eight rows a
-// thread, at most two blocks per CU (their partials are read again by pass 2).
+// Columns of the adjoint's thread layout, and its number of blocks: eight rows a thread or more, four
+// where that makes at most 60 blocks (whole adjoint, us, four : eight: N = 197, M = 64, Q = 15 11.9 : 13.4,
+// 953, 22, 13 (60) 11.5 : 12.5, 1000, 50, 2 (63) 9.6 : 9.2, 2000, 200, 16 31 : 27), at most two blocks per CU (their
+// partials are read again by pass 2).
 static int kfu_cols(int M) { return M <= 64 ? 64 : (M <= 128 ? 128 : 256); }
-static int kfu_blocks(int N, int M) { return (int)std::min<long>(512, gpx_cdiv(N, 8L * (256 / kfu_cols(M)))); }
+static int kfu_blocks(int N, int M) {
+  const int groups = 256 / kfu_cols(M), four = (int)std::min<long>(512, gpx_cdiv(N, 4L * groups));
+  return four <= 60 ? four : (int)std::min<long>(512, gpx_cdiv(N, 8L * groups));
+}
 
 long gpx_kfu_bwd_workspace(int N, int M, int Q) { return ((long)kfu_blocks(N, M) + 1) * M * (2 * Q + 1); }
 

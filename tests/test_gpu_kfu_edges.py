@@ -63,3 +63,21 @@ def test_se_rows_per_block(N, M, Q):
         assert torch.equal(K[r0:r1], dops.se(x[r0:r1].contiguous(), z, ls, sf))
     c = min(M, 16)
     assert torch.equal(K[:, :c], dops.se(x, z[:c].contiguous(), ls, sf))
+
+
+@pytest.mark.parametrize('N,M,Q', [(960, 30, 5), (961, 30, 5), (480, 100, 3), (481, 100, 9), (240, 200, 16), (241, 200, 2)])
+def test_kfu_rows_per_thread(N, M, Q):
+    """The adjoint on both sides of 60 blocks of four rows a thread, against two halves of the rows
+    (1e-12 of the sums' terms, of either sign: 1e-11 normwise)."""
+    from geepee_amd import dops
+    print('kfu rows', N, M, Q, flush=True)
+    rs = np.random.RandomState(N + Q)
+    x, z, ls, sf, G = [torch.as_tensor(a, device='cuda') for a in (rs.randn(N, Q), rs.randn(M, Q), 0.2 * rs.randn(Q) + 0.5,
+                                                                    np.array([0.3]), rs.rand(N, M))]
+    K = dops.se(x, z, ls, sf)
+    whole = dops.kfu_bwd(G, K, x, z, ls, sf, want_dx=True)
+    cut = [[t[a:b].contiguous() for t in (G, K, x)] for a, b in ((0, N // 2), (N // 2, N))]
+    parts = [dops.kfu_bwd(g, k, xx, z, ls, sf, want_dx=True) for g, k, xx in cut]
+    for i in range(3):
+        assert _nrel(whole[i].cpu().numpy(), (parts[0][i] + parts[1][i]).cpu().numpy()) < 1e-11
+    assert torch.equal(whole[3], torch.cat([p[3] for p in parts]))
