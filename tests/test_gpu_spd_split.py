@@ -82,3 +82,36 @@ def test_split_rule_and_capture():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize('M', [160, 177, 200, 256])
+@pytest.mark.parametrize('ridge', [1e-3, 1e-6])
+def test_split_matches_one_workgroup_ill_conditioned(M, ridge):
+    """Both forms do the same operations tile for tile, so on matrices of condition 1e6 and 1e9 they
+    give the same bits; their error against extended precision is within 4 cond eps."""
+    from geepee_amd import _lib as L
+    L.require_device()
+    print('spd ill-conditioned', M, ridge, flush=True)
+    rs = np.random.RandomState(M)
+    X = rs.randn(2, M, M // 2)
+    A = X @ X.transpose(0, 2, 1) + ridge * np.eye(M)
+    t = torch.as_tensor(A, device='cuda')
+    res = []
+    for split in (True, False):
+        out, ld = torch.empty_like(t), torch.empty(2, dtype=torch.float64, device='cuda')
+        info = torch.empty(2, dtype=torch.int32, device='cuda')
+        if split:
+            assert _call(L, M, 2, t, M, out, M, ld, info)[0] > 0
+        else:
+            L.call('gpx_spd_inv_batched', M, 2, L.P(t), M, M * M, L.P(out), M, M * M, L.P(ld), L.P(info), L.S())
+        assert info.cpu().tolist() == [0, 0]
+        res.append((out, ld))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+    for b in range(2):
+        w = np.linalg.eigvalsh(A[b])
+        R = np.linalg.inv(A[b]).astype(np.longdouble)
+        Al = A[b].astype(np.longdouble)
+        for _ in range(4):      # Newton steps in extended precision
+            R = R @ (2 * np.eye(M) - Al @ R)
+        err = np.linalg.norm((res[0][0][b].cpu().numpy() - R).astype(np.float64)) / np.linalg.norm(R.astype(np.float64))
+        assert err < 4 * (w[-1] / w[0]) * 2.0 ** -52, err
