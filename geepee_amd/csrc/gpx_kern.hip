@@ -342,10 +342,36 @@ __global__ __launch_bounds__(64) void kuu_tail_kernel(int M, int Q, const double
   else dls[j - 1] = dell[j - 1] * exp(ls[j - 1]) + 2.0 * s;
 }
 
-// mu_b = s_b S_b t_b (a wave per row), then P_b = S_b + mu_b mu_b^T (a thread per element).  Both launches
-// are latency, so their chains are as short as they get: us, M = 50, 2 matrices 5.7, 128, 10 6.2, 256, 4
-// 6.0, 256, 64 19; one launch that formed the means again in each workgroup 5.8, 8.8, -, -; four rows a
-// wave in both 9.6 and 19 at M = 256.
+// mu_b = s_b S_b t_b and P_b = S_b + mu_b mu_b^T.  M <= 64: one launch, a workgroup per matrix, whose waves
+// keep their rows in registers between the two.  Above, the means (a wave per row) and then P (a thread
+// per element): all of it is latency, and rows read again, or several rows a wave, cost more than the
+// launch (us: M = 50, 2 matrices 4.2, two launches 5.4; M = 100, 10 6.0, one launch that formed the means
+// again in each workgroup 8.5; 256, 4 6.0, four rows a wave in both 9.6).
+__global__ __launch_bounds__(1024) void moments_kernel(int D, int M, const double *__restrict__ S,
+                                                       const double *__restrict__ theta, double s0, double s1,
+                                                       double *__restrict__ mu, double *__restrict__ P) {
+  __shared__ double m[64];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, c = min(lane, M - 1);
+  const double *Sb = S + (long)b * M * M;
+  const double t = lane < M ? theta[(long)(b % D) * M + c] : 0.0, scale = b < D ? s0 : s1;
+  double v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = Sb[(long)min(w + 16 * u, M - 1) * M + c];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const double s = gpx_wave_sum(lane < M ? v[u] * t : 0.0);
+    if (lane == 0 && w + 16 * u < M) m[w + 16 * u] = scale * s;
+  }
+  __syncthreads();
+  if (lane >= M) return;
+  if (w == 0) mu[(long)b * M + lane] = m[lane];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int i = w + 16 * u;
+    if (i < M) P[(long)b * M * M + (long)i * M + lane] = m[i] * m[lane] + v[u];
+  }
+}
+
 __global__ __launch_bounds__(256) void mean_kernel(int D, int M, const double *__restrict__ S,
                                                    const double *__restrict__ theta, double s0, double s1,
                                                    double *__restrict__ mu) {
@@ -1177,6 +1203,11 @@ int gpx_moments(int batch, int D, int M, const double *S, const double *theta, d
   if (batch == 0) return GPX_OK;
   if (!S || !theta || !mu || !P) return GPX_EINVAL;
   hipStream_t st = (hipStream_t)stream;
+  if (M <= 64) {
+    hipLaunchKernelGGL(moments_kernel, dim3(batch), dim3(1024), 0, st, D, M, S, theta, s0, s1, mu, P);
+    GPX_CHECK_LAUNCH();
+    return GPX_OK;
+  }
   hipLaunchKernelGGL(mean_kernel, dim3(batch, gpx_cdiv(M, 4)), dim3(256), 0, st, D, M, S, theta, s0, s1, mu);
   GPX_CHECK_LAUNCH();
   hipLaunchKernelGGL(second_kernel, dim3(batch, gpx_cdiv(M * M, 256)), dim3(256), 0, st, M, S, (const double *)mu, P);
