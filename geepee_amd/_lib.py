@@ -75,7 +75,6 @@ SIGNATURES = {
                                  _p, _p, _p, _p]),
     'gpx_gram_workspace': (_l, [_i, _i, _i]),
     'gpx_gram': (_i, [_i, _i, _i, _p, _p, _i, _d, _p, _l, _p, _i, _p, _p]),
-    'gpx_rowscale': (_i, [_i, _i, _i, _p, _p, _p, _p]),
     'gpx_wsum': (_i, [_i, _i, _i, _d, _p, _p, _d, _p, _p]),
     'gpx_dmall': (_i, [_l, _p, _p, _p, _p, _p]),
     'gpx_hyper_grads': (_i, [_i, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p]),

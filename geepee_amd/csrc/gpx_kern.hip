@@ -888,18 +888,6 @@ __global__ __launch_bounds__(64) void emission_final(int nblk, int Nb, int Dout,
   }
 }
 
-// out[d][n][m] = w[n, d] * X[n][m]   (the dv-weighted rows of aep_models.py:464, 490)
-__global__ void rowscale_kernel(int N, int D, int M, const double *__restrict__ w,
-                                const double *__restrict__ X, double *__restrict__ out) {
-  const long e = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const long NM = (long)N * M;
-  if (e >= D * NM) return;
-  const int d = (int)(e / NM);
-  const long r = e % NM;
-  const int n = (int)(r / M);
-  out[e] = w[(long)n * D + d] * X[r];
-}
-
 // out[n][m] = alpha sum_d w[n, d] T[d][n][m] + beta out[n][m]   (aep_models.py:455)
 __global__ void wsum_kernel(int N, int D, int M, double alpha, const double *__restrict__ w,
                             const double *__restrict__ T, double beta, double *__restrict__ out) {
@@ -1446,15 +1434,6 @@ int gpx_emission_tilted(int Nb, int Dout, int Din, const double *C, const double
   GPX_CHECK_LAUNCH();
   hipLaunchKernelGGL(emission_final, dim3(Dout * Din + Dout + 1), dim3(64), 0, st, (int)nblk, Nb, Dout, Din, (const double *)work,
                      Rp, alpha, scale, dC, dR, scal);
-  GPX_CHECK_LAUNCH();
-  return GPX_OK;
-}
-
-int gpx_rowscale(int N, int D, int M, const double *w, const double *X, double *out, void *stream) {
-  if (N < 0 || D < 0 || M < 0 || !w || !X || !out) return GPX_EINVAL;
-  long n = (long)N * D * M;
-  if (n == 0) return GPX_OK;
-  hipLaunchKernelGGL(rowscale_kernel, dim3(gpx_cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, N, D, M, w, X, out);
   GPX_CHECK_LAUNCH();
   return GPX_OK;
 }

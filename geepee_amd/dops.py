@@ -152,14 +152,6 @@ def sym(X, a=0.5):
     return out
 
 
-def rowscale(w, X):
-    N, D = w.shape
-    M = X.shape[1]
-    out = empty(D, N, M, like=X)
-    call('gpx_rowscale', N, D, M, P(w), P(X), P(out), S())
-    return out
-
-
 def gram(w, X, E=None, gamma=0.0, splits=None):
     """(D, M, M): sum_n w_nd x_n x_n^T + gamma E, for w (N, D), X (N, M)."""
     N, D = w.shape
@@ -278,6 +270,7 @@ def kfu_bwd_reg(dm, dv, A, T, K, x, z, ls, sf):
 
 
 def dtrace(Mm, z, ls, sf):
+    """gsf, gls, gz of tr(Mm Kzz): the first half of kuu_tail by itself."""
     M, Q = z.shape
     outs = [empty(1, like=z), empty(Q, like=z), empty(M, Q, like=z)]
     work = empty(query('gpx_dtrace_workspace', M, Q), like=z)

@@ -239,10 +239,6 @@ long gpx_gram_workspace(int D, int M, int splits);
 int gpx_gram(int N, int D, int M, const double *w, const double *X, int ldx, double gamma, const double *E,
              long strideE, double *out, int splits, double *work, void *stream);
 
-/* out[d][n][m] = w[n,d] X[n][m]: the dv-weighted rows behind the syrk-like einsums
- * 'nd,na,nb->dab' (geepee/aep_models.py:464, 490). */
-int gpx_rowscale(int N, int D, int M, const double *w, const double *X, double *out, void *stream);
-
 /* out[n][m] = alpha sum_d w[n,d] T[d][n][m] + beta out[n][m]: the einsum
  * 'nd,dab,na->nb' (geepee/aep_models.py:455) with T[d] = kfu Bhat_det[d]. */
 int gpx_wsum(int N, int D, int M, double alpha, const double *w, const double *T, double beta,
