@@ -341,8 +341,9 @@ class SGP_Layer(object):
         M, D = self.M, self.Dout
         if not return_info and N > 0 and dops.fused_fits(M, mx.shape[1], D):
             # psi2 itself is not asked for: fold it into the contraction with B_sto instead of
-            # storing N M^2 of it (M = 100, Q = 4, one output, us: 1 point 53 -> 21, 1000 93 -> 30,
-            # 5000 447 -> 63; M = 256, Q = 10, D = 2: 1 point 57 -> 56, 5000 2245 -> 354)
+            # storing N M^2 of it (us a call, psi2 stored : folded: M = 100, Q = 4, one output, 1 point
+            # 43 : 27, 1000 70 : 35, 5000 316 : 66; M = 256, Q = 10, D = 2, 1 point 40 : 29, 5000
+            # 1336 : 359)
             # (a posterior formed without the operand: formed here and not kept, since another
             # stream, or work after a capture of this call, could not tell when it is there)
             Bp = self._Bp_post if self._Bp_post is not None else dops.sym_pairmajor(self.B_sto)
